@@ -366,7 +366,7 @@ __global__ void k_pair14(int32_t items, const int32_t *__restrict__ dl, const fl
                          const double *__restrict__ xd, const float *__restrict__ q,
                          const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
                          const double4 *__restrict__ lj14, DevParams P, int32_t n,
-                         long long *__restrict__ fout, long long *__restrict__ eacc) {
+                         long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = m < items;
     double ec = 0.0, el = 0.0;
@@ -377,15 +377,15 @@ __global__ void k_pair14(int32_t items, const int32_t *__restrict__ dl, const fl
         pair14_eval<F64POS>(it, pos4, xd, q, reps[r].box, reps[r].ibox, lj14, P, n, ec, el,
                             AtomicSink{it, fout, n});
     }
-    wave_add(to_efix(ec), live, r, eacc, E_COUL14);
-    wave_add(to_efix(el), live, r, eacc, E_POT14);
+    if (energies) wave_add(to_efix(ec), live, r, eacc, E_COUL14);
+    if (energies) wave_add(to_efix(el), live, r, eacc, E_POT14);
 }
 
 // Items whose type is <= 0 belong to a rigid water and are evaluated inside the SHAKE kernel.
 __global__ void k_bond(int32_t items, const int32_t *__restrict__ bl, const double *__restrict__ xd,
                        const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
                        const double *__restrict__ kb, const double *__restrict__ r0, int32_t n,
-                       long long *__restrict__ fout, long long *__restrict__ eacc) {
+                       long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = m < items && bl[(size_t)m * 3 + 2] >= 1;
     long long e = 0;
@@ -395,14 +395,14 @@ __global__ void k_bond(int32_t items, const int32_t *__restrict__ bl, const doub
         r = rep[it[0]];
         e = bond_eval(it, xd, reps[r].box, reps[r].ibox, kb, r0, n, AtomicSink{it, fout, n});
     }
-    wave_add(e, live, r, eacc, E_BOND);
+    if (energies) wave_add(e, live, r, eacc, E_BOND);
 }
 
 // (types <= 0: rigid-water angles, evaluated inside the SHAKE kernel)
 __global__ void k_angle(int32_t items, const int32_t *__restrict__ al, const double *__restrict__ xd,
                         const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
                         const double *__restrict__ ka, const double *__restrict__ th0, int32_t n,
-                        long long *__restrict__ fout, long long *__restrict__ eacc) {
+                        long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = m < items && al[(size_t)m * 4 + 3] >= 1;
     long long e = 0;
@@ -412,14 +412,14 @@ __global__ void k_angle(int32_t items, const int32_t *__restrict__ al, const dou
         r = rep[it[0]];
         e = angle_eval(it, xd, reps[r].box, reps[r].ibox, ka, th0, n, AtomicSink{it, fout, n});
     }
-    wave_add(e, live, r, eacc, E_ANGLE);
+    if (energies) wave_add(e, live, r, eacc, E_ANGLE);
 }
 
 __global__ void k_torsion(int32_t items, const int32_t *__restrict__ tl, const double *__restrict__ xd,
                           const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
                           const double *__restrict__ kk, const double *__restrict__ mult,
                           const double *__restrict__ shift_deg, const double *__restrict__ shift_cs,
-                          int32_t n, long long *__restrict__ fout, long long *__restrict__ eacc) {
+                          int32_t n, long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = m < items;
     double e = 0.0;
@@ -430,13 +430,13 @@ __global__ void k_torsion(int32_t items, const int32_t *__restrict__ tl, const d
         e = torsion_eval(it, xd, reps[r].box, reps[r].ibox, kk, mult, shift_deg, shift_cs, n,
                          AtomicSink{it, fout, n});
     }
-    wave_add(to_efix(e), live, r, eacc, E_DIHED);
+    if (energies) wave_add(to_efix(e), live, r, eacc, E_DIHED);
 }
 
 __global__ void k_improper(int32_t items, const int32_t *__restrict__ il, const double *__restrict__ xd,
                            const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
                            const double *__restrict__ kk, const double *__restrict__ chi0,
-                           int32_t n, long long *__restrict__ fout, long long *__restrict__ eacc) {
+                           int32_t n, long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = m < items;
     double e = 0.0;
@@ -446,14 +446,14 @@ __global__ void k_improper(int32_t items, const int32_t *__restrict__ il, const 
         r = rep[it[0]];
         e = improper_eval(it, xd, reps[r].box, reps[r].ibox, kk, chi0, n, AtomicSink{it, fout, n});
     }
-    wave_add(to_efix(e), live, r, eacc, E_IMPRO);
+    if (energies) wave_add(to_efix(e), live, r, eacc, E_IMPRO);
 }
 
 __global__ void k_improper_cvff(int32_t items, const int32_t *__restrict__ il,
                                 const double *__restrict__ xd, const int32_t *__restrict__ rep,
                                 const RepInfo *__restrict__ reps, const double *__restrict__ kk,
                                 const int32_t *__restrict__ dn, int32_t n,
-                                long long *__restrict__ fout, long long *__restrict__ eacc) {
+                                long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = m < items;
     double e = 0.0;
@@ -463,7 +463,7 @@ __global__ void k_improper_cvff(int32_t items, const int32_t *__restrict__ il,
         r = rep[it[0]];
         e = improper_cvff_eval(it, xd, reps[r].box, reps[r].ibox, kk, dn, n, AtomicSink{it, fout, n});
     }
-    wave_add(to_efix(e), live, r, eacc, E_IMPRO);
+    if (energies) wave_add(to_efix(e), live, r, eacc, E_IMPRO);
 }
 
 // real*4 positions promoted to an FP64 SoA copy, the input of the bonded kernels above
@@ -504,7 +504,7 @@ __global__ void __launch_bounds__(BUNDLE_THREADS)
 k_bonded_bundles(const int32_t *__restrict__ tstart, const int2 *__restrict__ terms,
                  const int32_t *__restrict__ sstart, const int32_t *__restrict__ slots,
                  BondedArgs A, DevParams P, long long *__restrict__ fout,
-                 long long *__restrict__ eacc) {
+                 long long *__restrict__ eacc, bool energies) {
     __shared__ unsigned long long s_f[3 * BUNDLE_SLOTS];
     const int b = blockIdx.x, lane = threadIdx.x;
     const int t0 = tstart[b], t1 = tstart[b + 1];
@@ -557,6 +557,7 @@ k_bonded_bundles(const int32_t *__restrict__ tstart, const int2 *__restrict__ te
             *p += (long long)s_f[3 * s + k];
         }
     }
+    if (!energies) return;
     wave_add(ec, true, r, eacc, E_COUL14);
     wave_add(el, true, r, eacc, E_POT14);
     wave_add(eb, true, r, eacc, E_BOND);
@@ -583,7 +584,7 @@ void launch_pair14(sofia_ctx *c, long long *fout) {
     if (!c->nd) return;
     hipLaunchKernelGGL(k_pair14<false>, dim3(nblocks(c->nd, 256)), dim3(256), 0, c->stream, c->nd,
                        c->dihedlist, c->a.pos4, c->a.xd, c->a.q, c->rep, c->reps_d, c->lj14, c->dp,
-                       c->N, fout, c->eacc);
+                       c->N, fout, c->eacc, true);
 }
 
 // The drop-in form of the bonded terms: every bond, angle, torsion and improper of the
@@ -596,26 +597,26 @@ void launch_bonded_dropin(sofia_ctx *c, long long *fout) {
     hipLaunchKernelGGL(k_pos_to_xd, dim3(nblocks(n, 256)), dim3(256), 0, c->stream, n, c->a.pos4, xd);
     if (c->nb && c->bond_k)
         hipLaunchKernelGGL(k_bond, dim3(nblocks(c->nb, 256)), dim3(256), 0, c->stream, c->nb,
-                           c->bondlist, xd, c->rep, c->reps_d, c->bond_k, c->bond_r0, n, fout, c->eacc);
+                           c->bondlist, xd, c->rep, c->reps_d, c->bond_k, c->bond_r0, n, fout, c->eacc, true);
     if (c->na && c->angle_k)
         hipLaunchKernelGGL(k_angle, dim3(nblocks(c->na, 256)), dim3(256), 0, c->stream, c->na,
                            c->anglelist, xd, c->rep, c->reps_d, c->angle_k, c->angle_th0, n, fout,
-                           c->eacc);
+                           c->eacc, true);
     if (c->ntor && c->tors_k)
         hipLaunchKernelGGL(k_torsion, dim3(nblocks(c->ntor, 256)), dim3(256), 0, c->stream, c->ntor,
                            c->torsions, xd, c->rep, c->reps_d, c->tors_k, c->tors_n, c->tors_shift,
-                           c->tors_cs, n, fout, c->eacc);
+                           c->tors_cs, n, fout, c->eacc, true);
     if (c->nimp && c->impro_style == 0)
         hipLaunchKernelGGL(k_improper, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream, c->nimp,
                            c->improlist, xd, c->rep, c->reps_d, c->impro_k, c->impro_chi0, n, fout,
-                           c->eacc);
+                           c->eacc, true);
     else if (c->nimp)
         hipLaunchKernelGGL(k_improper_cvff, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream,
                            c->nimp, c->improlist, xd, c->rep, c->reps_d, c->impro_k, c->impro_dn, n,
-                           fout, c->eacc);
+                           fout, c->eacc, true);
 }
 
-void launch_bonded_engine(sofia_ctx *c) {
+void launch_bonded_engine(sofia_ctx *c, bool energies) {
     const int n = c->N;
     if (c->bonded_bundles && c->nbundle > 0) {
         BondedArgs A{};
@@ -632,35 +633,35 @@ void launch_bonded_engine(sofia_ctx *c) {
         A.impro_style = c->impro_style;
         A.n = n;
         hipLaunchKernelGGL(k_bonded_bundles, dim3(c->nbundle), dim3(BUNDLE_THREADS), 0, c->stream, c->bund_tstart,
-                           c->bund_terms, c->bund_sstart, c->bund_slots, A, c->dp, c->fix, c->eacc);
+                           c->bund_terms, c->bund_sstart, c->bund_slots, A, c->dp, c->fix, c->eacc, energies);
         return;
     }
     if (c->nd)
         hipLaunchKernelGGL(k_pair14<true>, dim3(nblocks(c->nd, 256)), dim3(256), 0, c->stream, c->nd,
                            c->dihedlist, c->a.pos4, c->a.xd, c->a.q, c->rep, c->reps_d, c->lj14,
-                           c->dp, n, c->fix, c->eacc);
+                           c->dp, n, c->fix, c->eacc, energies);
     // with the rigid waters fused into SHAKE, the remaining items only
     const int nb = c->water_split ? c->nbe : c->nb, na = c->water_split ? c->nae : c->na;
     const int32_t *bl = c->water_split ? c->ebond : c->bondlist;
     const int32_t *al = c->water_split ? c->eangle : c->anglelist;
     if (nb && c->bond_k)
         hipLaunchKernelGGL(k_bond, dim3(nblocks(nb, 256)), dim3(256), 0, c->stream, nb, bl, c->a.xd,
-                           c->rep, c->reps_d, c->bond_k, c->bond_r0, n, c->fix, c->eacc);
+                           c->rep, c->reps_d, c->bond_k, c->bond_r0, n, c->fix, c->eacc, energies);
     if (na && c->angle_k)
         hipLaunchKernelGGL(k_angle, dim3(nblocks(na, 256)), dim3(256), 0, c->stream, na, al, c->a.xd,
-                           c->rep, c->reps_d, c->angle_k, c->angle_th0, n, c->fix, c->eacc);
+                           c->rep, c->reps_d, c->angle_k, c->angle_th0, n, c->fix, c->eacc, energies);
     if (c->ntor && c->tors_k)
         hipLaunchKernelGGL(k_torsion, dim3(nblocks(c->ntor, 256)), dim3(256), 0, c->stream, c->ntor,
                            c->torsions, c->a.xd, c->rep, c->reps_d, c->tors_k, c->tors_n,
-                           c->tors_shift, c->tors_cs, n, c->fix, c->eacc);
+                           c->tors_shift, c->tors_cs, n, c->fix, c->eacc, energies);
     if (c->nimp && c->impro_style == 0)
         hipLaunchKernelGGL(k_improper, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream, c->nimp,
                            c->improlist, c->a.xd, c->rep, c->reps_d, c->impro_k, c->impro_chi0, n,
-                           c->fix, c->eacc);
+                           c->fix, c->eacc, energies);
     else if (c->nimp)
         hipLaunchKernelGGL(k_improper_cvff, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream,
                            c->nimp, c->improlist, c->a.xd, c->rep, c->reps_d, c->impro_k,
-                           c->impro_dn, n, c->fix, c->eacc);
+                           c->impro_dn, n, c->fix, c->eacc, energies);
 }
 
 }  // namespace sofia

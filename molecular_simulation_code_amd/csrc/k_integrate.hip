@@ -509,7 +509,7 @@ struct ShakeArgs {
     int32_t n;
     double dt, dtsq, tol;
     int maxiter;
-    int32_t *err, *iters_max;
+    int32_t *err;
 };
 
 // The two O-H bonds and the H-O-H angle of a rigid water (atoms idx = O, H1, H2), added to
@@ -591,7 +591,6 @@ __device__ inline int shake_cluster(int m, const ShakeArgs &A, double vir[3], lo
         atomicOr(A.err, 1);
         return rr;
     }
-    atomicMax(A.iters_max, its);
     long long add[NA][3];
 #pragma unroll
     for (int a = 0; a < NA; ++a)
@@ -758,35 +757,45 @@ __device__ inline int settle_water(int m, const ShakeArgs &A, double vir[3], lon
 }
 
 // All engine constraints in one launch.  The first nb_it blocks run the iteratively solved
-// clusters of kidx (kinds 1, 3, 4, -3 in that order; e1..e4 are the ends of the groups), so
-// that a wavefront almost always runs a single solver.  Each wavefront of the other blocks
-// owns WSPAN consecutive atoms in their current (cell-sorted) order: it queues the SETTLE
-// waters whose oxygen lies there in LDS and solves them 64 at a time, so its waters come
-// from a few neighbouring cells and share cache lines, with every lane busy.
-constexpr int WSPAN = 512;
+// clusters of kidx (kinds 1, 3, 4, -3 in that order, each kind padded with -1 to whole
+// wavefronts; e1..e4 are the ends of the groups), so that a wavefront runs a single solver.
+// Each wavefront of the other blocks owns WSPAN consecutive atoms in their current
+// (cell-sorted) order: it queues the SETTLE waters whose oxygen lies there in LDS and solves
+// them 64 at a time, so its waters come from a few neighbouring cells and share cache lines.
+//
+// Bound by the latency of one solve (dependent gathers, FP64 divisions and square roots), not
+// by throughput, so the split aims at one solve per wavefront and many wavefronts: 160 atoms
+// hold about 53 waters (rarely more than the 64 of one round), where 512 atoms took three
+// rounds one after the other.  The energy and virial sums (ten 64-bit wave reductions and
+// five atomics) run on energy launches only.
+constexpr int WSPAN = 160;
 
+template <bool ENERGY>
 __global__ void __launch_bounds__(128)
 k_constraints(const int32_t *__restrict__ kidx, int32_t e1, int32_t e2, int32_t e3, int32_t e4,
               int32_t nb_it, const int32_t *__restrict__ wclus, ShakeArgs A,
               long long *__restrict__ eacc) {
-    if ((int)blockIdx.x < nb_it) {
-        double vir[3] = {0.0, 0.0, 0.0};
-        long long eb = 0, ea = 0;
-        int rr = 0;
-        const int t = blockIdx.x * blockDim.x + threadIdx.x;
-        const bool live = t < e4;
-        if (live) {
-            const int m = kidx[t];
-            if (t >= e3) rr = shake_cluster<-3>(m, A, vir, eb, ea);
-            else if (t >= e2) rr = shake_cluster<4>(m, A, vir, eb, ea);
-            else if (t >= e1) rr = shake_cluster<3>(m, A, vir, eb, ea);
-            else rr = shake_cluster<1>(m, A, vir, eb, ea);
-        }
+    auto energies = [&](const double vir[3], long long eb, long long ea, bool live, int rr) {
+        if (!ENERGY) return;
         wave_add(to_efix(vir[0]), live, rr, eacc, V_X);
         wave_add(to_efix(vir[1]), live, rr, eacc, V_Y);
         wave_add(to_efix(vir[2]), live, rr, eacc, V_Z);
         wave_add(eb, live, rr, eacc, E_BOND);
         wave_add(ea, live, rr, eacc, E_ANGLE);
+    };
+    if ((int)blockIdx.x < nb_it) {
+        double vir[3] = {0.0, 0.0, 0.0};
+        long long eb = 0, ea = 0;
+        int rr = 0;
+        const int t = blockIdx.x * blockDim.x + threadIdx.x;
+        const int m = t < e4 ? kidx[t] : -1;
+        if (m >= 0) {
+            if (t >= e3) rr = shake_cluster<-3>(m, A, vir, eb, ea);
+            else if (t >= e2) rr = shake_cluster<4>(m, A, vir, eb, ea);
+            else if (t >= e1) rr = shake_cluster<3>(m, A, vir, eb, ea);
+            else rr = shake_cluster<1>(m, A, vir, eb, ea);
+        }
+        energies(vir, eb, ea, m >= 0, rr);
         return;
     }
     __shared__ int32_t s_q[2][WSPAN];
@@ -796,7 +805,7 @@ k_constraints(const int32_t *__restrict__ kidx, int32_t e1, int32_t e2, int32_t 
     int cnt = 0;
     for (int k = 0; k < WSPAN; k += 64) {
         const int i = a0 + k + lane;
-        const int m = i < A.n ? wclus[i] : -1;
+        const int m = (k + lane < WSPAN && i < A.n) ? wclus[i] : -1;
         const uint64_t b = __ballot(m >= 0);
         if (m >= 0) s_q[wave][cnt + __popcll(b & lt_mask)] = m;
         cnt += __popcll(b);
@@ -808,11 +817,7 @@ k_constraints(const int32_t *__restrict__ kidx, int32_t e1, int32_t e2, int32_t 
         int rr = 0;
         const bool live = base + lane < cnt;
         if (live) rr = settle_water(s_q[wave][base + lane], A, vir, eb, ea);
-        wave_add(to_efix(vir[0]), live, rr, eacc, V_X);
-        wave_add(to_efix(vir[1]), live, rr, eacc, V_Y);
-        wave_add(to_efix(vir[2]), live, rr, eacc, V_Z);
-        wave_add(eb, live, rr, eacc, E_BOND);
-        wave_add(ea, live, rr, eacc, E_ANGLE);
+        energies(vir, eb, ea, live, rr);
     }
 }
 
@@ -999,19 +1004,23 @@ ShakeArgs shake_args(sofia_ctx *c) {
     A.mass = c->mass; A.rep = c->rep; A.reps = c->reps_d;
     A.bond_k = c->bond_k; A.bond_r0 = c->bond_r0; A.angle_k = c->angle_k; A.angle_th0 = c->angle_th0;
     A.n = c->N; A.dt = dt; A.dtsq = dtsq; A.tol = c->dp.shake_tol; A.maxiter = c->dp.shake_maxiter;
-    A.err = c->shake_err; A.iters_max = c->shake_iters;
+    A.err = c->shake_err;
     return A;
 }
 
-void launch_shake64(sofia_ctx *c) {
+void launch_shake64(sofia_ctx *c, bool energies) {
     if (!c->ns) return;
-    const int32_t *n = c->shake_kcount;
+    const int32_t *n = c->shake_kcount;   // group sizes in whole wavefronts
     const int e1 = n[0], e2 = e1 + n[1], e3 = e2 + n[2], e4 = e3 + n[3];
     const int nb_it = nblocks(e4, 128);
     const int nb_w = n[4] ? nblocks(c->N, 2 * WSPAN) : 0;
     if (nb_it + nb_w == 0) return;
-    hipLaunchKernelGGL(k_constraints, dim3(nb_it + nb_w), dim3(128), 0, c->stream, c->shake_kidx,
-                       e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), c->eacc);
+    if (energies)
+        hipLaunchKernelGGL(k_constraints<true>, dim3(nb_it + nb_w), dim3(128), 0, c->stream,
+                           c->shake_kidx, e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), c->eacc);
+    else
+        hipLaunchKernelGGL(k_constraints<false>, dim3(nb_it + nb_w), dim3(128), 0, c->stream,
+                           c->shake_kidx, e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), c->eacc);
 }
 
 void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb) {

@@ -1529,9 +1529,9 @@ int nb_mode(const sofia_ctx *c) {
 void force_sequence(sofia_ctx *c, bool energies) {
     launch_zero_forces(c, c->fix, energies);
     launch_nonbond(c, nb_mode(c), energies);
-    launch_bonded_engine(c);
+    launch_bonded_engine(c, energies);
     if (c->has_thermostat) launch_langevin64(c);
-    launch_shake64(c);
+    launch_shake64(c, energies);
 }
 
 void step_sequence(sofia_ctx *c, bool energies) {
@@ -1724,8 +1724,13 @@ int classify_shake(sofia_ctx *c) {
     }
     std::vector<int32_t> kidx;
     for (int q = 0; q < 5; ++q) {
-        if (q < 4) kidx.insert(kidx.end(), lists[q].begin(), lists[q].end());
-        c->shake_kcount[q] = (int32_t)lists[q].size();
+        if (q < 4) {
+            kidx.insert(kidx.end(), lists[q].begin(), lists[q].end());
+            kidx.resize((kidx.size() + 63) / 64 * 64, -1);
+            c->shake_kcount[q] = (int32_t)((lists[q].size() + 63) / 64 * 64);
+        } else {
+            c->shake_kcount[q] = (int32_t)lists[q].size();
+        }
     }
     if (!kidx.empty()) {
         TRY(dalloc(&c->shake_kidx, kidx.size()));
@@ -2157,7 +2162,7 @@ int sofia_minimize(sofia_ctx *c, int32_t nsteps, double gamma, double max_disp) 
     for (int s = 0; s < nsteps; ++s) {
         launch_zero_forces(c, c->fix, false);
         launch_nonbond(c, nb_mode(c), false);
-        launch_bonded_engine(c);
+        launch_bonded_engine(c, false);
         launch_water_bonded(c);
         launch_minimize_step(c, gamma, max_disp);
         launch_check_neighbor(c, true);
@@ -2297,10 +2302,10 @@ int sofia_profile_step(sofia_ctx *c, int32_t nsteps, int32_t full_rebuild, doubl
         launch_finish_rebuild(c, true); mark();
         launch_zero_forces(c, c->fix, false); mark();
         launch_nonbond(c, nb_mode(c), false); mark();
-        launch_bonded_engine(c); mark();
+        launch_bonded_engine(c, false); mark();
         if (c->has_thermostat) launch_langevin64(c);
         mark();
-        launch_shake64(c); mark();
+        launch_shake64(c, false); mark();
         launch_nve_v64(c, false); launch_step_advance(c); mark();
         rc = sync_check(c);
         for (int p = 0; p < NP && rc == SOFIA_OK; ++p) {

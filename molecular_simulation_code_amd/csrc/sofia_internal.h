@@ -154,7 +154,8 @@ struct sofia_ctx {
     int32_t rdf_cap = 0;
     size_t topo_stage_len = 0;
     // engine constraints: indices of the iteratively solved clusters grouped by kind 1, 3,
-    // 4, -3, and the count of symmetric rigid waters (SETTLE, found through AtomArrays::wclus);
+    // 4, -3 (each group padded with -1 to whole wavefronts, as the counts are), and the count
+    // of symmetric rigid waters (SETTLE, found through AtomArrays::wclus);
     // built when the engine sets up its lists
     int32_t *shake_kidx = nullptr;
     int32_t shake_kcount[5] = {0, 0, 0, 0, 0};
@@ -261,7 +262,7 @@ void launch_count_pairs(sofia_ctx *c, unsigned long long *out);
 // bonded (k_bonded.hip)
 void launch_correct(sofia_ctx *c, int which, long long *fout);
 void launch_pair14(sofia_ctx *c, long long *fout);
-void launch_bonded_engine(sofia_ctx *c);
+void launch_bonded_engine(sofia_ctx *c, bool energies);
 void launch_bonded_dropin(sofia_ctx *c, long long *fout);
 int build_bonded_bundles(sofia_ctx *c);   // host: molecules of the engine's bonded items
 void drop_bonded_bundles(sofia_ctx *c);
@@ -283,7 +284,7 @@ void launch_engine_to32(sofia_ctx *c);
 void launch_nve_v64(sofia_ctx *c, bool ke);
 void launch_nve_x64(sofia_ctx *c);
 void launch_langevin64(sofia_ctx *c);
-void launch_shake64(sofia_ctx *c);
+void launch_shake64(sofia_ctx *c, bool energies);
 void launch_water_bonded(sofia_ctx *c);
 void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst);
 void launch_type_range(sofia_ctx *c, const float4 *pos, int32_t *bad);
