@@ -350,7 +350,9 @@ int sofia_profile_copy(sofia_ctx *ctx, int64_t bytes, int32_t launches, double *
  * the average ms per step of each phase in phase_ms[SOFIA_NPHASE]: half-kick, drift,
  * displacement check, cell sort + gather + topology remap, list build, rebuild
  * bookkeeping, force zeroing, pair kernel, bonded (1-4, bond, angle, torsion, improper), Langevin,
- * SHAKE, second half-kick.  full_rebuild != 0 makes every replica rebuild on every step
+ * SHAKE, second half-kick.  The first entry's launch also drifts, checks the displacement,
+ * clears the force sum and adds the Langevin force, and the SHAKE launch keeps the rebuild
+ * books, so those entries read only the time between two events.  full_rebuild != 0 makes every replica rebuild on every step
  * (the cost of one full rebuild).  Energies are not reduced on these steps. */
 enum { SOFIA_NPHASE = 12 };
 int sofia_profile_step(sofia_ctx *ctx, int32_t nsteps, int32_t full_rebuild, double *phase_ms);

@@ -153,33 +153,23 @@ __device__ __forceinline__ PairOut pair_dsf(float dr2, float qq, const float4 &l
     return o;
 }
 
-constexpr uint32_t TYPE_BITS = 0x3fu;   // atom type in the low bits of X (types 1..63)
-
-// x -> round(x 2^32 / box) mod 2^32 per replica, type in the low bits of X, charge in w.
-// From the FP64 engine state (xd != nullptr) or from the float positions.
+// Every atom's record, from the FP64 engine state (xd != nullptr) or from the float positions.
+// An engine step writes its records with the positions (k_advance) and launches this only
+// where no step precedes the pair kernel.
 __global__ void k_fixpos(int32_t n, const double *__restrict__ xd, const float4 *__restrict__ pos4,
                          const float *__restrict__ q, const int32_t *__restrict__ rep,
                          const RepInfo *__restrict__ reps, int4 *__restrict__ pf) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float4 p = pos4[i];
-    const double s = 4294967296.0 / (double)reps[rep[i]].box;
+    const double s = reps[rep[i]].fscale;
     double x, y, z;
     if (xd) {
         x = xd[i]; y = xd[(size_t)n + i]; z = xd[2 * (size_t)n + i];
     } else {
         x = p.x; y = p.y; z = p.z;
     }
-    const uint32_t fx = (uint32_t)(unsigned long long)__double2ll_rn(x * s);
-    const int X = (int)((fx & ~TYPE_BITS) | ((uint32_t)__float_as_int(p.w) & TYPE_BITS));
-    const int Y = (int)(uint32_t)(unsigned long long)__double2ll_rn(y * s);
-    const int Z = (int)(uint32_t)(unsigned long long)__double2ll_rn(z * s);
-    if (q) {
-        pf[i] = make_int4(X, Y, Z, __float_as_int(q[i]));
-    } else {   // charges by type: 12-byte records
-        int *p3 = (int *)pf + 3 * (size_t)i;
-        p3[0] = X; p3[1] = Y; p3[2] = Z;
-    }
+    write_record(pf, i, x, y, z, s, (uint32_t)__float_as_int(p.w), q);
 }
 
 // L lanes per atom; lane s of a group walks list entries s, s+L, ... with the loads of the
@@ -534,13 +524,19 @@ void launch_compact(sofia_ctx *c, bool energies, float *ff32) {
 
 }  // namespace
 
-void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd) {
-    // 12-byte records while every atom of a type carries the type's charge (the compacting
-    // kernel reads 16-byte records)
+// 12-byte records while every atom of a type carries the type's charge (the compacting
+// kernel reads 16-byte records)
+int record_bytes(const sofia_ctx *c) {
+    if (c->p.precision != SOFIA_PREC_MIXED || c->p.coul_flag == SOFIA_COUL_EWALD) return 0;
+    return (c->q_by_type && c->ptab && c->lanes != 0) ? 12 : 16;
+}
+
+void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records) {
     const bool qt = c->q_by_type && c->ptab && c->lanes != 0;
-    hipLaunchKernelGGL(k_fixpos, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N,
-                       from_xd ? c->a.xd : nullptr, c->a.pos4, qt ? nullptr : c->a.q, c->rep,
-                       c->reps_d, c->pfix);
+    if (!records)
+        hipLaunchKernelGGL(k_fixpos, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N,
+                           from_xd ? c->a.xd : nullptr, c->a.pos4, qt ? nullptr : c->a.q, c->rep,
+                           c->reps_d, c->pfix);
     switch (c->lanes) {
         case 0: launch_compact(c, energies, ff32); break;
         case 4: launch_lanes<4>(c, energies, ff32, qt); break;

@@ -351,28 +351,77 @@ __global__ void k_nve_v64(int32_t n, double dthalf, const float4 *__restrict__ p
     if (ke) wave_add(to_efix(k), live, r, eacc, E_KE);
 }
 
-// x += dt v, displacement += dt v, wrap into (0, box], refresh the float4 copy
-__global__ void k_nve_x64(int32_t n, double dt, double *__restrict__ xd, const double *__restrict__ vd,
-                          double *__restrict__ drd, float4 *__restrict__ pos4,
-                          const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps) {
+__device__ inline double wrap64(double x, double box) {
+    for (int it = 0; it < 64 && x > box; ++it) x -= box;
+    for (int it = 0; it < 64 && x <= 0.0; ++it) x += box;
+    return x;
+}
+
+// Where an integration launch leaves what the rest of the step starts from: the rebuild flags
+// (an atom displaced by half the usable skin flags its replica; the first to do so raises
+// `any`), the fixed-point force sum (zero, or the Langevin term) and the mixed pair kernel's
+// position record (pf; q as in write_record).
+struct StepOut {
+    int32_t *rebuild, *any;
+    long long *fix;
+    int4 *pf;
+    const float *q;
+};
+
+__device__ inline void flag_rebuild(const StepOut &O, int r, const double dr[3], double chk2) {
+    if ((dr[0] * dr[0] + dr[1] * dr[1]) + dr[2] * dr[2] >= chk2 && atomicOr(&O.rebuild[r], 1) == 0)
+        atomicOr(O.any, 1);
+}
+
+// Everything between two force evaluations that one atom can do alone, in one pass over the
+// state: the previous step's second half kick (KICK2; the first step of a segment has none
+// left), this step's first half kick, the drift (wrapped into (0, box], the float4 copy
+// refreshed), the rebuild check, the Langevin force at the half-step velocity as the force
+// sum's first term, and the pair kernel's record.  These were seven launches; a launch costs
+// about 4.5 us in a step, so a 5,000-atom step (135 us) spent a quarter of its time on them.
+template <bool KICK2>
+__global__ void __launch_bounds__(256)
+k_advance(int32_t n, double dt, const double4 *__restrict__ mtab, double *__restrict__ xd,
+          double *__restrict__ vd, double *__restrict__ drd, float4 *__restrict__ pos4,
+          const double *__restrict__ fnb, const int32_t *__restrict__ gid,
+          const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
+          const uint64_t *__restrict__ step, int thermostat, StepOut O) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const double box = reps[rep[i]].box;
+    const int r = rep[i];
+    const RepInfo &R = reps[r];
+    const double box = R.box;
     float4 p = pos4[i];
-    float pf[3];
+    const uint32_t type = (uint32_t)__float_as_int(p.w);
+    const double4 mt = mtab[type - 1];
+    double v[3], x[3], dr[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const size_t o = (size_t)c * n + i;
-        const double d = dt * vd[o];
-        drd[o] += d;
-        double x = xd[o] + d;
-        for (int it = 0; it < 64 && x > box; ++it) x -= box;
-        for (int it = 0; it < 64 && x <= 0.0; ++it) x += box;
-        xd[o] = x;
-        pf[c] = (float)x;
+        const double f = fnb[o] + (double)O.fix[o] * FIX_INV;
+        v[c] = vd[o];
+        if (KICK2) v[c] += mt.y * f;
+        v[c] += mt.y * f;
+        vd[o] = v[c];
+        const double d = dt * v[c];
+        dr[c] = drd[o] + d;
+        drd[o] = dr[c];
+        x[c] = wrap64(xd[o] + d, box);
+        xd[o] = x[c];
     }
-    p.x = pf[0]; p.y = pf[1]; p.z = pf[2];
+    p.x = (float)x[0]; p.y = (float)x[1]; p.z = (float)x[2];
     pos4[i] = p;
+    flag_rebuild(O, r, dr, R.chk2);
+    long long q[3] = {0, 0, 0};
+    if (thermostat && !(R.fric == 0.0 && R.gconst == 0.0)) {
+        float u[3];
+        uniform3(R.seed, step[r], (uint32_t)gid[i], u);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) q[c] = to_fix(-R.fric * mt.x * v[c] + R.gconst * mt.z * (double)u[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) O.fix[(size_t)c * n + i] = q[c];
+    if (O.pf) write_record(O.pf, i, x[0], x[1], x[2], R.fscale, type, O.q);
 }
 
 // Langevin force -fric m v + gconst sqrt(m) U(-1/2,1/2) added to the fixed-point sum
@@ -502,7 +551,7 @@ struct ShakeArgs {
     const float4 *pos4;
     const double *xd, *vd, *fnb;
     long long *fix;
-    const double *mass;
+    const double4 *mtab;
     const int32_t *rep;
     const RepInfo *reps;
     const double *bond_k, *bond_r0, *angle_k, *angle_th0;
@@ -546,7 +595,7 @@ __device__ inline int shake_cluster(int m, const ShakeArgs &A, double vir[3], lo
 #pragma unroll
     for (int k = 0; k < NA; ++k) {
         idx[k] = A.atoms[4 * (size_t)m + k];
-        im[k] = 1.0 / A.mass[__float_as_int(A.pos4[idx[k]].w) - 1];
+        im[k] = A.mtab[__float_as_int(A.pos4[idx[k]].w) - 1].w;
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) bl[k] = A.bond[3 * (size_t)m + k];
@@ -634,8 +683,9 @@ __device__ inline int settle_water(int m, const ShakeArgs &A, double vir[3], lon
         int idx[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) idx[k] = A.atoms[4 * (size_t)m + k];
-        const double mo = A.mass[__float_as_int(A.pos4[idx[0]].w) - 1];
-        const double mh = A.mass[__float_as_int(A.pos4[idx[1]].w) - 1];
+        const double4 to4 = A.mtab[__float_as_int(A.pos4[idx[0]].w) - 1];
+        const double4 th4 = A.mtab[__float_as_int(A.pos4[idx[1]].w) - 1];
+        const double mo = to4.x, mh = th4.x;
         const double doh = A.bond[3 * (size_t)m], dhh = A.bond[3 * (size_t)m + 2];
         rr = A.rep[idx[0]];
         const double box = A.reps[rr].box, ibox = A.reps[rr].ibox;
@@ -649,7 +699,7 @@ __device__ inline int settle_water(int m, const ShakeArgs &A, double vir[3], lon
         const bool fused = w.w != 0;
         if (fused) water_bonded(w, A, idx, box, ibox, own, eb, ea);
         // old (b0, c0) and unconstrained new (x1) positions relative to the old O
-        const double im[3] = {1.0 / mo, 1.0 / mh, 1.0 / mh};
+        const double im[3] = {to4.w, th4.w, th4.w};
         double b0[3], c0[3], x1[3][3];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -770,11 +820,32 @@ __device__ inline int settle_water(int m, const ShakeArgs &A, double vir[3], lon
 // five atomics) run on energy launches only.
 constexpr int WSPAN = 160;
 
+// The end of an engine step, done by one extra workgroup of the constraint launch (the last of
+// the step): rebuilt replicas counted, every flag down, the step counters on by one.
+struct StepEnd {
+    int32_t nrep;          // 0: nothing to end
+    int32_t *rebuild, *nbuilds;
+    uint64_t *step;
+};
+__device__ inline void end_step(const StepEnd &S) {
+    for (int r = threadIdx.x; r <= S.nrep; r += blockDim.x) {
+        if (r < S.nrep) {
+            if (S.rebuild[r]) S.nbuilds[r] += 1;
+            S.step[r] += 1;
+        }
+        S.rebuild[r] = 0;   // [nrep] is `any`
+    }
+}
+
 template <bool ENERGY>
 __global__ void __launch_bounds__(128)
 k_constraints(const int32_t *__restrict__ kidx, int32_t e1, int32_t e2, int32_t e3, int32_t e4,
-              int32_t nb_it, const int32_t *__restrict__ wclus, ShakeArgs A,
+              int32_t nb_it, const int32_t *__restrict__ wclus, ShakeArgs A, StepEnd S,
               long long *__restrict__ eacc) {
+    if (S.nrep && blockIdx.x == gridDim.x - 1) {
+        end_step(S);
+        return;
+    }
     auto energies = [&](const double vir[3], long long eb, long long ea, bool live, int rr) {
         if (!ENERGY) return;
         wave_add(to_efix(vir[0]), live, rr, eacc, V_X);
@@ -878,38 +949,41 @@ __global__ void k_water_bonded(int32_t ns, const int32_t *__restrict__ num, Shak
     wave_add(ea, live, rr, eacc, E_ANGLE);
 }
 
-// Capped steepest descent: every atom moves along its force by min(gamma |F|, max_disp).
+// Capped steepest descent: every atom moves along its force by min(gamma |F|, max_disp); then,
+// as in k_advance, the rebuild check, a cleared force sum and the pair kernel's record.
 __global__ void k_minimize_step(int32_t n, double gamma, double max_disp, double *__restrict__ xd,
                                 double *__restrict__ drd, const double *__restrict__ fnb,
-                                const long long *__restrict__ fix, float4 *__restrict__ pos4,
-                                const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps) {
+                                float4 *__restrict__ pos4, const int32_t *__restrict__ rep,
+                                const RepInfo *__restrict__ reps, StepOut O) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const double box = reps[rep[i]].box;
-    double f[3], f2 = 0.0;
+    const int r = rep[i];
+    const RepInfo &R = reps[r];
+    const double box = R.box;
+    double f[3], x[3], dr[3], f2 = 0.0;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const size_t o = (size_t)c * n + i;
-        f[c] = fnb[o] + (double)fix[o] * FIX_INV;
+        f[c] = fnb[o] + (double)O.fix[o] * FIX_INV;
+        O.fix[o] = 0;
         f2 += f[c] * f[c];
     }
     const double fn = sqrt(f2);
     const double step = (fn > 0.0) ? fmin(gamma * fn, max_disp) / fn : 0.0;
     float4 p = pos4[i];
-    float pf[3];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const size_t o = (size_t)c * n + i;
         const double d = isfinite(f[c]) ? step * f[c] : 0.0;
-        drd[o] += d;
-        double x = xd[o] + d;
-        for (int it = 0; it < 64 && x > box; ++it) x -= box;
-        for (int it = 0; it < 64 && x <= 0.0; ++it) x += box;
-        xd[o] = x;
-        pf[c] = (float)x;
+        dr[c] = drd[o] + d;
+        drd[o] = dr[c];
+        x[c] = wrap64(xd[o] + d, box);
+        xd[o] = x[c];
     }
-    p.x = pf[0]; p.y = pf[1]; p.z = pf[2];
+    p.x = (float)x[0]; p.y = (float)x[1]; p.z = (float)x[2];
     pos4[i] = p;
+    flag_rebuild(O, r, dr, R.chk2);
+    if (O.pf) write_record(O.pf, i, x[0], x[1], x[2], R.fscale, (uint32_t)__float_as_int(p.w), O.q);
 }
 
 __global__ void k_step_add(int32_t nrep, uint64_t *step, long long delta) {
@@ -985,9 +1059,27 @@ void launch_nve_v64(sofia_ctx *c, bool ke) {
                        c->eacc);
 }
 
-void launch_nve_x64(sofia_ctx *c) {
-    hipLaunchKernelGGL(k_nve_x64, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N,
-                       (double)c->dp.dt, c->a.xd, c->a.vd, c->drd, c->a.pos4, c->rep, c->reps_d);
+StepOut step_out(sofia_ctx *c) {
+    const int rb = record_bytes(c);
+    return StepOut{c->rebuild, c->rebuild + c->nrep, c->fix, rb ? c->pfix : nullptr,
+                   rb == 16 ? c->a.q : nullptr};
+}
+
+void launch_advance(sofia_ctx *c, bool kick2) {
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N,
+                           (double)c->dp.dt, c->mtab, c->a.xd, c->a.vd, c->drd, c->a.pos4, c->fnb,
+                           c->a.gid, c->rep, c->reps_d, c->step_d, c->has_thermostat ? 1 : 0,
+                           step_out(c));
+    };
+    if (kick2) go(k_advance<true>);
+    else go(k_advance<false>);
+}
+
+void launch_zero_energies(sofia_ctx *c) {
+    const int ne = (int)eacc_len(c->nrep);
+    hipLaunchKernelGGL(k_zero, dim3(nblocks(ne, 256)), dim3(256), 0, c->stream, ne, c->eacc, 0,
+                       (long long *)nullptr);
 }
 
 void launch_langevin64(sofia_ctx *c) {
@@ -1001,26 +1093,27 @@ ShakeArgs shake_args(sofia_ctx *c) {
     ShakeArgs A;
     A.atoms = c->shake_atoms; A.bond = c->shake_bond; A.water = c->water;
     A.pos4 = c->a.pos4; A.xd = c->a.xd; A.vd = c->a.vd; A.fnb = c->fnb; A.fix = c->fix;
-    A.mass = c->mass; A.rep = c->rep; A.reps = c->reps_d;
+    A.mtab = c->mtab; A.rep = c->rep; A.reps = c->reps_d;
     A.bond_k = c->bond_k; A.bond_r0 = c->bond_r0; A.angle_k = c->angle_k; A.angle_th0 = c->angle_th0;
     A.n = c->N; A.dt = dt; A.dtsq = dtsq; A.tol = c->dp.shake_tol; A.maxiter = c->dp.shake_maxiter;
     A.err = c->shake_err;
     return A;
 }
 
-void launch_shake64(sofia_ctx *c, bool energies) {
-    if (!c->ns) return;
+void launch_shake64(sofia_ctx *c, bool energies, bool step) {
     const int32_t *n = c->shake_kcount;   // group sizes in whole wavefronts
     const int e1 = n[0], e2 = e1 + n[1], e3 = e2 + n[2], e4 = e3 + n[3];
     const int nb_it = nblocks(e4, 128);
     const int nb_w = n[4] ? nblocks(c->N, 2 * WSPAN) : 0;
-    if (nb_it + nb_w == 0) return;
+    const int grid = nb_it + nb_w + (step ? 1 : 0);
+    if (grid == 0) return;
+    StepEnd S{step ? c->nrep : 0, c->rebuild, c->nbuilds, c->step_d};
     if (energies)
-        hipLaunchKernelGGL(k_constraints<true>, dim3(nb_it + nb_w), dim3(128), 0, c->stream,
-                           c->shake_kidx, e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), c->eacc);
+        hipLaunchKernelGGL(k_constraints<true>, dim3(grid), dim3(128), 0, c->stream, c->shake_kidx,
+                           e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), S, c->eacc);
     else
-        hipLaunchKernelGGL(k_constraints<false>, dim3(nb_it + nb_w), dim3(128), 0, c->stream,
-                           c->shake_kidx, e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), c->eacc);
+        hipLaunchKernelGGL(k_constraints<false>, dim3(grid), dim3(128), 0, c->stream, c->shake_kidx,
+                           e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), S, c->eacc);
 }
 
 void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb) {
@@ -1046,11 +1139,7 @@ void launch_water_bonded(sofia_ctx *c) {
 
 void launch_minimize_step(sofia_ctx *c, double gamma, double max_disp) {
     hipLaunchKernelGGL(k_minimize_step, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N, gamma,
-                       max_disp, c->a.xd, c->drd, c->fnb, c->fix, c->a.pos4, c->rep, c->reps_d);
-}
-
-void launch_step_advance(sofia_ctx *c) {
-    launch_step_add(c, 1);
+                       max_disp, c->a.xd, c->drd, c->fnb, c->a.pos4, c->rep, c->reps_d, step_out(c));
 }
 
 void launch_step_add(sofia_ctx *c, long long delta) {

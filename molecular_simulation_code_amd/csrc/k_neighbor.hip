@@ -17,7 +17,7 @@
 // cell belongs to one replica and only replicas flagged for a rebuild do work.
 #include <algorithm>
 
-#include "sofia_internal.h"
+#include "sofia_device.h"
 
 namespace sofia {
 namespace {
@@ -53,171 +53,131 @@ __device__ inline float mimg32(float dx, float box, float ibox) {
 // with a fixed grid (at most GRID_CAP workgroups), which keeps such a step's launches short.
 constexpr int GRID_CAP = 2048;
 
-__global__ void k_cell_reset(int32_t ncell, const int32_t *__restrict__ cell_rep,
-                             const int32_t *__restrict__ rebuild, const int32_t *__restrict__ any,
-                             int32_t *__restrict__ ccount) {
-    if (!*any) return;
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < ncell; c += gridDim.x * blockDim.x)
-        if (rebuild[cell_rep[c]]) ccount[c] = 0;
-}
-
+// The sort is three launches.  k_bin counts each cell's atoms and drops their ids into the
+// cell's bucket; k_sort_gather orders a cell and moves its atoms' data to the gather target;
+// k_copyback puts them back (device pointers stay fixed, which keeps captured graphs valid),
+// re-indexes what names atoms and clears the binning counters for the next sort.
 __global__ void k_bin(int32_t n, const float4 *__restrict__ pos4, const int32_t *__restrict__ rep,
                       const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
-                      const int32_t *__restrict__ any, int32_t *__restrict__ ccount,
-                      int32_t *__restrict__ acell, int32_t *__restrict__ aslot) {
+                      const int32_t *__restrict__ any, int32_t *__restrict__ cbin,
+                      int32_t *__restrict__ acell, int32_t *__restrict__ bucket, int32_t cap) {
     if (!*any) return;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const int r = rep[i];
-        // perm and tt of a replica that rebuilds nothing are stale: every reader (scatter,
-        // cell sort, gather, copy-back, topology remap) skips such replicas
+        // tt of a replica that rebuilds nothing is stale: every reader skips such replicas
         if (!rebuild[r]) continue;
         const RepInfo R = reps[r];
         const int c = R.cell0 + xyz2bin_dev(pos4[i], R);
         acell[i] = c;
-        aslot[i] = atomicAdd(&ccount[c], 1);
+        const int slot = atomicAdd(&cbin[c], 1);
+        if (slot < cap) bucket[(size_t)c * cap + slot] = i;
     }
 }
 
-// One workgroup per replica: exclusive scan of its cell counts into absolute starts.
-__global__ void k_cell_scan(const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
-                            const int32_t *__restrict__ ccount, int32_t *__restrict__ cstart) {
-    const int r = blockIdx.x;
-    if (!rebuild[r]) return;
-    const RepInfo R = reps[r];
-    __shared__ int32_t s[1024];
-    __shared__ int32_t carry;
-    if (threadIdx.x == 0) carry = R.atom0;
-    __syncthreads();
-    for (int base = 0; base < R.ncellT; base += 1024) {
-        const int c = base + threadIdx.x;
-        const int v = (c < R.ncellT) ? ccount[R.cell0 + c] : 0;
-        s[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < 1024; off <<= 1) {          // Hillis-Steele inclusive scan
-            const int add = (threadIdx.x >= off) ? s[threadIdx.x - off] : 0;
-            __syncthreads();
-            s[threadIdx.x] += add;
-            __syncthreads();
-        }
-        if (c < R.ncellT) cstart[R.cell0 + c] = carry + s[threadIdx.x] - v;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry += s[1023];
-        __syncthreads();
-    }
-}
+// What the step's sort carries beyond the per-atom arrays (SORT_STEP), else null.
+struct StepArrays {
+    long long *fix, *fixb;   // the step's fixed-point forces and their gather target
+    int4 *pf;                // position records, rewritten from the moved positions
+    const float *q;          // null: 12-byte records
+};
 
-__global__ void k_scatter(int32_t n, const int32_t *__restrict__ rep,
-                          const int32_t *__restrict__ rebuild, const int32_t *__restrict__ any,
-                          const int32_t *__restrict__ acell, const int32_t *__restrict__ aslot,
-                          const int32_t *__restrict__ cstart, int32_t *__restrict__ sorted_ids) {
-    if (!*any) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        if (rebuild[rep[i]]) sorted_ids[cstart[acell[i]] + aslot[i]] = i;
-}
-
-// One workgroup per cell at a time: order the cell's atoms by descending old index (the
-// chain order of the reference's linked cells) by ranking, which is deterministic.
-__global__ void k_cell_sort(int32_t ncell, const int32_t *__restrict__ cell_rep,
-                            const int32_t *__restrict__ rebuild, const int32_t *__restrict__ any,
-                            const int32_t *__restrict__ ccount, const int32_t *__restrict__ cstart,
-                            const int32_t *__restrict__ sorted_ids, int32_t *__restrict__ perm,
-                            int32_t *__restrict__ tt, int32_t *__restrict__ atombin) {
-    if (!*any) return;
-    constexpr int CAP = 2048;
-    __shared__ int32_t ids[CAP];
-    for (int c = blockIdx.x; c < ncell; c += gridDim.x) {   // uniform over the workgroup
-        if (!rebuild[cell_rep[c]]) continue;
-        const int n = ccount[c], base = cstart[c];
-        const bool staged = n <= CAP;
-        if (staged)
-            for (int e = threadIdx.x; e < n; e += blockDim.x) ids[e] = sorted_ids[base + e];
-        __syncthreads();
-        for (int e = threadIdx.x; e < n; e += blockDim.x) {
-            const int me = staged ? ids[e] : sorted_ids[base + e];
-            int rank = 0;
-            for (int f = 0; f < n; ++f) {
-                const int other = staged ? ids[f] : sorted_ids[base + f];
-                rank += other > me;
-            }
-            perm[base + rank] = me;
-            tt[me] = base + rank;
-            atombin[base + rank] = c;
-        }
-        __syncthreads();   // ids is refilled for the next cell
-    }
-}
-
-// Gather every permuted per-atom array from `src` into `dst` (flagged replicas only),
-// remapping specbond entries through tt; FP64 engine state too when `engine`.
-__global__ void k_gather(int32_t n, const int32_t *__restrict__ rep,
-                         const int32_t *__restrict__ rebuild, const int32_t *__restrict__ any,
-                         const int32_t *__restrict__ perm, const int32_t *__restrict__ tt,
-                         AtomArrays src, AtomArrays dst, int engine) {
-    if (!*any) return;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        if (!rebuild[rep[k]]) continue;
-        const int o = perm[k];
-        dst.pos4[k] = src.pos4[o];
-        dst.q[k] = src.q[o];
-        dst.gid[k] = src.gid[o];
-        dst.num1[k] = src.num1[o];
-        dst.num2[k] = src.num2[o];
-        dst.num3[k] = src.num3[o];
-        dst.mol[k] = src.mol[o];
-        dst.wclus[k] = src.wclus[o];
+// Atom o of src to place k of dst; specbond entries go along unmapped.
+__device__ inline void move_atom(const AtomArrays &src, const AtomArrays &dst, int n, int o, int k,
+                                 int mode, const StepArrays &T) {
+    dst.pos4[k] = src.pos4[o];
+    dst.q[k] = src.q[o];
+    dst.gid[k] = src.gid[o];
+    dst.num1[k] = src.num1[o];
+    dst.num2[k] = src.num2[o];
+    dst.num3[k] = src.num3[o];
+    dst.mol[k] = src.mol[o];
+    dst.wclus[k] = src.wclus[o];
+    const int4 *s4 = (const int4 *)(src.spec + (size_t)o * SPEC);
+    int4 *d4 = (int4 *)(dst.spec + (size_t)k * SPEC);
 #pragma unroll
-        for (int l = 0; l < SPEC; ++l) {
-            const int s = src.spec[(size_t)o * SPEC + l];
-            dst.spec[(size_t)k * SPEC + l] = (s >= 0) ? tt[s] : -1;
-        }
+    for (int l = 0; l < SPEC / 4; ++l) d4[l] = s4[l];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) dst.v32[3 * (size_t)k + d] = src.v32[3 * (size_t)o + d];
-        if (engine) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                dst.xd[(size_t)d * n + k] = src.xd[(size_t)d * n + o];
-                dst.vd[(size_t)d * n + k] = src.vd[(size_t)d * n + o];
-            }
-        }
-    }
-}
-
-// Copy the gathered arrays back (flagged replicas only) so device pointers stay fixed,
-// which keeps captured graphs valid; zero the displacement accumulators.
-__global__ void k_copyback(int32_t n, const int32_t *__restrict__ rep,
-                           const int32_t *__restrict__ rebuild, const int32_t *__restrict__ any,
-                           AtomArrays src, AtomArrays dst, float *__restrict__ dr32,
-                           double *__restrict__ drd, int engine) {
-    if (!*any) return;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
-        if (!rebuild[rep[k]]) continue;
-        dst.pos4[k] = src.pos4[k];
-        dst.q[k] = src.q[k];
-        dst.gid[k] = src.gid[k];
-        dst.num1[k] = src.num1[k];
-        dst.num2[k] = src.num2[k];
-        dst.num3[k] = src.num3[k];
-        dst.mol[k] = src.mol[k];
-        dst.wclus[k] = src.wclus[k];
-#pragma unroll
-        for (int l = 0; l < SPEC; ++l) dst.spec[(size_t)k * SPEC + l] = src.spec[(size_t)k * SPEC + l];
+    for (int d = 0; d < 3; ++d) dst.v32[3 * (size_t)k + d] = src.v32[3 * (size_t)o + d];
+    if (mode != SORT_DROPIN) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            dst.v32[3 * (size_t)k + d] = src.v32[3 * (size_t)k + d];
-            dr32[(size_t)d * n + k] = 0.0f;
+            dst.xd[(size_t)d * n + k] = src.xd[(size_t)d * n + o];
+            dst.vd[(size_t)d * n + k] = src.vd[(size_t)d * n + o];
         }
-        if (engine) {
+    }
+    if (mode == SORT_STEP) {
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                dst.xd[(size_t)d * n + k] = src.xd[(size_t)d * n + k];
-                dst.vd[(size_t)d * n + k] = src.vd[(size_t)d * n + k];
-                drd[(size_t)d * n + k] = 0.0;
-            }
-        }
+        for (int d = 0; d < 3; ++d) T.fixb[(size_t)d * n + k] = T.fix[(size_t)d * n + o];
     }
 }
 
-// Every bonded list in one launch: item t of the concatenation falls in list L of S, whose
+// Atoms of a cell in descending old index (the chain order of the reference's linked cells),
+// by ranking, which is deterministic.  A wavefront owns `per` consecutive cells; it finds
+// their first atom by summing the replica's counts before its first cell (a scan kernel of one
+// workgroup per replica in the launch sequence cost every step more than these sums cost the
+// steps that rebuild).  A cell with more atoms than a bucket holds is read from acell.
+__global__ void __launch_bounds__(256)
+k_sort_gather(int32_t ncell, int32_t per, const int32_t *__restrict__ cell_rep,
+              const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
+              const int32_t *__restrict__ any, const int32_t *__restrict__ cbin,
+              const int32_t *__restrict__ acell, const int32_t *__restrict__ bucket, int32_t cap,
+              int32_t *__restrict__ ccount, int32_t *__restrict__ cstart, int32_t *__restrict__ tt,
+              int32_t *__restrict__ atombin, int32_t n, AtomArrays src, AtomArrays dst, int mode,
+              StepArrays T) {
+    if (!*any) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
+    const int c0 = wave * per, c1 = min(c0 + per, ncell);
+    int rcur = -1, base = 0;
+    for (int c = c0; c < c1; ++c) {
+        const int r = cell_rep[c];
+        if (!rebuild[r]) {
+            rcur = -1;
+            continue;
+        }
+        if (r != rcur) {   // first cell of this replica here: the atoms in the cells before it
+            int s = 0;
+            for (int k = reps[r].cell0 + lane; k < c; k += 64) s += cbin[k];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+            base = reps[r].atom0 + __builtin_amdgcn_readfirstlane(s);
+            rcur = r;
+        }
+        const int cnt = cbin[c];
+        if (lane == 0) {
+            cstart[c] = base;
+            ccount[c] = cnt;
+        }
+        auto place = [&](int me, int rank) {
+            tt[me] = base + rank;
+            atombin[base + rank] = c;
+            move_atom(src, dst, n, me, base + rank, mode, T);
+        };
+        if (cnt <= cap) {
+            const int32_t *ids = bucket + (size_t)c * cap;
+            for (int e = lane; e < cnt; e += 64) {
+                const int me = ids[e];
+                int rank = 0;
+                for (int f = 0; f < cnt; ++f) rank += ids[f] > me;
+                place(me, rank);
+            }
+        } else {
+            const int a0 = reps[r].atom0, a1 = a0 + reps[r].natom;
+            const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+            int done = 0;
+            for (int b = 0; b < a1 - a0; b += 64) {   // lanes in descending atom order
+                const int i = a1 - 1 - b - lane;
+                const bool in = i >= a0 && acell[i] == c;
+                const uint64_t m = __ballot(in);
+                if (in) place(i, done + __popcll(m & lt_mask));
+                done += __popcll(m);
+            }
+        }
+        base += cnt;
+    }
+}
+
+// Every bonded list of the context: item t of the concatenation falls in list L of S, whose
 // items are `width` ints with the first `nidx` atom ids (-1 = unused).  Items of replicas
 // that rebuild nothing this step are skipped (their atoms keep their places).
 struct RemapSet {
@@ -227,11 +187,40 @@ struct RemapSet {
     int32_t nlists;
 };
 
-__global__ void k_remap_all(RemapSet S, const int32_t *__restrict__ tt, const int32_t *__restrict__ rep,
-                            const int32_t *__restrict__ rebuild, const int32_t *__restrict__ any) {
-    if (!*any || S.nlists == 0) return;
-    const int total = S.end[S.nlists - 1];
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
+__global__ void k_copyback(int32_t n, const int32_t *__restrict__ rep,
+                           const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
+                           const int32_t *__restrict__ any, const int32_t *__restrict__ tt,
+                           AtomArrays src, AtomArrays dst, float *__restrict__ dr32,
+                           double *__restrict__ drd, int mode, StepArrays T, RemapSet S,
+                           int32_t ncell, const int32_t *__restrict__ cell_rep,
+                           int32_t *__restrict__ cbin) {
+    if (!*any) return;
+    const int t0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (int k = t0; k < n; k += stride) {
+        const int r = rep[k];
+        if (!rebuild[r]) continue;
+        move_atom(src, dst, n, k, k, mode == SORT_STEP ? (int)SORT_ENGINE : mode, T);
+#pragma unroll
+        for (int l = 0; l < SPEC; ++l) {
+            const int s = src.spec[(size_t)k * SPEC + l];
+            if (s >= 0) dst.spec[(size_t)k * SPEC + l] = tt[s];
+        }
+#pragma unroll
+        for (int d = 0; d < 3; ++d) dr32[(size_t)d * n + k] = 0.0f;
+        if (mode != SORT_DROPIN) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) drd[(size_t)d * n + k] = 0.0;
+        }
+        if (mode == SORT_STEP) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) T.fix[(size_t)d * n + k] = T.fixb[(size_t)d * n + k];
+            if (T.pf)
+                write_record(T.pf, k, src.xd[k], src.xd[(size_t)n + k], src.xd[2 * (size_t)n + k],
+                             reps[r].fscale, (uint32_t)__float_as_int(src.pos4[k].w), T.q ? src.q : nullptr);
+        }
+    }
+    const int total = S.nlists ? S.end[S.nlists - 1] : 0;
+    for (int t = t0; t < total; t += stride) {
         int L = 0;
         while (t >= S.end[L]) ++L;
         const int m = t - (L ? S.end[L - 1] : 0);
@@ -243,6 +232,8 @@ __global__ void k_remap_all(RemapSet S, const int32_t *__restrict__ tt, const in
             if (v >= 0) item[k] = tt[v];
         }
     }
+    for (int c = t0; c < ncell; c += stride)
+        if (rebuild[cell_rep[c]]) cbin[c] = 0;
 }
 
 // A device topology array in the host's layout: in the first nidx columns of each item a
@@ -411,18 +402,6 @@ __global__ void k_check32(int32_t n, const int32_t *__restrict__ rep, const floa
     if (d2 >= rvrc2 && atomicOr(&rebuild[rep[i]], 1) == 0) atomicOr(any, 1);
 }
 
-// Engine criterion: per-replica threshold that keeps every pair inside the force cutoff in
-// the list (half the usable skin), so forces do not depend on when the list was built.
-__global__ void k_check64(int32_t n, const int32_t *__restrict__ rep, const double *__restrict__ dr,
-                          const RepInfo *__restrict__ reps, int32_t *__restrict__ rebuild,
-                          int32_t *__restrict__ any) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int r = rep[i];
-    const double x = dr[i], y = dr[(size_t)n + i], z = dr[2 * (size_t)n + i];
-    if ((x * x + y * y) + z * z >= reps[r].chk2 && atomicOr(&rebuild[r], 1) == 0) atomicOr(any, 1);
-}
-
 // rebuild[0..nrep) and `any` = rebuild[nrep] to value
 __global__ void k_set_flags(int32_t nrep, int32_t *__restrict__ rebuild, int32_t value) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
@@ -446,37 +425,20 @@ inline int nblk(int n, int b) { return (n + b - 1) / b; }
 inline int capped(int n, int b) { return std::max(1, std::min(nblk(n, b), GRID_CAP)); }
 inline const int32_t *any_flag(const sofia_ctx *c) { return c->rebuild + c->nrep; }
 
-void launch_cell_reset(sofia_ctx *c, bool) {
-    hipLaunchKernelGGL(k_cell_reset, dim3(capped(c->ncell_total, 256)), dim3(256), 0, c->stream,
-                       c->ncell_total, c->cell_rep, c->rebuild, any_flag(c), c->ccount);
-}
-
-void launch_bin(sofia_ctx *c) {
+void launch_sort(sofia_ctx *c, SortMode mode) {
     hipLaunchKernelGGL(k_bin, dim3(capped(c->N, 256)), dim3(256), 0, c->stream, c->N, c->a.pos4,
-                       c->rep, c->reps_d, c->rebuild, any_flag(c), c->ccount, c->acell, c->aslot);
-}
-
-void launch_cell_scan(sofia_ctx *c) {
-    hipLaunchKernelGGL(k_cell_scan, dim3(c->nrep), dim3(1024), 0, c->stream, c->reps_d, c->rebuild,
-                       c->ccount, c->cstart);
-}
-
-void launch_scatter_sort(sofia_ctx *c) {
-    hipLaunchKernelGGL(k_scatter, dim3(capped(c->N, 256)), dim3(256), 0, c->stream, c->N, c->rep,
-                       c->rebuild, any_flag(c), c->acell, c->aslot, c->cstart, c->sorted_ids);
-    hipLaunchKernelGGL(k_cell_sort, dim3(capped(c->ncell_total, 1)), dim3(256), 0, c->stream,
-                       c->ncell_total, c->cell_rep, c->rebuild, any_flag(c), c->ccount, c->cstart,
-                       c->sorted_ids, c->perm, c->tt, c->atombin);
-}
-
-void launch_gather(sofia_ctx *c, bool engine) {
-    hipLaunchKernelGGL(k_gather, dim3(capped(c->N, 256)), dim3(256), 0, c->stream, c->N, c->rep,
-                       c->rebuild, any_flag(c), c->perm, c->tt, c->a, c->b, engine ? 1 : 0);
-    hipLaunchKernelGGL(k_copyback, dim3(capped(c->N, 256)), dim3(256), 0, c->stream, c->N, c->rep,
-                       c->rebuild, any_flag(c), c->b, c->a, c->dr32, c->drd, engine ? 1 : 0);
-}
-
-void launch_remap_topology(sofia_ctx *c) {
+                       c->rep, c->reps_d, c->rebuild, any_flag(c), c->cbin, c->acell, c->bucket,
+                       c->bucket_cap);
+    StepArrays T{};
+    if (mode == SORT_STEP) {
+        const int rb = record_bytes(c);
+        T = StepArrays{c->fix, c->fscratch, rb ? c->pfix : nullptr, rb == 16 ? c->a.q : nullptr};
+    }
+    const int per = nblk(c->ncell_total, 4 * GRID_CAP);   // cells per wavefront
+    hipLaunchKernelGGL(k_sort_gather, dim3(nblk(nblk(c->ncell_total, per), 4)), dim3(256), 0, c->stream,
+                       c->ncell_total, per, c->cell_rep, c->reps_d, c->rebuild, any_flag(c), c->cbin,
+                       c->acell, c->bucket, c->bucket_cap, c->ccount, c->cstart, c->tt, c->atombin,
+                       c->N, c->a, c->b, (int)mode, T);
     RemapSet S{};
     int total = 0;
     auto add = [&](int32_t *lst, int items, int width, int nidx) {
@@ -496,9 +458,10 @@ void launch_remap_topology(sofia_ctx *c) {
     add(c->shake_atoms, c->ns, 4, 4);
     add(c->ebond, c->nbe, 3, 2);
     add(c->eangle, c->nae, 4, 3);
-    if (total)
-        hipLaunchKernelGGL(k_remap_all, dim3(capped(total, 256)), dim3(256), 0, c->stream, S, c->tt,
-                           c->rep, c->rebuild, any_flag(c));
+    const int items = std::max({c->N, total, c->ncell_total});
+    hipLaunchKernelGGL(k_copyback, dim3(capped(items, 256)), dim3(256), 0, c->stream, c->N, c->rep,
+                       c->reps_d, c->rebuild, any_flag(c), c->tt, c->b, c->a, c->dr32, c->drd,
+                       (int)mode, T, S, c->ncell_total, c->cell_rep, c->cbin);
 }
 
 void launch_rdf(sofia_ctx *c, int32_t itype, int32_t jtype, double delta, int32_t nbins,
@@ -533,13 +496,9 @@ void launch_build_list(sofia_ctx *c) {
 #undef LB
 }
 
-void launch_check_neighbor(sofia_ctx *c, bool engine) {
-    if (engine)
-        hipLaunchKernelGGL(k_check64, dim3(nblk(c->N, 256)), dim3(256), 0, c->stream, c->N, c->rep,
-                           c->drd, c->reps_d, c->rebuild, c->rebuild + c->nrep);
-    else
-        hipLaunchKernelGGL(k_check32, dim3(nblk(c->N, 256)), dim3(256), 0, c->stream, c->N, c->rep,
-                           c->dr32, c->dp.rvrc2, c->rebuild, c->rebuild + c->nrep);
+void launch_check_neighbor(sofia_ctx *c) {
+    hipLaunchKernelGGL(k_check32, dim3(nblk(c->N, 256)), dim3(256), 0, c->stream, c->N, c->rep,
+                       c->dr32, c->dp.rvrc2, c->rebuild, c->rebuild + c->nrep);
 }
 
 void launch_set_rebuild(sofia_ctx *c, int32_t value) {
@@ -547,7 +506,7 @@ void launch_set_rebuild(sofia_ctx *c, int32_t value) {
                        c->rebuild, value);
 }
 
-void launch_finish_rebuild(sofia_ctx *c, bool) {
+void launch_finish_rebuild(sofia_ctx *c) {
     hipLaunchKernelGGL(k_finish, dim3(nblk(c->nrep + 1, 256)), dim3(256), 0, c->stream, c->nrep,
                        c->rebuild, c->nbuilds);
 }

@@ -261,13 +261,13 @@ void launch_mode(sofia_ctx *c, bool energies, float *ff32) {
 // Drop-in launches (positions from the float copy the caller handed over).
 void launch_nonbond_out(sofia_ctx *c, int mode, bool energies, float *ff32) {
     if (mode == 0) launch_mode<0>(c, energies, ff32);
-    else if (mode == 1) launch_dsf_mixed(c, energies, ff32, false);
+    else if (mode == 1) launch_dsf_mixed(c, energies, ff32, false, false);
     else launch_mode<2>(c, energies, ff32);
 }
 
 // Engine launches: the mixed kernel takes its fixed-point positions from the FP64 state.
-void launch_nonbond(sofia_ctx *c, int mode, bool energies) {
-    if (mode == 1) launch_dsf_mixed(c, energies, nullptr, c->engine_ready);
+void launch_nonbond(sofia_ctx *c, int mode, bool energies, bool records) {
+    if (mode == 1) launch_dsf_mixed(c, energies, nullptr, c->engine_ready, records);
     else launch_nonbond_out(c, mode, energies, nullptr);
 }
 

@@ -179,6 +179,35 @@ int ensure_list(sofia_ctx *c, int na) {
     return SOFIA_OK;
 }
 
+// Per-cell arrays for ncell cells of the current grids, and the binning buckets: twice a cell's
+// mean occupancy and 32 more (k_sort_gather handles fuller cells without one).
+int size_cells(sofia_ctx *c, int ncell) {
+    if (ncell > c->ncell_cap) {
+        dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep); dfree(c->cbin);
+        c->ncell_cap = 0;
+        TRY(dalloc(&c->ccount, ncell));
+        TRY(dalloc(&c->cstart, ncell));
+        TRY(dalloc(&c->cnum, (size_t)27 * ncell));
+        TRY(dalloc(&c->cell_rep, ncell));
+        TRY(dalloc(&c->cbin, ncell));
+        SOFIA_HIP(hipMemset(c->ccount, 0, sizeof(int32_t) * ncell));
+        SOFIA_HIP(hipMemset(c->cstart, 0, sizeof(int32_t) * ncell));
+        SOFIA_HIP(hipMemset(c->cbin, 0, sizeof(int32_t) * ncell));
+        c->ncell_cap = ncell;
+    }
+    int mean = 0;
+    for (const auto &R : c->reps_h) mean = std::max(mean, (R.natom + R.ncellT - 1) / R.ncellT);
+    c->bucket_cap = std::min((2 * mean + 32 + 15) / 16 * 16, 512);
+    const size_t need = (size_t)ncell * c->bucket_cap;
+    if (need > c->bucket_len) {
+        dfree(c->bucket);
+        c->bucket_len = 0;
+        TRY(dalloc(&c->bucket, need));
+        c->bucket_len = need;
+    }
+    return SOFIA_OK;
+}
+
 // Synchronous copies on the null stream; callers synchronise the context stream first
 // when kernels on it may still use the destination.
 int upload(void *dst, const void *src, size_t bytes) {
@@ -399,6 +428,7 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
         sofia::RepInfo R{};
         R.box = box[r];
         R.ibox = (float)(1.0 / (double)box[r]);      // ibox = 1.0d0/box, Source/get_started.f90:66
+        R.fscale = 4294967296.0 / (double)R.box;
         cell_grid(R.box, p->rcut, p->cut_coul, &R.rn, &R.ncellT, &R.ncellD);
         if (R.ncellD < 3)
             return fail(SOFIA_E_ARG, "box must hold at least 3 cells of max(rcut, cut_coul) per side");
@@ -412,7 +442,6 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
     }
     c->N = atom0;
     c->ncell_total = cell0;
-    c->ncell_cap = cell0;
     c->last_e.assign((size_t)nrep * SOFIA_NENERGY, 0.0);
     const int n = c->N;
     TRY(alloc_atoms(c->a, n));
@@ -425,16 +454,10 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
     TRY(dalloc(&c->fix, (size_t)3 * n));
     TRY(dalloc(&c->fscratch, (size_t)3 * n));
     TRY(dalloc(&c->stage32, (size_t)3 * n));
-    TRY(dalloc(&c->ccount, c->ncell_total));
-    TRY(dalloc(&c->cstart, c->ncell_total));
-    TRY(dalloc(&c->cnum, (size_t)27 * c->ncell_total));
-    TRY(dalloc(&c->cell_rep, c->ncell_total));
+    TRY(size_cells(c.get(), c->ncell_total));
     TRY(dalloc(&c->acell, n));
-    TRY(dalloc(&c->aslot, n));
-    TRY(dalloc(&c->perm, n));
     TRY(dalloc(&c->tt, n));
     TRY(dalloc(&c->atombin, n));
-    TRY(dalloc(&c->sorted_ids, n));
     TRY(dalloc(&c->numneigh, n));
     TRY(dalloc(&c->maxcnt, 1));
     TRY(dalloc(&c->rebuild, nrep + 1));   // nrep flags, then `any`
@@ -504,12 +527,7 @@ double E(const std::vector<long long> &e, int r, int slot) { return (double)e[(s
 
 // Full sort + list build of every flagged replica; grow-and-redo on overflow.
 int rebuild_now(sofia_ctx *c, bool engine, bool reference_growth) {
-    launch_cell_reset(c, true);
-    launch_bin(c);
-    launch_cell_scan(c);
-    launch_scatter_sort(c);
-    launch_gather(c, engine);
-    launch_remap_topology(c);
+    launch_sort(c, engine ? SORT_ENGINE : SORT_DROPIN);
     for (int attempt = 0; attempt < 8; ++attempt) {
         SOFIA_HIP(hipMemsetAsync(c->maxcnt, 0, sizeof(int32_t), c->stream));
         launch_build_list(c);
@@ -517,7 +535,7 @@ int rebuild_now(sofia_ctx *c, bool engine, bool reference_growth) {
         SOFIA_HIP(hipMemcpyAsync(&mx, c->maxcnt, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
         TRY(sync_check(c));
         if (mx <= c->neigh_alloc) {
-            launch_finish_rebuild(c, engine);
+            launch_finish_rebuild(c);
             c->have_list = true;
             return sync_check(c);
         }
@@ -744,7 +762,7 @@ int sofia_ctx_destroy(sofia_ctx *c) {
     dfree(c->gc_first); dfree(c->gc_refgid); dfree(c->gc_cnt); dfree(c->gc_dens); dfree(c->gc_sum);
     dfree(c->gc_refx); dfree(c->gc_com); dfree(c->gc_key); dfree(c->gc_surface);
     dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep); dfree(c->acell);
-    dfree(c->aslot); dfree(c->perm); dfree(c->tt); dfree(c->atombin); dfree(c->sorted_ids);
+    dfree(c->cbin); dfree(c->bucket); dfree(c->tt); dfree(c->atombin); dfree(c->mtab);
     dfree(c->nlist); dfree(c->numneigh); dfree(c->maxcnt); dfree(c->rebuild); dfree(c->nbuilds);
     dfree(c->bund_tstart); dfree(c->bund_sstart); dfree(c->bund_slots); dfree(c->bund_terms);
     dfree(c->shake_err); dfree(c->shake_iters); dfree(c->water); dfree(c->dsf_tab); dfree(c->pfix); dfree(c->ebond); dfree(c->eangle); dfree(c->bondlist); dfree(c->anglelist);
@@ -782,6 +800,7 @@ int sofia_set_forcefield(sofia_ctx *c, const float *lj1, const float *lj2, const
         TRY(dalloc(&c->ljtab, nt2));
         TRY(dalloc(&c->lj14, nt2));
         TRY(dalloc(&c->mass, c->p.ntypes));
+        TRY(dalloc(&c->mtab, c->p.ntypes));
     }
     TRY(sync_check(c));   // kernels in flight may still read the tables
     TRY(upload(c->ljtab, lj.data(), sizeof(float4) * nt2));
@@ -790,6 +809,11 @@ int sofia_set_forcefield(sofia_ctx *c, const float *lj1, const float *lj2, const
     drop_graph(c);          // a captured step may hold the 12-byte record layout
     TRY(upload(c->lj14, l14.data(), sizeof(double4) * nt2));
     TRY(upload(c->mass, mass, sizeof(double) * c->p.ntypes));
+    std::vector<double4> mt(c->p.ntypes);
+    const double dthalf = 0.5 * (double)c->dp.dt * (double)c->dp.kcal2amu;
+    for (int k = 0; k < c->p.ntypes; ++k)
+        mt[k] = make_double4(mass[k], dthalf / mass[k], std::sqrt(mass[k]), 1.0 / mass[k]);
+    TRY(upload(c->mtab, mt.data(), sizeof(double4) * mt.size()));
     c->have_ff = true;
     // a running engine takes the new coefficients into its type-pair table at once
     if (c->engine_ready) TRY(classify_charges(c));
@@ -1217,7 +1241,7 @@ int sofia_get_nlist(sofia_ctx *c, int32_t *nlist, int32_t *numneigh, int32_t *na
 int sofia_check_neighbor(sofia_ctx *c, int32_t *nflag) {
     if (!c || !nflag) return fail(SOFIA_E_ARG, "null argument");
     launch_set_rebuild(c, 0);
-    launch_check_neighbor(c, false);
+    launch_check_neighbor(c);
     std::vector<int32_t> f(c->nrep);
     SOFIA_HIP(hipMemcpyAsync(f.data(), c->rebuild, sizeof(int32_t) * c->nrep, hipMemcpyDeviceToHost, c->stream));
     TRY(sync_check(c));
@@ -1450,6 +1474,7 @@ int sofia_berendsen(sofia_ctx *c, const double *mu, float *box_out) {
         auto &R = c->reps_h[r];
         R.box = (float)((double)R.box * mu[r]);
         R.ibox = 1.0f / R.box;
+        R.fscale = 4294967296.0 / (double)R.box;
         if (box_out) box_out[r] = R.box;
     }
     TRY(reference_regrid(c));
@@ -1534,21 +1559,16 @@ void force_sequence(sofia_ctx *c, bool energies) {
     launch_shake64(c, energies);
 }
 
-void step_sequence(sofia_ctx *c, bool energies) {
-    launch_nve_v64(c, false);
-    launch_nve_x64(c);
-    launch_check_neighbor(c, true);
-    launch_cell_reset(c, false);
-    launch_bin(c);
-    launch_cell_scan(c);
-    launch_scatter_sort(c);
-    launch_gather(c, true);
-    launch_remap_topology(c);
+// One MD step up to its last half kick, which the next step's k_advance applies (kick2) or,
+// at a segment's end, launch_nve_v64.
+void step_sequence(sofia_ctx *c, bool kick2, bool energies) {
+    launch_advance(c, kick2);
+    launch_sort(c, SORT_STEP);
     launch_build_list(c);
-    launch_finish_rebuild(c, true);
-    force_sequence(c, energies);
-    launch_nve_v64(c, true);
-    launch_step_advance(c);
+    if (energies) launch_zero_energies(c);
+    launch_nonbond(c, nb_mode(c), energies, true);
+    launch_bonded_engine(c, energies);
+    launch_shake64(c, energies, true);
 }
 
 int collect_energies(sofia_ctx *c) {
@@ -1594,16 +1614,7 @@ int reference_regrid(sofia_ctx *c) {
         R.cell0 = cell0;
         cell0 += R.ncellT;
     }
-    if (cell0 > c->ncell_cap) {
-        dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep);
-        TRY(dalloc(&c->ccount, cell0));
-        TRY(dalloc(&c->cstart, cell0));
-        TRY(dalloc(&c->cnum, (size_t)27 * cell0));
-        TRY(dalloc(&c->cell_rep, cell0));
-        SOFIA_HIP(hipMemset(c->ccount, 0, sizeof(int32_t) * cell0));
-        SOFIA_HIP(hipMemset(c->cstart, 0, sizeof(int32_t) * cell0));
-        c->ncell_cap = cell0;
-    }
+    TRY(size_cells(c, cell0));
     c->ncell_total = cell0;
     c->n_stencil5 = 0;
     std::vector<int32_t> cnum((size_t)27 * cell0), crep(cell0);
@@ -1664,16 +1675,7 @@ int engine_regrid(sofia_ctx *c) {
         R.cell0 = cell0;
         cell0 += R.ncellT;
     }
-    if (cell0 > c->ncell_cap) {   // finer cells: re-size the per-cell arrays
-        dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep);
-        TRY(dalloc(&c->ccount, cell0));
-        TRY(dalloc(&c->cstart, cell0));
-        TRY(dalloc(&c->cnum, (size_t)27 * cell0));
-        TRY(dalloc(&c->cell_rep, cell0));
-        SOFIA_HIP(hipMemset(c->ccount, 0, sizeof(int32_t) * cell0));
-        SOFIA_HIP(hipMemset(c->cstart, 0, sizeof(int32_t) * cell0));
-        c->ncell_cap = cell0;
-    }
+    TRY(size_cells(c, cell0));
     c->ncell_total = cell0;
     c->n_stencil5 = n5;
     c->dp.rv2 = rv * rv;   // list radius of both build kernels from here on
@@ -1908,10 +1910,7 @@ int sofia_get_engine_config(sofia_ctx *c, int32_t *lanes, int32_t *list_waves,
     if (lanes) *lanes = c->lanes;
     if (list_waves) *list_waves = c->list_waves;
     if (bonded_mode) *bonded_mode = c->bonded_bundles ? 1 : 0;
-    if (record_bytes)
-        *record_bytes = c->p.precision != SOFIA_PREC_MIXED || c->p.coul_flag == SOFIA_COUL_EWALD
-                            ? 0
-                            : ((c->q_by_type && c->ptab && c->lanes != 0) ? 12 : 16);
+    if (record_bytes) *record_bytes = sofia::record_bytes(c);
     if (skin) *skin = c->skin >= 0.0 ? c->skin : std::sqrt(c->p.rv2) - std::sqrt(std::max(c->p.rcut2, c->p.cut_coulsq));
     return SOFIA_OK;
 }
@@ -2060,7 +2059,7 @@ int snapshot_restore(sofia_ctx *c, int32_t overflow) {
 int capture_steps(sofia_ctx *c, hipGraphExec_t *out, int k) {
     hipGraph_t g = nullptr;
     SOFIA_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    for (int s = 0; s < k; ++s) step_sequence(c, false);
+    for (int s = 0; s < k; ++s) step_sequence(c, true, false);
     SOFIA_HIP(hipStreamEndCapture(c->stream, &g));
     // the executable graph is independent of the captured one, which goes at once
     const hipError_t ie = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
@@ -2083,8 +2082,11 @@ int sofia_md_launch(sofia_ctx *c, int32_t nsteps, int32_t use_graph) {
         c->snap_nsteps = nsteps;
         c->snap_graph = use_graph;
     }
-    const int body = nsteps - 1;   // the last step also reduces energies
-    if (use_graph) {
+    // the first step has no half kick left from a step before it, the last one also reduces
+    // energies; the steps between are the captured ones
+    const int body = nsteps - 2;
+    if (nsteps > 1) step_sequence(c, false, false);
+    if (use_graph && body > 0) {
         const int k = c->graph_steps;
         if (!c->graph) TRY(capture_steps(c, &c->graph, 1));
         if (k > 1 && body >= k && !c->graphk) TRY(capture_steps(c, &c->graphk, k));
@@ -2093,9 +2095,10 @@ int sofia_md_launch(sofia_ctx *c, int32_t nsteps, int32_t use_graph) {
             for (; s + k <= body; s += k) SOFIA_HIP(hipGraphLaunch(c->graphk, c->stream));
         for (; s < body; ++s) SOFIA_HIP(hipGraphLaunch(c->graph, c->stream));
     } else {
-        for (int s = 0; s < body; ++s) step_sequence(c, false);
+        for (int s = 0; s < body; ++s) step_sequence(c, true, false);
     }
-    step_sequence(c, true);
+    step_sequence(c, nsteps > 1, true);
+    launch_nve_v64(c, true);
     c->step_h += nsteps;
     return SOFIA_OK;
 }
@@ -2159,21 +2162,15 @@ int sofia_minimize(sofia_ctx *c, int32_t nsteps, double gamma, double max_disp) 
     if (nsteps < 0 || !(gamma > 0.0) || !(max_disp > 0.0)) return fail(SOFIA_E_ARG, "bad minimizer arguments");
     const bool thermo = c->has_thermostat;
     c->has_thermostat = false;
+    launch_zero_forces(c, c->fix, false);
     for (int s = 0; s < nsteps; ++s) {
-        launch_zero_forces(c, c->fix, false);
-        launch_nonbond(c, nb_mode(c), false);
+        launch_nonbond(c, nb_mode(c), false, s > 0);
         launch_bonded_engine(c, false);
         launch_water_bonded(c);
         launch_minimize_step(c, gamma, max_disp);
-        launch_check_neighbor(c, true);
-        launch_cell_reset(c, false);
-        launch_bin(c);
-        launch_cell_scan(c);
-        launch_scatter_sort(c);
-        launch_gather(c, true);
-        launch_remap_topology(c);
+        launch_sort(c, SORT_STEP);
         launch_build_list(c);
-        launch_finish_rebuild(c, true);
+        launch_finish_rebuild(c);
     }
     c->has_thermostat = thermo;
     force_sequence(c, true);
@@ -2292,21 +2289,14 @@ int sofia_profile_step(sofia_ctx *c, int32_t nsteps, int32_t full_rebuild, doubl
         int k = 0;
         auto mark = [&]() { (void)hipEventRecord(ev[k++], c->stream); };
         mark();
-        launch_nve_v64(c, false); mark();
-        launch_nve_x64(c); mark();
+        launch_advance(c, false); mark(); mark(); mark();
         if (full_rebuild) launch_set_rebuild(c, 1);
-        launch_check_neighbor(c, true); mark();
-        launch_cell_reset(c, false); launch_bin(c); launch_cell_scan(c); launch_scatter_sort(c);
-        launch_gather(c, true); launch_remap_topology(c); mark();
-        launch_build_list(c); mark();
-        launch_finish_rebuild(c, true); mark();
-        launch_zero_forces(c, c->fix, false); mark();
-        launch_nonbond(c, nb_mode(c), false); mark();
-        launch_bonded_engine(c, false); mark();
-        if (c->has_thermostat) launch_langevin64(c);
-        mark();
-        launch_shake64(c, false); mark();
-        launch_nve_v64(c, false); launch_step_advance(c); mark();
+        launch_sort(c, SORT_STEP); mark();
+        launch_build_list(c); mark(); mark(); mark();
+        launch_nonbond(c, nb_mode(c), false, true); mark();
+        launch_bonded_engine(c, false); mark(); mark();
+        launch_shake64(c, false, true); mark();
+        launch_nve_v64(c, false); mark();
         rc = sync_check(c);
         for (int p = 0; p < NP && rc == SOFIA_OK; ++p) {
             float ms = 0.0f;

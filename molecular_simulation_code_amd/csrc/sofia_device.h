@@ -156,6 +156,23 @@ __device__ inline void uniform3(uint64_t seed, uint64_t step, uint32_t atom, flo
     for (int d = 0; d < 3; ++d) u[d] = (float)(c[d] >> 8) * (1.0f / 16777216.0f) - 0.5f;
 }
 
+// Position record of the mixed pair kernel: x -> round(x 2^32 / box) mod 2^32 (s = 2^32 / box),
+// the atom type in the low TYPE_BITS of X; q == nullptr: 12-byte records (charges by type).
+constexpr uint32_t TYPE_BITS = 0x3fu;   // types 1..63
+__device__ inline void write_record(int4 *pf, int i, double x, double y, double z, double s,
+                                    uint32_t type, const float *q) {
+    const uint32_t fx = (uint32_t)(unsigned long long)__double2ll_rn(x * s);
+    const int X = (int)((fx & ~TYPE_BITS) | (type & TYPE_BITS));
+    const int Y = (int)(uint32_t)(unsigned long long)__double2ll_rn(y * s);
+    const int Z = (int)(uint32_t)(unsigned long long)__double2ll_rn(z * s);
+    if (q) {
+        pf[i] = make_int4(X, Y, Z, __float_as_int(q[i]));
+    } else {
+        int *p3 = (int *)pf + 3 * (size_t)i;
+        p3[0] = X; p3[1] = Y; p3[2] = Z;
+    }
+}
+
 inline int nblocks(long long n, int b) { return (int)((n + b - 1) / b); }
 
 }  // namespace sofia

@@ -44,6 +44,7 @@ struct RepInfo {
     double gconst;    // noise amplitude * amu2e
     uint64_t seed;
     double chk2;      // engine rebuild threshold on |displacement|^2 (complete-list criterion)
+    double fscale;    // 2^32 / box: coordinate -> fixed-point record of the mixed pair kernel
 };
 
 // Scalars passed by value to every kernel.
@@ -125,8 +126,11 @@ struct sofia_ctx {
 
     // cells
     int32_t *ccount = nullptr, *cstart = nullptr, *cnum = nullptr, *cell_rep = nullptr;
-    int32_t *acell = nullptr, *aslot = nullptr, *perm = nullptr, *tt = nullptr;
-    int32_t *atombin = nullptr, *sorted_ids = nullptr;
+    int32_t *cbin = nullptr;        // binning counters (zero between sorts)
+    int32_t *bucket = nullptr;      // bucket_cap atom ids per cell, in binning order
+    int32_t bucket_cap = 0;
+    size_t bucket_len = 0;
+    int32_t *acell = nullptr, *tt = nullptr, *atombin = nullptr;
 
     // Verlet list
     int32_t *nlist = nullptr, *numneigh = nullptr;
@@ -175,6 +179,7 @@ struct sofia_ctx {
     float4 *ljtab = nullptr;    // (lj1, lj2, lj3, lj4) per type pair
     double4 *lj14 = nullptr;    // (lj14_1..4) per type pair
     double *mass = nullptr;     // per type
+    double4 *mtab = nullptr;    // per type: m, dt/2 kcal2amu / m, sqrt(m), 1/m
     double *bond_k = nullptr, *bond_r0 = nullptr, *angle_k = nullptr, *angle_th0 = nullptr;
     double *tors_k = nullptr, *tors_n = nullptr, *tors_shift = nullptr;
     double *tors_cs = nullptr;  // per torsion type: cos(shift), sin(shift)
@@ -239,24 +244,24 @@ namespace sofia {
 
 // ------------------------------------------------------------------ kernel launchers
 // neighbor build (k_neighbor.hip)
-void launch_cell_reset(sofia_ctx *c, bool all);
-void launch_bin(sofia_ctx *c);
-void launch_cell_scan(sofia_ctx *c);
-void launch_scatter_sort(sofia_ctx *c);
-void launch_gather(sofia_ctx *c, bool engine);
-void launch_remap_topology(sofia_ctx *c);
+// What the sort carries along with the atoms: the drop-in's real*4 state, the engine's FP64
+// state too, or (inside an engine step) also the fixed-point forces already set for the step
+// and the pair kernel's position records.
+enum SortMode { SORT_DROPIN = 0, SORT_ENGINE = 1, SORT_STEP = 2 };
+void launch_sort(sofia_ctx *c, SortMode mode);
 void launch_host_ids(sofia_ctx *c, const int32_t *src, int32_t *dst, size_t items, int width,
                      int nidx);
 void launch_rdf(sofia_ctx *c, int32_t itype, int32_t jtype, double delta, int32_t nbins,
                 uint32_t *hist);
 void launch_build_list(sofia_ctx *c);
 void launch_build_list_engine(sofia_ctx *c);
-void launch_check_neighbor(sofia_ctx *c, bool engine);
+void launch_check_neighbor(sofia_ctx *c);
 void launch_set_rebuild(sofia_ctx *c, int32_t value);
-void launch_finish_rebuild(sofia_ctx *c, bool engine);
+void launch_finish_rebuild(sofia_ctx *c);
 
 // nonbond (k_nonbond.hip): mode 0 = DSF FP64, 1 = DSF mixed, 2 = Ewald real space (FP32)
-void launch_nonbond(sofia_ctx *c, int mode, bool energies);
+// records: the mixed kernel's position records are already up to date
+void launch_nonbond(sofia_ctx *c, int mode, bool energies, bool records = false);
 void launch_count_pairs(sofia_ctx *c, unsigned long long *out);
 
 // bonded (k_bonded.hip)
@@ -266,7 +271,9 @@ void launch_bonded_engine(sofia_ctx *c, bool energies);
 void launch_bonded_dropin(sofia_ctx *c, long long *fout);
 int build_bonded_bundles(sofia_ctx *c);   // host: molecules of the engine's bonded items
 void drop_bonded_bundles(sofia_ctx *c);
-void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd);
+void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records);
+// bytes per position record the mixed pair kernel reads (12 or 16), 0 in the other modes
+int record_bytes(const sofia_ctx *c);
 
 // integration (k_integrate.hip)
 void launch_zero_forces(sofia_ctx *c, long long *f, bool energies);
@@ -282,14 +289,15 @@ void launch_langevin32(sofia_ctx *c, float fric, float gconst, uint64_t seed, ui
 void launch_engine_from32(sofia_ctx *c);
 void launch_engine_to32(sofia_ctx *c);
 void launch_nve_v64(sofia_ctx *c, bool ke);
-void launch_nve_x64(sofia_ctx *c);
+void launch_advance(sofia_ctx *c, bool kick2);
 void launch_langevin64(sofia_ctx *c);
-void launch_shake64(sofia_ctx *c, bool energies);
+// step: the launch also ends the engine step (rebuild flags down, step counters on)
+void launch_shake64(sofia_ctx *c, bool energies, bool step = false);
+void launch_zero_energies(sofia_ctx *c);
 void launch_water_bonded(sofia_ctx *c);
 void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst);
 void launch_type_range(sofia_ctx *c, const float4 *pos, int32_t *bad);
 void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb);
-void launch_step_advance(sofia_ctx *c);
 void launch_step_add(sofia_ctx *c, long long delta);
 void launch_minimize_step(sofia_ctx *c, double gamma, double max_disp);
 

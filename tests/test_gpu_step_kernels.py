@@ -42,3 +42,51 @@ def test_constraints_hold_at_span_and_wavefront_edges(ng, nw):
           flush=True)
     assert err[water].max() < 1e-8
     assert err[~water].max() < 3e-4
+
+
+@pytest.mark.parametrize("crowd", [79, 80, 81, 300])
+def test_sort_of_cells_fuller_than_their_bucket(crowd):
+    """A bucket holds twice the mean occupancy (21 atoms here) and 32 more, rounded up to 16: 80.
+    Cells just below, at and past that, and far past it, sort exactly as the oracle's chains."""
+    host = _host()
+    from oracle import oracle as O
+    s = S.make_system(10, 150, seed=5, params=S.Params(rcut=5.5, cut_coul=5.5, pad=1.0))
+    d = s.derived()
+    rn, nT, nD = O.cell_grid(d["box"], d["rcut"], d["cut_coul"])
+    rng = np.random.default_rng(crowd)
+    cell = np.floor(s.pos / float(rn)).astype(int).clip(0, nD - 1)
+    lone = np.where((cell == 0).all(1))[0]
+    others = rng.permutation(np.setdiff1d(np.arange(s.np), lone))
+    s.pos[others[:crowd - len(lone)]] = rng.uniform(0.05, 0.9 * float(rn), (crowd - len(lone), 3))
+    g = host.SofiaGPU(s)
+    try:
+        tt = g.neighbor_wrapper(0)
+        ott, perm, start, endp, atombin = O.sort_cells(s.pos, s.types, d["box"], rn, nT, nD)
+        st, en, ab, _ = g.get_cells()
+        assert (en - st + 1).max() == crowd
+        assert np.array_equal(tt, ott) and np.array_equal(ab, atombin)
+        assert np.array_equal(st, start) and np.array_equal(en, endp)
+        assert np.array_equal(g.position, s.pos[perm - 1])
+    finally:
+        g.close()
+
+
+@pytest.mark.parametrize("parts", [(1, 1, 1, 1, 1), (2, 3), (1, 4), (3, 2)])
+@pytest.mark.parametrize("graph", [True, False])
+def test_segments_of_any_length_join_bit_for_bit(parts, graph):
+    """A step's last half kick is applied by the next step's first launch inside a segment and
+    by its own launch at a segment's end: five steps in any split are the same five steps."""
+    host = _host()
+    s = S.make_system(8, 1000, seed=17)
+    out = []
+    for split in ((5,), parts):
+        e = host.Engine([host.ReplicaSpec(s, temp=300.0, gamma_ps=1.0, seed=3)])
+        try:
+            e.init()
+            for k in split:
+                e.run(k, use_graph=graph)
+            out.append((e.state()[0], e.energies(), e.steps()))
+        finally:
+            e.close()
+    assert np.array_equal(out[0][0][0], out[1][0][0]) and np.array_equal(out[0][0][1], out[1][0][1])
+    assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
