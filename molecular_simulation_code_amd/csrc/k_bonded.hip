@@ -361,12 +361,12 @@ struct AtomicSink {
 };
 
 // ------------------------------------------------------------------ one thread per item
-template <bool F64POS>
+// The drop-in 1-4 pair, on the real*4 positions.
 __global__ void k_pair14(int32_t items, const int32_t *__restrict__ dl, const float4 *__restrict__ pos4,
-                         const double *__restrict__ xd, const float *__restrict__ q,
-                         const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
-                         const double4 *__restrict__ lj14, DevParams P, int32_t n,
-                         long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
+                         const float *__restrict__ q, const int32_t *__restrict__ rep,
+                         const RepInfo *__restrict__ reps, const double4 *__restrict__ lj14,
+                         DevParams P, int32_t n, long long *__restrict__ fout,
+                         long long *__restrict__ eacc) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = m < items;
     double ec = 0.0, el = 0.0;
@@ -374,96 +374,11 @@ __global__ void k_pair14(int32_t items, const int32_t *__restrict__ dl, const fl
     if (live) {
         const int32_t *it = dl + (size_t)m * 5;
         r = rep[it[0]];
-        pair14_eval<F64POS>(it, pos4, xd, q, reps[r].box, reps[r].ibox, lj14, P, n, ec, el,
-                            AtomicSink{it, fout, n});
+        pair14_eval<false>(it, pos4, nullptr, q, reps[r].box, reps[r].ibox, lj14, P, n, ec, el,
+                           AtomicSink{it, fout, n});
     }
-    if (energies) wave_add(to_efix(ec), live, r, eacc, E_COUL14);
-    if (energies) wave_add(to_efix(el), live, r, eacc, E_POT14);
-}
-
-// Items whose type is <= 0 belong to a rigid water and are evaluated inside the SHAKE kernel.
-__global__ void k_bond(int32_t items, const int32_t *__restrict__ bl, const double *__restrict__ xd,
-                       const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
-                       const double *__restrict__ kb, const double *__restrict__ r0, int32_t n,
-                       long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = m < items && bl[(size_t)m * 3 + 2] >= 1;
-    long long e = 0;
-    int r = 0;
-    if (live) {
-        const int32_t *it = bl + (size_t)m * 3;
-        r = rep[it[0]];
-        e = bond_eval(it, xd, reps[r].box, reps[r].ibox, kb, r0, n, AtomicSink{it, fout, n});
-    }
-    if (energies) wave_add(e, live, r, eacc, E_BOND);
-}
-
-// (types <= 0: rigid-water angles, evaluated inside the SHAKE kernel)
-__global__ void k_angle(int32_t items, const int32_t *__restrict__ al, const double *__restrict__ xd,
-                        const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
-                        const double *__restrict__ ka, const double *__restrict__ th0, int32_t n,
-                        long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = m < items && al[(size_t)m * 4 + 3] >= 1;
-    long long e = 0;
-    int r = 0;
-    if (live) {
-        const int32_t *it = al + (size_t)m * 4;
-        r = rep[it[0]];
-        e = angle_eval(it, xd, reps[r].box, reps[r].ibox, ka, th0, n, AtomicSink{it, fout, n});
-    }
-    if (energies) wave_add(e, live, r, eacc, E_ANGLE);
-}
-
-__global__ void k_torsion(int32_t items, const int32_t *__restrict__ tl, const double *__restrict__ xd,
-                          const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
-                          const double *__restrict__ kk, const double *__restrict__ mult,
-                          const double *__restrict__ shift_deg, const double *__restrict__ shift_cs,
-                          int32_t n, long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = m < items;
-    double e = 0.0;
-    int r = 0;
-    if (live) {
-        const int32_t *it = tl + (size_t)m * 5;
-        r = rep[it[0]];
-        e = torsion_eval(it, xd, reps[r].box, reps[r].ibox, kk, mult, shift_deg, shift_cs, n,
-                         AtomicSink{it, fout, n});
-    }
-    if (energies) wave_add(to_efix(e), live, r, eacc, E_DIHED);
-}
-
-__global__ void k_improper(int32_t items, const int32_t *__restrict__ il, const double *__restrict__ xd,
-                           const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
-                           const double *__restrict__ kk, const double *__restrict__ chi0,
-                           int32_t n, long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = m < items;
-    double e = 0.0;
-    int r = 0;
-    if (live) {
-        const int32_t *it = il + (size_t)m * 5;
-        r = rep[it[0]];
-        e = improper_eval(it, xd, reps[r].box, reps[r].ibox, kk, chi0, n, AtomicSink{it, fout, n});
-    }
-    if (energies) wave_add(to_efix(e), live, r, eacc, E_IMPRO);
-}
-
-__global__ void k_improper_cvff(int32_t items, const int32_t *__restrict__ il,
-                                const double *__restrict__ xd, const int32_t *__restrict__ rep,
-                                const RepInfo *__restrict__ reps, const double *__restrict__ kk,
-                                const int32_t *__restrict__ dn, int32_t n,
-                                long long *__restrict__ fout, long long *__restrict__ eacc, bool energies) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool live = m < items;
-    double e = 0.0;
-    int r = 0;
-    if (live) {
-        const int32_t *it = il + (size_t)m * 5;
-        r = rep[it[0]];
-        e = improper_cvff_eval(it, xd, reps[r].box, reps[r].ibox, kk, dn, n, AtomicSink{it, fout, n});
-    }
-    if (energies) wave_add(to_efix(e), live, r, eacc, E_IMPRO);
+    wave_add(to_efix(ec), live, r, eacc, E_COUL14);
+    wave_add(to_efix(el), live, r, eacc, E_POT14);
 }
 
 // real*4 positions promoted to an FP64 SoA copy, the input of the bonded kernels above
@@ -499,6 +414,73 @@ struct BondedArgs {
     int32_t impro_style;
     int32_t n;
 };
+
+// Every kind in one launch, one thread per item, forces added with global atomics.  A
+// workgroup holds items of one kind (workgroups [0, end[0]) the first kind of ORDER, and so
+// on), so no wavefront runs two kinds' code; the kinds run side by side, where a launch each
+// took the sum of their latencies (five launches, 27 us at 5,000 atoms and 36 at 55,000, most
+// of it launch and FP64 latency).  Longest code first.  Items whose type is <= 0 belong to a
+// rigid water and are evaluated inside the constraint kernel.
+constexpr int ITEM_THREADS = 64;
+struct BondedItems {
+    int32_t items[BK_COUNT];   // per kind, 0 = none
+    int32_t end[BK_COUNT];     // cumulative workgroups, in the kernel's order of kinds
+};
+__device__ __host__ constexpr int bonded_order(int k) {
+    return k == 0 ? BK_TORSION : k == 1 ? BK_IMPRO : k == 2 ? BK_ANGLE : k == 3 ? BK_PAIR14 : BK_BOND;
+}
+
+__global__ void __launch_bounds__(ITEM_THREADS)
+k_bonded_items(BondedItems I, BondedArgs A, DevParams P, long long *__restrict__ fout,
+               long long *__restrict__ eacc, bool energies) {
+    int o = 0;
+    while ((int)blockIdx.x >= I.end[o]) ++o;
+    const int kind = bonded_order(o);
+    const int m = ((int)blockIdx.x - (o ? I.end[o - 1] : 0)) * ITEM_THREADS + (int)threadIdx.x;
+    const int width = bonded_width(kind);
+    const int32_t *it = A.lst[kind] + (size_t)m * width;
+    const bool live = m < I.items[kind] && (kind == BK_PAIR14 || it[width - 1] >= 1);
+    const int r = live ? A.rep[it[0]] : 0;
+    const float boxf = A.reps[r].box, iboxf = A.reps[r].ibox;
+    const double box = boxf, ibox = iboxf;
+    const AtomicSink add{it, fout, A.n};
+    long long e = 0, e2 = 0;
+    int slot = E_BOND;
+    switch (kind) {
+        case BK_PAIR14:
+            slot = E_COUL14;
+            if (live) {
+                double c14, l14;
+                pair14_eval<true>(it, A.pos4, A.xd, A.q, boxf, iboxf, A.lj14, P, A.n, c14, l14, add);
+                e = to_efix(c14);
+                e2 = to_efix(l14);
+            }
+            break;
+        case BK_BOND:
+            if (live) e = bond_eval(it, A.xd, box, ibox, A.bond_k, A.bond_r0, A.n, add);
+            break;
+        case BK_ANGLE:
+            slot = E_ANGLE;
+            if (live) e = angle_eval(it, A.xd, box, ibox, A.angle_k, A.angle_th0, A.n, add);
+            break;
+        case BK_TORSION:
+            slot = E_DIHED;
+            if (live)
+                e = to_efix(torsion_eval(it, A.xd, box, ibox, A.tors_k, A.tors_n, A.tors_shift,
+                                         A.tors_cs, A.n, add));
+            break;
+        default:
+            slot = E_IMPRO;
+            if (live)
+                e = to_efix(A.impro_style == 0
+                                ? improper_eval(it, A.xd, box, ibox, A.impro_k, A.impro_chi0, A.n, add)
+                                : improper_cvff_eval(it, A.xd, box, ibox, A.impro_k, A.impro_dn, A.n, add));
+            break;
+    }
+    if (!energies) return;
+    wave_add(e, live, r, eacc, slot);
+    if (kind == BK_PAIR14) wave_add(e2, live, r, eacc, E_POT14);
+}
 
 __global__ void __launch_bounds__(BUNDLE_THREADS)
 k_bonded_bundles(const int32_t *__restrict__ tstart, const int2 *__restrict__ terms,
@@ -582,10 +564,49 @@ void launch_correct(sofia_ctx *c, int which, long long *fout) {
 
 void launch_pair14(sofia_ctx *c, long long *fout) {
     if (!c->nd) return;
-    hipLaunchKernelGGL(k_pair14<false>, dim3(nblocks(c->nd, 256)), dim3(256), 0, c->stream, c->nd,
-                       c->dihedlist, c->a.pos4, c->a.xd, c->a.q, c->rep, c->reps_d, c->lj14, c->dp,
-                       c->N, fout, c->eacc, true);
+    hipLaunchKernelGGL(k_pair14, dim3(nblocks(c->nd, 256)), dim3(256), 0, c->stream, c->nd,
+                       c->dihedlist, c->a.pos4, c->a.q, c->rep, c->reps_d, c->lj14, c->dp, c->N,
+                       fout, c->eacc);
 }
+
+namespace {
+
+BondedArgs bonded_args(const sofia_ctx *c, const double *xd, const int32_t *bonds, const int32_t *angles) {
+    BondedArgs A{};
+    A.lst[BK_PAIR14] = c->dihedlist;
+    A.lst[BK_BOND] = bonds;
+    A.lst[BK_ANGLE] = angles;
+    A.lst[BK_TORSION] = c->torsions;
+    A.lst[BK_IMPRO] = c->improlist;
+    A.pos4 = c->a.pos4; A.xd = xd; A.q = c->a.q; A.rep = c->rep; A.reps = c->reps_d;
+    A.lj14 = c->lj14;
+    A.bond_k = c->bond_k; A.bond_r0 = c->bond_r0; A.angle_k = c->angle_k; A.angle_th0 = c->angle_th0;
+    A.tors_k = c->tors_k; A.tors_n = c->tors_n; A.tors_shift = c->tors_shift; A.tors_cs = c->tors_cs;
+    A.impro_k = c->impro_k; A.impro_chi0 = c->impro_chi0; A.impro_dn = c->impro_dn;
+    A.impro_style = c->impro_style;
+    A.n = c->N;
+    return A;
+}
+
+void launch_items(sofia_ctx *c, const BondedArgs &A, int n14, int nb, int na, long long *fout,
+                  bool energies) {
+    BondedItems I{};
+    I.items[BK_PAIR14] = n14;
+    I.items[BK_BOND] = c->bond_k ? nb : 0;
+    I.items[BK_ANGLE] = c->angle_k ? na : 0;
+    I.items[BK_TORSION] = c->tors_k ? c->ntor : 0;
+    I.items[BK_IMPRO] = c->nimp;
+    int total = 0;
+    for (int o = 0; o < BK_COUNT; ++o) {
+        total += nblocks(I.items[bonded_order(o)], ITEM_THREADS);
+        I.end[o] = total;
+    }
+    if (total)
+        hipLaunchKernelGGL(k_bonded_items, dim3(total), dim3(ITEM_THREADS), 0, c->stream, I, A, c->dp,
+                           fout, c->eacc, energies);
+}
+
+}  // namespace
 
 // The drop-in form of the bonded terms: every bond, angle, torsion and improper of the
 // uploaded lists (rigid waters included, as the reference's bond_harmonic / angle_harmonic
@@ -595,73 +616,21 @@ void launch_bonded_dropin(sofia_ctx *c, long long *fout) {
     const int n = c->N;
     double *xd = c->b.xd;
     hipLaunchKernelGGL(k_pos_to_xd, dim3(nblocks(n, 256)), dim3(256), 0, c->stream, n, c->a.pos4, xd);
-    if (c->nb && c->bond_k)
-        hipLaunchKernelGGL(k_bond, dim3(nblocks(c->nb, 256)), dim3(256), 0, c->stream, c->nb,
-                           c->bondlist, xd, c->rep, c->reps_d, c->bond_k, c->bond_r0, n, fout, c->eacc, true);
-    if (c->na && c->angle_k)
-        hipLaunchKernelGGL(k_angle, dim3(nblocks(c->na, 256)), dim3(256), 0, c->stream, c->na,
-                           c->anglelist, xd, c->rep, c->reps_d, c->angle_k, c->angle_th0, n, fout,
-                           c->eacc, true);
-    if (c->ntor && c->tors_k)
-        hipLaunchKernelGGL(k_torsion, dim3(nblocks(c->ntor, 256)), dim3(256), 0, c->stream, c->ntor,
-                           c->torsions, xd, c->rep, c->reps_d, c->tors_k, c->tors_n, c->tors_shift,
-                           c->tors_cs, n, fout, c->eacc, true);
-    if (c->nimp && c->impro_style == 0)
-        hipLaunchKernelGGL(k_improper, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream, c->nimp,
-                           c->improlist, xd, c->rep, c->reps_d, c->impro_k, c->impro_chi0, n, fout,
-                           c->eacc, true);
-    else if (c->nimp)
-        hipLaunchKernelGGL(k_improper_cvff, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream,
-                           c->nimp, c->improlist, xd, c->rep, c->reps_d, c->impro_k, c->impro_dn, n,
-                           fout, c->eacc, true);
+    launch_items(c, bonded_args(c, xd, c->bondlist, c->anglelist), 0, c->nb, c->na, fout, true);
 }
 
 void launch_bonded_engine(sofia_ctx *c, bool energies) {
-    const int n = c->N;
+    // with the rigid waters fused into the constraint kernel, the remaining items only
+    const BondedArgs A = bonded_args(c, c->a.xd, c->water_split ? c->ebond : c->bondlist,
+                                     c->water_split ? c->eangle : c->anglelist);
     if (c->bonded_bundles && c->nbundle > 0) {
-        BondedArgs A{};
-        A.lst[BK_PAIR14] = c->dihedlist;
-        A.lst[BK_BOND] = c->water_split ? c->ebond : c->bondlist;
-        A.lst[BK_ANGLE] = c->water_split ? c->eangle : c->anglelist;
-        A.lst[BK_TORSION] = c->torsions;
-        A.lst[BK_IMPRO] = c->improlist;
-        A.pos4 = c->a.pos4; A.xd = c->a.xd; A.q = c->a.q; A.rep = c->rep; A.reps = c->reps_d;
-        A.lj14 = c->lj14;
-        A.bond_k = c->bond_k; A.bond_r0 = c->bond_r0; A.angle_k = c->angle_k; A.angle_th0 = c->angle_th0;
-        A.tors_k = c->tors_k; A.tors_n = c->tors_n; A.tors_shift = c->tors_shift; A.tors_cs = c->tors_cs;
-        A.impro_k = c->impro_k; A.impro_chi0 = c->impro_chi0; A.impro_dn = c->impro_dn;
-        A.impro_style = c->impro_style;
-        A.n = n;
-        hipLaunchKernelGGL(k_bonded_bundles, dim3(c->nbundle), dim3(BUNDLE_THREADS), 0, c->stream, c->bund_tstart,
-                           c->bund_terms, c->bund_sstart, c->bund_slots, A, c->dp, c->fix, c->eacc, energies);
+        hipLaunchKernelGGL(k_bonded_bundles, dim3(c->nbundle), dim3(BUNDLE_THREADS), 0, c->stream,
+                           c->bund_tstart, c->bund_terms, c->bund_sstart, c->bund_slots, A, c->dp,
+                           c->fix, c->eacc, energies);
         return;
     }
-    if (c->nd)
-        hipLaunchKernelGGL(k_pair14<true>, dim3(nblocks(c->nd, 256)), dim3(256), 0, c->stream, c->nd,
-                           c->dihedlist, c->a.pos4, c->a.xd, c->a.q, c->rep, c->reps_d, c->lj14,
-                           c->dp, n, c->fix, c->eacc, energies);
-    // with the rigid waters fused into SHAKE, the remaining items only
-    const int nb = c->water_split ? c->nbe : c->nb, na = c->water_split ? c->nae : c->na;
-    const int32_t *bl = c->water_split ? c->ebond : c->bondlist;
-    const int32_t *al = c->water_split ? c->eangle : c->anglelist;
-    if (nb && c->bond_k)
-        hipLaunchKernelGGL(k_bond, dim3(nblocks(nb, 256)), dim3(256), 0, c->stream, nb, bl, c->a.xd,
-                           c->rep, c->reps_d, c->bond_k, c->bond_r0, n, c->fix, c->eacc, energies);
-    if (na && c->angle_k)
-        hipLaunchKernelGGL(k_angle, dim3(nblocks(na, 256)), dim3(256), 0, c->stream, na, al, c->a.xd,
-                           c->rep, c->reps_d, c->angle_k, c->angle_th0, n, c->fix, c->eacc, energies);
-    if (c->ntor && c->tors_k)
-        hipLaunchKernelGGL(k_torsion, dim3(nblocks(c->ntor, 256)), dim3(256), 0, c->stream, c->ntor,
-                           c->torsions, c->a.xd, c->rep, c->reps_d, c->tors_k, c->tors_n,
-                           c->tors_shift, c->tors_cs, n, c->fix, c->eacc, energies);
-    if (c->nimp && c->impro_style == 0)
-        hipLaunchKernelGGL(k_improper, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream, c->nimp,
-                           c->improlist, c->a.xd, c->rep, c->reps_d, c->impro_k, c->impro_chi0, n,
-                           c->fix, c->eacc, energies);
-    else if (c->nimp)
-        hipLaunchKernelGGL(k_improper_cvff, dim3(nblocks(c->nimp, 256)), dim3(256), 0, c->stream,
-                           c->nimp, c->improlist, c->a.xd, c->rep, c->reps_d, c->impro_k,
-                           c->impro_dn, n, c->fix, c->eacc, energies);
+    launch_items(c, A, c->nd, c->water_split ? c->nbe : c->nb, c->water_split ? c->nae : c->na,
+                 c->fix, energies);
 }
 
 }  // namespace sofia
