@@ -490,7 +490,7 @@ k_dsf_compact(int32_t n, const int4 *__restrict__ pf,
 
 template <int L>
 void launch_lanes(sofia_ctx *c, bool energies, float *ff32, bool qt) {
-    const int block = c->block;
+    const int block = mixed_block(c, energies);
     const long long threads = (long long)c->N * L;
     const int grid = (int)((threads + block - 1) / block);
     const int nt2 = c->dp.ntypes * c->dp.ntypes;
@@ -528,16 +528,16 @@ void launch_compact(sofia_ctx *c, bool energies, float *ff32) {
 // kernel reads 16-byte records)
 int record_bytes(const sofia_ctx *c) {
     if (c->p.precision != SOFIA_PREC_MIXED || c->p.coul_flag == SOFIA_COUL_EWALD) return 0;
-    return (c->q_by_type && c->ptab && c->lanes != 0) ? 12 : 16;
+    return (c->q_by_type && c->ptab && mixed_lanes(c) != 0) ? 12 : 16;
 }
 
 void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records) {
-    const bool qt = c->q_by_type && c->ptab && c->lanes != 0;
+    const bool qt = c->q_by_type && c->ptab && mixed_lanes(c) != 0;
     if (!records)
         hipLaunchKernelGGL(k_fixpos, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N,
                            from_xd ? c->a.xd : nullptr, c->a.pos4, qt ? nullptr : c->a.q, c->rep,
                            c->reps_d, c->pfix);
-    switch (c->lanes) {
+    switch (mixed_lanes(c, energies)) {
         case 0: launch_compact(c, energies, ff32); break;
         case 4: launch_lanes<4>(c, energies, ff32, qt); break;
         case 8: launch_lanes<8>(c, energies, ff32, qt); break;

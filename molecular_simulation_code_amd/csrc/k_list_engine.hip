@@ -210,10 +210,10 @@ inline int nblk(int n, int b) { return (n + b - 1) / b; }
 void launch_build_list_engine(sofia_ctx *c) {
     const float rv2 = (float)c->dp.rv2;
     const float rv = std::sqrt(rv2);
-    // at most 4 workgroups per CU fit (64 KiB of staged candidates each); a multiple of 8
-    const int grid = std::min(c->ncell_total, 2048);
+    // two workgroups of 16 wavefronts fit a CU (64 KiB of staged candidates each): more would
+    // only lengthen the launch of a step that rebuilds nothing
 #define LBE(W)                                                                                   \
-    hipLaunchKernelGGL(k_build_engine<W>, dim3(grid), dim3(W * 64), 0, c->stream,                \
+    hipLaunchKernelGGL(k_build_engine<W>, dim3(std::min(c->ncell_total, 8192 / W)), dim3(W * 64), 0, c->stream,                \
                        c->ncell_total, c->a.pos4, c->a.num3, c->a.spec, c->cstart, c->ccount,    \
                        c->cell_rep, c->reps_d, c->rebuild, c->rebuild + c->nrep, rv, rv2,        \
                        c->neigh_alloc, c->nlist, c->numneigh, c->maxcnt)

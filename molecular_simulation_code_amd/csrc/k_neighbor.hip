@@ -335,7 +335,7 @@ k_build_list(const float4 *__restrict__ pos4, const int32_t *__restrict__ num3,
     const int wave = tid >> 6, lane = tid & 63;
     const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     const int i0 = cstart[c], ni = ccount[c];
-    for (int ii = wave; ii < ni; ii += WAVES) {
+    for (int ii = blockIdx.y * WAVES + wave; ii < ni; ii += gridDim.y * WAVES) {
         const int i = i0 + ii;
         const float4 xi = pos4[i];
         const int n3 = num3[i];
@@ -483,9 +483,12 @@ void launch_host_ids(sofia_ctx *c, const int32_t *src, int32_t *dst, size_t item
 void launch_build_list(sofia_ctx *c) {
     if (c->n_stencil5 > 0) launch_build_list_engine(c);
     if (c->n_stencil5 == c->nrep) return;
+    // few cells (the reference's are a cutoff wide: 125 in a 13,500-atom box) leave most of the
+    // chip idle: their atoms go to several workgroups, each staging the stencil for itself
     const int w = c->list_waves;
+    const int parts = std::max(1, std::min(8, 1024 / c->ncell_total));
 #define LB(W)                                                                                    \
-    hipLaunchKernelGGL(k_build_list<W>, dim3(c->ncell_total), dim3(W * 64), 0, c->stream,       \
+    hipLaunchKernelGGL(k_build_list<W>, dim3(c->ncell_total, parts), dim3(W * 64), 0, c->stream, \
                        c->a.pos4, c->a.num3, c->a.spec, c->cstart, c->ccount, c->cnum,            \
                        c->cell_rep, c->reps_d, c->rebuild, c->dp.rv2, c->neigh_alloc, c->nlist,   \
                        c->numneigh, c->maxcnt)

@@ -229,7 +229,7 @@ k_nonbond(int32_t n, const float4 *__restrict__ pos4, const float *__restrict__ 
 
 template <int L, int MODE>
 void launch_t(sofia_ctx *c, bool energies, float *ff32) {
-    const int block = std::min(c->block, 256);   // this kernel's launch bound
+    const int block = c->block > 0 ? std::min(c->block, 256) : 256;   // this kernel's launch bound
     const long long threads = (long long)c->N * L;
     const int grid = (int)((threads + block - 1) / block);
     const int nt2 = c->dp.ntypes * c->dp.ntypes;
@@ -247,7 +247,7 @@ void launch_t(sofia_ctx *c, bool energies, float *ff32) {
 
 template <int MODE>
 void launch_mode(sofia_ctx *c, bool energies, float *ff32) {
-    switch (c->lanes) {
+    switch (ordered_lanes(c)) {
         case 4: launch_t<4, MODE>(c, energies, ff32); break;
         case 8: launch_t<8, MODE>(c, energies, ff32); break;
         case 32: launch_t<32, MODE>(c, energies, ff32); break;

@@ -1907,7 +1907,7 @@ int sofia_get_nlist_replica(sofia_ctx *c, int32_t rep, int32_t *nlist, int32_t *
 int sofia_get_engine_config(sofia_ctx *c, int32_t *lanes, int32_t *list_waves,
                             int32_t *bonded_mode, int32_t *record_bytes, double *skin) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
-    if (lanes) *lanes = c->lanes;
+    if (lanes) *lanes = nb_mode(c) == 1 ? mixed_lanes(c) : ordered_lanes(c);
     if (list_waves) *list_waves = c->list_waves;
     if (bonded_mode) *bonded_mode = c->bonded_bundles ? 1 : 0;
     if (record_bytes) *record_bytes = sofia::record_bytes(c);

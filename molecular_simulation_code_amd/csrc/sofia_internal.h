@@ -171,7 +171,9 @@ struct sofia_ctx {
     // engine bonded bundles (k_bonded_bundles): per bundle the ranges of its term and atom-slot
     // records; nbundle = 0 runs the per-kind kernels instead
     int32_t nbundle = 0;
-    bool bonded_bundles = false;   // run the bundles (tuning choice) rather than per-kind kernels
+    // run the bundles (tuning choice) rather than one thread per item: 10 against 11 us at
+    // 5,000 atoms, 11 / 17 at 55,000, 21 / 47 at 264,000, 16 / 39 at 204,000 (1,200 glycines)
+    bool bonded_bundles = true;
     int32_t *bund_tstart = nullptr, *bund_sstart = nullptr, *bund_slots = nullptr;
     int2 *bund_terms = nullptr;
 
@@ -207,10 +209,9 @@ struct sofia_ctx {
     double skin = -1.0;          // engine skin (A); < 0: the reference's pad
     uint64_t *step_d = nullptr;  // per-replica step counters (Langevin key)
     uint64_t step_h = 0;
-    // block: threads per workgroup of the mixed pair kernel.  Each workgroup stages the
-    // DSF table (16 KB) and the type-pair table in LDS, so fewer, larger workgroups spend
-    // less of the load path on it (1024 against 256: -4.8 % per launch on the batched mix)
-    int lanes = 16, block = 1024, list_waves = 4;
+    // lanes per atom of the pair kernels and threads per workgroup of the mixed one; < 0 and 0
+    // until the caller tunes them: chosen by kernel and size (mixed_lanes and its neighbours)
+    int lanes = -1, block = 0, list_waves = 16;
     hipGraphExec_t graph = nullptr;    // one MD step
     hipGraphExec_t graphk = nullptr;   // graph_steps MD steps
     int32_t graph_steps = 1;
@@ -309,6 +310,30 @@ int cluster_greatest(sofia_ctx *c, double denscut, int32_t densmin, int32_t *tot
 int cluster_greatest_noalloc(int32_t n, const double *x, const int32_t *gid, const int32_t *mol,
                              int32_t nmol, float box, double denscut, int32_t densmin,
                              int32_t *out, hipStream_t s);
+
+// Lanes per atom of the mixed pair kernel while the caller has not tuned them: its exact sums
+// do not depend on them.  Small systems need more lanes to spread over the chip (one launch,
+// 5,000 atoms: 12.7 us at 64 lanes, 13.6 at 32, 15.8 at 16), large ones fewer shuffles and
+// idle row tails (55,000: 76 / 64 / 60; 264,000: 433 / 353 / 321).  The energy sums lengthen
+// the tail of every lane, so launches with energies turn to 16 lanes earlier (a drop-in call,
+// 31,000 atoms: 371 us at 32, 346 at 16; 3,000 atoms: 133 / 150).
+inline int mixed_lanes(const sofia_ctx *c, bool energies = false) {
+    if (c->lanes >= 0) return c->lanes;
+    if (energies) return c->N < 6000 ? 32 : 16;
+    return c->N < 12000 ? 64 : (c->N < 40000 ? 32 : 16);
+}
+// The FP64 and Ewald kernels sum in floating point, in an order set by the lanes: one value
+// for every size, so that a replica's last bits do not depend on what it is batched with.
+inline int ordered_lanes(const sofia_ctx *c) { return c->lanes >= 0 ? c->lanes : 16; }
+// Threads per workgroup of the mixed pair kernel: each workgroup stages the DSF table (16 KB)
+// and the type-pair tables in LDS, so large workgroups spend less of the load path on it
+// (-4.8 % at 1,280,000 atoms), but a grid of few of them leaves compute units idle (5,000
+// atoms at 16 lanes: 22 us in 1024-thread workgroups, 16.5 in 256; 55,000: 65 / 60).
+inline int mixed_block(const sofia_ctx *c, bool energies) {
+    if (c->block > 0) return c->block;
+    if (energies) return 512;   // two tables to stage
+    return (long long)c->N * mixed_lanes(c) / 1024 < 1024 ? 256 : 1024;
+}
 
 // error helpers (sofia_api.cpp)
 int fail(int code, const std::string &msg);

@@ -90,3 +90,29 @@ def test_segments_of_any_length_join_bit_for_bit(parts, graph):
             e.close()
     assert np.array_equal(out[0][0][0], out[1][0][0]) and np.array_equal(out[0][0][1], out[1][0][1])
     assert np.array_equal(out[0][1], out[1][1]) and np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("nw", [1970, 2030, 3980, 4030, 13300, 13400])
+def test_default_lanes_by_size_keep_the_mixed_forces(nw):
+    """Untuned contexts pick the mixed kernel's lanes and workgroup by size (lines at 6,000,
+    12,000 and 40,000 atoms): forces equal those of the explicit 16-lane layout bit for bit."""
+    host = _host()
+    s = S.make_system(3, nw, seed=nw)
+    outs = []
+    for tuned in (False, True):
+        g = host.SofiaGPU(s.copy(), precision=host.PREC_MIXED)
+        e = host.Engine([host.ReplicaSpec(s, temp=300.0, gamma_ps=1.0, seed=3)])
+        try:
+            if tuned:
+                g.set_tuning(16, 1024, 4)
+                e.set_tuning(16, 1024, 4)
+            g.neighbor_wrapper(0)
+            g.lj_cut_coul_dsf_nonewton_mixed(0)
+            e.init()
+            e.run(3)
+            outs.append((g.ff64.copy(), e.state()[0][0], e.forces()[0]))
+        finally:
+            g.close()
+            e.close()
+    for a, b in zip(*outs):
+        assert np.array_equal(a, b)
