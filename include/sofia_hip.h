@@ -139,6 +139,10 @@ int sofia_get_state(sofia_ctx *ctx, sofia_ainfo *pos, sofia_coords *v, int32_t *
 /* FP64 positions/velocities of the engine (x, y, z interleaved per atom), may be NULL */
 int sofia_get_state_f64(sofia_ctx *ctx, double *x, double *v);
 int sofia_put_state_f64(sofia_ctx *ctx, const double *x, const double *v);
+/* Positions, velocities and the forces of sofia_get_forces_f64, each optional, with every
+ * replica's atoms in global-id order, re-ordered on the device.  *ordered is 0, and nothing is
+ * written, when some replica's global ids are not a permutation of 1..natoms. */
+int sofia_get_ordered_f64(sofia_ctx *ctx, double *x, double *v, double *f, int32_t *ordered);
 /* drx/dry/drz displacement accumulators since the last list build */
 int sofia_get_displacement(sofia_ctx *ctx, float *drx, float *dry, float *drz);
 int sofia_put_displacement(sofia_ctx *ctx, const float *drx, const float *dry, const float *drz);

@@ -71,6 +71,7 @@ SIGNATURES = {
     "sofia_get_state": [_vp] * 4,
     "sofia_get_state_f64": [_vp] * 3,
     "sofia_put_state_f64": [_vp] * 3,
+    "sofia_get_ordered_f64": [_vp] * 5,
     "sofia_get_displacement": [_vp] * 4,
     "sofia_put_displacement": [_vp] * 4,
     "sofia_host_alloc": [C.c_size_t, _vp],

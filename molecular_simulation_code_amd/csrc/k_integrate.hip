@@ -18,6 +18,67 @@ __global__ void k_zero(int32_t n3, long long *__restrict__ f, int32_t ne, long l
     if (e && i < ne) e[i] = 0;
 }
 
+__global__ void k_zero2(int32_t n3, long long *__restrict__ a, long long *__restrict__ b) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n3) {
+        a[i] = 0;
+        b[i] = 0;
+    }
+}
+
+// The ESPREAD copies of every energy slot summed (16 lanes a slot) and the device's flags, all
+// written to the host's page-locked words; the copies (and the solver's flags, whose engine
+// form stays up until the lists are set up again, on request) are cleared on the way.
+// A drop-in call used to copy the raw copies (26 KB) and each flag on their own.
+__global__ void k_report(int32_t slots, long long *__restrict__ eacc, int32_t *__restrict__ shake_err,
+                         int32_t *__restrict__ shake_iters, const int32_t *__restrict__ maxcnt,
+                         HostWords *__restrict__ hw, long long *__restrict__ hw_e, bool clear_shake) {
+    static_assert(ESPREAD == 16, "one lane per copy");
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int slot = t / ESPREAD;
+    long long v = 0;
+    if (slot < slots) {
+        long long *p = &eacc[(size_t)t * ECOPY];
+        v = *p;
+        *p = 0;
+    }
+#pragma unroll
+    for (int off = ESPREAD / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if (slot < slots && t % ESPREAD == 0) hw_e[slot] = v;
+    if (t == 0) {
+        hw->shake_err = *shake_err;
+        hw->shake_iters = *shake_iters;
+        hw->maxcnt = *maxcnt;
+        if (clear_shake) {
+            *shake_err = 0;
+            *shake_iters = 0;
+        }
+    }
+}
+
+// x | y | z of src (and FIX_INV fix) as x, y, z rows; with gid, the row of an atom is its global
+// id's place within its replica (ids a permutation of 1..natom).
+__global__ void k_soa_to_aos(int32_t n, const double *__restrict__ src, const long long *__restrict__ fix,
+                             const int32_t *__restrict__ gid, const int32_t *__restrict__ rep,
+                             const RepInfo *__restrict__ reps, double *__restrict__ dst) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const size_t row = gid ? (size_t)(reps[rep[i]].atom0 + gid[i] - 1) : (size_t)i;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const size_t o = (size_t)c * n + i;
+        // FIX_INV is a power of two: the product is exact, the sum the one k_nve_v64 forms
+        dst[3 * row + c] = fix ? src[o] + (double)fix[o] * FIX_INV : src[o];
+    }
+}
+
+__global__ void k_aos_to_soa(int32_t n, const double *__restrict__ src, double *__restrict__ dst) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) dst[(size_t)c * n + i] = src[3 * (size_t)i + c];
+}
+
 __global__ void k_fix_to_aos(int32_t n, const long long *__restrict__ f, float *__restrict__ out) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -917,14 +978,34 @@ __global__ void k_merge_forces(int32_t n, float *__restrict__ ff, const long lon
 // Atom types (the int bits of pos.w) outside 1..ntypes set *bad; any lane that finds one
 // writes the same value, so a plain store suffices.
 __global__ void k_type_range(int32_t n, const float4 *__restrict__ pos, int32_t ntypes,
-                             int32_t *__restrict__ bad) {
+                             int32_t *__restrict__ bad, HostWords *__restrict__ hw) {
     const int stride = gridDim.x * blockDim.x;
     bool out = false;
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
         const int t = __float_as_int(pos[k].w);
         out |= (t < 1) | (t > ntypes);
     }
-    if (__ballot(out) && __lane_id() == 0) *bad = 1;
+    if (__ballot(out) && __lane_id() == 0) {
+        *bad = 1;
+        hw->type_err = 1;
+    }
+}
+
+// An upload whose types are all in range goes from the staging set into the state: positions,
+// and v / q / gid where given.
+__global__ void k_put_state(int32_t n, const int32_t *__restrict__ bad, AtomArrays src, AtomArrays dst,
+                            bool v, bool q, bool gid) {
+    if (*bad) return;
+    const int stride = gridDim.x * blockDim.x;
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
+        dst.pos4[k] = src.pos4[k];
+        if (q) dst.q[k] = src.q[k];
+        if (gid) dst.gid[k] = src.gid[k];
+        if (v) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) dst.v32[(size_t)d * n + k] = src.v32[(size_t)d * n + k];
+        }
+    }
 }
 
 // The fused rigid-water bonded terms alone (steps that run no SHAKE: the minimiser).
@@ -994,6 +1075,7 @@ __global__ void k_step_add(int32_t nrep, uint64_t *step, long long delta) {
 }  // namespace
 
 void launch_zero_forces(sofia_ctx *c, long long *f, bool energies) {
+    if (energies) c->eacc_zero = false;
     const int n3 = 3 * c->N, ne = (int)eacc_len(c->nrep);
     hipLaunchKernelGGL(k_zero, dim3(nblocks(n3 > ne ? n3 : ne, 256)), dim3(256), 0, c->stream, n3, f,
                        ne, energies ? c->eacc : nullptr);
@@ -1076,7 +1158,11 @@ void launch_advance(sofia_ctx *c, bool kick2) {
     else go(k_advance<false>);
 }
 
+// Energy sums start from zero; skipped where the last report left them so.
 void launch_zero_energies(sofia_ctx *c) {
+    const bool zero = c->eacc_zero;
+    c->eacc_zero = false;
+    if (zero) return;
     const int ne = (int)eacc_len(c->nrep);
     hipLaunchKernelGGL(k_zero, dim3(nblocks(ne, 256)), dim3(256), 0, c->stream, ne, c->eacc, 0,
                        (long long *)nullptr);
@@ -1121,9 +1207,32 @@ void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const 
                        f14, fb);
 }
 
-void launch_type_range(sofia_ctx *c, const float4 *pos, int32_t *bad) {
-    hipLaunchKernelGGL(k_type_range, dim3(std::min(nblocks(c->N, 256), 1024)), dim3(256), 0,
-                       c->stream, c->N, pos, c->p.ntypes, bad);
+void launch_put_state(sofia_ctx *c, bool v, bool q, bool gid) {
+    const int grid = std::min(nblocks(c->N, 256), 1024);
+    hipLaunchKernelGGL(k_type_range, dim3(grid), dim3(256), 0, c->stream, c->N, c->b.pos4, c->p.ntypes,
+                       c->type_err, c->hw);
+    hipLaunchKernelGGL(k_put_state, dim3(grid), dim3(256), 0, c->stream, c->N, c->type_err, c->b, c->a,
+                       v, q, gid);
+}
+
+void launch_report(sofia_ctx *c, bool clear_shake) {
+    const int slots = c->nrep * NE;
+    hipLaunchKernelGGL(k_report, dim3(nblocks((long long)slots * ESPREAD, 256)), dim3(256), 0, c->stream,
+                       slots, c->eacc, c->shake_err, c->shake_iters, c->maxcnt, c->hw, c->hw_e, clear_shake);
+    c->eacc_zero = true;
+}
+
+void launch_zero2(sofia_ctx *c, long long *a, long long *b) {
+    hipLaunchKernelGGL(k_zero2, dim3(nblocks(3LL * c->N, 256)), dim3(256), 0, c->stream, 3 * c->N, a, b);
+}
+
+void launch_soa_to_aos(sofia_ctx *c, const double *src, const long long *fix, const int32_t *gid, double *dst) {
+    hipLaunchKernelGGL(k_soa_to_aos, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N, src, fix,
+                       gid, c->rep, c->reps_d, dst);
+}
+
+void launch_aos_to_soa(sofia_ctx *c, const double *src, double *dst) {
+    hipLaunchKernelGGL(k_aos_to_soa, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N, src, dst);
 }
 
 void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst) {
@@ -1133,6 +1242,7 @@ void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst) {
 
 void launch_water_bonded(sofia_ctx *c) {
     if (!c->ns || !c->water_split) return;
+    c->eacc_zero = false;
     hipLaunchKernelGGL(k_water_bonded, dim3(nblocks(c->ns, 128)), dim3(128), 0, c->stream, c->ns,
                        c->shake_num, shake_args(c), c->eacc);
 }

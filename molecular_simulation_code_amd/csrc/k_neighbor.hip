@@ -392,14 +392,16 @@ k_build_list(const float4 *__restrict__ pos4, const int32_t *__restrict__ num3,
     }
 }
 
-__global__ void k_check32(int32_t n, const int32_t *__restrict__ rep, const float *__restrict__ dr,
-                          double rvrc2, int32_t *__restrict__ rebuild, int32_t *__restrict__ any) {
+__global__ void k_check32(int32_t n, const float *__restrict__ dr,
+                          double rvrc2, HostWords *__restrict__ hw) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float x = dr[i], y = dr[(size_t)n + i], z = dr[2 * (size_t)n + i];
-    const double d2 = (double)((x * x + y * y) + z * z);
-    // the first atom to flag its replica also raises `any`
-    if (d2 >= rvrc2 && atomicOr(&rebuild[rep[i]], 1) == 0) atomicOr(any, 1);
+    bool moved = false;
+    if (i < n) {
+        const float x = dr[i], y = dr[(size_t)n + i], z = dr[2 * (size_t)n + i];
+        moved = (double)((x * x + y * y) + z * z) >= rvrc2;
+    }
+    // any atom of any replica: every wavefront that writes, writes the same
+    if (__ballot(moved) && (threadIdx.x & 63) == 0) hw->moved = 1;
 }
 
 // rebuild[0..nrep) and `any` = rebuild[nrep] to value
@@ -415,6 +417,21 @@ __global__ void k_finish(int32_t nrep, int32_t *__restrict__ rebuild, int32_t *_
         rebuild[r] = 0;
     }
     if (r == nrep) rebuild[r] = 0;   // any
+}
+
+// The end of a rebuild: the largest count to the host; if the lists fit, k_finish's books.
+__global__ void k_list_done(int32_t nrep, int32_t *__restrict__ rebuild, int32_t *__restrict__ nbuilds,
+                            const int32_t *__restrict__ maxcnt, int32_t na, HostWords *__restrict__ hw,
+                            int32_t n, const int32_t *__restrict__ tt, const int32_t *__restrict__ rep,
+                            const RepInfo *__restrict__ reps, int32_t *__restrict__ local) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int mx = *maxcnt;
+    if (t == 0) hw->maxcnt = mx;
+    if (mx <= na && t <= nrep) {
+        if (t < nrep && rebuild[t]) nbuilds[t] += 1;
+        rebuild[t] = 0;   // [nrep] is `any`
+    }
+    if (local && t < n) local[t] = tt[t] - reps[rep[t]].atom0 + 1;
 }
 
 inline int nblk(int n, int b) { return (n + b - 1) / b; }
@@ -500,8 +517,8 @@ void launch_build_list(sofia_ctx *c) {
 }
 
 void launch_check_neighbor(sofia_ctx *c) {
-    hipLaunchKernelGGL(k_check32, dim3(nblk(c->N, 256)), dim3(256), 0, c->stream, c->N, c->rep,
-                       c->dr32, c->dp.rvrc2, c->rebuild, c->rebuild + c->nrep);
+    hipLaunchKernelGGL(k_check32, dim3(nblk(c->N, 256)), dim3(256), 0, c->stream, c->N, c->dr32,
+                       c->dp.rvrc2, c->hw);
 }
 
 void launch_set_rebuild(sofia_ctx *c, int32_t value) {
@@ -512,6 +529,13 @@ void launch_set_rebuild(sofia_ctx *c, int32_t value) {
 void launch_finish_rebuild(sofia_ctx *c) {
     hipLaunchKernelGGL(k_finish, dim3(nblk(c->nrep + 1, 256)), dim3(256), 0, c->stream, c->nrep,
                        c->rebuild, c->nbuilds);
+}
+
+void launch_list_done(sofia_ctx *c, int32_t *local) {
+    const int threads = std::max(c->nrep + 1, local ? c->N : 1);
+    hipLaunchKernelGGL(k_list_done, dim3(nblk(threads, 256)), dim3(256), 0, c->stream, c->nrep,
+                       c->rebuild, c->nbuilds, c->maxcnt, c->neigh_alloc, c->hw, c->N, c->tt, c->rep,
+                       c->reps_d, local);
 }
 
 }  // namespace sofia

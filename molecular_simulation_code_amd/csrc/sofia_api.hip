@@ -68,32 +68,53 @@ void drop_graph(sofia_ctx *c) {
     c->graphk = nullptr;
 }
 
-int alloc_atoms(sofia::AtomArrays &A, int n) {
-    TRY(dalloc(&A.pos4, n));
-    TRY(dalloc(&A.q, n));
-    TRY(dalloc(&A.gid, n));
-    TRY(dalloc(&A.num1, n));
-    TRY(dalloc(&A.num2, n));
-    TRY(dalloc(&A.num3, n));
-    TRY(dalloc(&A.spec, (size_t)n * SPEC));
-    TRY(dalloc(&A.v32, (size_t)3 * n));
-    TRY(dalloc(&A.xd, (size_t)3 * n));
-    TRY(dalloc(&A.vd, (size_t)3 * n));
-    TRY(dalloc(&A.mol, n));
-    TRY(dalloc(&A.wclus, n));
-    SOFIA_HIP(hipMemset(A.mol, 0xff, sizeof(int32_t) * n));
-    SOFIA_HIP(hipMemset(A.wclus, 0xff, sizeof(int32_t) * n));
-    SOFIA_HIP(hipMemset(A.spec, 0xff, sizeof(int32_t) * (size_t)n * SPEC));
-    SOFIA_HIP(hipMemset(A.num1, 0, sizeof(int32_t) * n));
-    SOFIA_HIP(hipMemset(A.num2, 0, sizeof(int32_t) * n));
-    SOFIA_HIP(hipMemset(A.num3, 0, sizeof(int32_t) * n));
-    SOFIA_HIP(hipMemset(A.v32, 0, sizeof(float) * 3 * (size_t)n));
-    return SOFIA_OK;
+// Arrays of one context that are never re-sized, carved out of one allocation: dozens of
+// allocations made a context's creation and, with a device synchronisation per free, its
+// destruction cost milliseconds.
+class Block {
+public:
+    template <typename T>
+    void want(T **p, size_t count) {
+        *p = nullptr;
+        parts_.push_back({(void **)p, total_});
+        total_ += ((count ? count : 1) * sizeof(T) + 255) / 256 * 256;
+    }
+    // one zeroed allocation, owned by the context
+    int make(sofia_ctx *c) {
+        char *base = nullptr;
+        TRY(dalloc(&base, total_));
+        c->blocks.push_back(base);
+        SOFIA_HIP(hipMemset(base, 0, total_));
+        for (auto &x : parts_) *x.first = base + x.second;
+        return SOFIA_OK;
+    }
+
+private:
+    std::vector<std::pair<void **, size_t>> parts_;
+    size_t total_ = 0;
+};
+
+void want_atoms(Block &B, sofia::AtomArrays &A, size_t n) {
+    B.want(&A.pos4, n);
+    B.want(&A.q, n);
+    B.want(&A.gid, n);
+    B.want(&A.num1, n);
+    B.want(&A.num2, n);
+    B.want(&A.num3, n);
+    B.want(&A.spec, n * SPEC);
+    B.want(&A.v32, 3 * n);
+    B.want(&A.xd, 3 * n);
+    B.want(&A.vd, 3 * n);
+    B.want(&A.mol, n);
+    B.want(&A.wclus, n);
 }
 
-void free_atoms(sofia::AtomArrays &A) {
-    dfree(A.pos4); dfree(A.q); dfree(A.gid); dfree(A.num1); dfree(A.num2); dfree(A.num3);
-    dfree(A.spec); dfree(A.v32); dfree(A.xd); dfree(A.vd); dfree(A.mol); dfree(A.wclus);
+// "none" in the arrays whose empty value is -1 (the block is zeroed)
+int clear_atoms(sofia::AtomArrays &A, size_t n) {
+    SOFIA_HIP(hipMemset(A.mol, 0xff, sizeof(int32_t) * n));
+    SOFIA_HIP(hipMemset(A.wclus, 0xff, sizeof(int32_t) * n));
+    SOFIA_HIP(hipMemset(A.spec, 0xff, sizeof(int32_t) * n * SPEC));
+    return SOFIA_OK;
 }
 
 // Every per-atom array of one set into another, ordered on stream s.
@@ -218,6 +239,18 @@ int upload(void *dst, const void *src, size_t bytes) {
 int download(void *dst, const void *src, size_t bytes) {
     if (!bytes) return SOFIA_OK;
     SOFIA_HIP(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+    return SOFIA_OK;
+}
+
+// Copies ordered on the context's stream; the call that makes them synchronises once at its end.
+int up(sofia_ctx *c, void *dst, const void *src, size_t bytes) {
+    if (!bytes) return SOFIA_OK;
+    SOFIA_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+    return SOFIA_OK;
+}
+int down(sofia_ctx *c, void *dst, const void *src, size_t bytes) {
+    if (!bytes) return SOFIA_OK;
+    SOFIA_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
     return SOFIA_OK;
 }
 
@@ -444,38 +477,38 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
     c->ncell_total = cell0;
     c->last_e.assign((size_t)nrep * SOFIA_NENERGY, 0.0);
     const int n = c->N;
-    TRY(alloc_atoms(c->a, n));
-    TRY(alloc_atoms(c->b, n));
-    TRY(dalloc(&c->rep, n));
-    TRY(dalloc(&c->dr32, (size_t)3 * n));
-    TRY(dalloc(&c->drd, (size_t)3 * n));
-    TRY(dalloc(&c->fnb, (size_t)3 * n));
-    TRY(dalloc(&c->pfix, (size_t)n));
-    TRY(dalloc(&c->fix, (size_t)3 * n));
-    TRY(dalloc(&c->fscratch, (size_t)3 * n));
-    TRY(dalloc(&c->stage32, (size_t)3 * n));
+    Block B;
+    want_atoms(B, c->a, n);
+    want_atoms(B, c->b, n);
+    B.want(&c->rep, n);
+    B.want(&c->dr32, (size_t)3 * n);
+    B.want(&c->drd, (size_t)3 * n);
+    B.want(&c->fnb, (size_t)3 * n);
+    B.want(&c->pfix, (size_t)n);
+    B.want(&c->fix, (size_t)3 * n);
+    B.want(&c->fscratch, (size_t)3 * n);
+    B.want(&c->stage32, (size_t)3 * n);
+    B.want(&c->acell, n);
+    B.want(&c->tt, n);
+    B.want(&c->atombin, n);
+    B.want(&c->numneigh, n);
+    B.want(&c->maxcnt, 1);
+    B.want(&c->rebuild, nrep + 1);   // nrep flags, then `any`
+    B.want(&c->nbuilds, nrep);
+    B.want(&c->shake_err, 1);
+    B.want(&c->type_err, 1);
+    B.want(&c->shake_iters, 1);
+    B.want(&c->eacc, eacc_len(nrep));
+    B.want(&c->step_d, nrep);
+    B.want(&c->reps_d, nrep);
+    TRY(B.make(c.get()));
+    TRY(clear_atoms(c->a, n));
+    TRY(clear_atoms(c->b, n));
     TRY(size_cells(c.get(), c->ncell_total));
-    TRY(dalloc(&c->acell, n));
-    TRY(dalloc(&c->tt, n));
-    TRY(dalloc(&c->atombin, n));
-    TRY(dalloc(&c->numneigh, n));
-    TRY(dalloc(&c->maxcnt, 1));
-    TRY(dalloc(&c->rebuild, nrep + 1));   // nrep flags, then `any`
-    TRY(dalloc(&c->nbuilds, nrep));
-    TRY(dalloc(&c->shake_err, 1));
-    TRY(dalloc(&c->type_err, 1));
-    TRY(dalloc(&c->shake_iters, 1));
-    TRY(dalloc(&c->eacc, eacc_len(nrep)));
-    TRY(dalloc(&c->step_d, nrep));
-    TRY(dalloc(&c->reps_d, nrep));
-    SOFIA_HIP(hipMemset(c->dr32, 0, sizeof(float) * 3 * (size_t)n));
-    SOFIA_HIP(hipMemset(c->drd, 0, sizeof(double) * 3 * (size_t)n));
-    SOFIA_HIP(hipMemset(c->fix, 0, sizeof(long long) * 3 * (size_t)n));
-    SOFIA_HIP(hipMemset(c->fnb, 0, sizeof(double) * 3 * (size_t)n));
-    SOFIA_HIP(hipMemset(c->rebuild, 0, sizeof(int32_t) * (nrep + 1)));
-    SOFIA_HIP(hipMemset(c->nbuilds, 0, sizeof(int32_t) * nrep));
-    SOFIA_HIP(hipMemset(c->numneigh, 0, sizeof(int32_t) * n));
-    SOFIA_HIP(hipMemset(c->step_d, 0, sizeof(uint64_t) * nrep));
+    const size_t words = sizeof(sofia::HostWords) + sizeof(long long) * (size_t)nrep * NE;
+    SOFIA_HIP(hipHostMalloc((void **)&c->hw, words, hipHostMallocDefault));
+    std::memset((void *)c->hw, 0, words);
+    c->hw_e = (long long *)(c->hw + 1);
     std::vector<int32_t> rep(n), cnum((size_t)27 * c->ncell_total), crep(c->ncell_total);
     for (int r = 0; r < nrep; ++r) {
         const sofia::RepInfo &R = c->reps_h[r];
@@ -514,30 +547,30 @@ void sum_eacc(const long long *raw, int nrep, std::vector<long long> &e) {
         for (int cp = 0; cp < ESPREAD; ++cp) e[k] += raw[(k * ESPREAD + cp) * ECOPY];
 }
 
-int read_energies(sofia_ctx *c, std::vector<long long> &e) {
-    std::vector<long long> raw(eacc_len(c->nrep));
-    SOFIA_HIP(hipMemcpyAsync(raw.data(), c->eacc, sizeof(long long) * raw.size(), hipMemcpyDeviceToHost,
-                             c->stream));
+// Waits for the stream, the energy sums and flags (hw) with it.
+int read_energies(sofia_ctx *c, std::vector<long long> &e, bool clear_shake = false) {
+    launch_report(c, clear_shake);
     TRY(sync_check(c));
-    sum_eacc(raw.data(), c->nrep, e);
+    e.assign(c->hw_e, c->hw_e + (size_t)c->nrep * NE);
     return SOFIA_OK;
 }
 
 double E(const std::vector<long long> &e, int r, int slot) { return (double)e[(size_t)r * NE + slot] * EFIX_INV; }
 
-// Full sort + list build of every flagged replica; grow-and-redo on overflow.
-int rebuild_now(sofia_ctx *c, bool engine, bool reference_growth) {
+// Full sort + list build of every flagged replica; grow-and-redo on overflow.  tt (host,
+// optional): the sort's permutation, 1-based within each replica.
+int rebuild_now(sofia_ctx *c, bool engine, bool reference_growth, int32_t *tt = nullptr) {
     launch_sort(c, engine ? SORT_ENGINE : SORT_DROPIN);
     for (int attempt = 0; attempt < 8; ++attempt) {
         SOFIA_HIP(hipMemsetAsync(c->maxcnt, 0, sizeof(int32_t), c->stream));
         launch_build_list(c);
-        int32_t mx = 0;
-        SOFIA_HIP(hipMemcpyAsync(&mx, c->maxcnt, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
+        launch_list_done(c, tt ? (int32_t *)c->stage32 : nullptr);
+        if (tt) TRY(down(c, tt, c->stage32, sizeof(int32_t) * (size_t)c->N));
         TRY(sync_check(c));
+        const int32_t mx = c->hw->maxcnt;
         if (mx <= c->neigh_alloc) {
-            launch_finish_rebuild(c);
             c->have_list = true;
-            return sync_check(c);
+            return SOFIA_OK;
         }
         int na = reference_growth ? grow_alloc(mx) : engine_stride(c, mx);
         TRY(ensure_list(c, na));
@@ -752,28 +785,24 @@ int sofia_ctx_destroy(sofia_ctx *c) {
     if (!c) return SOFIA_OK;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     drop_graph(c);
-    free_atoms(c->a);
-    free_atoms(c->b);
-    free_atoms(c->snap);
-    dfree(c->snap_topo); dfree(c->snap_fnb); dfree(c->snap_drd); dfree(c->snap_fix);
-    dfree(c->snap_step); dfree(c->snap_nbuilds);
-    dfree(c->rep); dfree(c->dr32); dfree(c->drd); dfree(c->fnb); dfree(c->fix); dfree(c->fscratch); dfree(c->stage32);
+    for (void *p : c->blocks) (void)hipFree(p);
+    dfree(c->snap_topo);
     dfree(c->mol_rep); dfree(c->uf_parent); dfree(c->uf_size); dfree(c->uf_largest);
     dfree(c->gc_first); dfree(c->gc_refgid); dfree(c->gc_cnt); dfree(c->gc_dens); dfree(c->gc_sum);
     dfree(c->gc_refx); dfree(c->gc_com); dfree(c->gc_key); dfree(c->gc_surface);
-    dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep); dfree(c->acell);
-    dfree(c->cbin); dfree(c->bucket); dfree(c->tt); dfree(c->atombin); dfree(c->mtab);
-    dfree(c->nlist); dfree(c->numneigh); dfree(c->maxcnt); dfree(c->rebuild); dfree(c->nbuilds);
+    dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep);
+    dfree(c->cbin); dfree(c->bucket); dfree(c->mtab); dfree(c->nlist);
     dfree(c->bund_tstart); dfree(c->bund_sstart); dfree(c->bund_slots); dfree(c->bund_terms);
-    dfree(c->shake_err); dfree(c->shake_iters); dfree(c->water); dfree(c->dsf_tab); dfree(c->pfix); dfree(c->ebond); dfree(c->eangle); dfree(c->bondlist); dfree(c->anglelist);
+    dfree(c->water); dfree(c->dsf_tab); dfree(c->ebond); dfree(c->eangle); dfree(c->bondlist); dfree(c->anglelist);
     dfree(c->dihedlist); dfree(c->torsions); dfree(c->shake_num); dfree(c->shake_atoms); dfree(c->shake_kidx);
     dfree(c->ptab);
     dfree(c->shake_bond); dfree(c->ljtab); dfree(c->lj14); dfree(c->mass); dfree(c->bond_k);
     dfree(c->bond_r0); dfree(c->angle_k); dfree(c->angle_th0); dfree(c->tors_k); dfree(c->tors_n);
     dfree(c->tors_shift); dfree(c->tors_cs); dfree(c->improlist); dfree(c->impro_k);
-    dfree(c->impro_chi0); dfree(c->impro_dn); dfree(c->eacc); dfree(c->step_d); dfree(c->reps_d);
-    dfree(c->topo_stage); dfree(c->type_err); dfree(c->fix14); dfree(c->rdf_hist);
+    dfree(c->impro_chi0); dfree(c->impro_dn);
+    dfree(c->topo_stage); dfree(c->fix14); dfree(c->rdf_hist);
     if (c->pinned) (void)hipHostFree(c->pinned);
+    if (c->hw) (void)hipHostFree((void *)c->hw);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return SOFIA_OK;
@@ -1008,30 +1037,35 @@ int sofia_set_shake(sofia_ctx *c, int32_t ns, const int32_t *ns_rep, const int32
 int sofia_put_state(sofia_ctx *c, const sofia_ainfo *pos, const float *q, const sofia_coords *v,
                     const int32_t *gid) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
-    const int n = c->N;
-    TRY(sync_check(c));   // kernels in flight may still read the arrays replaced here
-    if (pos && n > 0) {
+    const size_t n = c->N;
+    // ordered on the stream behind kernels that may still read the arrays replaced here
+    if (pos) {
         // Types within 1..ntypes, checked on the device (a host pass over the array costs
         // more than the copy) on a staging copy, the sort's gather target, which holds nothing
         // between list builds; a rejected upload leaves the state as it was.
-        TRY(upload(c->b.pos4, pos, sizeof(float4) * n));
-        SOFIA_HIP(hipMemsetAsync(c->type_err, 0, sizeof(int32_t), c->stream));
-        launch_type_range(c, c->b.pos4, c->type_err);
-        int32_t bad = 0;
-        SOFIA_HIP(hipMemcpyAsync(&bad, c->type_err, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
+        c->hw->type_err = 0;
+        TRY(up(c, c->b.pos4, pos, sizeof(float4) * n));
+        if (q) TRY(up(c, c->b.q, q, sizeof(float) * n));
+        if (v) TRY(up(c, c->b.v32, v, sizeof(float) * 3 * n));
+        if (gid) TRY(up(c, c->b.gid, gid, sizeof(int32_t) * n));
+        launch_put_state(c, v != nullptr, q != nullptr, gid != nullptr);
         TRY(sync_check(c));
-        if (bad) return fail(SOFIA_E_ARG, "atom type out of range");
-        launch_copy16(c, (size_t)n, c->b.pos4, c->a.pos4);
-        c->q_by_type = false;   // types may have changed
+        if (c->hw->type_err) {
+            SOFIA_HIP(hipMemsetAsync(c->type_err, 0, sizeof(int32_t), c->stream));
+            TRY(sync_check(c));
+            return fail(SOFIA_E_ARG, "atom type out of range");
+        }
+    } else {
+        if (q) TRY(up(c, c->a.q, q, sizeof(float) * n));
+        if (v) TRY(up(c, c->a.v32, v, sizeof(float) * 3 * n));
+        if (gid) TRY(up(c, c->a.gid, gid, sizeof(int32_t) * n));
+        TRY(sync_check(c));
+    }
+    if (pos || q) {
+        c->q_by_type = false;   // types or charges may have changed
         drop_graph(c);
     }
-    if (q) {
-        TRY(upload(c->a.q, q, sizeof(float) * n));
-        c->q_by_type = false;
-        drop_graph(c);
-    }
-    if (v) TRY(upload(c->a.v32, v, sizeof(float) * 3 * (size_t)n));
-    if (gid) TRY(upload(c->a.gid, gid, sizeof(int32_t) * n));
+    if (gid) c->gid_perm = -1;
     // a running engine re-derives its charge records from the new types and charges
     if ((pos || q) && c->engine_ready) TRY(classify_charges(c));
     return SOFIA_OK;
@@ -1039,60 +1073,92 @@ int sofia_put_state(sofia_ctx *c, const sofia_ainfo *pos, const float *q, const 
 
 int sofia_get_state(sofia_ctx *c, sofia_ainfo *pos, sofia_coords *v, int32_t *gid) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
-    TRY(sync_check(c));
-    const int n = c->N;
-    if (pos) TRY(download(pos, c->a.pos4, sizeof(float4) * n));
-    if (v) TRY(download(v, c->a.v32, sizeof(float) * 3 * (size_t)n));
-    if (gid) TRY(download(gid, c->a.gid, sizeof(int32_t) * n));
-    return SOFIA_OK;
+    const size_t n = c->N;
+    if (pos) TRY(down(c, pos, c->a.pos4, sizeof(float4) * n));
+    if (v) TRY(down(c, v, c->a.v32, sizeof(float) * 3 * n));
+    if (gid) TRY(down(c, gid, c->a.gid, sizeof(int32_t) * n));
+    return sync_check(c);
 }
 
 int sofia_get_state_f64(sofia_ctx *c, double *x, double *v) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
-    TRY(sync_check(c));
-    const int n = c->N;
-    std::vector<double> t((size_t)3 * n);
-    for (int w = 0; w < 2; ++w) {
-        double *dst = w ? v : x;
-        if (!dst) continue;
-        TRY(download(t.data(), w ? c->a.vd : c->a.xd, sizeof(double) * t.size()));
-        for (int i = 0; i < n; ++i)
-            for (int d = 0; d < 3; ++d) dst[3 * (size_t)i + d] = t[(size_t)d * n + i];
+    const size_t bytes = sizeof(double) * 3 * (size_t)c->N;
+    // rows made on the device, in the sort's gather target (free between list builds)
+    if (x) {
+        launch_soa_to_aos(c, c->a.xd, nullptr, nullptr, c->b.xd);
+        TRY(down(c, x, c->b.xd, bytes));
     }
-    return SOFIA_OK;
+    if (v) {
+        launch_soa_to_aos(c, c->a.vd, nullptr, nullptr, c->b.vd);
+        TRY(down(c, v, c->b.vd, bytes));
+    }
+    return sync_check(c);
 }
 
 int sofia_put_state_f64(sofia_ctx *c, const double *x, const double *v) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
-    const int n = c->N;
-    std::vector<double> t((size_t)3 * n);
-    for (int w = 0; w < 2; ++w) {
-        const double *src = w ? v : x;
-        if (!src) continue;
-        for (int i = 0; i < n; ++i)
-            for (int d = 0; d < 3; ++d) t[(size_t)d * n + i] = src[3 * (size_t)i + d];
-        TRY(upload(w ? c->a.vd : c->a.xd, t.data(), sizeof(double) * t.size()));
+    const size_t bytes = sizeof(double) * 3 * (size_t)c->N;
+    if (x) {
+        TRY(up(c, c->b.xd, x, bytes));
+        launch_aos_to_soa(c, c->b.xd, c->a.xd);
     }
-    return SOFIA_OK;
+    if (v) {
+        TRY(up(c, c->b.vd, v, bytes));
+        launch_aos_to_soa(c, c->b.vd, c->a.vd);
+    }
+    return sync_check(c);
+}
+
+int sofia_get_ordered_f64(sofia_ctx *c, double *x, double *v, double *f, int32_t *ordered) {
+    if (!c || !ordered) return fail(SOFIA_E_ARG, "null argument");
+    if (f && !c->engine_ready) return fail(SOFIA_E_STATE, "call sofia_md_init first");
+    if (c->gid_perm < 0) {   // checked once per upload of the ids (the sort permutes them)
+        std::vector<int32_t> g(c->N);
+        TRY(down(c, g.data(), c->a.gid, sizeof(int32_t) * g.size()));
+        TRY(sync_check(c));
+        std::vector<char> seen(c->N, 0);
+        c->gid_perm = 1;
+        for (const auto &R : c->reps_h)
+            for (int k = 0; k < R.natom && c->gid_perm; ++k) {
+                const int id = g[R.atom0 + k];
+                if (id < 1 || id > R.natom || seen[R.atom0 + id - 1]) c->gid_perm = 0;
+                else seen[R.atom0 + id - 1] = 1;
+            }
+    }
+    *ordered = c->gid_perm;
+    if (!c->gid_perm) return SOFIA_OK;
+    const size_t bytes = sizeof(double) * 3 * (size_t)c->N;
+    if (x) {
+        launch_soa_to_aos(c, c->a.xd, nullptr, c->a.gid, c->b.xd);
+        TRY(down(c, x, c->b.xd, bytes));
+    }
+    if (v) {
+        launch_soa_to_aos(c, c->a.vd, nullptr, c->a.gid, c->b.vd);
+        TRY(down(c, v, c->b.vd, bytes));
+    }
+    if (f) {
+        launch_soa_to_aos(c, c->fnb, c->fix, c->a.gid, (double *)c->fscratch);
+        TRY(down(c, f, c->fscratch, bytes));
+    }
+    return sync_check(c);
 }
 
 int sofia_get_displacement(sofia_ctx *c, float *dx, float *dy, float *dz) {
     if (!c || !dx || !dy || !dz) return fail(SOFIA_E_ARG, "null argument");
-    TRY(sync_check(c));
-    const int n = c->N;
-    TRY(download(dx, c->dr32, sizeof(float) * n));
-    TRY(download(dy, c->dr32 + n, sizeof(float) * n));
-    TRY(download(dz, c->dr32 + 2 * (size_t)n, sizeof(float) * n));
-    return SOFIA_OK;
+    const size_t n = c->N;
+    TRY(down(c, dx, c->dr32, sizeof(float) * n));
+    TRY(down(c, dy, c->dr32 + n, sizeof(float) * n));
+    TRY(down(c, dz, c->dr32 + 2 * n, sizeof(float) * n));
+    return sync_check(c);
 }
 
 int sofia_put_displacement(sofia_ctx *c, const float *dx, const float *dy, const float *dz) {
     if (!c || !dx || !dy || !dz) return fail(SOFIA_E_ARG, "null argument");
-    const int n = c->N;
-    TRY(upload(c->dr32, dx, sizeof(float) * n));
-    TRY(upload(c->dr32 + n, dy, sizeof(float) * n));
-    TRY(upload(c->dr32 + 2 * (size_t)n, dz, sizeof(float) * n));
-    return SOFIA_OK;
+    const size_t n = c->N;
+    TRY(up(c, c->dr32, dx, sizeof(float) * n));
+    TRY(up(c, c->dr32 + n, dy, sizeof(float) * n));
+    TRY(up(c, c->dr32 + 2 * n, dz, sizeof(float) * n));
+    return sync_check(c);
 }
 
 int sofia_host_alloc(size_t bytes, void **out) {
@@ -1114,28 +1180,18 @@ int sofia_host_free(void *p) {
 int sofia_neighbor_wrapper(sofia_ctx *c, int32_t, int32_t *tt) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
     launch_set_rebuild(c, 1);
-    TRY(rebuild_now(c, c->engine_ready, true));
-    if (tt) {
-        std::vector<int32_t> t(c->N);
-        TRY(download(t.data(), c->tt, sizeof(int32_t) * c->N));
-        for (int r = 0; r < c->nrep; ++r) {
-            const auto &R = c->reps_h[r];
-            for (int k = 0; k < R.natom; ++k) tt[R.atom0 + k] = t[R.atom0 + k] - R.atom0 + 1;
-        }
-    }
-    return SOFIA_OK;
+    return rebuild_now(c, c->engine_ready, true, tt);
 }
 
 int sofia_get_topology(sofia_ctx *c, float *q, int32_t *num1bond, int32_t *num2bond,
                        int32_t *num3bond, int32_t *specbond, int32_t *bondlist, int32_t *anglelist,
                        int32_t *dihedlist, int32_t *improlist, int32_t *shake_atoms) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
-    TRY(sync_check(c));
     const size_t n = c->N;
-    if (q) TRY(download(q, c->a.q, sizeof(float) * n));
-    if (num1bond) TRY(download(num1bond, c->a.num1, sizeof(int32_t) * n));
-    if (num2bond) TRY(download(num2bond, c->a.num2, sizeof(int32_t) * n));
-    if (num3bond) TRY(download(num3bond, c->a.num3, sizeof(int32_t) * n));
+    if (q) TRY(down(c, q, c->a.q, sizeof(float) * n));
+    if (num1bond) TRY(down(c, num1bond, c->a.num1, sizeof(int32_t) * n));
+    if (num2bond) TRY(down(c, num2bond, c->a.num2, sizeof(int32_t) * n));
+    if (num3bond) TRY(down(c, num3bond, c->a.num3, sizeof(int32_t) * n));
     struct Arr {
         int32_t *dst;
         const int32_t *src;
@@ -1148,22 +1204,23 @@ int sofia_get_topology(sofia_ctx *c, float *q, int32_t *num1bond, int32_t *num2b
                         {dihedlist, c->dihedlist, (size_t)c->nd, 5, 4},
                         {improlist, c->improlist, (size_t)c->nimp, 5, 4},
                         {shake_atoms, c->shake_atoms, (size_t)c->ns, 4, 4}};
-    size_t need = 0;
+    size_t need = 0;   // every array has its own stretch of the staging buffer
     for (const Arr &x : arrs)
-        if (x.dst) need = std::max(need, x.items * x.width);
+        if (x.dst) need += x.items * x.width;
     if (need > c->topo_stage_len) {
         dfree(c->topo_stage);
         c->topo_stage_len = 0;
         TRY(dalloc(&c->topo_stage, need));
         c->topo_stage_len = need;
     }
+    size_t off = 0;
     for (const Arr &x : arrs) {
         if (!x.dst || !x.items) continue;
-        launch_host_ids(c, x.src, c->topo_stage, x.items, x.width, x.nidx);
-        TRY(sync_check(c));
-        TRY(download(x.dst, c->topo_stage, sizeof(int32_t) * x.items * x.width));
+        launch_host_ids(c, x.src, c->topo_stage + off, x.items, x.width, x.nidx);
+        TRY(down(c, x.dst, c->topo_stage + off, sizeof(int32_t) * x.items * x.width));
+        off += x.items * x.width;
     }
-    return SOFIA_OK;
+    return sync_check(c);
 }
 
 int sofia_rdf_calc(sofia_ctx *c, int32_t itype, int32_t jtype, float rdf_delta, int32_t nbins,
@@ -1217,8 +1274,9 @@ int sofia_get_cells(sofia_ctx *c, int32_t *start, int32_t *endposit, int32_t *at
 int sofia_get_nlist(sofia_ctx *c, int32_t *nlist, int32_t *numneigh, int32_t *na) {
     if (!c) return fail(SOFIA_E_ARG, "null context");
     if (!c->have_list) return fail(SOFIA_E_STATE, "no list built yet");
-    TRY(sync_check(c));
     if (na) *na = c->neigh_alloc;
+    if (!nlist && !numneigh) return SOFIA_OK;
+    TRY(sync_check(c));
     std::vector<int32_t> nn(c->N);
     TRY(download(nn.data(), c->numneigh, sizeof(int32_t) * c->N));
     if (numneigh) std::memcpy(numneigh, nn.data(), sizeof(int32_t) * c->N);
@@ -1241,14 +1299,11 @@ int sofia_get_nlist(sofia_ctx *c, int32_t *nlist, int32_t *numneigh, int32_t *na
 int sofia_check_neighbor(sofia_ctx *c, int32_t *nflag) {
     if (!c || !nflag) return fail(SOFIA_E_ARG, "null argument");
     launch_set_rebuild(c, 0);
+    c->hw->moved = 0;
     launch_check_neighbor(c);
-    std::vector<int32_t> f(c->nrep);
-    SOFIA_HIP(hipMemcpyAsync(f.data(), c->rebuild, sizeof(int32_t) * c->nrep, hipMemcpyDeviceToHost, c->stream));
     TRY(sync_check(c));
-    *nflag = 0;
-    for (int v : f) *nflag |= v;
-    launch_set_rebuild(c, 0);
-    return sync_check(c);
+    *nflag = c->hw->moved;
+    return SOFIA_OK;
 }
 
 static int nonbond_dropin(sofia_ctx *c, int mode, sofia_coords *ff, double *ff64, double *pot,
@@ -1256,18 +1311,16 @@ static int nonbond_dropin(sofia_ctx *c, int mode, sofia_coords *ff, double *ff64
     if (!c) return fail(SOFIA_E_ARG, "null context");
     if (!c->have_list) return fail(SOFIA_E_STATE, "no Verlet list: call sofia_neighbor_wrapper first");
     if (!c->have_ff) return fail(SOFIA_E_STATE, "force field not set");
-    launch_zero_forces(c, c->fscratch, true);
+    launch_zero_energies(c);
     launch_nonbond_out(c, mode, true, staging_f32(c));
+    const size_t n = c->N;
+    if (ff) TRY(down(c, ff, staging_f32(c), sizeof(float) * 3 * n));
+    if (ff64) {
+        launch_soa_to_aos(c, c->fnb, nullptr, nullptr, (double *)c->fscratch);
+        TRY(down(c, ff64, c->fscratch, sizeof(double) * 3 * n));
+    }
     std::vector<long long> e;
     TRY(read_energies(c, e));
-    const int n = c->N;
-    if (ff) TRY(download(ff, staging_f32(c), sizeof(float) * 3 * (size_t)n));
-    if (ff64) {
-        std::vector<double> t((size_t)3 * n);
-        TRY(download(t.data(), c->fnb, sizeof(double) * t.size()));
-        for (int i = 0; i < n; ++i)
-            for (int d = 0; d < 3; ++d) ff64[3 * (size_t)i + d] = t[(size_t)d * n + i];
-    }
     double sp = 0, se = 0, vx = 0, vy = 0, vz = 0;
     for (int r = 0; r < c->nrep; ++r) {
         sp += E(e, r, E_LJ); se += E(e, r, E_COUL);
@@ -1293,7 +1346,7 @@ int sofia_lj_cut_coul_dsf_async(sofia_ctx *c, int32_t mixed) {
         c->pinned_bytes = fbytes + ebytes;
     }
     const int mode = mixed ? 1 : 0;
-    launch_zero_forces(c, c->fscratch, true);
+    launch_zero_forces(c, c->fscratch, true);   // (the raw sums are read, not reported)
     launch_nonbond_out(c, mode, true, staging_f32(c));
     SOFIA_HIP(hipMemcpyAsync(c->pinned, staging_f32(c), fbytes, hipMemcpyDeviceToHost, c->stream));
     SOFIA_HIP(hipMemcpyAsync((char *)c->pinned + fbytes, c->eacc, ebytes, hipMemcpyDeviceToHost, c->stream));
@@ -1343,9 +1396,9 @@ int sofia_correct_bonds(sofia_ctx *c, int32_t which, sofia_coords *ff, double *e
     launch_correct(c, which, c->fscratch);
     float *st = staging_f32(c);
     launch_fix_to_coords(c, c->fscratch, st);
+    if (ff) TRY(down(c, ff, st, sizeof(float) * 3 * (size_t)c->N));
     std::vector<long long> e;
     TRY(read_energies(c, e));
-    if (ff) TRY(download(ff, st, sizeof(float) * 3 * (size_t)c->N));
     double s = 0, vx = 0, vy = 0, vz = 0;
     for (int r = 0; r < c->nrep; ++r) {
         s += E(e, r, E_CORR); vx += E(e, r, V_X); vy += E(e, r, V_Y); vz += E(e, r, V_Z);
@@ -1362,9 +1415,9 @@ int sofia_pair14_dsf(sofia_ctx *c, sofia_coords *ffh, double *ec14, double *pot1
     launch_pair14(c, c->fscratch);
     float *st = staging_f32(c);
     launch_fix_to_coords(c, c->fscratch, st);
+    if (ffh) TRY(down(c, ffh, st, sizeof(float) * 3 * (size_t)c->N));
     std::vector<long long> e;
     TRY(read_energies(c, e));
-    if (ffh) TRY(download(ffh, st, sizeof(float) * 3 * (size_t)c->N));
     double a = 0, b = 0;
     for (int r = 0; r < c->nrep; ++r) { a += E(e, r, E_COUL14); b += E(e, r, E_POT14); }
     if (ec14) *ec14 += a;
@@ -1381,9 +1434,9 @@ int sofia_bonded_forces(sofia_ctx *c, sofia_coords *ff, double *e_bond, double *
     launch_bonded_dropin(c, c->fscratch);
     float *st = staging_f32(c);
     launch_fix_to_coords(c, c->fscratch, st);
+    if (ff) TRY(down(c, ff, st, sizeof(float) * 3 * (size_t)c->N));
     std::vector<long long> e;
     TRY(read_energies(c, e));
-    if (ff) TRY(download(ff, st, sizeof(float) * 3 * (size_t)c->N));
     double sb = 0, sa = 0, sd = 0, si = 0;
     for (int r = 0; r < c->nrep; ++r) {
         sb += E(e, r, E_BOND); sa += E(e, r, E_ANGLE); sd += E(e, r, E_DIHED); si += E(e, r, E_IMPRO);
@@ -1405,15 +1458,15 @@ int sofia_force_wrapper_dsf(sofia_ctx *c, sofia_coords *ff, double *e, double *v
     const int n = c->N;
     if (!c->fix14) TRY(dalloc(&c->fix14, (size_t)3 * n));
     float *st = staging_f32(c);
-    launch_zero_forces(c, c->fscratch, true);   // energies zeroed once: the terms use their own slots
-    launch_zero_forces(c, c->fix14, false);
+    launch_zero_energies(c);   // once: the terms use their own slots
+    launch_zero2(c, c->fscratch, c->fix14);
     launch_nonbond_out(c, 0, true, st);
     launch_pair14(c, c->fix14);
     launch_bonded_dropin(c, c->fscratch);
     launch_merge_forces(c, st, c->fix14, c->fscratch);
+    if (ff) TRY(down(c, ff, st, sizeof(float) * 3 * (size_t)n));
     std::vector<long long> es;
     TRY(read_energies(c, es));
-    if (ff) TRY(download(ff, st, sizeof(float) * 3 * (size_t)n));
     // summed over replicas first, then added, as each routine of its own adds its sums
     const int slot[8] = {E_LJ, E_COUL, E_COUL14, E_POT14, E_BOND, E_ANGLE, E_DIHED, E_IMPRO};
     double sum[8] = {0, 0, 0, 0, 0, 0, 0, 0}, vx = 0, vy = 0, vz = 0;
@@ -1431,8 +1484,8 @@ int sofia_nve_v(sofia_ctx *c, float dt_partial, const sofia_coords *ff, double *
     if (!c || !ff) return fail(SOFIA_E_ARG, "null argument");
     if (!c->have_ff) return fail(SOFIA_E_STATE, "force field not set");
     float *st = staging_f32(c);
-    TRY(upload(st, ff, sizeof(float) * 3 * (size_t)c->N));
-    SOFIA_HIP(hipMemsetAsync(c->eacc, 0, sizeof(long long) * eacc_len(c->nrep), c->stream));
+    TRY(up(c, st, ff, sizeof(float) * 3 * (size_t)c->N));
+    launch_zero_energies(c);
     launch_nve_v32(c, dt_partial, st);
     std::vector<long long> e;
     TRY(read_energies(c, e));
@@ -1491,17 +1544,17 @@ int sofia_shake(sofia_ctx *c, int32_t iflag, sofia_coords *ff, double *vir, int3
     if (!c || !ff) return fail(SOFIA_E_ARG, "null argument");
     if (!c->have_ff) return fail(SOFIA_E_STATE, "force field not set");
     float *st = staging_f32(c);
-    TRY(upload(st, ff, sizeof(float) * 3 * (size_t)c->N));
-    SOFIA_HIP(hipMemsetAsync(c->eacc, 0, sizeof(long long) * eacc_len(c->nrep), c->stream));
-    SOFIA_HIP(hipMemsetAsync(c->shake_err, 0, sizeof(int32_t), c->stream));
-    SOFIA_HIP(hipMemsetAsync(c->shake_iters, 0, sizeof(int32_t), c->stream));
+    TRY(up(c, st, ff, sizeof(float) * 3 * (size_t)c->N));
+    launch_zero_energies(c);
+    if (c->engine_ready) {   // (the last report of a drop-in call cleared them)
+        SOFIA_HIP(hipMemsetAsync(c->shake_err, 0, sizeof(int32_t), c->stream));
+        SOFIA_HIP(hipMemsetAsync(c->shake_iters, 0, sizeof(int32_t), c->stream));
+    }
     launch_shake32(c, iflag, st, nullptr);
+    TRY(down(c, ff, st, sizeof(float) * 3 * (size_t)c->N));
     std::vector<long long> e;
-    TRY(read_energies(c, e));
-    int32_t err = 0, its = 0;
-    TRY(download(&err, c->shake_err, sizeof(int32_t)));
-    TRY(download(&its, c->shake_iters, sizeof(int32_t)));
-    TRY(download(ff, st, sizeof(float) * 3 * (size_t)c->N));
+    TRY(read_energies(c, e, true));
+    const int32_t err = c->hw->shake_err, its = c->hw->shake_iters;
     if (vir)
         for (int r = 0; r < c->nrep; ++r) {
             vir[0] += E(e, r, V_X); vir[1] += E(e, r, V_Y); vir[2] += E(e, r, V_Z);
@@ -1517,8 +1570,8 @@ int sofia_langevin(sofia_ctx *c, float fric, float gconst, uint64_t seed, uint64
     if (!c->have_ff) return fail(SOFIA_E_STATE, "force field not set");
     float *st = staging_f32(c);
     launch_langevin32(c, fric, gconst, seed, step, st);
-    TRY(sync_check(c));
-    return download(ff_lang, st, sizeof(float) * 3 * (size_t)c->N);
+    TRY(down(c, ff_lang, st, sizeof(float) * 3 * (size_t)c->N));
+    return sync_check(c);
 }
 
 // ------------------------------------------------------------------ engine
@@ -1571,23 +1624,31 @@ void step_sequence(sofia_ctx *c, bool kick2, bool energies) {
     launch_shake64(c, energies, true);
 }
 
-int collect_energies(sofia_ctx *c) {
-    std::vector<long long> e;
-    TRY(read_energies(c, e));
+// Energies of the last report into last_e.
+void take_energies(sofia_ctx *c) {
+    const std::vector<long long> e(c->hw_e, c->hw_e + (size_t)c->nrep * NE);
     for (int r = 0; r < c->nrep; ++r) {
         double *o = c->last_e.data() + (size_t)r * SOFIA_NENERGY;
         o[0] = E(e, r, E_LJ); o[1] = E(e, r, E_COUL); o[2] = E(e, r, E_POT14);
         o[3] = E(e, r, E_COUL14); o[4] = E(e, r, E_BOND); o[5] = E(e, r, E_ANGLE);
         o[6] = E(e, r, E_DIHED); o[7] = E(e, r, E_KE); o[8] = E(e, r, E_IMPRO);
     }
+}
+
+int report(sofia_ctx *c) {
+    launch_report(c);
+    return sync_check(c);
+}
+
+int collect_energies(sofia_ctx *c) {
+    TRY(report(c));
+    take_energies(c);
     return SOFIA_OK;
 }
 
+// The flags of the last report.
 int check_engine_flags(sofia_ctx *c, int32_t *overflow = nullptr) {
-    int32_t err = 0, mx = 0;
-    SOFIA_HIP(hipMemcpyAsync(&err, c->shake_err, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    SOFIA_HIP(hipMemcpyAsync(&mx, c->maxcnt, sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    TRY(sync_check(c));
+    const int32_t err = c->hw->shake_err, mx = c->hw->maxcnt;
     if (overflow) *overflow = mx > c->neigh_alloc ? mx : 0;
     if (mx > c->neigh_alloc) return fail(SOFIA_E_OVERFLOW, "Verlet list overflow during an MD segment");
     if (err)
@@ -1843,16 +1904,9 @@ int sofia_md_resume(sofia_ctx *c) {
 int sofia_get_forces_f64(sofia_ctx *c, double *f) {
     if (!c || !f) return fail(SOFIA_E_ARG, "null argument");
     if (!c->engine_ready) return fail(SOFIA_E_STATE, "call sofia_md_init first");
-    TRY(sync_check(c));
-    const size_t n = (size_t)c->N;
-    std::vector<double> nb(3 * n);
-    std::vector<long long> fx(3 * n);
-    TRY(download(nb.data(), c->fnb, sizeof(double) * nb.size()));
-    TRY(download(fx.data(), c->fix, sizeof(long long) * fx.size()));
-    // the sum k_nve_v64 forms (FIX_INV is a power of two, so the product is exact)
-    for (size_t i = 0; i < n; ++i)
-        for (int d = 0; d < 3; ++d) f[3 * i + d] = nb[d * n + i] + (double)fx[d * n + i] * FIX_INV;
-    return SOFIA_OK;
+    launch_soa_to_aos(c, c->fnb, c->fix, nullptr, c->b.xd);
+    TRY(down(c, f, c->b.xd, sizeof(double) * 3 * (size_t)c->N));
+    return sync_check(c);
 }
 
 int sofia_md_pair_forces(sofia_ctx *c, double *f, double *e) {
@@ -1988,12 +2042,14 @@ std::vector<std::pair<int32_t *, size_t>> sorted_lists(sofia_ctx *c) {
 int snapshot_take(sofia_ctx *c) {
     const size_t n = (size_t)c->N;
     if (!c->snap.pos4) {
-        TRY(alloc_atoms(c->snap, c->N));
-        TRY(dalloc(&c->snap_fnb, 3 * n));
-        TRY(dalloc(&c->snap_drd, 3 * n));
-        TRY(dalloc(&c->snap_fix, 3 * n));
-        TRY(dalloc(&c->snap_step, c->nrep));
-        TRY(dalloc(&c->snap_nbuilds, c->nrep));
+        Block B;
+        want_atoms(B, c->snap, n);
+        B.want(&c->snap_fnb, 3 * n);
+        B.want(&c->snap_drd, 3 * n);
+        B.want(&c->snap_fix, 3 * n);
+        B.want(&c->snap_step, c->nrep);
+        B.want(&c->snap_nbuilds, c->nrep);
+        TRY(B.make(c));
     }
     size_t topo = 0;
     for (auto &l : sorted_lists(c)) topo += l.first ? l.second : 0;
@@ -2108,6 +2164,7 @@ int sofia_md_finish(sofia_ctx *c) {
     if (!c->engine_ready) return fail(SOFIA_E_STATE, "call sofia_md_init first");
     for (int attempt = 0;; ++attempt) {
         int32_t overflow = 0;
+        TRY(report(c));
         const int rc = check_engine_flags(c, &overflow);
         if (rc == SOFIA_E_OVERFLOW && c->snap_valid && attempt < 4) {
             // grow and redo the segment (the reference grows neigh_alloc and rebuilds)
@@ -2119,8 +2176,8 @@ int sofia_md_finish(sofia_ctx *c) {
             continue;
         }
         c->snap_valid = false;
-        if (rc != SOFIA_OK) return rc;
-        return collect_energies(c);
+        if (rc == SOFIA_OK) take_energies(c);
+        return rc;
     }
 }
 
@@ -2308,6 +2365,7 @@ int sofia_profile_step(sofia_ctx *c, int32_t nsteps, int32_t full_rebuild, doubl
     TRY(rc);
     c->step_h += nsteps;
     for (int p = 0; p < NP; ++p) phase_ms[p] = acc[p] / nsteps;
+    TRY(report(c));
     return check_engine_flags(c);
 }
 

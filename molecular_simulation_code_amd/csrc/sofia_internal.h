@@ -75,6 +75,10 @@ __host__ __device__ inline int bonded_width(int kind) {
     return kind == BK_BOND ? 3 : (kind == BK_ANGLE ? 4 : 5);
 }
 
+struct HostWords {
+    int32_t maxcnt, shake_err, shake_iters, type_err, moved, pad[11];
+};
+
 // Per-atom arrays that the cell sort permutes (one set; the context keeps two).
 struct AtomArrays {
     float4 *pos4 = nullptr;     // x, y, z, type (int bits)
@@ -200,6 +204,14 @@ struct sofia_ctx {
 
     // energies (int64 fixed point, per replica x NE)
     long long *eacc = nullptr;
+    bool eacc_zero = false;      // eacc is known to be all zero (launch_report cleared it)
+    // page-locked words the device writes for the host (launch_report, launch_list_done,
+    // k_check32): read after one synchronisation, with no copy of their own
+    sofia::HostWords *hw = nullptr;
+    long long *hw_e = nullptr;   // nrep x NE energy sums, behind hw
+    // blocks that hold the context's fixed-size arrays (one allocation instead of dozens)
+    std::vector<void *> blocks;
+    int gid_perm = -1;           // global ids of every replica a permutation: 1, 0, -1 unknown
     std::vector<double> last_e;
 
     // engine
@@ -259,6 +271,9 @@ void launch_build_list_engine(sofia_ctx *c);
 void launch_check_neighbor(sofia_ctx *c);
 void launch_set_rebuild(sofia_ctx *c, int32_t value);
 void launch_finish_rebuild(sofia_ctx *c);
+// Ends a rebuild whose lists fit (counts it, lowers the flags) and tells the host the largest
+// count either way; local (optional): tt as 1-based ids within the replica.
+void launch_list_done(sofia_ctx *c, int32_t *local);
 
 // nonbond (k_nonbond.hip): mode 0 = DSF FP64, 1 = DSF mixed, 2 = Ewald real space (FP32)
 // records: the mixed kernel's position records are already up to date
@@ -297,8 +312,14 @@ void launch_shake64(sofia_ctx *c, bool energies, bool step = false);
 void launch_zero_energies(sofia_ctx *c);
 void launch_water_bonded(sofia_ctx *c);
 void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst);
-void launch_type_range(sofia_ctx *c, const float4 *pos, int32_t *bad);
+void launch_put_state(sofia_ctx *c, bool v, bool q, bool gid);
 void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb);
+// Energy sums (cleared on the device) and flags to the host words
+void launch_report(sofia_ctx *c, bool clear_shake = false);
+void launch_zero2(sofia_ctx *c, long long *a, long long *b);
+// FP64 SoA (plus fixed point) <-> AoS; with gid, dst rows in global-id order of each replica
+void launch_soa_to_aos(sofia_ctx *c, const double *src, const long long *fix, const int32_t *gid, double *dst);
+void launch_aos_to_soa(sofia_ctx *c, const double *src, double *dst);
 void launch_step_add(sofia_ctx *c, long long delta);
 void launch_minimize_step(sofia_ctx *c, double gamma, double max_disp);
 

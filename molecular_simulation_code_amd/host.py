@@ -852,9 +852,8 @@ class Engine:
 
     def _by_gid(self, arrays):
         """Split device-order (N, 3) arrays per replica, each re-ordered by global id."""
-        a = np.empty((self.N, 4), f32)
         gid = np.empty(self.N, i32)
-        check(lib().sofia_get_state(self.ctx, ptr(a), None, ptr(gid)))
+        check(lib().sofia_get_state(self.ctx, None, None, ptr(gid)))
         out = []
         off = 0
         for n in self.natoms:
@@ -864,11 +863,25 @@ class Engine:
             off += n
         return out
 
+    def _ordered(self, x=None, v=None, f=None) -> bool:
+        """Fill the (N, 3) arrays in global-id order on the device; False when some replica's
+        global ids are not a permutation (nothing is filled)."""
+        ok = C.c_int32()
+        check(lib().sofia_get_ordered_f64(self.ctx, ptr(x), ptr(v), ptr(f), C.byref(ok)))
+        return bool(ok.value)
+
+    def _split(self, arrays):
+        """The arrays' rows per replica (views)."""
+        off = np.concatenate([[0], np.cumsum(self.natoms)])
+        return [tuple(x[a:b] for x in arrays) for a, b in zip(off[:-1], off[1:])]
+
     def state(self):
         """FP64 positions/velocities per replica, in each replica's own original atom
         order (global_id order)."""
         x = np.empty((self.N, 3), f64)
         v = np.empty((self.N, 3), f64)
+        if self._ordered(x=x, v=v):
+            return self._split((x, v))
         check(lib().sofia_get_state_f64(self.ctx, ptr(x), ptr(v)))
         return self._by_gid((x, v))
 
@@ -885,6 +898,8 @@ class Engine:
         """Total force per replica after the last step (global_id order): the force the
         next step's first half-kick uses."""
         f = np.empty((self.N, 3), f64)
+        if self._ordered(f=f):
+            return [t[0] for t in self._split((f,))]
         check(lib().sofia_get_forces_f64(self.ctx, ptr(f)))
         return [t[0] for t in self._by_gid((f,))]
 
