@@ -24,22 +24,6 @@ namespace {
 
 constexpr int LIST_CAP = 4096;   // staged candidates per cell (64 KiB of LDS)
 
-__device__ inline int xyz2bin_dev(float4 p, const RepInfo &R) {
-    const double irn = 1.0 / (double)R.rn;
-    const double bx = (double)R.box;
-    const double c[3] = {(double)p.x, (double)p.y, (double)p.z};
-    int ix[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        int v = (c[d] < bx) ? (int)(c[d] * irn) : R.ncellD - 1;
-        // the reference clamps ncellD back into range; negative inputs are not produced
-        // by pbc() but are clamped here so a bad coordinate cannot index out of bounds
-        v = v >= R.ncellD ? R.ncellD - 1 : (v < 0 ? 0 : v);
-        ix[d] = v;
-    }
-    return ix[0] + ix[1] * R.ncellD + ix[2] * R.ncellD * R.ncellD;
-}
-
 // real*4 minimum image: (s + sign(2^23,s)) - sign(2^23,dx) is round-to-nearest-even of
 // s = dx*ibox for |s| < 2^22, i.e. rintf.
 __device__ inline float mimg32(float dx, float box, float ibox) {
@@ -53,25 +37,14 @@ __device__ inline float mimg32(float dx, float box, float ibox) {
 // with a fixed grid (at most GRID_CAP workgroups), which keeps such a step's launches short.
 constexpr int GRID_CAP = 2048;
 
-// The sort is three launches.  k_bin counts each cell's atoms and drops their ids into the
-// cell's bucket; k_sort_gather orders a cell and moves its atoms' data to the gather target;
+// The sort is three launches.  k_bin (in a step with bonded bundles k_bonded_bundles, which
+// shares its launch) counts each cell's atoms and drops their ids into the cell's bucket;
+// k_sort_gather orders a cell and moves its atoms' data to the gather target;
 // k_copyback puts them back (device pointers stay fixed, which keeps captured graphs valid),
 // re-indexes what names atoms and clears the binning counters for the next sort.
-__global__ void k_bin(int32_t n, const float4 *__restrict__ pos4, const int32_t *__restrict__ rep,
-                      const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
-                      const int32_t *__restrict__ any, int32_t *__restrict__ cbin,
-                      int32_t *__restrict__ acell, int32_t *__restrict__ bucket, int32_t cap) {
-    if (!*any) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const int r = rep[i];
-        // tt of a replica that rebuilds nothing is stale: every reader skips such replicas
-        if (!rebuild[r]) continue;
-        const RepInfo R = reps[r];
-        const int c = R.cell0 + xyz2bin_dev(pos4[i], R);
-        acell[i] = c;
-        const int slot = atomicAdd(&cbin[c], 1);
-        if (slot < cap) bucket[(size_t)c * cap + slot] = i;
-    }
+__global__ void k_bin(BinArgs A) {
+    if (!*A.any) return;
+    bin_atoms(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 // What the step's sort carries beyond the per-atom arrays (SORT_STEP), else null.
@@ -412,11 +385,7 @@ __global__ void k_set_flags(int32_t nrep, int32_t *__restrict__ rebuild, int32_t
 
 __global__ void k_finish(int32_t nrep, int32_t *__restrict__ rebuild, int32_t *__restrict__ nbuilds) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nrep && rebuild[r]) {
-        nbuilds[r] += 1;
-        rebuild[r] = 0;
-    }
-    if (r == nrep) rebuild[r] = 0;   // any
+    if (r <= nrep) finish_rebuild(r, nrep, rebuild, nbuilds);
 }
 
 // The end of a rebuild: the largest count to the host; if the lists fit, k_finish's books.
@@ -442,10 +411,12 @@ inline int nblk(int n, int b) { return (n + b - 1) / b; }
 inline int capped(int n, int b) { return std::max(1, std::min(nblk(n, b), GRID_CAP)); }
 inline const int32_t *any_flag(const sofia_ctx *c) { return c->rebuild + c->nrep; }
 
-void launch_sort(sofia_ctx *c, SortMode mode) {
-    hipLaunchKernelGGL(k_bin, dim3(capped(c->N, 256)), dim3(256), 0, c->stream, c->N, c->a.pos4,
-                       c->rep, c->reps_d, c->rebuild, any_flag(c), c->cbin, c->acell, c->bucket,
-                       c->bucket_cap);
+void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies) {
+    const BinArgs B{c->N, c->bucket_cap, c->a.pos4, c->rep, c->reps_d, c->rebuild, any_flag(c),
+                    c->cbin, c->acell, c->bucket};
+    const int bin_grid = capped(c->N, 256);
+    if (bonded) launch_bundles_bin(c, B, bin_grid, energies);
+    else hipLaunchKernelGGL(k_bin, dim3(bin_grid), dim3(256), 0, c->stream, B);
     StepArrays T{};
     if (mode == SORT_STEP) {
         const int rb = record_bytes(c);

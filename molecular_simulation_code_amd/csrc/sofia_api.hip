@@ -1615,12 +1615,13 @@ void force_sequence(sofia_ctx *c, bool energies) {
 // One MD step up to its last half kick, which the next step's k_advance applies (kick2) or,
 // at a segment's end, launch_nve_v64.
 void step_sequence(sofia_ctx *c, bool kick2, bool energies) {
+    const bool bonded = sort_takes_bonded(c);
     launch_advance(c, kick2);
-    launch_sort(c, SORT_STEP);
-    launch_build_list(c);
     if (energies) launch_zero_energies(c);
+    launch_sort(c, SORT_STEP, bonded, energies);
+    launch_build_list(c);
     launch_nonbond(c, nb_mode(c), energies, true);
-    launch_bonded_engine(c, energies);
+    if (!bonded) launch_bonded_engine(c, energies);
     launch_shake64(c, energies, true);
 }
 
@@ -2220,15 +2221,16 @@ int sofia_minimize(sofia_ctx *c, int32_t nsteps, double gamma, double max_disp) 
     const bool thermo = c->has_thermostat;
     c->has_thermostat = false;
     launch_zero_forces(c, c->fix, false);
+    const bool with_sort = sort_takes_bonded(c);   // after a move, the next one's bonded terms
     for (int s = 0; s < nsteps; ++s) {
         launch_nonbond(c, nb_mode(c), false, s > 0);
-        launch_bonded_engine(c, false);
+        if (s == 0 || !with_sort) launch_bonded_engine(c, false);
         launch_water_bonded(c);
         launch_minimize_step(c, gamma, max_disp);
-        launch_sort(c, SORT_STEP);
+        launch_sort(c, SORT_STEP, with_sort && s + 1 < nsteps);
         launch_build_list(c);
-        launch_finish_rebuild(c);
     }
+    if (nsteps > 0) launch_finish_rebuild(c);
     c->has_thermostat = thermo;
     force_sequence(c, true);
     TRY(collect_energies(c));

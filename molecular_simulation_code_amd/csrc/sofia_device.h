@@ -173,6 +173,50 @@ __device__ inline void write_record(int4 *pf, int i, double x, double y, double 
     }
 }
 
+__device__ inline int xyz2bin_dev(float4 p, const RepInfo &R) {
+    const double irn = 1.0 / (double)R.rn;
+    const double bx = (double)R.box;
+    const double c[3] = {(double)p.x, (double)p.y, (double)p.z};
+    int ix[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        int v = (c[d] < bx) ? (int)(c[d] * irn) : R.ncellD - 1;
+        // the reference clamps ncellD back into range; negative inputs are not produced
+        // by pbc() but are clamped here so a bad coordinate cannot index out of bounds
+        v = v >= R.ncellD ? R.ncellD - 1 : (v < 0 ? 0 : v);
+        ix[d] = v;
+    }
+    return ix[0] + ix[1] * R.ncellD + ix[2] * R.ncellD * R.ncellD;
+}
+
+// Binning: counts each cell's atoms and drops their ids into the cell's bucket.  tt of a
+// replica that rebuilds nothing is stale: every reader skips such replicas.
+struct BinArgs {
+    int32_t n, cap;
+    const float4 *pos4;
+    const int32_t *rep;
+    const RepInfo *reps;
+    const int32_t *rebuild, *any;
+    int32_t *cbin, *acell, *bucket;
+};
+__device__ inline void bin_atoms(const BinArgs &A, int t0, int stride) {
+    for (int i = t0; i < A.n; i += stride) {
+        const int r = A.rep[i];
+        if (!A.rebuild[r]) continue;
+        const RepInfo R = A.reps[r];
+        const int c = R.cell0 + xyz2bin_dev(A.pos4[i], R);
+        A.acell[i] = c;
+        const int slot = atomicAdd(&A.cbin[c], 1);
+        if (slot < A.cap) A.bucket[(size_t)c * A.cap + slot] = i;
+    }
+}
+
+// The books of a finished rebuild, replica r (r == nrep: the `any` flag).
+__device__ inline void finish_rebuild(int r, int nrep, int32_t *rebuild, int32_t *nbuilds) {
+    if (r < nrep && rebuild[r]) nbuilds[r] += 1;
+    rebuild[r] = 0;
+}
+
 inline int nblocks(long long n, int b) { return (int)((n + b - 1) / b); }
 
 }  // namespace sofia

@@ -261,7 +261,11 @@ namespace sofia {
 // state too, or (inside an engine step) also the fixed-point forces already set for the step
 // and the pair kernel's position records.
 enum SortMode { SORT_DROPIN = 0, SORT_ENGINE = 1, SORT_STEP = 2 };
-void launch_sort(sofia_ctx *c, SortMode mode);
+// bonded: with the step's bonded terms (where sort_takes_bonded)
+void launch_sort(sofia_ctx *c, SortMode mode, bool bonded = false, bool energies = false);
+bool sort_takes_bonded(const sofia_ctx *c);
+struct BinArgs;
+void launch_bundles_bin(sofia_ctx *c, const BinArgs &B, int bin_grid, bool energies);
 void launch_host_ids(sofia_ctx *c, const int32_t *src, int32_t *dst, size_t items, int width,
                      int nidx);
 void launch_rdf(sofia_ctx *c, int32_t itype, int32_t jtype, double delta, int32_t nbins,
@@ -310,7 +314,7 @@ void launch_langevin64(sofia_ctx *c);
 // step: the launch also ends the engine step (rebuild flags down, step counters on)
 void launch_shake64(sofia_ctx *c, bool energies, bool step = false);
 void launch_zero_energies(sofia_ctx *c);
-void launch_water_bonded(sofia_ctx *c);
+void launch_water_bonded(sofia_ctx *c);   // and the books of the rebuild before it
 void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst);
 void launch_put_state(sofia_ctx *c, bool v, bool q, bool gid);
 void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb);

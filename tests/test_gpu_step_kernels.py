@@ -146,3 +146,30 @@ def test_ordered_state_equals_the_host_reorder(permutation):
             assert np.array_equal(f[k], hf)
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("sizes", [((1, 1060),), ((19, 1000), (21, 1500)), ((90, 900), (1, 1400), (40, 2000))])
+def test_bonded_terms_with_the_sort_equal_those_after_it(sizes):
+    """The bundles run before the sort's binning moves anything, the per-item kernels after the
+    lists: the same integer forces and energies, so the minimised and the moving states agree
+    bit for bit, with one bundle and many, and replicas that rebuild at different steps."""
+    host = _host()
+    out = []
+    for mode in (0, 1):
+        e = host.Engine([host.ReplicaSpec(S.make_system(g, w, seed=60 + k), temp=300.0 + 200.0 * k,
+                                          gamma_ps=5.0, seed=k) for k, (g, w) in enumerate(sizes)])
+        try:
+            e.init()
+            e.set_bonded_mode(mode)
+            e.minimize(40)
+            built = e.rebuilds().tolist()
+            e.run(60)
+            out.append((e.state(), built, e.rebuilds().tolist(), e.energies()))
+        finally:
+            e.close()
+    (s0, m0, r0, e0), (s1, m1, r1, e1) = out
+    assert m0 == m1 and r0 == r1 and min(r0) > 1
+    for (x0, v0), (x1, v1) in zip(s0, s1):
+        np.testing.assert_array_equal(x0, x1)
+        np.testing.assert_array_equal(v0, v1)
+    np.testing.assert_array_equal(e0, e1)
