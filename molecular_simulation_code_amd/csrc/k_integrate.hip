@@ -7,6 +7,8 @@
 //    langevin_debug_intel (Source/mod_langevin.f90:15-43);
 //  * engine ("64"): the same algorithms on FP64 positions and velocities, with forces read
 //    as FP64 nonbond sums + int64 fixed-point sums of every other term.
+#include <type_traits>
+
 #include "sofia_device.h"
 
 namespace sofia {
@@ -191,169 +193,199 @@ __global__ void k_langevin32(int32_t n, const float4 *__restrict__ pos4, const f
 // shake4 (0,1),(0,2),(0,3), shake3angle (0,1),(0,2),(1,2).  The Lagrange multipliers solve
 // |s_k + sum_l cpl[k][l] lambda_l r_l|^2 = d_k^2 by the reference's iteration: linear
 // system with the quadratic terms lagged, stopped when every |delta lambda| <= tol.
-struct ShakeCluster {
-    int nc;          // constraints
-    int P[3], Q[3];
-    int idx[4];
-    double im[4];
-    double bl[3];
-};
+// The solver is instantiated per cluster kind, so that the constraint topology is known at
+// compile time and the arrays stay in registers.  Cluster atoms are exclusive to their cluster.
+template <int KIND> __device__ constexpr int topo_nc() { return KIND == 1 ? 1 : (KIND == 3 ? 2 : 3); }
+template <int KIND> __device__ constexpr int topo_na() { return KIND == 1 ? 2 : (KIND == 4 ? 4 : 3); }
+template <int KIND> __device__ constexpr int topo_p(int k) { return (KIND == -3 && k == 2) ? 1 : 0; }
+template <int KIND> __device__ constexpr int topo_q(int k) { return (KIND == -3 && k == 2) ? 2 : k + 1; }
 
-__device__ inline bool shake_solve(const ShakeCluster &S, const double (*r)[3], const double (*s)[3],
-                                   double tol, int maxiter, double lam[3], int *iters) {
-    if (S.nc == 1) {   // shake2: closed-form root of the quadratic (Source/mod_shake.f90:133-168)
+template <int KIND>
+__device__ inline bool shake_solve_t(const double *im, const double *bl, const double (*r)[3],
+                                     const double (*s)[3], double tol, int maxiter, double *lam,
+                                     int *iters) {
+    constexpr int NC = topo_nc<KIND>();
+    if constexpr (NC == 1) {   // closed-form root of the quadratic (Source/mod_shake.f90:133-168)
         const double r01sq = r[0][0] * r[0][0] + r[0][1] * r[0][1] + r[0][2] * r[0][2];
         const double s01sq = s[0][0] * s[0][0] + s[0][1] * s[0][1] + s[0][2] * s[0][2];
-        const double ims = S.im[0] + S.im[1];
+        const double ims = im[0] + im[1];
         const double a = ims * ims * r01sq;
         const double b = 2.0 * ims * (s[0][0] * r[0][0] + s[0][1] * r[0][1] + s[0][2] * r[0][2]);
-        const double cc = s01sq - S.bl[0] * S.bl[0];
+        const double cc = s01sq - bl[0] * bl[0];
         const double det = b * b - 4.0 * a * cc;
         if (det < 0.0) return false;
         const double l1 = (-b + sqrt(det)) / (2.0 * a), l2 = (-b - sqrt(det)) / (2.0 * a);
         lam[0] = (fabs(l1) <= fabs(l2)) ? l1 : l2;
         *iters = 1;
         return true;
-    }
-    const int nc = S.nc;
-    double cpl[3][3], A[3][3], G[3][3], ssq[3];
-    for (int k = 0; k < nc; ++k) {
-        ssq[k] = s[k][0] * s[k][0] + s[k][1] * s[k][1] + s[k][2] * s[k][2];
-        for (int l = 0; l < nc; ++l) {
-            double c = 0.0;
-            if (S.P[k] == S.P[l]) c += S.im[S.P[k]];
-            if (S.P[k] == S.Q[l]) c -= S.im[S.P[k]];
-            if (S.Q[k] == S.P[l]) c -= S.im[S.Q[k]];
-            if (S.Q[k] == S.Q[l]) c += S.im[S.Q[k]];
-            cpl[k][l] = c;
-            A[k][l] = 2.0 * c * (s[k][0] * r[l][0] + s[k][1] * r[l][1] + s[k][2] * r[l][2]);
-            G[k][l] = r[k][0] * r[l][0] + r[k][1] * r[l][1] + r[k][2] * r[l][2];
-        }
-    }
-    double Ai[3][3];
-    if (nc == 2) {
-        const double det = A[0][0] * A[1][1] - A[0][1] * A[1][0];
-        if (det == 0.0) return false;
-        const double di = 1.0 / det;
-        Ai[0][0] = A[1][1] * di; Ai[0][1] = -A[0][1] * di;
-        Ai[1][0] = -A[1][0] * di; Ai[1][1] = A[0][0] * di;
     } else {
-        const double det = A[0][0] * A[1][1] * A[2][2] + A[0][1] * A[1][2] * A[2][0] +
-                           A[0][2] * A[1][0] * A[2][1] - A[0][0] * A[1][2] * A[2][1] -
-                           A[0][1] * A[1][0] * A[2][2] - A[0][2] * A[1][1] * A[2][0];
-        if (det == 0.0) return false;
-        const double di = 1.0 / det;
-        Ai[0][0] = di * (A[1][1] * A[2][2] - A[1][2] * A[2][1]);
-        Ai[0][1] = -di * (A[0][1] * A[2][2] - A[0][2] * A[2][1]);
-        Ai[0][2] = di * (A[0][1] * A[1][2] - A[0][2] * A[1][1]);
-        Ai[1][0] = -di * (A[1][0] * A[2][2] - A[1][2] * A[2][0]);
-        Ai[1][1] = di * (A[0][0] * A[2][2] - A[0][2] * A[2][0]);
-        Ai[1][2] = -di * (A[0][0] * A[1][2] - A[0][2] * A[1][0]);
-        Ai[2][0] = di * (A[1][0] * A[2][1] - A[1][1] * A[2][0]);
-        Ai[2][1] = -di * (A[0][0] * A[2][1] - A[0][1] * A[2][0]);
-        Ai[2][2] = di * (A[0][0] * A[1][1] - A[0][1] * A[1][0]);
+        double cpl[NC][NC], A[NC][NC], G[NC][NC], ssq[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            ssq[k] = s[k][0] * s[k][0] + s[k][1] * s[k][1] + s[k][2] * s[k][2];
+#pragma unroll
+            for (int l = 0; l < NC; ++l) {
+                double c = 0.0;
+                if (topo_p<KIND>(k) == topo_p<KIND>(l)) c += im[topo_p<KIND>(k)];
+                if (topo_p<KIND>(k) == topo_q<KIND>(l)) c -= im[topo_p<KIND>(k)];
+                if (topo_q<KIND>(k) == topo_p<KIND>(l)) c -= im[topo_q<KIND>(k)];
+                if (topo_q<KIND>(k) == topo_q<KIND>(l)) c += im[topo_q<KIND>(k)];
+                cpl[k][l] = c;
+                A[k][l] = 2.0 * c * (s[k][0] * r[l][0] + s[k][1] * r[l][1] + s[k][2] * r[l][2]);
+                G[k][l] = r[k][0] * r[l][0] + r[k][1] * r[l][1] + r[k][2] * r[l][2];
+            }
+        }
+        double Ai[NC][NC];
+        if constexpr (NC == 2) {
+            const double det = A[0][0] * A[1][1] - A[0][1] * A[1][0];
+            if (det == 0.0) return false;
+            const double di = 1.0 / det;
+            Ai[0][0] = A[1][1] * di; Ai[0][1] = -A[0][1] * di;
+            Ai[1][0] = -A[1][0] * di; Ai[1][1] = A[0][0] * di;
+        } else {
+            const double det = A[0][0] * A[1][1] * A[2][2] + A[0][1] * A[1][2] * A[2][0] +
+                               A[0][2] * A[1][0] * A[2][1] - A[0][0] * A[1][2] * A[2][1] -
+                               A[0][1] * A[1][0] * A[2][2] - A[0][2] * A[1][1] * A[2][0];
+            if (det == 0.0) return false;
+            const double di = 1.0 / det;
+            Ai[0][0] = di * (A[1][1] * A[2][2] - A[1][2] * A[2][1]);
+            Ai[0][1] = -di * (A[0][1] * A[2][2] - A[0][2] * A[2][1]);
+            Ai[0][2] = di * (A[0][1] * A[1][2] - A[0][2] * A[1][1]);
+            Ai[1][0] = -di * (A[1][0] * A[2][2] - A[1][2] * A[2][0]);
+            Ai[1][1] = di * (A[0][0] * A[2][2] - A[0][2] * A[2][0]);
+            Ai[1][2] = -di * (A[0][0] * A[1][2] - A[0][2] * A[1][0]);
+            Ai[2][0] = di * (A[1][0] * A[2][1] - A[1][1] * A[2][0]);
+            Ai[2][1] = -di * (A[0][0] * A[2][1] - A[0][1] * A[2][0]);
+            Ai[2][2] = di * (A[0][0] * A[1][1] - A[0][1] * A[1][0]);
+        }
+#pragma unroll
+        for (int k = 0; k < NC; ++k) lam[k] = 0.0;
+        int it = 0;
+        bool done = false;
+        while (!done && it < maxiter) {
+            double bb[NC], nl[NC];
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                double qd = 0.0;
+#pragma unroll
+                for (int l = 0; l < NC; ++l)
+#pragma unroll
+                    for (int m = 0; m < NC; ++m) qd += cpl[k][l] * cpl[k][m] * G[l][m] * lam[l] * lam[m];
+                bb[k] = bl[k] * bl[k] - ssq[k] - qd;
+            }
+            done = true;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                double v = 0.0;
+#pragma unroll
+                for (int l = 0; l < NC; ++l) v += Ai[k][l] * bb[l];
+                nl[k] = v;
+            }
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {
+                if (fabs(nl[k] - lam[k]) > tol) done = false;
+                lam[k] = nl[k];
+            }
+            ++it;
+        }
+        *iters = it;
+        return true;
     }
-    lam[0] = lam[1] = lam[2] = 0.0;
-    int it = 0;
-    bool done = false;
-    while (!done && it < maxiter) {
-        double bb[3], nl[3];
-        for (int k = 0; k < nc; ++k) {
-            double qd = 0.0;
-            for (int l = 0; l < nc; ++l)
-                for (int m = 0; m < nc; ++m) qd += cpl[k][l] * cpl[k][m] * G[l][m] * lam[l] * lam[m];
-            bb[k] = S.bl[k] * S.bl[k] - ssq[k] - qd;
-        }
-        done = true;
-        for (int k = 0; k < nc; ++k) {
-            double v = 0.0;
-            for (int l = 0; l < nc; ++l) v += Ai[k][l] * bb[l];
-            nl[k] = v;
-        }
-        for (int k = 0; k < nc; ++k) {
-            if (fabs(nl[k] - lam[k]) > tol) done = false;
-            lam[k] = nl[k];
-        }
-        ++it;
-    }
-    *iters = it;
-    return true;
 }
 
-__device__ inline ShakeCluster make_cluster(int num, const int32_t *at, const double *bd,
-                                            const double *mass, const float4 *pos4) {
-    ShakeCluster S;
-    for (int k = 0; k < 4; ++k) {
-        S.idx[k] = at[k];
-        S.im[k] = (at[k] >= 0) ? 1.0 / mass[__float_as_int(pos4[at[k]].w) - 1] : 0.0;
+// One cluster of the drop-in SHAKE.  Returns the iterations, or -1 where the system has no
+// solution; adds to the virial.
+template <int KIND>
+__device__ inline int shake32_cluster(const int4 at, const double *__restrict__ bond,
+                                      const float4 *__restrict__ pos4, const float *__restrict__ v,
+                                      float *__restrict__ ff, const double4 *__restrict__ mtab,
+                                      float box, float ibox, float dt, double dtsq, double tol,
+                                      int maxiter, double vir[3]) {
+    constexpr int NA = topo_na<KIND>(), NC = topo_nc<KIND>();
+    const int all[4] = {at.x, at.y, at.z, at.w};
+    double im[NA], bl[3], xs[NA][3];
+    float pp[NA][3], f[NA][3];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+        const size_t i = (size_t)all[a];
+        const float4 p = pos4[i];
+        im[a] = mtab[__float_as_int(p.w) - 1].w;
+        pp[a][0] = p.x; pp[a][1] = p.y; pp[a][2] = p.z;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            f[a][c] = ff[3 * i + c];
+            xs[a][c] = (double)(pp[a][c] + dt * v[3 * i + c]) + dtsq * im[a] * (double)f[a][c];
+        }
     }
-    for (int k = 0; k < 3; ++k) S.bl[k] = bd[k];
-    if (num == 1) {
-        S.nc = 1; S.P[0] = 0; S.Q[0] = 1;
-    } else if (num == 3) {
-        S.nc = 2; S.P[0] = 0; S.Q[0] = 1; S.P[1] = 0; S.Q[1] = 2;
-    } else if (num == 4) {
-        S.nc = 3; S.P[0] = 0; S.Q[0] = 1; S.P[1] = 0; S.Q[1] = 2; S.P[2] = 0; S.Q[2] = 3;
-    } else {   // -3: rigid triangle, constraints 0-1, 0-2, 1-2
-        S.nc = 3; S.P[0] = 0; S.Q[0] = 1; S.P[1] = 0; S.Q[1] = 2; S.P[2] = 1; S.Q[2] = 2;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) bl[k] = bond[k];
+    double r[NC][3], s[NC][3], lam[NC];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const int a = topo_p<KIND>(k), b = topo_q<KIND>(k);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const double d = (double)(pp[a][c] - pp[b][c]);
+            r[k][c] = d - (double)(box * (float)(int)round((double)ibox * d));
+            const double e = xs[a][c] - xs[b][c];
+            s[k][c] = e - (double)(box * (float)(int)round((double)ibox * e));
+        }
     }
-    return S;
+    int its = 0;
+    if (!shake_solve_t<KIND>(im, bl, r, s, tol, maxiter, lam, &its)) return -1;
+    // the force is real*4 after every constraint, as in the reference
+#pragma unroll
+    for (int k = 0; k < NC; ++k) {
+        const double l = lam[k] / dtsq;
+        const int a = topo_p<KIND>(k), b = topo_q<KIND>(k);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            f[a][c] = (float)((double)f[a][c] + l * r[k][c]);
+            f[b][c] = (float)((double)f[b][c] - l * r[k][c]);
+            vir[c] += r[k][c] * r[k][c] * l;
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) ff[3 * (size_t)all[a] + c] = f[a][c];
+    return its;
 }
 
-// drop-in: real*4 positions/velocities/forces, FP64 solve (Source/mod_shake.f90:8-85, 888-913)
-__global__ void k_shake32(int32_t ns, const int32_t *__restrict__ num, const int32_t *__restrict__ atoms,
-                          const double *__restrict__ bond, const float4 *__restrict__ pos4,
-                          const float *__restrict__ v, float *__restrict__ ff,
-                          const double *__restrict__ mass, const int32_t *__restrict__ rep,
-                          const RepInfo *__restrict__ reps, float dt, double dtsq, double tol,
-                          int maxiter, int32_t *__restrict__ err, int32_t *__restrict__ iters_max,
-                          long long *__restrict__ eacc) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
+// drop-in: real*4 positions/velocities/forces, FP64 solve (Source/mod_shake.f90:8-85, 888-913).
+// Few wavefronts (one per SIMD at 204,000 atoms) walk a chain of FP64 steps, so the time is that
+// chain's: with the solver's arrays indexed by the cluster's kind at run time, in scratch, it
+// took 54 us at 13,500 atoms and 83 at 204,000; with one instance per kind and one iteration
+// count per wavefront 10 and 21.
+__global__ void __launch_bounds__(64)
+k_shake32(int32_t ns, const int32_t *__restrict__ num, const int4 *__restrict__ atoms,
+          const double *__restrict__ bond, const float4 *__restrict__ pos4,
+          const float *__restrict__ v, float *__restrict__ ff, const double4 *__restrict__ mtab,
+          const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps, float dt, double dtsq,
+          double tol, int maxiter, int32_t *__restrict__ err, int32_t *__restrict__ iters_max,
+          long long *__restrict__ eacc) {
+    const int m = blockIdx.x * 64 + threadIdx.x;
     const bool live = m < ns;
     double vir[3] = {0.0, 0.0, 0.0};
-    int rr = 0;
+    int rr = 0, its = 0;
     if (live) {
-        const ShakeCluster S = make_cluster(num[m], atoms + 4 * (size_t)m, bond + 3 * (size_t)m, mass, pos4);
-        rr = rep[S.idx[0]];
+        const int kind = num[m];
+        const int4 at = atoms[m];
+        rr = rep[at.x];
         const float box = reps[rr].box, ibox = reps[rr].ibox;
-        double xs[4][3];
-        for (int a = 0; a < 4; ++a) {
-            if (S.idx[a] < 0) continue;
-            const int i = S.idx[a];
-            const float4 p = pos4[i];
-            const float pp[3] = {p.x, p.y, p.z};
-            for (int c = 0; c < 3; ++c)
-                xs[a][c] = (double)(pp[c] + dt * v[3 * (size_t)i + c]) +
-                           dtsq * S.im[a] * (double)ff[3 * (size_t)i + c];
-        }
-        double r[3][3], s[3][3];
-        for (int k = 0; k < S.nc; ++k) {
-            const float4 pa = pos4[S.idx[S.P[k]]], pb = pos4[S.idx[S.Q[k]]];
-            const float df[3] = {pa.x - pb.x, pa.y - pb.y, pa.z - pb.z};
-            for (int c = 0; c < 3; ++c) {
-                const double d = (double)df[c];
-                r[k][c] = d - (double)(box * (float)(int)round((double)ibox * d));
-                const double e = xs[S.P[k]][c] - xs[S.Q[k]][c];
-                s[k][c] = e - (double)(box * (float)(int)round((double)ibox * e));
-            }
-        }
-        double lam[3];
-        int its = 0;
-        if (!shake_solve(S, r, s, tol, maxiter, lam, &its)) {
-            atomicOr(err, 1);
-        } else {
-            atomicMax(iters_max, its);
-            for (int k = 0; k < S.nc; ++k) {
-                const double l = lam[k] / dtsq;
-                const int a = S.idx[S.P[k]], b = S.idx[S.Q[k]];
-                for (int c = 0; c < 3; ++c) {
-                    ff[3 * (size_t)a + c] = (float)((double)ff[3 * (size_t)a + c] + l * r[k][c]);
-                    ff[3 * (size_t)b + c] = (float)((double)ff[3 * (size_t)b + c] - l * r[k][c]);
-                    vir[c] += r[k][c] * r[k][c] * l;
-                }
-            }
-        }
+        auto solve = [&](auto k) {
+            its = shake32_cluster<decltype(k)::value>(at, bond + 3 * (size_t)m, pos4, v, ff, mtab, box,
+                                                      ibox, dt, dtsq, tol, maxiter, vir);
+        };
+        if (kind == 1) solve(std::integral_constant<int, 1>{});
+        else if (kind == 3) solve(std::integral_constant<int, 3>{});
+        else if (kind == 4) solve(std::integral_constant<int, 4>{});
+        else solve(std::integral_constant<int, -3>{});   // rigid triangle
+        if (its < 0) atomicOr(err, 1);
     }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) its = max(its, __shfl_xor(its, off, 64));
+    if (threadIdx.x == 0 && its > 0) atomicMax(iters_max, its);
     wave_add(to_efix(vir[0]), live, rr, eacc, V_X);
     wave_add(to_efix(vir[1]), live, rr, eacc, V_Y);
     wave_add(to_efix(vir[2]), live, rr, eacc, V_Z);
@@ -501,107 +533,6 @@ __global__ void k_langevin64(int32_t n, const float4 *__restrict__ pos4, const d
     for (int c = 0; c < 3; ++c) {
         const size_t o = (size_t)c * n + i;
         fix[o] += to_fix(-R.fric * m * vd[o] + R.gconst * sqrt(m) * (double)u[c]);
-    }
-}
-
-// Engine SHAKE.  The solver is instantiated per cluster kind so the constraint topology is
-// known at compile time (the arrays stay in registers); the arithmetic is the one of
-// shake_solve.  Cluster atoms are exclusive to their cluster.
-template <int KIND> __device__ constexpr int topo_nc() { return KIND == 1 ? 1 : (KIND == 3 ? 2 : 3); }
-template <int KIND> __device__ constexpr int topo_na() { return KIND == 1 ? 2 : (KIND == 4 ? 4 : 3); }
-template <int KIND> __device__ constexpr int topo_p(int k) { return (KIND == -3 && k == 2) ? 1 : 0; }
-template <int KIND> __device__ constexpr int topo_q(int k) { return (KIND == -3 && k == 2) ? 2 : k + 1; }
-
-template <int KIND>
-__device__ inline bool shake_solve_t(const double *im, const double *bl, const double (*r)[3],
-                                     const double (*s)[3], double tol, int maxiter, double *lam,
-                                     int *iters) {
-    constexpr int NC = topo_nc<KIND>();
-    if constexpr (NC == 1) {
-        const double r01sq = r[0][0] * r[0][0] + r[0][1] * r[0][1] + r[0][2] * r[0][2];
-        const double s01sq = s[0][0] * s[0][0] + s[0][1] * s[0][1] + s[0][2] * s[0][2];
-        const double ims = im[0] + im[1];
-        const double a = ims * ims * r01sq;
-        const double b = 2.0 * ims * (s[0][0] * r[0][0] + s[0][1] * r[0][1] + s[0][2] * r[0][2]);
-        const double cc = s01sq - bl[0] * bl[0];
-        const double det = b * b - 4.0 * a * cc;
-        if (det < 0.0) return false;
-        const double l1 = (-b + sqrt(det)) / (2.0 * a), l2 = (-b - sqrt(det)) / (2.0 * a);
-        lam[0] = (fabs(l1) <= fabs(l2)) ? l1 : l2;
-        *iters = 1;
-        return true;
-    } else {
-        double cpl[NC][NC], A[NC][NC], G[NC][NC], ssq[NC];
-#pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            ssq[k] = s[k][0] * s[k][0] + s[k][1] * s[k][1] + s[k][2] * s[k][2];
-#pragma unroll
-            for (int l = 0; l < NC; ++l) {
-                double c = 0.0;
-                if (topo_p<KIND>(k) == topo_p<KIND>(l)) c += im[topo_p<KIND>(k)];
-                if (topo_p<KIND>(k) == topo_q<KIND>(l)) c -= im[topo_p<KIND>(k)];
-                if (topo_q<KIND>(k) == topo_p<KIND>(l)) c -= im[topo_q<KIND>(k)];
-                if (topo_q<KIND>(k) == topo_q<KIND>(l)) c += im[topo_q<KIND>(k)];
-                cpl[k][l] = c;
-                A[k][l] = 2.0 * c * (s[k][0] * r[l][0] + s[k][1] * r[l][1] + s[k][2] * r[l][2]);
-                G[k][l] = r[k][0] * r[l][0] + r[k][1] * r[l][1] + r[k][2] * r[l][2];
-            }
-        }
-        double Ai[NC][NC];
-        if constexpr (NC == 2) {
-            const double det = A[0][0] * A[1][1] - A[0][1] * A[1][0];
-            if (det == 0.0) return false;
-            const double di = 1.0 / det;
-            Ai[0][0] = A[1][1] * di; Ai[0][1] = -A[0][1] * di;
-            Ai[1][0] = -A[1][0] * di; Ai[1][1] = A[0][0] * di;
-        } else {
-            const double det = A[0][0] * A[1][1] * A[2][2] + A[0][1] * A[1][2] * A[2][0] +
-                               A[0][2] * A[1][0] * A[2][1] - A[0][0] * A[1][2] * A[2][1] -
-                               A[0][1] * A[1][0] * A[2][2] - A[0][2] * A[1][1] * A[2][0];
-            if (det == 0.0) return false;
-            const double di = 1.0 / det;
-            Ai[0][0] = di * (A[1][1] * A[2][2] - A[1][2] * A[2][1]);
-            Ai[0][1] = -di * (A[0][1] * A[2][2] - A[0][2] * A[2][1]);
-            Ai[0][2] = di * (A[0][1] * A[1][2] - A[0][2] * A[1][1]);
-            Ai[1][0] = -di * (A[1][0] * A[2][2] - A[1][2] * A[2][0]);
-            Ai[1][1] = di * (A[0][0] * A[2][2] - A[0][2] * A[2][0]);
-            Ai[1][2] = -di * (A[0][0] * A[1][2] - A[0][2] * A[1][0]);
-            Ai[2][0] = di * (A[1][0] * A[2][1] - A[1][1] * A[2][0]);
-            Ai[2][1] = -di * (A[0][0] * A[2][1] - A[0][1] * A[2][0]);
-            Ai[2][2] = di * (A[0][0] * A[1][1] - A[0][1] * A[1][0]);
-        }
-#pragma unroll
-        for (int k = 0; k < NC; ++k) lam[k] = 0.0;
-        int it = 0;
-        bool done = false;
-        while (!done && it < maxiter) {
-            double bb[NC], nl[NC];
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                double qd = 0.0;
-#pragma unroll
-                for (int l = 0; l < NC; ++l)
-#pragma unroll
-                    for (int m = 0; m < NC; ++m) qd += cpl[k][l] * cpl[k][m] * G[l][m] * lam[l] * lam[m];
-                bb[k] = bl[k] * bl[k] - ssq[k] - qd;
-            }
-            done = true;
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                double v = 0.0;
-#pragma unroll
-                for (int l = 0; l < NC; ++l) v += Ai[k][l] * bb[l];
-                nl[k] = v;
-            }
-#pragma unroll
-            for (int k = 0; k < NC; ++k) {
-                if (fabs(nl[k] - lam[k]) > tol) done = false;
-                lam[k] = nl[k];
-            }
-            ++it;
-        }
-        *iters = it;
-        return true;
     }
 }
 
@@ -1111,8 +1042,8 @@ void launch_shake32(sofia_ctx *c, int iflag, float *ff, double *) {
     if (!c->ns) return;
     const float dt = c->dp.dt, k2a = c->dp.kcal2amu;
     const double dtsq = (iflag == 0) ? (double)(((0.5f * dt) * dt) * k2a) : (double)((dt * dt) * k2a);
-    hipLaunchKernelGGL(k_shake32, dim3(nblocks(c->ns, 128)), dim3(128), 0, c->stream, c->ns,
-                       c->shake_num, c->shake_atoms, c->shake_bond, c->a.pos4, c->a.v32, ff, c->mass,
+    hipLaunchKernelGGL(k_shake32, dim3(nblocks(c->ns, 64)), dim3(64), 0, c->stream, c->ns, c->shake_num,
+                       (const int4 *)c->shake_atoms, c->shake_bond, c->a.pos4, c->a.v32, ff, c->mtab,
                        c->rep, c->reps_d, dt, dtsq, c->dp.shake_tol, c->dp.shake_maxiter,
                        c->shake_err, c->shake_iters, c->eacc);
 }

@@ -173,3 +173,36 @@ def test_bonded_terms_with_the_sort_equal_those_after_it(sizes):
         np.testing.assert_array_equal(x0, x1)
         np.testing.assert_array_equal(v0, v1)
     np.testing.assert_array_equal(e0, e1)
+
+
+@pytest.mark.parametrize("ns", [1, 63, 64, 65, 129])
+def test_dropin_shake_of_mixed_kinds(ns):
+    """Clusters of all four kinds shuffled within wavefronts, at the edges of one.  The solve
+    is FP64; the real*4 force rounds once per constraint, at most three times an atom, so the
+    oracle's is met within 3 x 2^-23 of the largest force, with the same iteration count."""
+    host = _host()
+    from oracle import oracle as O
+    s = S.make_system(16, 160, seed=31, params=S.Params(rcut=5.5, cut_coul=5.5, pad=1.0))
+    rng = np.random.default_rng(ns)
+    kinds = [np.where(s.shake_num == k)[0] for k in (-3, 3, 4)]
+    pick = np.concatenate([kinds[2], kinds[1], kinds[0]])[:max(ns, 1)] if ns > 1 else kinds[0][:1]
+    pick = rng.permutation(pick)
+    s.shake_num, s.shake_atoms, s.shake_bond = (np.ascontiguousarray(a[pick]) for a in
+                                                (s.shake_num, s.shake_atoms, s.shake_bond))
+    one = np.where(s.shake_num == 3)[0][::2]      # two-bond clusters cut to their first bond
+    s.shake_num[one] = 1
+    g = host.SofiaGPU(s)
+    try:
+        d, mass = s.derived(), S.type_mass()
+        ff0 = (rng.standard_normal((s.np, 3)) * 10).astype(np.float32)
+        g.ff = ff0.copy()
+        ref, vir, st, its = O.shake(1, g.position, g.type, g.v, ff0, mass, d["dt"], S.KCAL2AMU,
+                                    d["box"], d["ibox"], s.shake_num, s.shake_atoms, s.shake_bond,
+                                    float(S.SHAKE_TOL), S.SHAKE_MAXITER)
+        g.virial = np.zeros(3)
+        g.shake(1)
+        assert st == 0 and g.shake_iters == its
+        assert np.abs(g.ff - ref).max() <= 3 * 2.0 ** -23 * np.abs(ref).max()
+        np.testing.assert_allclose(g.virial, vir, rtol=1e-6)
+    finally:
+        g.close()
