@@ -68,6 +68,14 @@ void drop_graph(sofia_ctx *c) {
     c->graphk = nullptr;
 }
 
+// hipMemset returns before the device has cleared the memory, and does so on the null stream,
+// for which the contexts' streams (non-blocking) do not wait: whoever clears memory with it
+// settles before a stream may use the memory.
+int settle() {
+    SOFIA_HIP(hipStreamSynchronize(nullptr));
+    return SOFIA_OK;
+}
+
 // Arrays of one context that are never re-sized, carved out of one allocation: dozens of
 // allocations made a context's creation and, with a device synchronisation per free, its
 // destruction cost milliseconds.
@@ -79,12 +87,12 @@ public:
         parts_.push_back({(void **)p, total_});
         total_ += ((count ? count : 1) * sizeof(T) + 255) / 256 * 256;
     }
-    // one zeroed allocation, owned by the context
-    int make(sofia_ctx *c) {
+    // one allocation, owned by the context (zero: cleared, once settled)
+    int make(sofia_ctx *c, bool zero) {
         char *base = nullptr;
         TRY(dalloc(&base, total_));
         c->blocks.push_back(base);
-        SOFIA_HIP(hipMemset(base, 0, total_));
+        if (zero) SOFIA_HIP(hipMemset(base, 0, total_));
         for (auto &x : parts_) *x.first = base + x.second;
         return SOFIA_OK;
     }
@@ -214,6 +222,7 @@ int size_cells(sofia_ctx *c, int ncell) {
         SOFIA_HIP(hipMemset(c->ccount, 0, sizeof(int32_t) * ncell));
         SOFIA_HIP(hipMemset(c->cstart, 0, sizeof(int32_t) * ncell));
         SOFIA_HIP(hipMemset(c->cbin, 0, sizeof(int32_t) * ncell));
+        TRY(settle());
         c->ncell_cap = ncell;
     }
     int mean = 0;
@@ -304,7 +313,7 @@ int unsplit_water(sofia_ctx *c) {
     c->nbe = c->nae = 0;
     if (c->water) SOFIA_HIP(hipMemset(c->water, 0, sizeof(int4) * c->ns));
     c->water_split = false;
-    return SOFIA_OK;
+    return settle();
 }
 
 int split_water(sofia_ctx *c) {
@@ -501,9 +510,10 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
     B.want(&c->eacc, eacc_len(nrep));
     B.want(&c->step_d, nrep);
     B.want(&c->reps_d, nrep);
-    TRY(B.make(c.get()));
+    TRY(B.make(c.get(), true));
     TRY(clear_atoms(c->a, n));
     TRY(clear_atoms(c->b, n));
+    TRY(settle());
     TRY(size_cells(c.get(), c->ncell_total));
     const size_t words = sizeof(sofia::HostWords) + sizeof(long long) * (size_t)nrep * NE;
     SOFIA_HIP(hipHostMalloc((void **)&c->hw, words, hipHostMallocDefault));
@@ -1010,6 +1020,7 @@ int sofia_set_shake(sofia_ctx *c, int32_t ns, const int32_t *ns_rep, const int32
     for (int q = 0; q < 5; ++q) c->shake_kcount[q] = 0;
     TRY(sync_check(c));
     SOFIA_HIP(hipMemset(c->a.wclus, 0xff, sizeof(int32_t) * c->N));   // no SETTLE waters yet
+    TRY(settle());
     c->ns = 0;
     if (!ns) return SOFIA_OK;
     for (int k = 0; k < ns; ++k)
@@ -1030,6 +1041,7 @@ int sofia_set_shake(sofia_ctx *c, int32_t ns, const int32_t *ns_rep, const int32
     TRY(upload(c->shake_bond, bond, sizeof(double) * 3 * ns));
     TRY(dalloc(&c->water, ns));
     SOFIA_HIP(hipMemset(c->water, 0, sizeof(int4) * ns));
+    TRY(settle());
     c->ns = ns;
     return SOFIA_OK;
 }
@@ -2050,7 +2062,7 @@ int snapshot_take(sofia_ctx *c) {
         B.want(&c->snap_fix, 3 * n);
         B.want(&c->snap_step, c->nrep);
         B.want(&c->snap_nbuilds, c->nrep);
-        TRY(B.make(c));
+        TRY(B.make(c, false));   // the copies below fill it
     }
     size_t topo = 0;
     for (auto &l : sorted_lists(c)) topo += l.first ? l.second : 0;
