@@ -1817,16 +1817,14 @@ int classify_shake(sofia_ctx *c) {
     return upload(c->a.wclus, wclus.data(), sizeof(int32_t) * wclus.size());
 }
 
-// Charges by atom type (and fewer than 2^24 atoms)?  Then the mixed pair kernel reads
-// 12-byte position records and takes C q_i q_j from a per-type-pair table, formed in float32
-// exactly as the kernel forms it from per-atom charges ((C q_i) q_j), so the forces do not
-// change.
+// Charges by atom type (and fewer than 2^24 atoms)?  Then the pair kernels take C q_i q_j from
+// a per-type-pair table, formed exactly as from per-atom charges ((C q_i) q_j, in float32 or,
+// in the FP64 kernel, from the table's charges), so the forces do not change, and the mixed
+// kernel reads 12-byte position records.
 int classify_charges(sofia_ctx *c) {
     c->q_by_type = false;
     // 12-byte record offsets are formed with a 24-bit multiply: fewer than 2^24 atoms
-    if (c->p.precision != SOFIA_PREC_MIXED || c->p.coul_flag == SOFIA_COUL_EWALD || c->lj_host.empty() ||
-        c->N >= (1 << 24))
-        return SOFIA_OK;
+    if (c->lj_host.empty() || c->N >= (1 << 24)) return SOFIA_OK;
     TRY(sync_check(c));
     const int n = c->N, nt = c->p.ntypes;
     std::vector<float> q(n);
@@ -1851,7 +1849,7 @@ int classify_charges(sofia_ctx *c) {
             const float4 l = c->lj_host[(size_t)a * nt + b];
             volatile float qc = c->dp.coulpre * qt[a];
             volatile float qq = qc * qt[b];
-            pt[(size_t)a * nt + b] = make_float4(l.x, l.y, qq, 0.0f);
+            pt[(size_t)a * nt + b] = make_float4(l.x, l.y, qq, qt[b]);
         }
     if (!c->ptab) TRY(dalloc(&c->ptab, pt.size()));
     TRY(upload(c->ptab, pt.data(), sizeof(float4) * pt.size()));

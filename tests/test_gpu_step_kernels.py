@@ -206,3 +206,34 @@ def test_dropin_shake_of_mixed_kinds(ns):
         np.testing.assert_allclose(g.virial, vir, rtol=1e-6)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("ewald", [False, True])
+@pytest.mark.parametrize("ng,nw", [(1, 1060), (7, 1337)])
+def test_charges_by_type_in_the_fp64_and_ewald_kernels(ewald, ng, nw):
+    """One atom's charge a last bit off makes the kernels read every atom's own charge: the
+    same products otherwise, so the forces agree bit for bit but for what that charge moves,
+    2^-23 of its own pairs' Coulomb forces (bounded by 2^-20 of the largest force here)."""
+    host = _host()
+    kw = dict(precision=host.PREC_MIXED, coul_flag=host.COUL_EWALD) if ewald else dict(precision=host.PREC_FP64)
+    out = []
+    for one_off in (False, True):
+        s = S.make_system(ng, nw, seed=ng, params=S.Params(gewald=0.3))
+        if one_off:
+            s.q[s.np - 1] = np.nextafter(s.q[s.np - 1], np.float32(2.0))
+        e = host.Engine([host.ReplicaSpec(s, temp=300.0, gamma_ps=1.0, seed=3)], **kw)
+        try:
+            e.init()
+            out.append((e.forces()[0], e.energies()[0, :2].copy(), s))
+        finally:
+            e.close()
+    (f0, e0, s), (f1, e1, _) = out
+    d = np.abs(f0 - f1).max(1)
+    L = float(s.box)
+    r = s.pos - s.pos[-1]
+    r -= L * np.round(r / L)
+    # molecules beyond the cutoff of the changed atom (a constraint takes a force across its own)
+    far = ~np.isin(s.mol, s.mol[np.sqrt((r * r).sum(1)) < 10.1])
+    assert far.sum() > 100 and d[far].max() == 0.0
+    assert d.max() <= 2.0 ** -20 * np.abs(f0).max()
+    np.testing.assert_allclose(e0, e1, rtol=1e-5)
