@@ -425,6 +425,7 @@ constexpr int ITEM_THREADS = 64;
 struct BondedItems {
     int32_t items[BK_COUNT];   // per kind, 0 = none
     int32_t end[BK_COUNT];     // cumulative workgroups, in the kernel's order of kinds
+    long long *f14;            // the drop-in 1-4 pairs (on the real*4 positions): their own sum
 };
 __device__ __host__ constexpr int bonded_order(int k) {
     return k == 0 ? BK_TORSION : k == 1 ? BK_IMPRO : k == 2 ? BK_ANGLE : k == 3 ? BK_PAIR14 : BK_BOND;
@@ -451,7 +452,11 @@ k_bonded_items(BondedItems I, BondedArgs A, DevParams P, long long *__restrict__
             slot = E_COUL14;
             if (live) {
                 double c14, l14;
-                pair14_eval<true>(it, A.pos4, A.xd, A.q, boxf, iboxf, A.lj14, P, A.n, c14, l14, add);
+                if (I.f14)
+                    pair14_eval<false>(it, A.pos4, nullptr, A.q, boxf, iboxf, A.lj14, P, A.n, c14, l14,
+                                       AtomicSink{it, I.f14, A.n});
+                else
+                    pair14_eval<true>(it, A.pos4, A.xd, A.q, boxf, iboxf, A.lj14, P, A.n, c14, l14, add);
                 e = to_efix(c14);
                 e2 = to_efix(l14);
             }
@@ -600,8 +605,9 @@ BondedArgs bonded_args(const sofia_ctx *c, const double *xd, const int32_t *bond
 }
 
 void launch_items(sofia_ctx *c, const BondedArgs &A, int n14, int nb, int na, long long *fout,
-                  bool energies) {
+                  bool energies, long long *f14 = nullptr) {
     BondedItems I{};
+    I.f14 = f14;
     I.items[BK_PAIR14] = n14;
     I.items[BK_BOND] = c->bond_k ? nb : 0;
     I.items[BK_ANGLE] = c->angle_k ? na : 0;
@@ -628,6 +634,11 @@ void launch_bonded_dropin(sofia_ctx *c, long long *fout) {
     double *xd = c->b.xd;
     hipLaunchKernelGGL(k_pos_to_xd, dim3(nblocks(n, 256)), dim3(256), 0, c->stream, n, c->a.pos4, xd);
     launch_items(c, bonded_args(c, xd, c->bondlist, c->anglelist), 0, c->nb, c->na, fout, true);
+}
+
+// The same with the 1-4 pairs (into f14) in the launch, on an FP64 copy that is there.
+void launch_bonded_wrapper(sofia_ctx *c, const double *xd, long long *fout, long long *f14) {
+    launch_items(c, bonded_args(c, xd, c->bondlist, c->anglelist), c->nd, c->nb, c->na, fout, true, f14);
 }
 
 namespace {

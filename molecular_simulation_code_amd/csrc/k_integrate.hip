@@ -20,11 +20,20 @@ __global__ void k_zero(int32_t n3, long long *__restrict__ f, int32_t ne, long l
     if (e && i < ne) e[i] = 0;
 }
 
-__global__ void k_zero2(int32_t n3, long long *__restrict__ a, long long *__restrict__ b) {
+// What the force wrapper's terms start from: two force sums at zero, and the real*4 positions
+// promoted to the FP64 copy that the bonded kernels read.
+__global__ void k_start_forces(int32_t n, long long *__restrict__ a, long long *__restrict__ b,
+                               const float4 *__restrict__ pos4, double *__restrict__ xd) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n3) {
-        a[i] = 0;
-        b[i] = 0;
+    if (i >= n) return;
+    const float4 p = pos4[i];
+    const float x[3] = {p.x, p.y, p.z};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const size_t o = (size_t)c * n + i;
+        a[o] = 0;
+        b[o] = 0;
+        xd[o] = x[c];
     }
 }
 
@@ -32,31 +41,38 @@ __global__ void k_zero2(int32_t n3, long long *__restrict__ a, long long *__rest
 // written to the host's page-locked words; the copies (and the solver's flags, whose engine
 // form stays up until the lists are set up again, on request) are cleared on the way.
 // A drop-in call used to copy the raw copies (26 KB) and each flag on their own.
-__global__ void k_report(int32_t slots, long long *__restrict__ eacc, int32_t *__restrict__ shake_err,
-                         int32_t *__restrict__ shake_iters, const int32_t *__restrict__ maxcnt,
-                         HostWords *__restrict__ hw, long long *__restrict__ hw_e, bool clear_shake) {
+struct ReportArgs {
+    int32_t slots;
+    long long *eacc;
+    int32_t *shake_err, *shake_iters;
+    const int32_t *maxcnt;
+    HostWords *hw;
+    long long *hw_e;
+    bool clear_shake;
+};
+__device__ inline void report_words(const ReportArgs &A, int t) {
     static_assert(ESPREAD == 16, "one lane per copy");
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int slot = t / ESPREAD;
     long long v = 0;
-    if (slot < slots) {
-        long long *p = &eacc[(size_t)t * ECOPY];
+    if (slot < A.slots) {
+        long long *p = &A.eacc[(size_t)t * ECOPY];
         v = *p;
         *p = 0;
     }
 #pragma unroll
     for (int off = ESPREAD / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    if (slot < slots && t % ESPREAD == 0) hw_e[slot] = v;
+    if (slot < A.slots && t % ESPREAD == 0) A.hw_e[slot] = v;
     if (t == 0) {
-        hw->shake_err = *shake_err;
-        hw->shake_iters = *shake_iters;
-        hw->maxcnt = *maxcnt;
-        if (clear_shake) {
-            *shake_err = 0;
-            *shake_iters = 0;
+        A.hw->shake_err = *A.shake_err;
+        A.hw->shake_iters = *A.shake_iters;
+        A.hw->maxcnt = *A.maxcnt;
+        if (A.clear_shake) {
+            *A.shake_err = 0;
+            *A.shake_iters = 0;
         }
     }
 }
+__global__ void k_report(ReportArgs A) { report_words(A, blockIdx.x * blockDim.x + threadIdx.x); }
 
 // x | y | z of src (and FIX_INV fix) as x, y, z rows; with gid, the row of an atom is its global
 // id's place within its replica (ids a permutation of 1..natom).
@@ -893,10 +909,17 @@ __global__ void k_copy16(size_t n16, const float4 *__restrict__ src, float4 *__r
 
 // The force wrapper's merge: each term rounded to real*4 as its own routine returns it (the
 // fixed-point sums as k_fix_to_aos rounds them), then pair + 1-4 + bonded summed in FP64 and
-// stored real*4 into ff (which holds the pair term on entry).
-__global__ void k_merge_forces(int32_t n, float *__restrict__ ff, const long long *__restrict__ f14,
-                               const long long *__restrict__ fb) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+// stored real*4 into ff (which holds the pair term on entry).  Workgroups past the atoms'
+// write the report, for which the merge need not wait.
+__global__ void __launch_bounds__(256)
+k_merge_report(int32_t n, float *__restrict__ ff, const long long *__restrict__ f14,
+               const long long *__restrict__ fb, ReportArgs A) {
+    const int merge = (n + 255) / 256;
+    if ((int)blockIdx.x >= merge) {
+        report_words(A, ((int)blockIdx.x - merge) * 256 + threadIdx.x);
+        return;
+    }
+    const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -906,37 +929,31 @@ __global__ void k_merge_forces(int32_t n, float *__restrict__ ff, const long lon
     }
 }
 
-// Atom types (the int bits of pos.w) outside 1..ntypes set *bad; any lane that finds one
-// writes the same value, so a plain store suffices.
-__global__ void k_type_range(int32_t n, const float4 *__restrict__ pos, int32_t ntypes,
-                             int32_t *__restrict__ bad, HostWords *__restrict__ hw) {
+// An upload changes places with the state (positions, and v / q / gid where given), and a type
+// (the int bits of pos.w) outside 1..ntypes is told to the host, which then runs the exchange
+// once more and has the state as it was.  (A check of its own before the move was a launch in
+// every call of the drop-in step: 3.4 us, and one in front of the other.)
+__global__ void k_put_state(int32_t n, AtomArrays up, AtomArrays state, bool v, bool q, bool gid,
+                            int32_t ntypes, HostWords *__restrict__ hw) {
     const int stride = gridDim.x * blockDim.x;
     bool out = false;
+    auto exchange = [](auto &a, auto &b) {
+        const auto x = a;
+        a = b;
+        b = x;
+    };
     for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
-        const int t = __float_as_int(pos[k].w);
+        exchange(state.pos4[k], up.pos4[k]);
+        const int t = __float_as_int(state.pos4[k].w);
         out |= (t < 1) | (t > ntypes);
-    }
-    if (__ballot(out) && __lane_id() == 0) {
-        *bad = 1;
-        hw->type_err = 1;
-    }
-}
-
-// An upload whose types are all in range goes from the staging set into the state: positions,
-// and v / q / gid where given.
-__global__ void k_put_state(int32_t n, const int32_t *__restrict__ bad, AtomArrays src, AtomArrays dst,
-                            bool v, bool q, bool gid) {
-    if (*bad) return;
-    const int stride = gridDim.x * blockDim.x;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
-        dst.pos4[k] = src.pos4[k];
-        if (q) dst.q[k] = src.q[k];
-        if (gid) dst.gid[k] = src.gid[k];
+        if (q) exchange(state.q[k], up.q[k]);
+        if (gid) exchange(state.gid[k], up.gid[k]);
         if (v) {
 #pragma unroll
-            for (int d = 0; d < 3; ++d) dst.v32[(size_t)d * n + k] = src.v32[(size_t)d * n + k];
+            for (int d = 0; d < 3; ++d) exchange(state.v32[(size_t)d * n + k], up.v32[(size_t)d * n + k]);
         }
     }
+    if (__ballot(out) && __lane_id() == 0) hw->type_err = 1;   // every lane writes the same
 }
 
 // The fused rigid-water bonded terms alone (steps that run no SHAKE: the minimiser), their
@@ -1131,28 +1148,34 @@ void launch_shake64(sofia_ctx *c, bool energies, bool step) {
                            e1, e2, e3, e4, nb_it, c->a.wclus, shake_args(c), S, c->eacc);
 }
 
-void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb) {
-    hipLaunchKernelGGL(k_merge_forces, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N, ff32,
-                       f14, fb);
-}
-
 void launch_put_state(sofia_ctx *c, bool v, bool q, bool gid) {
     const int grid = std::min(nblocks(c->N, 256), 1024);
-    hipLaunchKernelGGL(k_type_range, dim3(grid), dim3(256), 0, c->stream, c->N, c->b.pos4, c->p.ntypes,
-                       c->type_err, c->hw);
-    hipLaunchKernelGGL(k_put_state, dim3(grid), dim3(256), 0, c->stream, c->N, c->type_err, c->b, c->a,
-                       v, q, gid);
+    hipLaunchKernelGGL(k_put_state, dim3(grid), dim3(256), 0, c->stream, c->N, c->b, c->a, v, q, gid,
+                       c->p.ntypes, c->hw);
 }
+
+namespace {
+ReportArgs report_args(sofia_ctx *c, bool clear_shake) {
+    c->eacc_zero = true;
+    return ReportArgs{c->nrep * NE, c->eacc, c->shake_err, c->shake_iters, c->maxcnt, c->hw, c->hw_e,
+                      clear_shake};
+}
+inline int report_blocks(const sofia_ctx *c) { return nblocks((long long)c->nrep * NE * ESPREAD, 256); }
+}  // namespace
 
 void launch_report(sofia_ctx *c, bool clear_shake) {
-    const int slots = c->nrep * NE;
-    hipLaunchKernelGGL(k_report, dim3(nblocks((long long)slots * ESPREAD, 256)), dim3(256), 0, c->stream,
-                       slots, c->eacc, c->shake_err, c->shake_iters, c->maxcnt, c->hw, c->hw_e, clear_shake);
-    c->eacc_zero = true;
+    hipLaunchKernelGGL(k_report, dim3(report_blocks(c)), dim3(256), 0, c->stream,
+                       report_args(c, clear_shake));
 }
 
-void launch_zero2(sofia_ctx *c, long long *a, long long *b) {
-    hipLaunchKernelGGL(k_zero2, dim3(nblocks(3LL * c->N, 256)), dim3(256), 0, c->stream, 3 * c->N, a, b);
+void launch_merge_report(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb) {
+    hipLaunchKernelGGL(k_merge_report, dim3(nblocks(c->N, 256) + report_blocks(c)), dim3(256), 0,
+                       c->stream, c->N, ff32, f14, fb, report_args(c, false));
+}
+
+void launch_start_forces(sofia_ctx *c, long long *a, long long *b, double *xd) {
+    hipLaunchKernelGGL(k_start_forces, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N, a, b,
+                       c->a.pos4, xd);
 }
 
 void launch_soa_to_aos(sofia_ctx *c, const double *src, const long long *fix, const int32_t *gid, double *dst) {

@@ -365,10 +365,12 @@ k_build_list(const float4 *__restrict__ pos4, const int32_t *__restrict__ num3,
     }
 }
 
-__global__ void k_check32(int32_t n, const float *__restrict__ dr,
-                          double rvrc2, HostWords *__restrict__ hw) {
+// check_neighbor; the rebuild flags are cleared with it.
+__global__ void k_check32(int32_t n, const float *__restrict__ dr, double rvrc2, int32_t nrep,
+                          int32_t *__restrict__ rebuild, HostWords *__restrict__ hw) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     bool moved = false;
+    if (i <= nrep) rebuild[i] = 0;   // [nrep] is `any`
     if (i < n) {
         const float x = dr[i], y = dr[(size_t)n + i], z = dr[2 * (size_t)n + i];
         moved = (double)((x * x + y * y) + z * z) >= rvrc2;
@@ -488,8 +490,8 @@ void launch_build_list(sofia_ctx *c) {
 }
 
 void launch_check_neighbor(sofia_ctx *c) {
-    hipLaunchKernelGGL(k_check32, dim3(nblk(c->N, 256)), dim3(256), 0, c->stream, c->N, c->dr32,
-                       c->dp.rvrc2, c->hw);
+    hipLaunchKernelGGL(k_check32, dim3(nblk(std::max(c->N, c->nrep + 1), 256)), dim3(256), 0, c->stream,
+                       c->N, c->dr32, c->dp.rvrc2, c->nrep, c->rebuild, c->hw);
 }
 
 void launch_set_rebuild(sofia_ctx *c, int32_t value) {

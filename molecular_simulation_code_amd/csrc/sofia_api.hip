@@ -505,7 +505,6 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
     B.want(&c->rebuild, nrep + 1);   // nrep flags, then `any`
     B.want(&c->nbuilds, nrep);
     B.want(&c->shake_err, 1);
-    B.want(&c->type_err, 1);
     B.want(&c->shake_iters, 1);
     B.want(&c->eacc, eacc_len(nrep));
     B.want(&c->step_d, nrep);
@@ -1053,8 +1052,9 @@ int sofia_put_state(sofia_ctx *c, const sofia_ainfo *pos, const float *q, const 
     // ordered on the stream behind kernels that may still read the arrays replaced here
     if (pos) {
         // Types within 1..ntypes, checked on the device (a host pass over the array costs
-        // more than the copy) on a staging copy, the sort's gather target, which holds nothing
-        // between list builds; a rejected upload leaves the state as it was.
+        // more than the copy) as a staging copy, in the sort's gather target, which holds
+        // nothing between list builds, changes places with the state; a rejected upload leaves
+        // the state as it was.
         c->hw->type_err = 0;
         TRY(up(c, c->b.pos4, pos, sizeof(float4) * n));
         if (q) TRY(up(c, c->b.q, q, sizeof(float) * n));
@@ -1063,7 +1063,7 @@ int sofia_put_state(sofia_ctx *c, const sofia_ainfo *pos, const float *q, const 
         launch_put_state(c, v != nullptr, q != nullptr, gid != nullptr);
         TRY(sync_check(c));
         if (c->hw->type_err) {
-            SOFIA_HIP(hipMemsetAsync(c->type_err, 0, sizeof(int32_t), c->stream));
+            launch_put_state(c, v != nullptr, q != nullptr, gid != nullptr);
             TRY(sync_check(c));
             return fail(SOFIA_E_ARG, "atom type out of range");
         }
@@ -1158,6 +1158,10 @@ int sofia_get_ordered_f64(sofia_ctx *c, double *x, double *v, double *f, int32_t
 int sofia_get_displacement(sofia_ctx *c, float *dx, float *dy, float *dz) {
     if (!c || !dx || !dy || !dz) return fail(SOFIA_E_ARG, "null argument");
     const size_t n = c->N;
+    if (dy == dx + n && dz == dy + n) {   // one array of three rows
+        TRY(down(c, dx, c->dr32, sizeof(float) * 3 * n));
+        return sync_check(c);
+    }
     TRY(down(c, dx, c->dr32, sizeof(float) * n));
     TRY(down(c, dy, c->dr32 + n, sizeof(float) * n));
     TRY(down(c, dz, c->dr32 + 2 * n, sizeof(float) * n));
@@ -1167,6 +1171,10 @@ int sofia_get_displacement(sofia_ctx *c, float *dx, float *dy, float *dz) {
 int sofia_put_displacement(sofia_ctx *c, const float *dx, const float *dy, const float *dz) {
     if (!c || !dx || !dy || !dz) return fail(SOFIA_E_ARG, "null argument");
     const size_t n = c->N;
+    if (dy == dx + n && dz == dy + n) {
+        TRY(up(c, c->dr32, dx, sizeof(float) * 3 * n));
+        return sync_check(c);
+    }
     TRY(up(c, c->dr32, dx, sizeof(float) * n));
     TRY(up(c, c->dr32 + n, dy, sizeof(float) * n));
     TRY(up(c, c->dr32 + 2 * n, dz, sizeof(float) * n));
@@ -1310,7 +1318,6 @@ int sofia_get_nlist(sofia_ctx *c, int32_t *nlist, int32_t *numneigh, int32_t *na
 
 int sofia_check_neighbor(sofia_ctx *c, int32_t *nflag) {
     if (!c || !nflag) return fail(SOFIA_E_ARG, "null argument");
-    launch_set_rebuild(c, 0);
     c->hw->moved = 0;
     launch_check_neighbor(c);
     TRY(sync_check(c));
@@ -1471,14 +1478,13 @@ int sofia_force_wrapper_dsf(sofia_ctx *c, sofia_coords *ff, double *e, double *v
     if (!c->fix14) TRY(dalloc(&c->fix14, (size_t)3 * n));
     float *st = staging_f32(c);
     launch_zero_energies(c);   // once: the terms use their own slots
-    launch_zero2(c, c->fscratch, c->fix14);
+    launch_start_forces(c, c->fscratch, c->fix14, c->b.xd);
     launch_nonbond_out(c, 0, true, st);
-    launch_pair14(c, c->fix14);
-    launch_bonded_dropin(c, c->fscratch);
-    launch_merge_forces(c, st, c->fix14, c->fscratch);
+    launch_bonded_wrapper(c, c->b.xd, c->fscratch, c->fix14);
+    launch_merge_report(c, st, c->fix14, c->fscratch);
     if (ff) TRY(down(c, ff, st, sizeof(float) * 3 * (size_t)n));
-    std::vector<long long> es;
-    TRY(read_energies(c, es));
+    TRY(sync_check(c));
+    const std::vector<long long> es(c->hw_e, c->hw_e + (size_t)c->nrep * NE);
     // summed over replicas first, then added, as each routine of its own adds its sums
     const int slot[8] = {E_LJ, E_COUL, E_COUL14, E_POT14, E_BOND, E_ANGLE, E_DIHED, E_IMPRO};
     double sum[8] = {0, 0, 0, 0, 0, 0, 0, 0}, vx = 0, vy = 0, vz = 0;

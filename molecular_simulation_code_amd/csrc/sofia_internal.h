@@ -147,7 +147,6 @@ struct sofia_ctx {
     int32_t *rebuild = nullptr;     // per replica
     int32_t *nbuilds = nullptr;     // per replica
     int32_t *shake_err = nullptr;   // device scalar
-    int32_t *type_err = nullptr;    // device scalar: put_state's type check
     int32_t *shake_iters = nullptr; // device scalar
 
     // topology (global 0-based indices)
@@ -289,6 +288,7 @@ void launch_correct(sofia_ctx *c, int which, long long *fout);
 void launch_pair14(sofia_ctx *c, long long *fout);
 void launch_bonded_engine(sofia_ctx *c, bool energies);
 void launch_bonded_dropin(sofia_ctx *c, long long *fout);
+void launch_bonded_wrapper(sofia_ctx *c, const double *xd, long long *fout, long long *f14);
 int build_bonded_bundles(sofia_ctx *c);   // host: molecules of the engine's bonded items
 void drop_bonded_bundles(sofia_ctx *c);
 void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records);
@@ -317,10 +317,11 @@ void launch_zero_energies(sofia_ctx *c);
 void launch_water_bonded(sofia_ctx *c);   // and the books of the rebuild before it
 void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst);
 void launch_put_state(sofia_ctx *c, bool v, bool q, bool gid);
-void launch_merge_forces(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb);
+// with the report of the call
+void launch_merge_report(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb);
 // Energy sums (cleared on the device) and flags to the host words
 void launch_report(sofia_ctx *c, bool clear_shake = false);
-void launch_zero2(sofia_ctx *c, long long *a, long long *b);
+void launch_start_forces(sofia_ctx *c, long long *a, long long *b, double *xd);
 // FP64 SoA (plus fixed point) <-> AoS; with gid, dst rows in global-id order of each replica
 void launch_soa_to_aos(sofia_ctx *c, const double *src, const long long *fix, const int32_t *gid, double *dst);
 void launch_aos_to_soa(sofia_ctx *c, const double *src, double *dst);
