@@ -16,6 +16,7 @@
 // the output keeps the reference's order.  Several replicas share one launch: every
 // cell belongs to one replica and only replicas flagged for a rebuild do work.
 #include <algorithm>
+#include <cmath>
 
 #include "sofia_device.h"
 
@@ -90,7 +91,7 @@ __device__ inline void move_atom(const AtomArrays &src, const AtomArrays &dst, i
 // workgroup per replica in the launch sequence cost every step more than these sums cost the
 // steps that rebuild).  A cell with more atoms than a bucket holds is read from acell.
 __global__ void __launch_bounds__(256)
-k_sort_gather(int32_t ncell, int32_t per, const int32_t *__restrict__ cell_rep,
+k_sort_gather(int32_t ncell, int32_t per, int32_t split, const int32_t *__restrict__ cell_rep,
               const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
               const int32_t *__restrict__ any, const int32_t *__restrict__ cbin,
               const int32_t *__restrict__ acell, const int32_t *__restrict__ bucket, int32_t cap,
@@ -100,7 +101,8 @@ k_sort_gather(int32_t ncell, int32_t per, const int32_t *__restrict__ cell_rep,
     if (!*any) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
-    const int c0 = wave * per, c1 = min(c0 + per, ncell);
+    const int part = wave % split;   // split > 1: per = 1
+    const int c0 = wave / split * per, c1 = min(c0 + per, ncell);
     int rcur = -1, base = 0;
     for (int c = c0; c < c1; ++c) {
         const int r = cell_rep[c];
@@ -117,7 +119,7 @@ k_sort_gather(int32_t ncell, int32_t per, const int32_t *__restrict__ cell_rep,
             rcur = r;
         }
         const int cnt = cbin[c];
-        if (lane == 0) {
+        if (lane == 0 && part == 0) {
             cstart[c] = base;
             ccount[c] = cnt;
         }
@@ -128,13 +130,18 @@ k_sort_gather(int32_t ncell, int32_t per, const int32_t *__restrict__ cell_rep,
         };
         if (cnt <= cap) {
             const int32_t *ids = bucket + (size_t)c * cap;
-            for (int e = lane; e < cnt; e += 64) {
-                const int me = ids[e];
+            for (int e0 = 64 * part; e0 < cnt; e0 += 64 * split) {
+                const bool in = e0 + lane < cnt;
+                const int me = in ? ids[e0 + lane] : 0;
                 int rank = 0;
-                for (int f = 0; f < cnt; ++f) rank += ids[f] > me;
-                place(me, rank);
+                for (int f0 = 0; f0 < cnt; f0 += 64) {
+                    const int other = f0 + lane < cnt ? ids[f0 + lane] : -1;
+                    const int m = min(64, cnt - f0);
+                    for (int f = 0; f < m; ++f) rank += __builtin_amdgcn_readlane(other, f) > me;
+                }
+                if (in) place(me, rank);
             }
-        } else {
+        } else if (part == 0) {
             const int a0 = reps[r].atom0, a1 = a0 + reps[r].natom;
             const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
             int done = 0;
@@ -256,59 +263,182 @@ __global__ void k_rdf(int32_t n, const float4 *__restrict__ pos4, const int32_t 
     }
 }
 
+// The drop-in list of one cell (or of a share of its atoms, blockIdx.y).
+//
+// Where the box has at least 5 cells a side and every staged coordinate lies in [0, box], the
+// image of a stencil cell is the same for all its atoms: separations inside the box are at
+// most 0.4 box, across it at least 0.6 box, so the reference's rounded shift is 0 or +-1 as the
+// cell lies, and the distance takes that shift directly -- the same two real*4 operations
+// without the product and the rounding.  (4 cells a side: the two shifts can differ only at
+// half a box, which is no neighbour by either where rv is less.)  A wavefront then sweeps two atoms at once over the
+// cells that come within rv of either (CULL_MARGIN is far above the rounding of positions and
+// cells).  Candidates are staged three loads at a time from all 27 cells, which one after the
+// other were a chain of 27 loads.  97 -> 60 us at 13,500 atoms, 1010 -> 560 at 204,000; the
+// second launch bound keeps two workgroups of 16 wavefronts on a CU.
+constexpr float CULL_MARGIN = 0.01f;  // A
+
 template <int WAVES>
-__global__ void __launch_bounds__(WAVES * 64)
+__global__ void __launch_bounds__(WAVES * 64, WAVES >= 4 ? WAVES * 2 / 4 : 1)
 k_build_list(const float4 *__restrict__ pos4, const int32_t *__restrict__ num3,
              const int32_t *__restrict__ spec, const int32_t *__restrict__ cstart,
              const int32_t *__restrict__ ccount, const int32_t *__restrict__ cnum,
              const int32_t *__restrict__ cell_rep, const RepInfo *__restrict__ reps,
-             const int32_t *__restrict__ rebuild, double rv2, int32_t na,
+             const int32_t *__restrict__ rebuild, float rv2, float rvm2, int32_t na,
              int32_t *__restrict__ nlist, int32_t *__restrict__ numneigh,
              int32_t *__restrict__ maxcnt) {
     const int c = blockIdx.x;
     const int r = cell_rep[c];
     if (!rebuild[r] || reps[r].stencil5) return;
-    const float box = reps[r].box, ibox = reps[r].ibox;
+    const float box = reps[r].box, ibox = reps[r].ibox, rn = reps[r].rn;
+    const int nD = reps[r].ncellD, lc = c - reps[r].cell0;
 
-    __shared__ int32_t s_cell[27];
     __shared__ int32_t s_start[27];
     __shared__ int32_t s_off[28];
     __shared__ float4 s_j[LIST_CAP];
 
     const int tid = threadIdx.x;
-    if (tid < 27) {
-        const int nc = cnum[27 * c + tid];
-        s_cell[tid] = nc;
-        s_start[tid] = cstart[nc];
-    }
-    __syncthreads();
-    if (tid == 0) {
-        int acc = 0;
-        for (int k = 0; k < 27; ++k) {
-            s_off[k] = acc;
-            acc += ccount[s_cell[k]];
+    if (tid < 64) {
+        int start = 0, count = 0;
+        if (tid < 27) {
+            const int nc = cnum[27 * c + tid];
+            start = cstart[nc];
+            count = ccount[nc];
+            s_start[tid] = start;
         }
-        s_off[27] = acc;
+        int v = count;
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) {
+            const int u = __shfl_up(v, o, 64);
+            if (tid >= o) v += u;
+        }
+        if (tid < 28) s_off[tid] = v - count;
     }
     __syncthreads();
     const int total = s_off[27];
     const bool staged = total <= LIST_CAP;
+    bool outside = false;
     if (staged) {
-        for (int k = 0; k < 27; ++k) {
-            const int cnt = s_off[k + 1] - s_off[k], st = s_start[k];
-            for (int t = tid; t < cnt; t += WAVES * 64) {
-                float4 p = pos4[st + t];
-                p.w = __int_as_float(st + t);
-                s_j[s_off[k] + t] = p;
+        constexpr int U = 3;   // loads in flight per thread
+        for (int t0 = tid; t0 < total; t0 += U * WAVES * 64) {
+            float4 p[U];
+            int id[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int t = min(t0 + u * WAVES * 64, total - 1);
+                int k = 0;   // the last cell that starts at or before t
+#pragma unroll
+                for (int s = 16; s > 0; s >>= 1)
+                    if (k + s < 27 && s_off[k + s] <= t) k += s;
+                id[u] = s_start[k] + t - s_off[k];
+                p[u] = pos4[id[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int t = t0 + u * WAVES * 64;
+                if (t >= total) continue;
+                outside |= !(p[u].x >= 0.0f && p[u].x <= box && p[u].y >= 0.0f && p[u].y <= box &&
+                             p[u].z >= 0.0f && p[u].z <= box);
+                p[u].w = __int_as_float(id[u]);
+                s_j[t] = p[u];
             }
         }
     }
-    __syncthreads();
+    const bool inside = !__syncthreads_or(outside);   // (and the staged candidates are there)
+    const bool direct = staged && inside && (nD >= 5 || (nD == 4 && 0.49f * box > sqrtf(rvm2)));
 
-    const int wave = tid >> 6, lane = tid & 63;
-    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int i0 = cstart[c], ni = ccount[c];
-    for (int ii = blockIdx.y * WAVES + wave; ii < ni; ii += gridDim.y * WAVES) {
+    const int first = blockIdx.y * WAVES + wave, step = gridDim.y * WAVES;
+
+    if (direct) {
+        // lane k < 27: stencil cell k's place (the centre first, then z, y, x ascending), the
+        // shift of its image, and where its candidates lie
+        const int j = lane == 0 ? 13 : (lane <= 13 ? lane - 1 : lane);
+        const int at[3] = {lc % nD + j % 3 - 1, (lc / nD) % nD + j / 3 % 3 - 1, lc / (nD * nD) + j / 9 - 1};
+        float sh[3], low[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            sh[d] = at[d] < 0 ? -box : (at[d] >= nD ? box : 0.0f);
+            low[d] = (float)at[d] * rn;
+        }
+        const int o0 = s_off[min(lane, 27)], o1 = s_off[min(lane + 1, 27)];
+        const int id0 = s_start[min(lane, 26)], id1 = id0 + o1 - o0;   // the cell's atom ids
+        for (int ii = 2 * first; ii < ni; ii += 2 * step) {
+            const int ia = i0 + ii;
+            const bool two = ii + 1 < ni;
+            const int ib = two ? ia + 1 : ia;
+            const float4 xa = pos4[ia], xb = pos4[ib];
+            const float lima = rv2, limb = two ? rv2 : -1.0f;
+            // exclusions: lanes 0..11 those of a, 16..27 those of b
+            const int who = lane < 16 ? ia : ib, e = lane & 15;
+            const bool has = lane < 32 && e < SPEC && e < num3[who];
+            const int ex = has ? spec[(size_t)who * SPEC + e] : -1;
+            const uint64_t exs = __ballot(has);
+            bool holds = false;   // an excluded atom of either
+            for (uint64_t m = exs; m; m &= m - 1) {
+                const int v = __builtin_amdgcn_readlane(ex, __builtin_ctzll(m));
+                holds |= v >= id0 && v < id1;
+            }
+            const uint64_t excells = __ballot(lane < 27 && holds);
+            auto gap = [&](const float4 &x) {
+                const float g[3] = {x.x, x.y, x.z};
+                float d2 = 0.0f;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const float w = fmaxf(0.0f, fmaxf(low[d] - g[d], g[d] - (low[d] + rn)) - CULL_MARGIN);
+                    d2 += w * w;
+                }
+                return d2;
+            };
+            uint64_t cells = __ballot(lane < 27 && o1 > o0 && fminf(gap(xa), gap(xb)) < rvm2);
+            int cnta = 0, cntb = 0;
+            int32_t *outa = nlist + (size_t)ia * na, *outb = nlist + (size_t)ib * na;
+            while (cells) {
+                const int k = __builtin_ctzll(cells);
+                cells &= cells - 1;
+                const uint64_t exk = (excells >> k & 1) ? exs : 0ull;
+                const int lo = __builtin_amdgcn_readlane(o0, k), hi = __builtin_amdgcn_readlane(o1, k);
+                const float sx = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sh[0]), k));
+                const float sy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sh[1]), k));
+                const float sz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(sh[2]), k));
+                for (int base = lo; base < hi; base += 64) {
+                    const int t = base + lane;
+                    const float4 pj = s_j[min(t, hi - 1)];
+                    const int z = __float_as_int(pj.w);
+                    const bool in = t < hi;
+                    const float ax = (xa.x - pj.x) - sx, ay = (xa.y - pj.y) - sy, az = (xa.z - pj.z) - sz;
+                    const float bx = (xb.x - pj.x) - sx, by = (xb.y - pj.y) - sy, bz = (xb.z - pj.z) - sz;
+                    bool ha = in & ((ax * ax + ay * ay) + az * az <= lima) & (z != ia);
+                    bool hb = in & ((bx * bx + by * by) + bz * bz <= limb) & (z != ib);
+                    for (uint64_t m = exk; m; m &= m - 1) {   // exclusions of a and of b
+                        const int l = __builtin_ctzll(m);
+                        const int v = __builtin_amdgcn_readlane(ex, l);
+                        if (l < 16) ha = ha & (z != v);
+                        else hb = hb & (z != v);
+                    }
+                    const uint64_t ma = __ballot(ha), mb = __ballot(hb);
+                    const int pa = cnta + (int)__builtin_amdgcn_mbcnt_hi(
+                                              (uint32_t)(ma >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ma, 0u));
+                    const int pb = cntb + (int)__builtin_amdgcn_mbcnt_hi(
+                                              (uint32_t)(mb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mb, 0u));
+                    if (ha & (pa < na)) outa[pa] = z;
+                    if (hb & (pb < na)) outb[pb] = z;
+                    cnta += __popcll(ma);
+                    cntb += __popcll(mb);
+                }
+            }
+            if (lane == 0) {
+                numneigh[ia] = cnta;
+                if (two) numneigh[ib] = cntb;
+                const int mx = max(cnta, cntb);
+                if (mx > na) atomicMax(maxcnt, mx);
+            }
+        }
+        return;
+    }
+
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    for (int ii = first; ii < ni; ii += step) {
         const int i = i0 + ii;
         const float4 xi = pos4[i];
         const int n3 = num3[i];
@@ -343,7 +473,7 @@ k_build_list(const float4 *__restrict__ pos4, const int32_t *__restrict__ num3,
                 const float dy = mimg32(xi.y - pj.y, box, ibox);
                 const float dz = mimg32(xi.z - pj.z, box, ibox);
                 const float dr2 = (dx * dx + dy * dy) + dz * dz;
-                pred = (z != i) && ((double)dr2 < rv2);
+                pred = (z != i) && (dr2 <= rv2);
             }
             const bool maybe = pred && z >= exmin && z <= exmax;
             if (__any(maybe)) {
@@ -425,8 +555,11 @@ void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies) {
         T = StepArrays{c->fix, c->fscratch, rb ? c->pfix : nullptr, rb == 16 ? c->a.q : nullptr};
     }
     const int per = nblk(c->ncell_total, 4 * GRID_CAP);   // cells per wavefront
-    hipLaunchKernelGGL(k_sort_gather, dim3(nblk(nblk(c->ncell_total, per), 4)), dim3(256), 0, c->stream,
-                       c->ncell_total, per, c->cell_rep, c->reps_d, c->rebuild, any_flag(c), c->cbin,
+    // or wavefronts per cell, where a cell holds more atoms than a wavefront has lanes (the
+    // reference's cells: 30 -> 22 us at 13,500 atoms in 125 cells, 33 -> 15 at 31,000)
+    const int split = per > 1 ? 1 : std::max(1, std::min(8, nblk(c->N, 64 * c->ncell_total)));
+    hipLaunchKernelGGL(k_sort_gather, dim3(nblk(nblk(c->ncell_total, per) * split, 4)), dim3(256), 0, c->stream,
+                       c->ncell_total, per, split, c->cell_rep, c->reps_d, c->rebuild, any_flag(c), c->cbin,
                        c->acell, c->bucket, c->bucket_cap, c->ccount, c->cstart, c->tt, c->atombin,
                        c->N, c->a, c->b, (int)mode, T);
     RemapSet S{};
@@ -477,10 +610,14 @@ void launch_build_list(sofia_ctx *c) {
     // chip idle: their atoms go to several workgroups, each staging the stencil for itself
     const int w = c->list_waves;
     const int parts = std::max(1, std::min(8, 1024 / c->ncell_total));
+    // the largest real*4 value whose real*8 promotion is below rv2: the same comparison in real*4
+    float rv2 = (float)c->dp.rv2;
+    if ((double)rv2 >= c->dp.rv2) rv2 = std::nextafterf(rv2, 0.0f);
+    const float rvm = (float)std::sqrt(c->dp.rv2) + CULL_MARGIN;
 #define LB(W)                                                                                    \
     hipLaunchKernelGGL(k_build_list<W>, dim3(c->ncell_total, parts), dim3(W * 64), 0, c->stream, \
                        c->a.pos4, c->a.num3, c->a.spec, c->cstart, c->ccount, c->cnum,            \
-                       c->cell_rep, c->reps_d, c->rebuild, c->dp.rv2, c->neigh_alloc, c->nlist,   \
+                       c->cell_rep, c->reps_d, c->rebuild, rv2, rvm * rvm, c->neigh_alloc, c->nlist,  \
                        c->numneigh, c->maxcnt)
     if (w <= 2) LB(2);
     else if (w <= 4) LB(4);

@@ -279,3 +279,44 @@ def test_a_rejected_upload_is_exchanged_back(where):
             np.testing.assert_array_equal(np.array(rows), d)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("edge", ["wrapped", "on the faces", "outside"])
+@pytest.mark.parametrize("ng,nw,cells", [(10, 260, 3), (10, 400, 4), (10, 700, 5), (20, 1500, 6)])
+def test_dropin_list_by_cell_images_is_the_references(ng, nw, cells, edge):
+    """3 to 6 cells a side (the image of a stencil cell is fixed from 4 on), atoms on the box's
+    faces, and atoms just outside it (every pair then by its own minimum image): the entries
+    and their order are the oracle's, also in a second build from the sorted order."""
+    host = _host()
+    from oracle import oracle as O
+    s = S.make_system(ng, nw, seed=5, params=S.Params(rcut=5.5, cut_coul=5.5, pad=1.0))
+    d = s.derived()
+    rn, nT, nD = O.cell_grid(d["box"], d["rcut"], d["cut_coul"])
+    assert nD == cells
+    rng = np.random.default_rng(nw)
+    some = rng.choice(s.np, 12, replace=False)
+    if edge == "on the faces":
+        s.pos[some[:6], rng.integers(0, 3, 6)] = 0.0
+        s.pos[some[6:], rng.integers(0, 3, 6)] = d["box"]
+    elif edge == "outside":
+        s.pos[some, rng.integers(0, 3, 12)] = np.float32(d["box"]) + np.float32(0.01)
+    g = host.SofiaGPU(s)
+    na = S.NEIGH_ALLOC0
+    try:
+        for _ in range(2):
+            pos, types, n3, sp = g.position.copy(), g.type.copy(), g.num3bond.copy(), g.specbond.copy()
+            tt = g.neighbor_wrapper(0)
+            ott, perm, start, endp, atombin = O.sort_cells(pos, types, d["box"], rn, nT, nD)
+            np.testing.assert_array_equal(tt, ott)
+            inv = perm - 1
+            spec = np.where(sp[inv] > 0, ott[np.maximum(sp[inv], 1) - 1], 0).astype(np.int32)
+            onl, onn, ona = O.build_neighbor(pos[inv], types[inv], atombin, start, endp, O.neighcell(nT, nD),
+                                             n3[inv], spec, d["box"], d["ibox"], d["rv2"], na)
+            nl, nn, na = g.get_nlist()
+            assert na == ona
+            np.testing.assert_array_equal(nn, onn)
+            a, o = nl.reshape(s.np, na), onl.reshape(s.np, ona)
+            for i in range(s.np):
+                assert np.array_equal(a[i, :nn[i]], o[i, :nn[i]])
+    finally:
+        g.close()
