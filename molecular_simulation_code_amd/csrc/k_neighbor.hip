@@ -18,7 +18,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "sofia_device.h"
+#include "sort_device.h"
 
 namespace sofia {
 namespace {
@@ -40,49 +40,11 @@ constexpr int GRID_CAP = 2048;
 
 // The sort is three launches.  k_bin (in a step with bonded bundles k_bonded_bundles, which
 // shares its launch) counts each cell's atoms and drops their ids into the cell's bucket;
-// k_sort_gather orders a cell and moves its atoms' data to the gather target;
-// k_copyback puts them back (device pointers stay fixed, which keeps captured graphs valid),
-// re-indexes what names atoms and clears the binning counters for the next sort.
+// k_sort_gather orders a cell and moves its atoms' data to the gather target; k_copyback (in an
+// engine step the first workgroups of the list build) puts them back.
 __global__ void k_bin(BinArgs A) {
     if (!*A.any) return;
     bin_atoms(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
-}
-
-// What the step's sort carries beyond the per-atom arrays (SORT_STEP), else null.
-struct StepArrays {
-    long long *fix, *fixb;   // the step's fixed-point forces and their gather target
-    int4 *pf;                // position records, rewritten from the moved positions
-    const float *q;          // null: 12-byte records
-};
-
-// Atom o of src to place k of dst; specbond entries go along unmapped.
-__device__ inline void move_atom(const AtomArrays &src, const AtomArrays &dst, int n, int o, int k,
-                                 int mode, const StepArrays &T) {
-    dst.pos4[k] = src.pos4[o];
-    dst.q[k] = src.q[o];
-    dst.gid[k] = src.gid[o];
-    dst.num1[k] = src.num1[o];
-    dst.num2[k] = src.num2[o];
-    dst.num3[k] = src.num3[o];
-    dst.mol[k] = src.mol[o];
-    dst.wclus[k] = src.wclus[o];
-    const int4 *s4 = (const int4 *)(src.spec + (size_t)o * SPEC);
-    int4 *d4 = (int4 *)(dst.spec + (size_t)k * SPEC);
-#pragma unroll
-    for (int l = 0; l < SPEC / 4; ++l) d4[l] = s4[l];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) dst.v32[3 * (size_t)k + d] = src.v32[3 * (size_t)o + d];
-    if (mode != SORT_DROPIN) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            dst.xd[(size_t)d * n + k] = src.xd[(size_t)d * n + o];
-            dst.vd[(size_t)d * n + k] = src.vd[(size_t)d * n + o];
-        }
-    }
-    if (mode == SORT_STEP) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) T.fixb[(size_t)d * n + k] = T.fix[(size_t)d * n + o];
-    }
 }
 
 // Atoms of a cell in descending old index (the chain order of the reference's linked cells),
@@ -157,63 +119,9 @@ k_sort_gather(int32_t ncell, int32_t per, int32_t split, const int32_t *__restri
     }
 }
 
-// Every bonded list of the context: item t of the concatenation falls in list L of S, whose
-// items are `width` ints with the first `nidx` atom ids (-1 = unused).  Items of replicas
-// that rebuild nothing this step are skipped (their atoms keep their places).
-struct RemapSet {
-    int32_t *lst[8];
-    int32_t end[8];           // cumulative item counts
-    int32_t width[8], nidx[8];
-    int32_t nlists;
-};
-
-__global__ void k_copyback(int32_t n, const int32_t *__restrict__ rep,
-                           const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
-                           const int32_t *__restrict__ any, const int32_t *__restrict__ tt,
-                           AtomArrays src, AtomArrays dst, float *__restrict__ dr32,
-                           double *__restrict__ drd, int mode, StepArrays T, RemapSet S,
-                           int32_t ncell, const int32_t *__restrict__ cell_rep,
-                           int32_t *__restrict__ cbin) {
-    if (!*any) return;
-    const int t0 = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
-    for (int k = t0; k < n; k += stride) {
-        const int r = rep[k];
-        if (!rebuild[r]) continue;
-        move_atom(src, dst, n, k, k, mode == SORT_STEP ? (int)SORT_ENGINE : mode, T);
-#pragma unroll
-        for (int l = 0; l < SPEC; ++l) {
-            const int s = src.spec[(size_t)k * SPEC + l];
-            if (s >= 0) dst.spec[(size_t)k * SPEC + l] = tt[s];
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d) dr32[(size_t)d * n + k] = 0.0f;
-        if (mode != SORT_DROPIN) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) drd[(size_t)d * n + k] = 0.0;
-        }
-        if (mode == SORT_STEP) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) T.fix[(size_t)d * n + k] = T.fixb[(size_t)d * n + k];
-            if (T.pf)
-                write_record(T.pf, k, src.xd[k], src.xd[(size_t)n + k], src.xd[2 * (size_t)n + k],
-                             reps[r].fscale, (uint32_t)__float_as_int(src.pos4[k].w), T.q ? src.q : nullptr);
-        }
-    }
-    const int total = S.nlists ? S.end[S.nlists - 1] : 0;
-    for (int t = t0; t < total; t += stride) {
-        int L = 0;
-        while (t >= S.end[L]) ++L;
-        const int m = t - (L ? S.end[L - 1] : 0);
-        int32_t *item = S.lst[L] + (size_t)m * S.width[L];
-        const int a0 = item[0];
-        if (a0 < 0 || !rebuild[rep[a0]]) continue;
-        for (int k = 0; k < S.nidx[L]; ++k) {
-            const int v = item[k];
-            if (v >= 0) item[k] = tt[v];
-        }
-    }
-    for (int c = t0; c < ncell; c += stride)
-        if (rebuild[cell_rep[c]]) cbin[c] = 0;
+__global__ void k_copyback(CopyArgs A) {
+    if (!*A.any) return;
+    copy_back(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 // A device topology array in the host's layout: in the first nidx columns of each item a
@@ -543,25 +451,13 @@ inline int nblk(int n, int b) { return (n + b - 1) / b; }
 inline int capped(int n, int b) { return std::max(1, std::min(nblk(n, b), GRID_CAP)); }
 inline const int32_t *any_flag(const sofia_ctx *c) { return c->rebuild + c->nrep; }
 
-void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies) {
-    const BinArgs B{c->N, c->bucket_cap, c->a.pos4, c->rep, c->reps_d, c->rebuild, any_flag(c),
-                    c->cbin, c->acell, c->bucket};
-    const int bin_grid = capped(c->N, 256);
-    if (bonded) launch_bundles_bin(c, B, bin_grid, energies);
-    else hipLaunchKernelGGL(k_bin, dim3(bin_grid), dim3(256), 0, c->stream, B);
-    StepArrays T{};
-    if (mode == SORT_STEP) {
-        const int rb = record_bytes(c);
-        T = StepArrays{c->fix, c->fscratch, rb ? c->pfix : nullptr, rb == 16 ? c->a.q : nullptr};
-    }
-    const int per = nblk(c->ncell_total, 4 * GRID_CAP);   // cells per wavefront
-    // or wavefronts per cell, where a cell holds more atoms than a wavefront has lanes (the
-    // reference's cells: 30 -> 22 us at 13,500 atoms in 125 cells, 33 -> 15 at 31,000)
-    const int split = per > 1 ? 1 : std::max(1, std::min(8, nblk(c->N, 64 * c->ncell_total)));
-    hipLaunchKernelGGL(k_sort_gather, dim3(nblk(nblk(c->ncell_total, per) * split, 4)), dim3(256), 0, c->stream,
-                       c->ncell_total, per, split, c->cell_rep, c->reps_d, c->rebuild, any_flag(c), c->cbin,
-                       c->acell, c->bucket, c->bucket_cap, c->ccount, c->cstart, c->tt, c->atombin,
-                       c->N, c->a, c->b, (int)mode, T);
+StepArrays step_arrays(sofia_ctx *c, SortMode mode) {
+    if (mode != SORT_STEP) return StepArrays{};
+    const int rb = record_bytes(c);
+    return StepArrays{c->fix, c->fscratch, rb ? c->pfix : nullptr, rb == 16 ? c->a.q : nullptr};
+}
+
+CopyArgs copy_args(sofia_ctx *c, SortMode mode, int *items) {
     RemapSet S{};
     int total = 0;
     auto add = [&](int32_t *lst, int items, int width, int nidx) {
@@ -581,10 +477,29 @@ void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies) {
     add(c->shake_atoms, c->ns, 4, 4);
     add(c->ebond, c->nbe, 3, 2);
     add(c->eangle, c->nae, 4, 3);
-    const int items = std::max({c->N, total, c->ncell_total});
-    hipLaunchKernelGGL(k_copyback, dim3(capped(items, 256)), dim3(256), 0, c->stream, c->N, c->rep,
-                       c->reps_d, c->rebuild, any_flag(c), c->tt, c->b, c->a, c->dr32, c->drd,
-                       (int)mode, T, S, c->ncell_total, c->cell_rep, c->cbin);
+    *items = std::max({c->N, total, c->ncell_total});
+    return CopyArgs{c->N, c->ncell_total, (int)mode, c->rep, c->rebuild, any_flag(c), c->tt, c->cell_rep,
+                    c->reps_d, c->b, c->a, c->dr32, c->drd, step_arrays(c, mode), S, c->cbin};
+}
+
+void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies, bool leave_copy) {
+    const BinArgs B{c->N, c->bucket_cap, c->a.pos4, c->rep, c->reps_d, c->rebuild, any_flag(c),
+                    c->cbin, c->acell, c->bucket};
+    const int bin_grid = capped(c->N, 256);
+    if (bonded) launch_bundles_bin(c, B, bin_grid, energies);
+    else hipLaunchKernelGGL(k_bin, dim3(bin_grid), dim3(256), 0, c->stream, B);
+    const int per = nblk(c->ncell_total, 4 * GRID_CAP);   // cells per wavefront
+    // or wavefronts per cell, where a cell holds more atoms than a wavefront has lanes (the
+    // reference's cells: 30 -> 22 us at 13,500 atoms in 125 cells, 33 -> 15 at 31,000)
+    const int split = per > 1 ? 1 : std::max(1, std::min(8, nblk(c->N, 64 * c->ncell_total)));
+    hipLaunchKernelGGL(k_sort_gather, dim3(nblk(nblk(c->ncell_total, per) * split, 4)), dim3(256), 0, c->stream,
+                       c->ncell_total, per, split, c->cell_rep, c->reps_d, c->rebuild, any_flag(c), c->cbin,
+                       c->acell, c->bucket, c->bucket_cap, c->ccount, c->cstart, c->tt, c->atombin,
+                       c->N, c->a, c->b, (int)mode, step_arrays(c, mode));
+    if (leave_copy) return;
+    int items = 0;
+    const CopyArgs A = copy_args(c, mode, &items);
+    hipLaunchKernelGGL(k_copyback, dim3(capped(items, 256)), dim3(256), 0, c->stream, A);
 }
 
 void launch_rdf(sofia_ctx *c, int32_t itype, int32_t jtype, double delta, int32_t nbins,
@@ -603,8 +518,11 @@ void launch_host_ids(sofia_ctx *c, const int32_t *src, int32_t *dst, size_t item
                        dst, c->rep, c->reps_d);
 }
 
-void launch_build_list(sofia_ctx *c) {
-    if (c->n_stencil5 > 0) launch_build_list_engine(c);
+// The sort's copy back rides with the engine's list build where that builds every list.
+bool list_takes_copy(const sofia_ctx *c) { return c->n_stencil5 == c->nrep; }
+
+void launch_build_list(sofia_ctx *c, bool copy) {
+    if (c->n_stencil5 > 0) launch_build_list_engine(c, copy);
     if (c->n_stencil5 == c->nrep) return;
     // few cells (the reference's are a cutoff wide: 125 in a 13,500-atom box) leave most of the
     // chip idle: their atoms go to several workgroups, each staging the stencil for itself

@@ -1633,11 +1633,11 @@ void force_sequence(sofia_ctx *c, bool energies) {
 // One MD step up to its last half kick, which the next step's k_advance applies (kick2) or,
 // at a segment's end, launch_nve_v64.
 void step_sequence(sofia_ctx *c, bool kick2, bool energies) {
-    const bool bonded = sort_takes_bonded(c);
+    const bool bonded = sort_takes_bonded(c), copy = list_takes_copy(c);
     launch_advance(c, kick2);
     if (energies) launch_zero_energies(c);
-    launch_sort(c, SORT_STEP, bonded, energies);
-    launch_build_list(c);
+    launch_sort(c, SORT_STEP, bonded, energies, copy);
+    launch_build_list(c, copy);
     launch_nonbond(c, nb_mode(c), energies, true);
     if (!bonded) launch_bonded_engine(c, energies);
     launch_shake64(c, energies, true);
@@ -2243,8 +2243,8 @@ int sofia_minimize(sofia_ctx *c, int32_t nsteps, double gamma, double max_disp) 
         if (s == 0 || !with_sort) launch_bonded_engine(c, false);
         launch_water_bonded(c);
         launch_minimize_step(c, gamma, max_disp);
-        launch_sort(c, SORT_STEP, with_sort && s + 1 < nsteps);
-        launch_build_list(c);
+        launch_sort(c, SORT_STEP, with_sort && s + 1 < nsteps, false, list_takes_copy(c));
+        launch_build_list(c, list_takes_copy(c));
     }
     if (nsteps > 0) launch_finish_rebuild(c);
     c->has_thermostat = thermo;
@@ -2366,8 +2366,8 @@ int sofia_profile_step(sofia_ctx *c, int32_t nsteps, int32_t full_rebuild, doubl
         mark();
         launch_advance(c, false); mark(); mark(); mark();
         if (full_rebuild) launch_set_rebuild(c, 1);
-        launch_sort(c, SORT_STEP); mark();
-        launch_build_list(c); mark(); mark(); mark();
+        launch_sort(c, SORT_STEP, false, false, list_takes_copy(c)); mark();
+        launch_build_list(c, list_takes_copy(c)); mark(); mark(); mark();
         launch_nonbond(c, nb_mode(c), false, true); mark();
         launch_bonded_engine(c, false); mark(); mark();
         launch_shake64(c, false, true); mark();

@@ -261,7 +261,10 @@ namespace sofia {
 // and the pair kernel's position records.
 enum SortMode { SORT_DROPIN = 0, SORT_ENGINE = 1, SORT_STEP = 2 };
 // bonded: with the step's bonded terms (where sort_takes_bonded)
-void launch_sort(sofia_ctx *c, SortMode mode, bool bonded = false, bool energies = false);
+// (leave_copy: its copy back is left to launch_build_list, where list_takes_copy)
+void launch_sort(sofia_ctx *c, SortMode mode, bool bonded = false, bool energies = false,
+                 bool leave_copy = false);
+bool list_takes_copy(const sofia_ctx *c);
 bool sort_takes_bonded(const sofia_ctx *c);
 struct BinArgs;
 void launch_bundles_bin(sofia_ctx *c, const BinArgs &B, int bin_grid, bool energies);
@@ -269,8 +272,8 @@ void launch_host_ids(sofia_ctx *c, const int32_t *src, int32_t *dst, size_t item
                      int nidx);
 void launch_rdf(sofia_ctx *c, int32_t itype, int32_t jtype, double delta, int32_t nbins,
                 uint32_t *hist);
-void launch_build_list(sofia_ctx *c);
-void launch_build_list_engine(sofia_ctx *c);
+void launch_build_list(sofia_ctx *c, bool copy = false);   // copy: with a step's copy back
+void launch_build_list_engine(sofia_ctx *c, bool copy);
 void launch_check_neighbor(sofia_ctx *c);
 void launch_set_rebuild(sofia_ctx *c, int32_t value);
 void launch_finish_rebuild(sofia_ctx *c);

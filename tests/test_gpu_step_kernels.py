@@ -320,3 +320,30 @@ def test_dropin_list_by_cell_images_is_the_references(ng, nw, cells, edge):
                 assert np.array_equal(a[i, :nn[i]], o[i, :nn[i]])
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("sizes,skin", [(((4, 1500), (40, 2500)), 1.5), (((4, 1500), (10, 1000)), 3.0)])
+@pytest.mark.parametrize("waves", [4, 8, 16])
+def test_list_built_beside_the_copy_back(sizes, skin, waves):
+    """Lists of a step's rebuild, read from the sort's target with exclusions re-indexed on the
+    way, and where a replica's box holds fewer than 5 half-width cells a side and keeps the
+    separate copy (the second sizes: 31.5 A against 2.5 x 13 A): every pair inside the cutoff, both ways round, and no excluded one."""
+    host = _host()
+    from test_gpu_engine import _engine_pairs, _excluded, _pairs_within
+    systems = [S.make_system(g, w, seed=70 + k) for k, (g, w) in enumerate(sizes)]
+    e = host.Engine([host.ReplicaSpec(s, temp=700.0, gamma_ps=5.0, seed=3) for s in systems])
+    try:
+        e.set_tuning(16, 256, waves)
+        e.set_skin(skin)
+        e.init()
+        e.minimize(30)
+        e.run(60 if skin < 2.0 else 250)
+        assert e.rebuilds().min() > 1
+        d = systems[0].derived()
+        rc = float(np.sqrt(max(d["rcut2"], d["cut_coulsq"])))
+        for s, (x, gid, pairs) in zip(systems, _engine_pairs(e)):
+            ex = _excluded(s, gid)
+            assert _pairs_within(x, float(s.box), rc) - ex <= pairs
+            assert not pairs & ex
+    finally:
+        e.close()
