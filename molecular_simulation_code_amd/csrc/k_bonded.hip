@@ -494,9 +494,8 @@ k_bonded_items(BondedItems I, BondedArgs A, DevParams P, long long *__restrict__
 // steps with a rebuild, 518 and 509 (the binning loses nothing to the bundles' 225 registers).
 template <bool BIN>
 __global__ void __launch_bounds__(BUNDLE_THREADS)
-k_bonded_bundles(int32_t nbundle, const int32_t *__restrict__ tstart, const int2 *__restrict__ terms,
-                 const int32_t *__restrict__ sstart, const int32_t *__restrict__ slots,
-                 BondedArgs A, DevParams P, long long *__restrict__ fout,
+k_bonded_bundles(int32_t nbundle, const int4 *__restrict__ heads, const int2 *__restrict__ terms,
+                 const int32_t *__restrict__ slots, BondedArgs A, DevParams P, long long *__restrict__ fout,
                  long long *__restrict__ eacc, bool energies, BinArgs B) {
     __shared__ unsigned long long s_f[3 * BUNDLE_SLOTS];
     const int b = blockIdx.x, lane = threadIdx.x;
@@ -505,14 +504,24 @@ k_bonded_bundles(int32_t nbundle, const int32_t *__restrict__ tstart, const int2
             bin_atoms(B, (b - nbundle) * BUNDLE_THREADS + lane, (gridDim.x - nbundle) * BUNDLE_THREADS);
         return;
     }
-    const int t0 = tstart[b], t1 = tstart[b + 1];
-    const int s0 = sstart[b], ns = sstart[b + 1] - s0;
-    for (int k = lane; k < 3 * ns; k += BUNDLE_THREADS) s_f[k] = 0ull;
-    // the bundle's replica, from its first atom
-    const uint32_t first = (uint32_t)slots[s0];
-    const int r = A.rep[A.lst[first >> 29][first & 0x1fffffffu]];
+    const int4 head = heads[b];
+    const int t0 = head.x, t1 = head.y, s0 = head.z, ns = head.w & 0xff, r = head.w >> 8;
     const float boxf = A.reps[r].box, iboxf = A.reps[r].ibox;
     const double box = boxf, ibox = iboxf;
+    // a thread's slot: its atom and what the sums hold for it, fetched beside the terms (a
+    // bundle is a chain of dependent loads; this one stood at its end)
+    static_assert(BUNDLE_SLOTS <= BUNDLE_THREADS && BUNDLE_SLOTS < 256, "one slot per thread");
+    int atom = 0;
+    long long held[3] = {0, 0, 0};
+    if (lane < ns) {
+        const uint32_t rec = (uint32_t)slots[s0 + lane];
+        atom = A.lst[rec >> 29][rec & 0x1fffffffu];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            s_f[3 * lane + k] = 0ull;
+            held[k] = fout[(size_t)k * A.n + atom];
+        }
+    }
     __syncthreads();
     // energies in quanta per item, as the per-item kernels form them
     long long ec = 0, el = 0, ed = 0, ei = 0, eb = 0, ea = 0;
@@ -546,14 +555,10 @@ k_bonded_bundles(int32_t nbundle, const int32_t *__restrict__ tstart, const int2
         }
     }
     __syncthreads();
-    for (int s = lane; s < ns; s += BUNDLE_THREADS) {
-        const uint32_t rec = (uint32_t)slots[s0 + s];
-        const int atom = A.lst[rec >> 29][rec & 0x1fffffffu];
+    if (lane < ns) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            long long *p = &fout[(size_t)k * A.n + atom];
-            *p += (long long)s_f[3 * s + k];
-        }
+        for (int k = 0; k < 3; ++k)
+            fout[(size_t)k * A.n + atom] = held[k] + (long long)s_f[3 * lane + k];
     }
     if (!energies) return;
     wave_add(ec, true, r, eacc, E_COUL14);
@@ -658,15 +663,15 @@ bool sort_takes_bonded(const sofia_ctx *c) {
 
 void launch_bundles_bin(sofia_ctx *c, const BinArgs &B, int bin_grid, bool energies) {
     hipLaunchKernelGGL(k_bonded_bundles<true>, dim3(c->nbundle + bin_grid), dim3(BUNDLE_THREADS), 0,
-                       c->stream, c->nbundle, c->bund_tstart, c->bund_terms, c->bund_sstart,
-                       c->bund_slots, engine_args(c), c->dp, c->fix, c->eacc, energies, B);
+                       c->stream, c->nbundle, c->bund_heads, c->bund_terms, c->bund_slots, engine_args(c),
+                       c->dp, c->fix, c->eacc, energies, B);
 }
 
 void launch_bonded_engine(sofia_ctx *c, bool energies) {
     const BondedArgs A = engine_args(c);
     if (c->bonded_bundles && c->nbundle > 0) {
         hipLaunchKernelGGL(k_bonded_bundles<false>, dim3(c->nbundle), dim3(BUNDLE_THREADS), 0, c->stream,
-                           c->nbundle, c->bund_tstart, c->bund_terms, c->bund_sstart, c->bund_slots, A,
+                           c->nbundle, c->bund_heads, c->bund_terms, c->bund_slots, A,
                            c->dp, c->fix, c->eacc, energies, BinArgs{});
         return;
     }

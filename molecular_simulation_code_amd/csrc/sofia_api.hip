@@ -590,7 +590,7 @@ int rebuild_now(sofia_ctx *c, bool engine, bool reference_growth, int32_t *tt = 
 }  // namespace
 
 void drop_bonded_bundles(sofia_ctx *c) {
-    dfree(c->bund_tstart); dfree(c->bund_sstart); dfree(c->bund_slots); dfree(c->bund_terms);
+    dfree(c->bund_heads); dfree(c->bund_slots); dfree(c->bund_terms);
     c->nbundle = 0;
     drop_graph(c);
 }
@@ -703,7 +703,9 @@ int build_bonded_bundles(sofia_ctx *c) {
     };
     std::sort(order.begin(), order.end(), [&](int a, int b) { return mol_min[a] < mol_min[b]; });
     // pack; a bundle's items go out sorted by kind (the record's top bits)
-    std::vector<int32_t> tstart{0}, sstart{0}, slots, local(n, -1);
+    std::vector<int32_t> slots, local(n, -1);
+    std::vector<int4> heads;
+    int t0 = 0, s0 = 0;   // of the bundle being filled
     std::vector<int2> recs, open_recs;
     int cur_rep = -1, cur_slots = 0;
     auto close = [&]() {
@@ -712,8 +714,10 @@ int build_bonded_bundles(sofia_ctx *c) {
         });
         recs.insert(recs.end(), open_recs.begin(), open_recs.end());
         open_recs.clear();
-        tstart.push_back((int32_t)recs.size());
-        sstart.push_back((int32_t)slots.size());
+        const int t1 = (int)recs.size(), s1 = (int)slots.size();
+        heads.push_back(int4{t0, t1, s0, cur_rep << 8 | (s1 - s0)});
+        t0 = t1;
+        s0 = s1;
         cur_slots = 0;
     };
     for (int m : order) {
@@ -738,16 +742,13 @@ int build_bonded_bundles(sofia_ctx *c) {
         }
     }
     if (!open_recs.empty()) close();
-    const int nb = (int)tstart.size() - 1;
-    TRY(dalloc(&c->bund_tstart, tstart.size()));
-    TRY(dalloc(&c->bund_sstart, sstart.size()));
+    TRY(dalloc(&c->bund_heads, heads.size()));
     TRY(dalloc(&c->bund_slots, slots.size()));
     TRY(dalloc(&c->bund_terms, recs.size()));
-    TRY(upload(c->bund_tstart, tstart.data(), sizeof(int32_t) * tstart.size()));
-    TRY(upload(c->bund_sstart, sstart.data(), sizeof(int32_t) * sstart.size()));
+    TRY(upload(c->bund_heads, heads.data(), sizeof(int4) * heads.size()));
     TRY(upload(c->bund_slots, slots.data(), sizeof(int32_t) * slots.size()));
     TRY(upload(c->bund_terms, recs.data(), sizeof(int2) * recs.size()));
-    c->nbundle = nb;
+    c->nbundle = (int32_t)heads.size();
     return SOFIA_OK;
 }
 
@@ -801,7 +802,7 @@ int sofia_ctx_destroy(sofia_ctx *c) {
     dfree(c->gc_refx); dfree(c->gc_com); dfree(c->gc_key); dfree(c->gc_surface);
     dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep);
     dfree(c->cbin); dfree(c->bucket); dfree(c->mtab); dfree(c->nlist);
-    dfree(c->bund_tstart); dfree(c->bund_sstart); dfree(c->bund_slots); dfree(c->bund_terms);
+    dfree(c->bund_heads); dfree(c->bund_slots); dfree(c->bund_terms);
     dfree(c->water); dfree(c->dsf_tab); dfree(c->ebond); dfree(c->eangle); dfree(c->bondlist); dfree(c->anglelist);
     dfree(c->dihedlist); dfree(c->torsions); dfree(c->shake_num); dfree(c->shake_atoms); dfree(c->shake_kidx);
     dfree(c->ptab);

@@ -174,10 +174,11 @@ struct sofia_ctx {
     // engine bonded bundles (k_bonded_bundles): per bundle the ranges of its term and atom-slot
     // records; nbundle = 0 runs the per-kind kernels instead
     int32_t nbundle = 0;
-    // run the bundles (tuning choice) rather than one thread per item: 10 against 11 us at
-    // 5,000 atoms, 11 / 17 at 55,000, 21 / 47 at 264,000, 16 / 39 at 204,000 (1,200 glycines)
+    // run the bundles (tuning choice) rather than one thread per item: 7 against 11 us at
+    // 5,000 atoms, 8 / 17 at 55,000, 16 / 47 at 264,000, 12 / 39 at 204,000 (1,200 glycines)
     bool bonded_bundles = true;
-    int32_t *bund_tstart = nullptr, *bund_sstart = nullptr, *bund_slots = nullptr;
+    int4 *bund_heads = nullptr;   // first and last term, first slot, replica << 8 | slots
+    int32_t *bund_slots = nullptr;
     int2 *bund_terms = nullptr;
 
     // force field
@@ -356,12 +357,14 @@ inline int mixed_lanes(const sofia_ctx *c, bool energies = false) {
 inline int ordered_lanes(const sofia_ctx *c) { return c->lanes >= 0 ? c->lanes : 16; }
 // Threads per workgroup of the mixed pair kernel: each workgroup stages the DSF table (16 KB)
 // and the type-pair tables in LDS, so large workgroups spend less of the load path on it
-// (-4.8 % at 1,280,000 atoms), but a grid of few of them leaves compute units idle (5,000
-// atoms at 16 lanes: 22 us in 1024-thread workgroups, 16.5 in 256; 55,000: 65 / 60).
+// (-4.8 % at 1,280,000 atoms), but a grid of few of them leaves compute units idle: by
+// workgroups of 256 / 512 / 1024 threads and the lanes above, 12.6 / 13.1 / 14.8 us at 5,000
+// atoms, 28.5 / 27.4 / 30.6 at 20,000, 63 / 61 / 66 at 55,000.
 inline int mixed_block(const sofia_ctx *c, bool energies) {
     if (c->block > 0) return c->block;
     if (energies) return 512;   // two tables to stage
-    return (long long)c->N * mixed_lanes(c) / 1024 < 1024 ? 256 : 1024;
+    if ((long long)c->N * mixed_lanes(c) / 1024 >= 1024) return 1024;
+    return c->N < 6000 ? 256 : 512;
 }
 
 // error helpers (sofia_api.cpp)
