@@ -91,7 +91,11 @@ k_nonbond(int32_t n, const float4 *__restrict__ pos4, const float *__restrict__ 
     const int r = rep[ii];
     const float box = reps[r].box, ibox = reps[r].ibox;
     const int nn = live ? min(numneigh[ii], na) : 0;   // a row never reads past its stride
-    const int32_t *lst = nlist + (size_t)ii * na;
+    // the list by 32-bit offsets from the row of the wavefront's first atom
+    const int iw = __builtin_amdgcn_readfirstlane(ii);
+    const uint32_t *lists = (const uint32_t *)nlist + (size_t)iw * na;
+    const uint32_t row0 = (uint32_t)(ii - iw) * (uint32_t)na * 4u;
+    const uint32_t row1 = row0 + 4u * (uint32_t)max(nn - 1, 0);   // its last entry
     const float4 *ljrow = s_lj + ti * P.ntypes - 1;   // index by jtype (1-based)
     const double2 *ljrow64 = s_lj64 + 2 * (ti * P.ntypes - 1);
     // QT (charges by atom type): C qi qj from a type-pair table, formed as from the atoms'
@@ -111,19 +115,22 @@ k_nonbond(int32_t n, const float4 *__restrict__ pos4, const float *__restrict__ 
         const double a2 = P.alpha * P.alpha, pa = P.ewald_p * P.alpha;
         // software pipeline: an entry's data is loaded one iteration ahead; loads past the
         // end of the row re-read its last entry (clamped index), so no branch is needed
-        const int last = max(nn - 1, 0);
-        const uint32_t *ulst = (const uint32_t *)lst;
-        const uint32_t j0 = (nn > 0) ? ulst[min(sub, last)] : (uint32_t)ii;
-        uint32_t jnn = (nn > 0) ? ulst[min(sub + L, last)] : (uint32_t)ii;
-        float4 pn = pos4[j0];
-        float qn = QT ? 0.0f : q[j0];
-#pragma unroll 2
+        uint32_t at = row0 + 4u * (uint32_t)sub;
+        const uint32_t j0 = (nn > 0) ? elem(lists, min(at, row1)) : (uint32_t)ii;
+        at += 4u * L;
+        uint32_t jnn = (nn > 0) ? elem(lists, min(at, row1)) : (uint32_t)ii;
+        float4 pn = elem(pos4, 16u * j0);
+        float qn = QT ? 0.0f : elem(q, 4u * j0);
+        // (not unrolled: two entries at a time cost the wavefronts that hide the latency, 91
+        // registers against 70, and the FP64 kernel 4 % at 204,000 atoms)
+#pragma unroll 1
         for (int k = sub; k < nn; k += L) {
             const float4 pj = pn;
             const float qj = qn;
-            pn = pos4[jnn];
-            if (!QT) qn = q[jnn];
-            jnn = ulst[min(k + 2 * L, last)];
+            pn = elem(pos4, 16u * jnn);
+            if (!QT) qn = elem(q, 4u * jnn);
+            at += 4u * L;
+            jnn = elem(lists, min(at, row1));
             double dx = x1 - (double)pj.x, dy = y1 - (double)pj.y, dz = z1 - (double)pj.z;
             dx -= bx * __builtin_rint(dx * ib);
             dy -= bx * __builtin_rint(dy * ib);
@@ -168,19 +175,22 @@ k_nonbond(int32_t n, const float4 *__restrict__ pos4, const float *__restrict__ 
                     A5 = (float)P.a5;
         // software pipeline: an entry's data is loaded one iteration ahead; loads past the
         // end of the row re-read its last entry (clamped index), so no branch is needed
-        const int last = max(nn - 1, 0);
-        const uint32_t *ulst = (const uint32_t *)lst;
-        const uint32_t j0 = (nn > 0) ? ulst[min(sub, last)] : (uint32_t)ii;
-        uint32_t jnn = (nn > 0) ? ulst[min(sub + L, last)] : (uint32_t)ii;
-        float4 pn = pos4[j0];
-        float qn = QT ? 0.0f : q[j0];
-#pragma unroll 2
+        uint32_t at = row0 + 4u * (uint32_t)sub;
+        const uint32_t j0 = (nn > 0) ? elem(lists, min(at, row1)) : (uint32_t)ii;
+        at += 4u * L;
+        uint32_t jnn = (nn > 0) ? elem(lists, min(at, row1)) : (uint32_t)ii;
+        float4 pn = elem(pos4, 16u * j0);
+        float qn = QT ? 0.0f : elem(q, 4u * j0);
+        // (not unrolled: two entries at a time cost the wavefronts that hide the latency, 91
+        // registers against 70, and the FP64 kernel 4 % at 204,000 atoms)
+#pragma unroll 1
         for (int k = sub; k < nn; k += L) {
             const float4 pj = pn;
             const float qj = qn;
-            pn = pos4[jnn];
-            if (!QT) qn = q[jnn];
-            jnn = ulst[min(k + 2 * L, last)];
+            pn = elem(pos4, 16u * jnn);
+            if (!QT) qn = elem(q, 4u * jnn);
+            at += 4u * L;
+            jnn = elem(lists, min(at, row1));
             float dx = xi.x - pj.x, dy = xi.y - pj.y, dz = xi.z - pj.z;
             dx -= box * __builtin_rintf(dx * ibox);
             dy -= box * __builtin_rintf(dy * ibox);

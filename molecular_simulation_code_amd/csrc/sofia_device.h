@@ -232,6 +232,13 @@ __device__ inline void finish_rebuild(int r, int nrep, int32_t *rebuild, int32_t
     rebuild[r] = 0;
 }
 
+// Element of a wave-uniform array by a 32-bit byte offset: one address register, where a
+// 64-bit index takes two and the instructions that widen it.
+template <class T>
+__device__ __forceinline__ const T &elem(const T *base, uint32_t byte) {
+    return *(const T *)((const char *)base + byte);
+}
+
 inline int nblocks(long long n, int b) { return (int)((n + b - 1) / b); }
 
 }  // namespace sofia
