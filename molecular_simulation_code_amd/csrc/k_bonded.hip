@@ -9,7 +9,7 @@
 // Drop-in variants read the real*4 positions and follow the reference's precision
 // (real*4 coordinate difference and charge product, double for the rest); the engine
 // variants read the FP64 positions of the device-resident state.
-#include "sofia_device.h"
+#include "water_device.h"
 
 namespace sofia {
 namespace {
@@ -492,16 +492,24 @@ k_bonded_items(BondedItems I, BondedArgs A, DevParams P, long long *__restrict__
 // rebuilds nothing is an empty launch otherwise.  A step took 51.9 us at 5,000 atoms and 128
 // at 55,000 with the two apart, and takes 49.9 and 126; 264,000 atoms in 12 replicas, most
 // steps with a rebuild, 518 and 509 (the binning loses nothing to the bundles' 225 registers).
+// nbin: the workgroups that bin; those past them take the rigid waters' own terms in the
+// minimiser, whose moves run no constraint kernel (51 -> 45.5 us a move at 20,000 atoms; in
+// MD steps, taking them out of the constraint kernel, they cost a second pass: 45 -> 49 us a
+// step at 5,000 atoms, 122 -> 128 at 55,000).
 template <bool BIN>
 __global__ void __launch_bounds__(BUNDLE_THREADS)
 k_bonded_bundles(int32_t nbundle, const int4 *__restrict__ heads, const int2 *__restrict__ terms,
                  const int32_t *__restrict__ slots, BondedArgs A, DevParams P, long long *__restrict__ fout,
-                 long long *__restrict__ eacc, bool energies, BinArgs B) {
+                 long long *__restrict__ eacc, bool energies, int32_t nbin, BinArgs B,
+                 const int32_t *__restrict__ shake_num, int32_t ns_water, ShakeArgs W) {
     __shared__ unsigned long long s_f[3 * BUNDLE_SLOTS];
     const int b = blockIdx.x, lane = threadIdx.x;
+    if (BIN && b >= nbundle + nbin) {
+        water_terms(ns_water, shake_num, W, (b - nbundle - nbin) * BUNDLE_THREADS + lane);
+        return;
+    }
     if (BIN && b >= nbundle) {
-        if (*B.any)
-            bin_atoms(B, (b - nbundle) * BUNDLE_THREADS + lane, (gridDim.x - nbundle) * BUNDLE_THREADS);
+        if (*B.any) bin_atoms(B, (b - nbundle) * BUNDLE_THREADS + lane, nbin * BUNDLE_THREADS);
         return;
     }
     const int4 head = heads[b];
@@ -661,10 +669,11 @@ bool sort_takes_bonded(const sofia_ctx *c) {
     return c->bonded_bundles && c->nbundle > 0;
 }
 
-void launch_bundles_bin(sofia_ctx *c, const BinArgs &B, int bin_grid, bool energies) {
-    hipLaunchKernelGGL(k_bonded_bundles<true>, dim3(c->nbundle + bin_grid), dim3(BUNDLE_THREADS), 0,
+void launch_bundles_bin(sofia_ctx *c, const BinArgs &B, int bin_grid, bool energies, bool water) {
+    const int nw = water && c->water_split ? nblocks(c->ns, BUNDLE_THREADS) : 0;
+    hipLaunchKernelGGL(k_bonded_bundles<true>, dim3(c->nbundle + bin_grid + nw), dim3(BUNDLE_THREADS), 0,
                        c->stream, c->nbundle, c->bund_heads, c->bund_terms, c->bund_slots, engine_args(c),
-                       c->dp, c->fix, c->eacc, energies, B);
+                       c->dp, c->fix, c->eacc, energies, bin_grid, B, c->shake_num, c->ns, shake_args(c));
 }
 
 void launch_bonded_engine(sofia_ctx *c, bool energies) {
@@ -672,7 +681,7 @@ void launch_bonded_engine(sofia_ctx *c, bool energies) {
     if (c->bonded_bundles && c->nbundle > 0) {
         hipLaunchKernelGGL(k_bonded_bundles<false>, dim3(c->nbundle), dim3(BUNDLE_THREADS), 0, c->stream,
                            c->nbundle, c->bund_heads, c->bund_terms, c->bund_slots, A,
-                           c->dp, c->fix, c->eacc, energies, BinArgs{});
+                           c->dp, c->fix, c->eacc, energies, 0, BinArgs{}, nullptr, 0, ShakeArgs{});
         return;
     }
     launch_items(c, A, c->nd, c->water_split ? c->nbe : c->nb, c->water_split ? c->nae : c->na,

@@ -181,7 +181,8 @@ k_dsf_mixed(int32_t n, const int4 *__restrict__ pf,
             const int32_t *__restrict__ nlist, const int32_t *__restrict__ numneigh, int32_t na,
             const float4 *__restrict__ ljtab, const float4 *__restrict__ ptab,
             const float4 *__restrict__ tab, DevParams P,
-            double *__restrict__ fnb, float *__restrict__ ff32, long long *__restrict__ eacc) {
+            double *__restrict__ fnb, float *__restrict__ ff32, long long *__restrict__ eacc, Books B) {
+    close_books(B);
     // QT: charges by atom type; 12-byte records (x, y, z) and a pair table (lj1, lj2,
     // C q_i q_j) in place of the charge in the record
     extern __shared__ float4 s_dyn[];
@@ -362,7 +363,8 @@ k_dsf_compact(int32_t n, const int4 *__restrict__ pf,
               const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
               const int32_t *__restrict__ nlist, const int32_t *__restrict__ numneigh, int32_t na,
               const float4 *__restrict__ ljtab, const float4 *__restrict__ tab, DevParams P,
-              double *__restrict__ fnb, float *__restrict__ ff32, long long *__restrict__ eacc) {
+              double *__restrict__ fnb, float *__restrict__ ff32, long long *__restrict__ eacc, Books B) {
+    close_books(B);
     extern __shared__ float4 s_dyn[];
     const int nt2 = P.ntypes * P.ntypes;
     const int tn = P.tab_n;
@@ -489,7 +491,7 @@ k_dsf_compact(int32_t n, const int4 *__restrict__ pf,
 }
 
 template <int L>
-void launch_lanes(sofia_ctx *c, bool energies, float *ff32, bool qt) {
+void launch_lanes(sofia_ctx *c, bool energies, float *ff32, bool qt, const Books &B) {
     const int block = mixed_block(c, energies);
     const long long threads = (long long)c->N * L;
     const int grid = (int)((threads + block - 1) / block);
@@ -498,7 +500,7 @@ void launch_lanes(sofia_ctx *c, bool energies, float *ff32, bool qt) {
 #define DSF_LAUNCH(E, Q)                                                                          \
     hipLaunchKernelGGL((k_dsf_mixed<L, E, Q>), dim3(grid), dim3(block), lds, c->stream, c->N,       \
                        c->pfix, c->rep, c->reps_d, c->nlist, c->numneigh, c->neigh_alloc,          \
-                       c->ljtab, c->ptab, c->dsf_tab, c->dp, c->fnb, ff32, c->eacc)
+                       c->ljtab, c->ptab, c->dsf_tab, c->dp, c->fnb, ff32, c->eacc, B)
     if (energies) {
         if (qt) DSF_LAUNCH(true, true); else DSF_LAUNCH(true, false);
     } else {
@@ -507,7 +509,7 @@ void launch_lanes(sofia_ctx *c, bool energies, float *ff32, bool qt) {
 #undef DSF_LAUNCH
 }
 
-void launch_compact(sofia_ctx *c, bool energies, float *ff32) {
+void launch_compact(sofia_ctx *c, bool energies, float *ff32, const Books &B) {
     const int grid = (c->N + 3) / 4;
     const int nt2 = c->dp.ntypes * c->dp.ntypes;
     const size_t lds = sizeof(float4) * (nt2 + (energies ? 2 : 1) * (c->dp.tab_n + 1) + 4 * QRING) +
@@ -515,11 +517,11 @@ void launch_compact(sofia_ctx *c, bool energies, float *ff32) {
     if (energies)
         hipLaunchKernelGGL(k_dsf_compact<true>, dim3(grid), dim3(256), lds, c->stream, c->N,
                            c->pfix, c->rep, c->reps_d, c->nlist, c->numneigh,
-                           c->neigh_alloc, c->ljtab, c->dsf_tab, c->dp, c->fnb, ff32, c->eacc);
+                           c->neigh_alloc, c->ljtab, c->dsf_tab, c->dp, c->fnb, ff32, c->eacc, B);
     else
         hipLaunchKernelGGL(k_dsf_compact<false>, dim3(grid), dim3(256), lds, c->stream, c->N,
                            c->pfix, c->rep, c->reps_d, c->nlist, c->numneigh,
-                           c->neigh_alloc, c->ljtab, c->dsf_tab, c->dp, c->fnb, ff32, c->eacc);
+                           c->neigh_alloc, c->ljtab, c->dsf_tab, c->dp, c->fnb, ff32, c->eacc, B);
 }
 
 }  // namespace
@@ -531,19 +533,20 @@ int record_bytes(const sofia_ctx *c) {
     return (c->q_by_type && c->ptab && mixed_lanes(c) != 0) ? 12 : 16;
 }
 
-void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records) {
+void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records, bool close) {
+    const Books B = books(c, close);
     const bool qt = c->q_by_type && c->ptab && mixed_lanes(c) != 0;
     if (!records)
         hipLaunchKernelGGL(k_fixpos, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N,
                            from_xd ? c->a.xd : nullptr, c->a.pos4, qt ? nullptr : c->a.q, c->rep,
                            c->reps_d, c->pfix);
     switch (mixed_lanes(c, energies)) {
-        case 0: launch_compact(c, energies, ff32); break;
-        case 4: launch_lanes<4>(c, energies, ff32, qt); break;
-        case 8: launch_lanes<8>(c, energies, ff32, qt); break;
-        case 32: launch_lanes<32>(c, energies, ff32, qt); break;
-        case 64: launch_lanes<64>(c, energies, ff32, qt); break;
-        default: launch_lanes<16>(c, energies, ff32, qt); break;
+        case 0: launch_compact(c, energies, ff32, B); break;
+        case 4: launch_lanes<4>(c, energies, ff32, qt, B); break;
+        case 8: launch_lanes<8>(c, energies, ff32, qt, B); break;
+        case 32: launch_lanes<32>(c, energies, ff32, qt, B); break;
+        case 64: launch_lanes<64>(c, energies, ff32, qt, B); break;
+        default: launch_lanes<16>(c, energies, ff32, qt, B); break;
     }
 }
 

@@ -9,7 +9,7 @@
 //    as FP64 nonbond sums + int64 fixed-point sums of every other term.
 #include <type_traits>
 
-#include "sofia_device.h"
+#include "water_device.h"
 
 namespace sofia {
 namespace {
@@ -552,44 +552,6 @@ __global__ void k_langevin64(int32_t n, const float4 *__restrict__ pos4, const d
     }
 }
 
-struct ShakeArgs {
-    const int32_t *atoms;
-    const double *bond;
-    const int4 *water;        // per cluster: bond types (O-H1, O-H2), angle type, fused flag
-    const float4 *pos4;
-    const double *xd, *vd, *fnb;
-    long long *fix;
-    const double4 *mtab;
-    const int32_t *rep;
-    const RepInfo *reps;
-    const double *bond_k, *bond_r0, *angle_k, *angle_th0;
-    int32_t n;
-    double dt, dtsq, tol;
-    int maxiter;
-    int32_t *err;
-};
-
-// The two O-H bonds and the H-O-H angle of a rigid water (atoms idx = O, H1, H2), added to
-// the atoms' fixed-point sums with the quanta the bond and angle kernels would add.
-__device__ inline void water_bonded(const int4 w, const ShakeArgs &A, const int *idx, double box,
-                                    double ibox, long long (*own)[3], long long &eb, long long &ea) {
-    long long f[3], f1[3], f3[3];
-    eb += bond_term(A.xd, A.n, idx[0], idx[1], box, ibox, A.bond_k[w.x - 1], A.bond_r0[w.x - 1], f);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) { own[0][c] += f[c]; own[1][c] -= f[c]; }
-    eb += bond_term(A.xd, A.n, idx[0], idx[2], box, ibox, A.bond_k[w.y - 1], A.bond_r0[w.y - 1], f);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) { own[0][c] += f[c]; own[2][c] -= f[c]; }
-    ea += angle_term(A.xd, A.n, idx[1], idx[0], idx[2], box, ibox, A.angle_k[w.z - 1],
-                     A.angle_th0[w.z - 1], f1, f3);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        own[1][c] += f1[c];
-        own[0][c] -= f1[c] + f3[c];
-        own[2][c] += f3[c];
-    }
-}
-
 // One cluster of kind KIND.  A fused rigid water (KIND -3, water flag set) also evaluates its
 // two O-H bonds and its H-O-H angle here -- with the same fixed-point quanta the bond and
 // angle kernels would add -- and owns its three atoms, so it writes their force sums without
@@ -956,24 +918,9 @@ __global__ void k_put_state(int32_t n, AtomArrays up, AtomArrays state, bool v, 
     if (__ballot(out) && __lane_id() == 0) hw->type_err = 1;   // every lane writes the same
 }
 
-// The fused rigid-water bonded terms alone (steps that run no SHAKE: the minimiser), their
-// energies left to the closing force evaluation; the rebuild flags are cleared here instead of
-// by a launch (with the bonded terms beside the binning 59 -> 54 us a move at 20,000 atoms).
-__global__ void k_water_bonded(int32_t ns, const int32_t *__restrict__ num, ShakeArgs A, int32_t nrep,
-                               int32_t *__restrict__ rebuild, int32_t *__restrict__ nbuilds) {
-    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-    if (m <= nrep) finish_rebuild(m, nrep, rebuild, nbuilds);
-    if (m < ns && num[m] != 1 && num[m] != 3 && num[m] != 4 && A.water[m].w != 0) {
-        int idx[3];
-        for (int k = 0; k < 3; ++k) idx[k] = A.atoms[4 * (size_t)m + k];
-        const int rr = A.rep[idx[0]];
-        long long own[3][3], eb = 0, ea = 0;
-        for (int a = 0; a < 3; ++a)
-            for (int c = 0; c < 3; ++c) own[a][c] = A.fix[(size_t)c * A.n + idx[a]];
-        water_bonded(A.water[m], A, idx, A.reps[rr].box, A.reps[rr].ibox, own, eb, ea);
-        for (int a = 0; a < 3; ++a)
-            for (int c = 0; c < 3; ++c) A.fix[(size_t)c * A.n + idx[a]] = own[a][c];
-    }
+// The fused rigid-water bonded terms alone (steps that run no SHAKE: the minimiser).
+__global__ void k_water_bonded(int32_t ns, const int32_t *__restrict__ num, ShakeArgs A) {
+    water_terms(ns, num, A, blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // Capped steepest descent: every atom moves along its force by min(gamma |F|, max_disp); then,
@@ -1193,12 +1140,9 @@ void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst) {
 }
 
 void launch_water_bonded(sofia_ctx *c) {
-    if (!c->ns || !c->water_split) {
-        launch_finish_rebuild(c);
-        return;
-    }
-    hipLaunchKernelGGL(k_water_bonded, dim3(nblocks(std::max(c->ns, c->nrep + 1), 128)), dim3(128), 0,
-                       c->stream, c->ns, c->shake_num, shake_args(c), c->nrep, c->rebuild, c->nbuilds);
+    if (!c->ns || !c->water_split) return;
+    hipLaunchKernelGGL(k_water_bonded, dim3(nblocks(c->ns, 128)), dim3(128), 0, c->stream, c->ns,
+                       c->shake_num, shake_args(c));
 }
 
 void launch_minimize_step(sofia_ctx *c, double gamma, double max_disp) {

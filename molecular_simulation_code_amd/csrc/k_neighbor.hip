@@ -482,11 +482,11 @@ CopyArgs copy_args(sofia_ctx *c, SortMode mode, int *items) {
                     c->reps_d, c->b, c->a, c->dr32, c->drd, step_arrays(c, mode), S, c->cbin};
 }
 
-void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies, bool leave_copy) {
+void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies, bool leave_copy, bool water) {
     const BinArgs B{c->N, c->bucket_cap, c->a.pos4, c->rep, c->reps_d, c->rebuild, any_flag(c),
                     c->cbin, c->acell, c->bucket};
     const int bin_grid = capped(c->N, 256);
-    if (bonded) launch_bundles_bin(c, B, bin_grid, energies);
+    if (bonded) launch_bundles_bin(c, B, bin_grid, energies, water);
     else hipLaunchKernelGGL(k_bin, dim3(bin_grid), dim3(256), 0, c->stream, B);
     const int per = nblk(c->ncell_total, 4 * GRID_CAP);   // cells per wavefront
     // or wavefronts per cell, where a cell holds more atoms than a wavefront has lanes (the

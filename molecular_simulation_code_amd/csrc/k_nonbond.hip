@@ -52,7 +52,8 @@ k_nonbond(int32_t n, const float4 *__restrict__ pos4, const float *__restrict__ 
           const int32_t *__restrict__ rep, const RepInfo *__restrict__ reps,
           const int32_t *__restrict__ nlist, const int32_t *__restrict__ numneigh, int32_t na,
           const float4 *__restrict__ ljtab, const float4 *__restrict__ ptab, DevParams P,
-          double *__restrict__ fnb, float *__restrict__ ff32, long long *__restrict__ eacc) {
+          double *__restrict__ fnb, float *__restrict__ ff32, long long *__restrict__ eacc, Books B) {
+    close_books(B);
     // LDS, sized at launch: the LJ table (FP64 mode: as doubles, then the 64 values 2^(k/64)
     // of exp_tab)
     static_assert(MODE == 0 || MODE == 2, "mode 1 is k_dsf_mixed");
@@ -251,7 +252,7 @@ k_nonbond(int32_t n, const float4 *__restrict__ pos4, const float *__restrict__ 
 }
 
 template <int L, int MODE>
-void launch_t(sofia_ctx *c, bool energies, float *ff32) {
+void launch_t(sofia_ctx *c, bool energies, float *ff32, bool close) {
     const int block = c->block > 0 ? std::min(c->block, 256) : 256;   // this kernel's launch bound
     const long long threads = (long long)c->N * L;
     const int grid = (int)((threads + block - 1) / block);
@@ -262,7 +263,7 @@ void launch_t(sofia_ctx *c, bool energies, float *ff32) {
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(grid), dim3(block), lds, c->stream, c->N, c->a.pos4, c->a.q,
                            c->rep, c->reps_d, c->nlist, c->numneigh, c->neigh_alloc, c->ljtab, c->ptab,
-                           c->dp, c->fnb, ff32, c->eacc);
+                           c->dp, c->fnb, ff32, c->eacc, books(c, close));
     };
     if (qt) {
         if (energies) go(k_nonbond<L, MODE, true, true>);
@@ -274,13 +275,13 @@ void launch_t(sofia_ctx *c, bool energies, float *ff32) {
 }
 
 template <int MODE>
-void launch_mode(sofia_ctx *c, bool energies, float *ff32) {
+void launch_mode(sofia_ctx *c, bool energies, float *ff32, bool close) {
     switch (ordered_lanes(c)) {
-        case 4: launch_t<4, MODE>(c, energies, ff32); break;
-        case 8: launch_t<8, MODE>(c, energies, ff32); break;
-        case 32: launch_t<32, MODE>(c, energies, ff32); break;
-        case 64: launch_t<64, MODE>(c, energies, ff32); break;
-        default: launch_t<16, MODE>(c, energies, ff32); break;
+        case 4: launch_t<4, MODE>(c, energies, ff32, close); break;
+        case 8: launch_t<8, MODE>(c, energies, ff32, close); break;
+        case 32: launch_t<32, MODE>(c, energies, ff32, close); break;
+        case 64: launch_t<64, MODE>(c, energies, ff32, close); break;
+        default: launch_t<16, MODE>(c, energies, ff32, close); break;
     }
 }
 
@@ -288,15 +289,16 @@ void launch_mode(sofia_ctx *c, bool energies, float *ff32) {
 
 // Drop-in launches (positions from the float copy the caller handed over).
 void launch_nonbond_out(sofia_ctx *c, int mode, bool energies, float *ff32) {
-    if (mode == 0) launch_mode<0>(c, energies, ff32);
-    else if (mode == 1) launch_dsf_mixed(c, energies, ff32, false, false);
-    else launch_mode<2>(c, energies, ff32);
+    if (mode == 0) launch_mode<0>(c, energies, ff32, false);
+    else if (mode == 1) launch_dsf_mixed(c, energies, ff32, false, false, false);
+    else launch_mode<2>(c, energies, ff32, false);
 }
 
 // Engine launches: the mixed kernel takes its fixed-point positions from the FP64 state.
-void launch_nonbond(sofia_ctx *c, int mode, bool energies, bool records) {
-    if (mode == 1) launch_dsf_mixed(c, energies, nullptr, c->engine_ready, records);
-    else launch_nonbond_out(c, mode, energies, nullptr);
+void launch_nonbond(sofia_ctx *c, int mode, bool energies, bool records, bool close) {
+    if (mode == 1) launch_dsf_mixed(c, energies, nullptr, c->engine_ready, records, close);
+    else if (mode == 0) launch_mode<0>(c, energies, nullptr, close);
+    else launch_mode<2>(c, energies, nullptr, close);
 }
 
 // Number of list entries inside the force cutoff (the algorithmic pair count of a launch).

@@ -2238,14 +2238,17 @@ int sofia_minimize(sofia_ctx *c, int32_t nsteps, double gamma, double max_disp) 
     const bool thermo = c->has_thermostat;
     c->has_thermostat = false;
     launch_zero_forces(c, c->fix, false);
-    const bool with_sort = sort_takes_bonded(c);   // after a move, the next one's bonded terms
+    // a move's sort carries the next one's bonded terms, its pair launch closes the rebuild
+    const bool with_sort = sort_takes_bonded(c), copy = list_takes_copy(c);
     for (int s = 0; s < nsteps; ++s) {
-        launch_nonbond(c, nb_mode(c), false, s > 0);
-        if (s == 0 || !with_sort) launch_bonded_engine(c, false);
-        launch_water_bonded(c);
+        launch_nonbond(c, nb_mode(c), false, s > 0, s > 0);
+        if (s == 0 || !with_sort) {
+            launch_bonded_engine(c, false);
+            launch_water_bonded(c);
+        }
         launch_minimize_step(c, gamma, max_disp);
-        launch_sort(c, SORT_STEP, with_sort && s + 1 < nsteps, false, list_takes_copy(c));
-        launch_build_list(c, list_takes_copy(c));
+        launch_sort(c, SORT_STEP, with_sort && s + 1 < nsteps, false, copy, true);
+        launch_build_list(c, copy);
     }
     if (nsteps > 0) launch_finish_rebuild(c);
     c->has_thermostat = thermo;

@@ -231,6 +231,18 @@ __device__ inline void finish_rebuild(int r, int nrep, int32_t *rebuild, int32_t
     if (r < nrep && rebuild[r]) nbuilds[r] += 1;
     rebuild[r] = 0;
 }
+// The same for every replica, by one workgroup of a launch that follows the list build.
+struct Books {
+    int32_t nrep;          // 0: none to close
+    int32_t *rebuild, *nbuilds;
+};
+__device__ inline void close_books(const Books &B) {
+    if (B.nrep && blockIdx.x == 0)
+        for (int r = threadIdx.x; r <= B.nrep; r += blockDim.x) finish_rebuild(r, B.nrep, B.rebuild, B.nbuilds);
+}
+inline Books books(const sofia_ctx *c, bool close) {
+    return Books{close ? c->nrep : 0, c->rebuild, c->nbuilds};
+}
 
 // Element of a wave-uniform array by a 32-bit byte offset: one address register, where a
 // 64-bit index takes two and the instructions that widen it.

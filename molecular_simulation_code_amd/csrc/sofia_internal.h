@@ -262,13 +262,14 @@ namespace sofia {
 // and the pair kernel's position records.
 enum SortMode { SORT_DROPIN = 0, SORT_ENGINE = 1, SORT_STEP = 2 };
 // bonded: with the step's bonded terms (where sort_takes_bonded)
-// (leave_copy: its copy back is left to launch_build_list, where list_takes_copy)
+// (leave_copy: its copy back is left to launch_build_list, where list_takes_copy; water: and
+// with the rigid waters' own terms)
 void launch_sort(sofia_ctx *c, SortMode mode, bool bonded = false, bool energies = false,
-                 bool leave_copy = false);
+                 bool leave_copy = false, bool water = false);
 bool list_takes_copy(const sofia_ctx *c);
 bool sort_takes_bonded(const sofia_ctx *c);
 struct BinArgs;
-void launch_bundles_bin(sofia_ctx *c, const BinArgs &B, int bin_grid, bool energies);
+void launch_bundles_bin(sofia_ctx *c, const BinArgs &B, int bin_grid, bool energies, bool water);
 void launch_host_ids(sofia_ctx *c, const int32_t *src, int32_t *dst, size_t items, int width,
                      int nidx);
 void launch_rdf(sofia_ctx *c, int32_t itype, int32_t jtype, double delta, int32_t nbins,
@@ -284,7 +285,8 @@ void launch_list_done(sofia_ctx *c, int32_t *local);
 
 // nonbond (k_nonbond.hip): mode 0 = DSF FP64, 1 = DSF mixed, 2 = Ewald real space (FP32)
 // records: the mixed kernel's position records are already up to date
-void launch_nonbond(sofia_ctx *c, int mode, bool energies, bool records = false);
+// close: the books of the rebuild before it
+void launch_nonbond(sofia_ctx *c, int mode, bool energies, bool records = false, bool close = false);
 void launch_count_pairs(sofia_ctx *c, unsigned long long *out);
 
 // bonded (k_bonded.hip)
@@ -295,7 +297,7 @@ void launch_bonded_dropin(sofia_ctx *c, long long *fout);
 void launch_bonded_wrapper(sofia_ctx *c, const double *xd, long long *fout, long long *f14);
 int build_bonded_bundles(sofia_ctx *c);   // host: molecules of the engine's bonded items
 void drop_bonded_bundles(sofia_ctx *c);
-void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records);
+void launch_dsf_mixed(sofia_ctx *c, bool energies, float *ff32, bool from_xd, bool records, bool close);
 // bytes per position record the mixed pair kernel reads (12 or 16), 0 in the other modes
 int record_bytes(const sofia_ctx *c);
 
@@ -318,7 +320,7 @@ void launch_langevin64(sofia_ctx *c);
 // step: the launch also ends the engine step (rebuild flags down, step counters on)
 void launch_shake64(sofia_ctx *c, bool energies, bool step = false);
 void launch_zero_energies(sofia_ctx *c);
-void launch_water_bonded(sofia_ctx *c);   // and the books of the rebuild before it
+void launch_water_bonded(sofia_ctx *c);
 void launch_copy16(sofia_ctx *c, size_t n16, const void *src, void *dst);
 void launch_put_state(sofia_ctx *c, bool v, bool q, bool gid);
 // with the report of the call
