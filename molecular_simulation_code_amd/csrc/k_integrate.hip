@@ -486,8 +486,8 @@ __device__ inline void flag_rebuild(const StepOut &O, int r, const double dr[3],
 // state: the previous step's second half kick (KICK2; the first step of a segment has none
 // left), this step's first half kick, the drift (wrapped into (0, box], the float4 copy
 // refreshed), the rebuild check, the Langevin force at the half-step velocity as the force
-// sum's first term, and the pair kernel's record.  These were seven launches; a launch costs
-// about 4.5 us in a step, so a 5,000-atom step (135 us) spent a quarter of its time on them.
+// sum's first term, and the pair kernel's record.  These were seven launches of 1.5 to 4.5 us, a
+// quarter of a 5,000-atom step (138 us); the one takes 4.3 us there, 12.5 at 204,000 atoms (HBM).
 template <bool KICK2>
 __global__ void __launch_bounds__(256)
 k_advance(int32_t n, double dt, const double4 *__restrict__ mtab, double *__restrict__ xd,
