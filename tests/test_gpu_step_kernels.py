@@ -347,3 +347,41 @@ def test_list_built_beside_the_copy_back(sizes, skin, waves):
             assert not pairs & ex
     finally:
         e.close()
+
+
+def test_list_by_two_cells_equals_the_list_by_one():
+    """From 2,048 half-width cells a workgroup of 16 wavefronts takes two neighbouring cells, one
+    of 8 takes one.  Boxes of odd and even cell counts a side, so that pairs break at the ends of
+    rows and replicas: rows in order, state and rebuilds equal bit for bit."""
+    host = _host()
+    from molecular_simulation_code_amd._lib import lib, check, ptr
+    import ctypes as C
+    systems = [S.make_system(10, w, seed=90 + k) for k, w in enumerate((1500, 3000, 2000, 3500, 2000))]
+    d = systems[0].derived()
+    rv = float(np.sqrt(max(d["rcut2"], d["cut_coulsq"]))) + 0.3
+    side = [int(float(s.box) / (0.5 * rv)) for s in systems]
+    assert sum(n ** 3 for n in side) >= 2048 and {n % 2 for n in side} == {0, 1}
+    out = []
+    for waves in (8, 16):
+        e = host.Engine([host.ReplicaSpec(s, temp=300.0, gamma_ps=5.0, seed=3) for s in systems])
+        try:
+            e.set_tuning(16, 256, waves)
+            e.set_skin(0.3)
+            e.init()
+            e.minimize(20)
+            e.run(20)
+            na = C.c_int32()
+            check(lib().sofia_get_nlist(e.ctx, None, None, C.byref(na)))
+            nl, nn = np.zeros((e.N, na.value), np.int32), np.zeros(e.N, np.int32)
+            check(lib().sofia_get_nlist(e.ctx, ptr(nl), ptr(nn), C.byref(na)))
+            out.append((nn, [nl[i, :k].copy() for i, k in enumerate(nn)], e.state(), e.rebuilds()))
+        finally:
+            e.close()
+    (nn, rows, st, rb), (nn2, rows2, st2, rb2) = out
+    np.testing.assert_array_equal(rb, rb2)
+    assert rb.min() > 1
+    np.testing.assert_array_equal(nn, nn2)
+    assert all(np.array_equal(a, b) for a, b in zip(rows, rows2))
+    for a, b in zip(st, st2):
+        for u, v in zip(a, b):
+            np.testing.assert_array_equal(u, v)
