@@ -280,7 +280,9 @@ int sofia_md_init(sofia_ctx *ctx);
 int sofia_md_run(sofia_ctx *ctx, int32_t nsteps, int32_t use_graph);
 /* sofia_md_run in two halves: md_launch enqueues the steps on the context's stream and
  * returns at once; md_finish waits for them, reduces the energies and reports a list
- * overflow or SHAKE failure.  Several contexts launched back to back run concurrently. */
+ * overflow or SHAKE failure.  Several contexts launched back to back run concurrently.
+ * A finish with no launched segment (a second one, or after a launch of 0 steps) leaves the
+ * energies of the last segment as they are. */
 int sofia_md_launch(sofia_ctx *ctx, int32_t nsteps, int32_t use_graph);
 int sofia_md_finish(sofia_ctx *ctx);
 /* Grow-and-redo (the engine's form of neighbor_wrapper's grow-and-rebuild,

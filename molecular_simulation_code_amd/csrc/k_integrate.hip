@@ -968,7 +968,10 @@ __global__ void k_step_add(int32_t nrep, uint64_t *step, long long delta) {
 }  // namespace
 
 void launch_zero_forces(sofia_ctx *c, long long *f, bool energies) {
-    if (energies) c->eacc_zero = false;
+    if (energies) {
+        launch_save_segment(c);
+        c->eacc_zero = false;
+    }
     const int n3 = 3 * c->N, ne = (int)eacc_len(c->nrep);
     hipLaunchKernelGGL(k_zero, dim3(nblocks(n3 > ne ? n3 : ne, 256)), dim3(256), 0, c->stream, n3, f,
                        ne, energies ? c->eacc : nullptr);
@@ -1053,6 +1056,7 @@ void launch_advance(sofia_ctx *c, bool kick2) {
 
 // Energy sums start from zero; skipped where the last report left them so.
 void launch_zero_energies(sofia_ctx *c) {
+    launch_save_segment(c);
     const bool zero = c->eacc_zero;
     c->eacc_zero = false;
     if (zero) return;
@@ -1113,6 +1117,14 @@ inline int report_blocks(const sofia_ctx *c) { return nblocks((long long)c->nrep
 void launch_report(sofia_ctx *c, bool clear_shake) {
     hipLaunchKernelGGL(k_report, dim3(report_blocks(c)), dim3(256), 0, c->stream,
                        report_args(c, clear_shake));
+}
+
+void launch_save_segment(sofia_ctx *c) {
+    if (c->segment != sofia_ctx::SEG_EACC) return;
+    ReportArgs A = report_args(c, false);
+    A.hw_e = c->hw_seg;
+    hipLaunchKernelGGL(k_report, dim3(report_blocks(c)), dim3(256), 0, c->stream, A);
+    c->segment = sofia_ctx::SEG_SAVED;
 }
 
 void launch_merge_report(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb) {

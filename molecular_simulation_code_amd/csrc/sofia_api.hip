@@ -514,10 +514,11 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
     TRY(clear_atoms(c->b, n));
     TRY(settle());
     TRY(size_cells(c.get(), c->ncell_total));
-    const size_t words = sizeof(sofia::HostWords) + sizeof(long long) * (size_t)nrep * NE;
+    const size_t words = sizeof(sofia::HostWords) + 2 * sizeof(long long) * (size_t)nrep * NE;
     SOFIA_HIP(hipHostMalloc((void **)&c->hw, words, hipHostMallocDefault));
     std::memset((void *)c->hw, 0, words);
     c->hw_e = (long long *)(c->hw + 1);
+    c->hw_seg = c->hw_e + (size_t)nrep * NE;
     std::vector<int32_t> rep(n), cnum((size_t)27 * c->ncell_total), crep(c->ncell_total);
     for (int r = 0; r < nrep; ++r) {
         const sofia::RepInfo &R = c->reps_h[r];
@@ -1644,9 +1645,11 @@ void step_sequence(sofia_ctx *c, bool kick2, bool energies) {
     launch_shake64(c, energies, true);
 }
 
-// Energies of the last report into last_e.
+// Energies of the last report (or of a segment put aside) into last_e.
 void take_energies(sofia_ctx *c) {
-    const std::vector<long long> e(c->hw_e, c->hw_e + (size_t)c->nrep * NE);
+    const long long *w = c->segment == sofia_ctx::SEG_SAVED ? c->hw_seg : c->hw_e;
+    const std::vector<long long> e(w, w + (size_t)c->nrep * NE);
+    c->segment = sofia_ctx::SEG_NONE;
     for (int r = 0; r < c->nrep; ++r) {
         double *o = c->last_e.data() + (size_t)r * SOFIA_NENERGY;
         o[0] = E(e, r, E_LJ); o[1] = E(e, r, E_COUL); o[2] = E(e, r, E_POT14);
@@ -1660,8 +1663,10 @@ int report(sofia_ctx *c) {
     return sync_check(c);
 }
 
+// Energies of a force evaluation just launched; those of a segment before it are superseded.
 int collect_energies(sofia_ctx *c) {
     TRY(report(c));
+    c->segment = sofia_ctx::SEG_NONE;
     take_energies(c);
     return SOFIA_OK;
 }
@@ -2173,6 +2178,7 @@ int sofia_md_launch(sofia_ctx *c, int32_t nsteps, int32_t use_graph) {
     }
     step_sequence(c, nsteps > 1, true);
     launch_nve_v64(c, true);
+    c->segment = sofia_ctx::SEG_EACC;
     c->step_h += nsteps;
     return SOFIA_OK;
 }
@@ -2187,6 +2193,7 @@ int sofia_md_finish(sofia_ctx *c) {
         if (rc == SOFIA_E_OVERFLOW && c->snap_valid && attempt < 4) {
             // grow and redo the segment (the reference grows neigh_alloc and rebuilds)
             const int32_t nsteps = c->snap_nsteps, graph = c->snap_graph;
+            c->segment = sofia_ctx::SEG_NONE;   // its sums are of the run that overflowed
             TRY(snapshot_restore(c, overflow));
             c->step_h -= nsteps;
             ++c->redos;
@@ -2194,7 +2201,10 @@ int sofia_md_finish(sofia_ctx *c) {
             continue;
         }
         c->snap_valid = false;
-        if (rc == SOFIA_OK) take_energies(c);
+        // the report cleared the sums it read: without a segment to take, the energies of the
+        // last one stay
+        if (rc == SOFIA_OK && c->segment != sofia_ctx::SEG_NONE) take_energies(c);
+        c->segment = sofia_ctx::SEG_NONE;
         return rc;
     }
 }
@@ -2387,6 +2397,7 @@ int sofia_profile_step(sofia_ctx *c, int32_t nsteps, int32_t full_rebuild, doubl
     TRY(rc);
     c->step_h += nsteps;
     for (int p = 0; p < NP; ++p) phase_ms[p] = acc[p] / nsteps;
+    launch_save_segment(c);
     TRY(report(c));
     return check_engine_flags(c);
 }

@@ -209,6 +209,10 @@ struct sofia_ctx {
     // k_check32): read after one synchronisation, with no copy of their own
     sofia::HostWords *hw = nullptr;
     long long *hw_e = nullptr;   // nrep x NE energy sums, behind hw
+    // a launched segment whose energies the host has not taken yet: their sums stand in eacc,
+    // or (another call needed eacc since) in hw_seg, which a report ahead of that call wrote
+    enum { SEG_NONE, SEG_EACC, SEG_SAVED } segment = SEG_NONE;
+    long long *hw_seg = nullptr; // nrep x NE, behind hw_e
     // blocks that hold the context's fixed-size arrays (one allocation instead of dozens)
     std::vector<void *> blocks;
     int gid_perm = -1;           // global ids of every replica a permutation: 1, 0, -1 unknown
@@ -327,6 +331,8 @@ void launch_put_state(sofia_ctx *c, bool v, bool q, bool gid);
 void launch_merge_report(sofia_ctx *c, float *ff32, const long long *f14, const long long *fb);
 // Energy sums (cleared on the device) and flags to the host words
 void launch_report(sofia_ctx *c, bool clear_shake = false);
+// ahead of whatever clears or reads the energy sums: those of a launched segment put aside
+void launch_save_segment(sofia_ctx *c);
 void launch_start_forces(sofia_ctx *c, long long *a, long long *b, double *xd);
 // FP64 SoA (plus fixed point) <-> AoS; with gid, dst rows in global-id order of each replica
 void launch_soa_to_aos(sofia_ctx *c, const double *src, const long long *fix, const int32_t *gid, double *dst);

@@ -385,3 +385,86 @@ def test_list_by_two_cells_equals_the_list_by_one():
     for a, b in zip(st, st2):
         for u, v in zip(a, b):
             np.testing.assert_array_equal(u, v)
+
+
+def _one(host, s, **kw):
+    return host.Engine([host.ReplicaSpec(s, temp=300.0, gamma_ps=1.0, seed=3)], **kw)
+
+
+@pytest.mark.parametrize("prec", ["mixed", "fp64"])
+def test_a_finish_without_a_segment_keeps_the_energies(prec):
+    """Every finish but the one that ends a segment reads nothing new: energies and temperature
+    stay those of the last segment, set-up or minimisation."""
+    host = _host()
+    e = _one(host, S.make_system(5, 1000, seed=41),
+             precision=host.PREC_FP64 if prec == "fp64" else host.PREC_MIXED)
+    try:
+        e.init()
+        for last in (lambda: None, lambda: e.minimize(20), lambda: e.run(4), lambda: e.run(1)):
+            last()
+            want, temp = e.energies(), e.temperatures()
+            assert want[0, :2].all()
+            for again in (e.finish, lambda: (e.launch(0), e.finish()), lambda: e.profile_step(1), e.finish,
+                          lambda: e.pair_forces(), e.finish):
+                again()
+                np.testing.assert_array_equal(e.energies(), want)
+                np.testing.assert_array_equal(e.temperatures(), temp)
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("between", ["another launch", "pair forces", "profiled launches", "minimisation"])
+def test_a_segments_energies_outlast_calls_before_its_finish(between):
+    """Calls that need the energy sums between a launch and its finish leave the segment its
+    own; a minimisation after it replaces them."""
+    host = _host()
+    s = S.make_system(5, 1000, seed=42)
+    a, b = _one(host, s.copy()), _one(host, s.copy())
+    try:
+        for e in (a, b):
+            e.init()
+            e.minimize(20)
+        if between == "another launch":
+            a.run(5)
+            b.launch(2)
+            b.launch(3)
+        elif between == "minimisation":
+            a.run(3)
+            a.minimize(5)
+            b.launch(3)
+            b.minimize(5)
+        else:
+            a.run(3)
+            b.launch(3)
+            b.pair_forces() if between == "pair forces" else b.profile_nonbond(2)
+        b.finish()
+        np.testing.assert_array_equal(a.energies(), b.energies())
+        assert a.energies()[0, 7] > 0.0 or between == "minimisation"
+    finally:
+        a.close()
+        b.close()
+
+
+@pytest.mark.parametrize("policy", ["cohort", "rebatch"])
+@pytest.mark.parametrize("beside", [False, True])
+def test_a_served_request_of_no_steps_has_its_energies(beside, policy):
+    """Alone, and beside a request of 50 steps that goes on without it: the energies are those
+    an engine of the same requests starts from."""
+    host = _host()
+    from molecular_simulation_code_amd import server
+    systems = [S.make_system(4, 1000, seed=43), S.make_system(6, 1100, seed=44)][:2 if beside else 1]
+    server.relax(systems, 30)
+    for k, s in enumerate(systems):
+        s.v = S.maxwell_boltzmann(s, 300.0, np.random.default_rng(k))
+    reqs = [server.Request(rid=k, arrival=0.0, system=s, seed=k + 1, temp=300.0, nsteps=50 * k)
+            for k, s in enumerate(systems)]
+    e = host.Engine([host.ReplicaSpec(s, temp=300.0, gamma_ps=1.0, seed=k + 1) for k, s in enumerate(systems)])
+    try:
+        e.put_state([(s.pos.astype(np.float64), s.v.astype(np.float64)) for s in systems])
+        e.resume()
+        want = e.energies()
+    finally:
+        e.close()
+    res, _, _ = server.SegmentServer(hbm_budget_gb=8.0, segment=25, policy=policy).serve(reqs, realtime=False)
+    np.testing.assert_array_equal(res[0].energies, want[0])
+    assert res[0].energies[0] != 0.0 and [len(r.clusters) for r in res] == [1, 3][:len(res)]
