@@ -349,15 +349,15 @@ int cluster_greatest_noalloc(int32_t n, const double *x, const int32_t *gid, con
                              int32_t nmol, float box, double denscut, int32_t densmin,
                              int32_t *out, hipStream_t s);
 
-// Lanes per atom of the mixed pair kernel while the caller has not tuned them: its exact sums
-// do not depend on them.  Small systems need more lanes to spread over the chip (one launch,
+// Lanes per atom of the mixed pair kernel while the caller has not tuned them: its exact force
+// sums do not depend on them.  Small systems need more lanes to spread over the chip (one launch,
 // 5,000 atoms: 12.7 us at 64 lanes, 13.6 at 32, 15.8 at 16), large ones fewer shuffles and
-// idle row tails (55,000: 76 / 64 / 60; 264,000: 433 / 353 / 321).  The energy sums lengthen
-// the tail of every lane, so launches with energies turn to 16 lanes earlier (a drop-in call,
-// 31,000 atoms: 371 us at 32, 346 at 16; 3,000 atoms: 133 / 150).
+// idle row tails (55,000: 76 / 64 / 60; 264,000: 433 / 353 / 321).  An atom's energies and virial
+// are summed in floating point, in an order set by the lanes: launches with energies take one
+// value for every size, so that a replica's energies do not depend on what it is batched with.
 inline int mixed_lanes(const sofia_ctx *c, bool energies = false) {
     if (c->lanes >= 0) return c->lanes;
-    if (energies) return c->N < 6000 ? 32 : 16;
+    if (energies) return 16;
     return c->N < 12000 ? 64 : (c->N < 40000 ? 32 : 16);
 }
 // The FP64 and Ewald kernels sum in floating point, in an order set by the lanes: one value

@@ -468,3 +468,34 @@ def test_a_served_request_of_no_steps_has_its_energies(beside, policy):
     res, _, _ = server.SegmentServer(hbm_budget_gb=8.0, segment=25, policy=policy).serve(reqs, realtime=False)
     np.testing.assert_array_equal(res[0].energies, want[0])
     assert res[0].energies[0] != 0.0 and [len(r.clusters) for r in res] == [1, 3][:len(res)]
+
+
+@pytest.mark.parametrize("kernel", ["mixed", "ewald", "fp64"])
+@pytest.mark.parametrize("others", [(1200,), (1100, 5000, 9000), (1300, 2000)])
+def test_untuned_energies_alone_equal_those_in_a_batch(others, kernel):
+    """A 3,180-atom replica alone and in batches past the size lines of the untuned layouts:
+    energies and pair virial bit for bit.  Two waters sit 0.62 A from another: the sums of
+    their oxygens (2e8 kcal/mol, an ulp of half the 2^-24 quantum they are kept in) round
+    differently in almost any other order, and the total stays below 2^53 quanta."""
+    host = _host()
+    kw = {"mixed": dict(precision=host.PREC_MIXED), "fp64": dict(precision=host.PREC_FP64),
+          "ewald": dict(precision=host.PREC_MIXED, coul_flag=host.COUL_EWALD)}[kernel]
+    systems = [S.make_system(6, w, seed=w, params=S.Params(gewald=0.3)) for w in (1040,) + others]
+    s = systems[0]
+    oxygen = np.where(s.moltype == 2)[0].reshape(-1, 3)
+    for a, b in oxygen[[0, 100, 500, 900]].reshape(-1, 2, 3):
+        s.pos[a] += s.pos[b[0]] - s.pos[a[0]] + np.float32([0.62, 0.0, 0.0])
+    for x in systems:   # (no constraint has a solution under such forces)
+        x.shake_num, x.shake_atoms, x.shake_bond = x.shake_num[:0], x.shake_atoms[:0], x.shake_bond[:0]
+    out = []
+    for batch in (systems[:1], systems):
+        e = host.Engine([host.ReplicaSpec(x.copy(), temp=300.0, gamma_ps=1.0, seed=3) for x in batch], **kw)
+        try:
+            e.init()
+            out.append((e.energies()[0], e.pair_forces()[1][0]))
+        finally:
+            e.close()
+    assert s.np < 6000 < sum(x.np for x in systems)
+    assert 2e8 < out[0][0][0] < 5e8
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
