@@ -51,15 +51,16 @@ __global__ void k_bin(BinArgs A) {
 // by ranking, which is deterministic.  A wavefront owns `per` consecutive cells; it finds
 // their first atom by summing the replica's counts before its first cell (a scan kernel of one
 // workgroup per replica in the launch sequence cost every step more than these sums cost the
-// steps that rebuild).  A cell with more atoms than a bucket holds is read from acell.
+// steps that rebuild).  A cell with more atoms than a bucket holds first gathers them, from its
+// bucket and the list of atoms past full buckets, where its places will be (in fat).
 __global__ void __launch_bounds__(256)
 k_sort_gather(int32_t ncell, int32_t per, int32_t split, const int32_t *__restrict__ cell_rep,
               const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
               const int32_t *__restrict__ any, const int32_t *__restrict__ cbin,
-              const int32_t *__restrict__ acell, const int32_t *__restrict__ bucket, int32_t cap,
-              int32_t *__restrict__ ccount, int32_t *__restrict__ cstart, int32_t *__restrict__ tt,
-              int32_t *__restrict__ atombin, int32_t n, AtomArrays src, AtomArrays dst, int mode,
-              StepArrays T) {
+              const int32_t *__restrict__ bucket, int32_t cap, const int32_t *__restrict__ nover,
+              const int2 *__restrict__ over, int32_t *fat, int32_t *__restrict__ ccount,
+              int32_t *__restrict__ cstart, int32_t *__restrict__ tt, int32_t *__restrict__ atombin,
+              int32_t n, AtomArrays src, AtomArrays dst, int mode, StepArrays T) {
     if (!*any) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
@@ -85,34 +86,36 @@ k_sort_gather(int32_t ncell, int32_t per, int32_t split, const int32_t *__restri
             cstart[c] = base;
             ccount[c] = cnt;
         }
-        auto place = [&](int me, int rank) {
-            tt[me] = base + rank;
-            atombin[base + rank] = c;
-            move_atom(src, dst, n, me, base + rank, mode, T);
-        };
-        if (cnt <= cap) {
-            const int32_t *ids = bucket + (size_t)c * cap;
-            for (int e0 = 64 * part; e0 < cnt; e0 += 64 * split) {
-                const bool in = e0 + lane < cnt;
-                const int me = in ? ids[e0 + lane] : 0;
-                int rank = 0;
-                for (int f0 = 0; f0 < cnt; f0 += 64) {
-                    const int other = f0 + lane < cnt ? ids[f0 + lane] : -1;
-                    const int m = min(64, cnt - f0);
-                    for (int f = 0; f < m; ++f) rank += __builtin_amdgcn_readlane(other, f) > me;
-                }
-                if (in) place(me, rank);
-            }
-        } else if (part == 0) {
-            const int a0 = reps[r].atom0, a1 = a0 + reps[r].natom;
+        const int32_t *ids = bucket + (size_t)c * cap;
+        if (cnt > cap) {   // every part of a split writes the same ids to the same places
             const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-            int done = 0;
-            for (int b = 0; b < a1 - a0; b += 64) {   // lanes in descending atom order
-                const int i = a1 - 1 - b - lane;
-                const bool in = i >= a0 && acell[i] == c;
+            for (int e = lane; e < cap; e += 64) fat[base + e] = ids[e];
+            const int no = *nover;
+            int done = cap;
+#pragma unroll 4
+            for (int b = 0; b < no; b += 64) {
+                const int2 o = over[min(b + lane, no - 1)];
+                const bool in = b + lane < no && o.x == c;
                 const uint64_t m = __ballot(in);
-                if (in) place(i, done + __popcll(m & lt_mask));
+                if (in) fat[base + done + __popcll(m & lt_mask)] = o.y;
                 done += __popcll(m);
+            }
+            __threadfence_block();   // other lanes read them
+            ids = fat + base;
+        }
+        for (int e0 = 64 * part; e0 < cnt; e0 += 64 * split) {
+            const bool in = e0 + lane < cnt;
+            const int me = in ? ids[e0 + lane] : 0;
+            int rank = 0;
+            for (int f0 = 0; f0 < cnt; f0 += 64) {
+                const int other = f0 + lane < cnt ? ids[f0 + lane] : -1;
+                const int m = min(64, cnt - f0);
+                for (int f = 0; f < m; ++f) rank += __builtin_amdgcn_readlane(other, f) > me;
+            }
+            if (in) {
+                tt[me] = base + rank;
+                atombin[base + rank] = c;
+                move_atom(src, dst, n, me, base + rank, mode, T);
             }
         }
         base += cnt;
@@ -479,12 +482,12 @@ CopyArgs copy_args(sofia_ctx *c, SortMode mode, int *items) {
     add(c->eangle, c->nae, 4, 3);
     *items = std::max({c->N, total, c->ncell_total});
     return CopyArgs{c->N, c->ncell_total, (int)mode, c->rep, c->rebuild, any_flag(c), c->tt, c->cell_rep,
-                    c->reps_d, c->b, c->a, c->dr32, c->drd, step_arrays(c, mode), S, c->cbin};
+                    c->reps_d, c->b, c->a, c->dr32, c->drd, step_arrays(c, mode), S, c->cbin, c->nover};
 }
 
 void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies, bool leave_copy, bool water) {
     const BinArgs B{c->N, c->bucket_cap, c->a.pos4, c->rep, c->reps_d, c->rebuild, any_flag(c),
-                    c->cbin, c->acell, c->bucket};
+                    c->cbin, c->bucket, c->nover, c->over};
     const int bin_grid = capped(c->N, 256);
     if (bonded) launch_bundles_bin(c, B, bin_grid, energies, water);
     else hipLaunchKernelGGL(k_bin, dim3(bin_grid), dim3(256), 0, c->stream, B);
@@ -494,8 +497,8 @@ void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies, bool l
     const int split = per > 1 ? 1 : std::max(1, std::min(8, nblk(c->N, 64 * c->ncell_total)));
     hipLaunchKernelGGL(k_sort_gather, dim3(nblk(nblk(c->ncell_total, per) * split, 4)), dim3(256), 0, c->stream,
                        c->ncell_total, per, split, c->cell_rep, c->reps_d, c->rebuild, any_flag(c), c->cbin,
-                       c->acell, c->bucket, c->bucket_cap, c->ccount, c->cstart, c->tt, c->atombin,
-                       c->N, c->a, c->b, (int)mode, step_arrays(c, mode));
+                       c->bucket, c->bucket_cap, c->nover, c->over, c->fat, c->ccount, c->cstart, c->tt,
+                       c->atombin, c->N, c->a, c->b, (int)mode, step_arrays(c, mode));
     if (leave_copy) return;
     int items = 0;
     const CopyArgs A = copy_args(c, mode, &items);

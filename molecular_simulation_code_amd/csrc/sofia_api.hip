@@ -208,8 +208,14 @@ int ensure_list(sofia_ctx *c, int na) {
     return SOFIA_OK;
 }
 
-// Per-cell arrays for ncell cells of the current grids, and the binning buckets: twice a cell's
-// mean occupancy and 32 more (k_sort_gather handles fuller cells without one).
+// Per-cell arrays for ncell cells of the current grids, and the binning buckets: 32 atoms more
+// than twice a cell's mean occupancy, and 32 more than a cell holds at 0.15 atoms per cubic A,
+// half as dense again as water, since the mean of a box that is part empty says little.  (By the
+// mean alone, every cell of a droplet in eight times its volume is past its bucket; when such a
+// cell searched all atoms for its own, a drop-in sort and list of 204,000 took 2.14 ms, and takes
+// 0.70 so, 0.66 in a full box.)  The second only as far as all buckets stay within BUCKET_WORDS;
+// k_sort_gather orders fuller cells too.
+constexpr size_t BUCKET_WORDS = size_t(1) << 27;   // 512 MB, a box of 1000 A a side nearly empty
 int size_cells(sofia_ctx *c, int ncell) {
     if (ncell > c->ncell_cap) {
         dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep); dfree(c->cbin);
@@ -225,9 +231,15 @@ int size_cells(sofia_ctx *c, int ncell) {
         TRY(settle());
         c->ncell_cap = ncell;
     }
-    int mean = 0;
-    for (const auto &R : c->reps_h) mean = std::max(mean, (R.natom + R.ncellT - 1) / R.ncellT);
-    c->bucket_cap = std::min((2 * mean + 32 + 15) / 16 * 16, 512);
+    int twice = 0;
+    double dense = 0.0;
+    for (const auto &R : c->reps_h) {
+        twice = std::max(twice, 2 * ((R.natom + R.ncellT - 1) / R.ncellT));
+        dense = std::max(dense, std::min(0.15 * std::pow((double)R.rn, 3.0), (double)R.natom));
+    }
+    auto words = [](double atoms) { return ((size_t)atoms + 32 + 15) / 16 * 16; };
+    const size_t most = std::min(words(dense), BUCKET_WORDS / ncell / 16 * 16);
+    c->bucket_cap = (int32_t)std::max(words(twice), most);
     const size_t need = (size_t)ncell * c->bucket_cap;
     if (need > c->bucket_len) {
         dfree(c->bucket);
@@ -497,7 +509,9 @@ int create(const sofia_params *p, int nrep, const int32_t *natoms, const float *
     B.want(&c->fix, (size_t)3 * n);
     B.want(&c->fscratch, (size_t)3 * n);
     B.want(&c->stage32, (size_t)3 * n);
-    B.want(&c->acell, n);
+    B.want(&c->nover, 1);
+    B.want(&c->over, n);
+    B.want(&c->fat, n);
     B.want(&c->tt, n);
     B.want(&c->atombin, n);
     B.want(&c->numneigh, n);

@@ -189,15 +189,16 @@ __device__ inline int xyz2bin_dev(float4 p, const RepInfo &R) {
     return ix[0] + ix[1] * R.ncellD + ix[2] * R.ncellD * R.ncellD;
 }
 
-// Binning: counts each cell's atoms and drops their ids into the cell's bucket.  tt of a
-// replica that rebuilds nothing is stale: every reader skips such replicas.
+// Binning: counts each cell's atoms and drops their ids into the cell's bucket, those past a
+// full one into a list of all cells.  tt of a replica that rebuilds nothing is stale: every reader skips such replicas.
 struct BinArgs {
     int32_t n, cap;
     const float4 *pos4;
     const int32_t *rep;
     const RepInfo *reps;
     const int32_t *rebuild, *any;
-    int32_t *cbin, *acell, *bucket;
+    int32_t *cbin, *bucket, *nover;
+    int2 *over;
 };
 __device__ inline void bin_atoms(const BinArgs &A, int t0, int stride) {
     const uint64_t lt_mask = (threadIdx.x & 63) ? ~0ull >> (64 - (threadIdx.x & 63)) : 0ull;
@@ -206,7 +207,6 @@ __device__ inline void bin_atoms(const BinArgs &A, int t0, int stride) {
         if (!A.rebuild[r]) continue;
         const RepInfo R = A.reps[r];
         const int c = R.cell0 + xyz2bin_dev(A.pos4[i], R);
-        A.acell[i] = c;
         // lanes of one cell (atoms come in the last sort's order, so a wavefront holds few
         // cells) share one count: wide cells' counters are hit by a hundred atoms each, and
         // 13,500 atoms in 125 cells took 34 us one by one, 3.9 so
@@ -222,7 +222,12 @@ __device__ inline void bin_atoms(const BinArgs &A, int t0, int stride) {
             if (!left) break;
         }
         if (left >> (threadIdx.x & 63) & 1) slot = atomicAdd(&A.cbin[c], 1);
-        if (slot < A.cap) A.bucket[(size_t)c * A.cap + slot] = i;
+        if (slot < A.cap) {
+            A.bucket[(size_t)c * A.cap + slot] = i;
+        } else {
+            const int k = atomicAdd(A.nover, 1);
+            if (k < A.n) A.over[k] = make_int2(c, i);
+        }
     }
 }
 

@@ -134,7 +134,11 @@ struct sofia_ctx {
     int32_t *bucket = nullptr;      // bucket_cap atom ids per cell, in binning order
     int32_t bucket_cap = 0;
     size_t bucket_len = 0;
-    int32_t *acell = nullptr, *tt = nullptr, *atombin = nullptr;
+    // atoms past a full bucket: how many (zero between sorts), their (cell, id), and the ids of
+    // such cells' atoms gathered for the ranking
+    int32_t *nover = nullptr, *fat = nullptr;
+    int2 *over = nullptr;
+    int32_t *tt = nullptr, *atombin = nullptr;
 
     // Verlet list
     int32_t *nlist = nullptr, *numneigh = nullptr;

@@ -64,7 +64,7 @@ struct CopyArgs {
     double *drd;
     StepArrays T;
     RemapSet S;
-    int32_t *cbin;
+    int32_t *cbin, *nover;
 };
 __device__ inline void copy_back(const CopyArgs &A, int t0, int stride) {
     const int n = A.n, mode = A.mode;
@@ -116,6 +116,7 @@ __device__ inline void copy_back(const CopyArgs &A, int t0, int stride) {
     }
     for (int c = t0; c < ncell; c += stride)
         if (rebuild[cell_rep[c]]) cbin[c] = 0;
+    if (t0 == 0) *A.nover = 0;
 }
 // The arguments of the context's copy back; *items: how many threads find work.
 CopyArgs copy_args(sofia_ctx *c, SortMode mode, int *items);
