@@ -47,20 +47,39 @@ __global__ void k_bin(BinArgs A) {
     bin_atoms(A, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
+// Atoms in each run of cells, a run a workgroup.
+__global__ void __launch_bounds__(1 << CHUNK_SHIFT)
+k_chunk_sums(int32_t ncell, const int32_t *__restrict__ any, const int32_t *__restrict__ cbin,
+             int32_t *__restrict__ chunk) {
+    if (!*any) return;
+    __shared__ int32_t s_w[(1 << CHUNK_SHIFT) / 64];
+    const int c = (blockIdx.x << CHUNK_SHIFT) + threadIdx.x;
+    int s = c < ncell ? cbin[c] : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x) return;
+    s = 0;
+    for (int w = 0; w < (1 << CHUNK_SHIFT) / 64; ++w) s += s_w[w];
+    chunk[blockIdx.x] = s;
+}
+
 // Atoms of a cell in descending old index (the chain order of the reference's linked cells),
 // by ranking, which is deterministic.  A wavefront owns `per` consecutive cells; it finds
 // their first atom by summing the replica's counts before its first cell (a scan kernel of one
 // workgroup per replica in the launch sequence cost every step more than these sums cost the
-// steps that rebuild).  A cell with more atoms than a bucket holds first gathers them, from its
+// steps that rebuild), by runs of cells where k_chunk_sums counted those.  A cell with more atoms than a bucket holds first gathers them, from its
 // bucket and the list of atoms past full buckets, where its places will be (in fat).
 __global__ void __launch_bounds__(256)
 k_sort_gather(int32_t ncell, int32_t per, int32_t split, const int32_t *__restrict__ cell_rep,
               const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,
               const int32_t *__restrict__ any, const int32_t *__restrict__ cbin,
-              const int32_t *__restrict__ bucket, int32_t cap, const int32_t *__restrict__ nover,
-              const int2 *__restrict__ over, int32_t *fat, int32_t *__restrict__ ccount,
-              int32_t *__restrict__ cstart, int32_t *__restrict__ tt, int32_t *__restrict__ atombin,
-              int32_t n, AtomArrays src, AtomArrays dst, int mode, StepArrays T) {
+              const int32_t *__restrict__ chunk, const int32_t *__restrict__ bucket, int32_t cap,
+              const int32_t *__restrict__ nover, const int2 *__restrict__ over, int32_t *fat,
+              int32_t *__restrict__ ccount, int32_t *__restrict__ cstart, int32_t *__restrict__ tt,
+              int32_t *__restrict__ atombin, int32_t n, AtomArrays src, AtomArrays dst, int mode,
+              StepArrays T) {
     if (!*any) return;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
@@ -75,7 +94,14 @@ k_sort_gather(int32_t ncell, int32_t per, int32_t split, const int32_t *__restri
         }
         if (r != rcur) {   // first cell of this replica here: the atoms in the cells before it
             int s = 0;
-            for (int k = reps[r].cell0 + lane; k < c; k += 64) s += cbin[k];
+            const int first = reps[r].cell0;
+            // whole runs of cells [h, t), the cells before and after them one by one
+            const int h = chunk ? (first + (1 << CHUNK_SHIFT) - 1) >> CHUNK_SHIFT : 0;
+            const int t = chunk ? c >> CHUNK_SHIFT : 0;
+            const int a = h < t ? h << CHUNK_SHIFT : c, b = h < t ? t << CHUNK_SHIFT : c;
+            for (int k = first + lane; k < a; k += 64) s += cbin[k];
+            for (int k = h + lane; k < t; k += 64) s += chunk[k];
+            for (int k = b + lane; k < c; k += 64) s += cbin[k];
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
             base = reps[r].atom0 + __builtin_amdgcn_readfirstlane(s);
@@ -491,14 +517,18 @@ void launch_sort(sofia_ctx *c, SortMode mode, bool bonded, bool energies, bool l
     const int bin_grid = capped(c->N, 256);
     if (bonded) launch_bundles_bin(c, B, bin_grid, energies, water);
     else hipLaunchKernelGGL(k_bin, dim3(bin_grid), dim3(256), 0, c->stream, B);
+    const int32_t *chunk = c->chunked ? c->chunk : nullptr;
+    if (chunk)
+        hipLaunchKernelGGL(k_chunk_sums, dim3(nblk(c->ncell_total, 1 << CHUNK_SHIFT)), dim3(1 << CHUNK_SHIFT), 0,
+                           c->stream, c->ncell_total, any_flag(c), c->cbin, c->chunk);
     const int per = nblk(c->ncell_total, 4 * GRID_CAP);   // cells per wavefront
     // or wavefronts per cell, where a cell holds more atoms than a wavefront has lanes (the
     // reference's cells: 30 -> 22 us at 13,500 atoms in 125 cells, 33 -> 15 at 31,000)
     const int split = per > 1 ? 1 : std::max(1, std::min(8, nblk(c->N, 64 * c->ncell_total)));
     hipLaunchKernelGGL(k_sort_gather, dim3(nblk(nblk(c->ncell_total, per) * split, 4)), dim3(256), 0, c->stream,
                        c->ncell_total, per, split, c->cell_rep, c->reps_d, c->rebuild, any_flag(c), c->cbin,
-                       c->bucket, c->bucket_cap, c->nover, c->over, c->fat, c->ccount, c->cstart, c->tt,
-                       c->atombin, c->N, c->a, c->b, (int)mode, step_arrays(c, mode));
+                       chunk, c->bucket, c->bucket_cap, c->nover, c->over, c->fat, c->ccount, c->cstart,
+                       c->tt, c->atombin, c->N, c->a, c->b, (int)mode, step_arrays(c, mode));
     if (leave_copy) return;
     int items = 0;
     const CopyArgs A = copy_args(c, mode, &items);

@@ -215,16 +215,25 @@ int ensure_list(sofia_ctx *c, int na) {
 // cell searched all atoms for its own, a drop-in sort and list of 204,000 took 2.14 ms, and takes
 // 0.70 so, 0.66 in a full box.)  The second only as far as all buckets stay within BUCKET_WORDS;
 // k_sort_gather orders fuller cells too.
+//
+// Whether the sort's prefix goes by runs of cells: one launch a step, against each wavefront
+// reading the counts of all cells before its own, quadratic in the cells of a replica.  One
+// replica's steps, of which one in eight sorts (and a full sort), one by one / by runs:
+// 2,500 cells 11 / 14 us (33 / 27), 4,700 12.5 / 13 (46 / 33), 9,700 17 / 14.7 (80 / 51),
+// 19,000 25 / 18 (139 / 76), 47,000 62 / 39 (425 / 235); a droplet's 77,000 cells 53 / 22
+// (371 / 113), 600,000 280 / 26 (2,190 / 143).
 constexpr size_t BUCKET_WORDS = size_t(1) << 27;   // 512 MB, a box of 1000 A a side nearly empty
+constexpr int CHUNK_CELLS = 6000;                  // of one replica, from which it goes by runs
 int size_cells(sofia_ctx *c, int ncell) {
     if (ncell > c->ncell_cap) {
-        dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep); dfree(c->cbin);
+        dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep); dfree(c->cbin); dfree(c->chunk);
         c->ncell_cap = 0;
         TRY(dalloc(&c->ccount, ncell));
         TRY(dalloc(&c->cstart, ncell));
         TRY(dalloc(&c->cnum, (size_t)27 * ncell));
         TRY(dalloc(&c->cell_rep, ncell));
         TRY(dalloc(&c->cbin, ncell));
+        TRY(dalloc(&c->chunk, (ncell >> CHUNK_SHIFT) + 1));
         SOFIA_HIP(hipMemset(c->ccount, 0, sizeof(int32_t) * ncell));
         SOFIA_HIP(hipMemset(c->cstart, 0, sizeof(int32_t) * ncell));
         SOFIA_HIP(hipMemset(c->cbin, 0, sizeof(int32_t) * ncell));
@@ -233,7 +242,9 @@ int size_cells(sofia_ctx *c, int ncell) {
     }
     int twice = 0;
     double dense = 0.0;
+    c->chunked = false;
     for (const auto &R : c->reps_h) {
+        c->chunked |= R.ncellT >= CHUNK_CELLS;
         twice = std::max(twice, 2 * ((R.natom + R.ncellT - 1) / R.ncellT));
         dense = std::max(dense, std::min(0.15 * std::pow((double)R.rn, 3.0), (double)R.natom));
     }
@@ -816,7 +827,7 @@ int sofia_ctx_destroy(sofia_ctx *c) {
     dfree(c->gc_first); dfree(c->gc_refgid); dfree(c->gc_cnt); dfree(c->gc_dens); dfree(c->gc_sum);
     dfree(c->gc_refx); dfree(c->gc_com); dfree(c->gc_key); dfree(c->gc_surface);
     dfree(c->ccount); dfree(c->cstart); dfree(c->cnum); dfree(c->cell_rep);
-    dfree(c->cbin); dfree(c->bucket); dfree(c->mtab); dfree(c->nlist);
+    dfree(c->cbin); dfree(c->chunk); dfree(c->bucket); dfree(c->mtab); dfree(c->nlist);
     dfree(c->bund_heads); dfree(c->bund_slots); dfree(c->bund_terms);
     dfree(c->water); dfree(c->dsf_tab); dfree(c->ebond); dfree(c->eangle); dfree(c->bondlist); dfree(c->anglelist);
     dfree(c->dihedlist); dfree(c->torsions); dfree(c->shake_num); dfree(c->shake_atoms); dfree(c->shake_kidx);

@@ -66,6 +66,8 @@ struct DevParams {
 
 constexpr int DSF_TAB_BINS = 1024;
 
+constexpr int CHUNK_SHIFT = 8;   // cells to a run of the sort's prefix: 256
+
 // Engine bonded work in bundles of whole molecules: item kinds and the widths of their lists.
 enum BondedKind { BK_PAIR14 = 0, BK_BOND = 1, BK_ANGLE = 2, BK_TORSION = 3, BK_IMPRO = 4, BK_COUNT = 5 };
 constexpr int BUNDLE_SLOTS = 192;   // atoms per bundle (its forces sit in LDS)
@@ -138,6 +140,10 @@ struct sofia_ctx {
     // such cells' atoms gathered for the ranking
     int32_t *nover = nullptr, *fat = nullptr;
     int2 *over = nullptr;
+    // where a replica has many cells: atoms in each run of 1 << CHUNK_SHIFT cells, which the
+    // sort's prefix takes instead of their counts one by one
+    int32_t *chunk = nullptr;
+    bool chunked = false;
     int32_t *tt = nullptr, *atombin = nullptr;
 
     // Verlet list

@@ -563,3 +563,68 @@ def test_a_droplet_sorts_and_lists_as_fast_as_a_full_box():
         best.append(min(ts))
     print(f"[droplet] full box {1e3 * best[0]:.2f} ms, droplet {1e3 * best[1]:.2f} ms", flush=True)
     assert best[1] < 1.8 * best[0]
+
+
+def _in_larger_box(s, factor):
+    """The system's molecules, whole, in the middle of a box `factor` times as wide."""
+    x, b = s.copy(), float(s.box)
+    p = s.pos.astype(np.float64)
+    first = p[np.searchsorted(s.mol, s.mol)]
+    x.pos = np.ascontiguousarray(p - b * np.rint((p - first) / b) + 0.5 * (factor - 1.0) * b, np.float32)
+    x.box = np.float32(b * factor)
+    return x
+
+
+@pytest.mark.parametrize("box", [103.0, 130.0, 175.0])
+def test_sort_of_many_cells(box):
+    """5,832 cells (summed one by one), 12,167 and 29,791 (by runs of 256, the last of them cut),
+    2,900 atoms all over them: sorted as the oracle's chains."""
+    host = _host()
+    s = S.make_system(20, 900, seed=4, params=S.Params(rcut=5.5, cut_coul=5.5, pad=1.0))
+    s.box = np.float32(box)
+    s.pos = np.random.default_rng(1).uniform(0.01, box - 0.01, s.pos.shape).astype(np.float32)
+    g = host.SofiaGPU(s)
+    try:
+        _sorts_as_the_oracle(g, s, 2)
+    finally:
+        g.close()
+
+
+def test_runs_of_cells_shared_by_replicas():
+    """Replicas of 125 and of some 8,000 cells in turn, so that runs begin and end inside
+    replicas: each one's state after rebuilds is the one it reaches alone, bit for bit."""
+    host = _host()
+    systems = [S.make_system(6, 1040 + 40 * k, seed=50 + k) for k in range(4)]
+    systems = [_in_larger_box(s, 4.0) if k % 2 else s for k, s in enumerate(systems)]
+    out = []
+    for batch in (systems, *[[s] for s in systems]):
+        e = host.Engine([host.ReplicaSpec(s.copy(), temp=700.0, gamma_ps=5.0, seed=3) for s in batch])
+        try:
+            e.init()
+            e.minimize(30)
+            e.run(60)
+            assert e.rebuilds().min() > 2
+            out += e.state()
+        finally:
+            e.close()
+    for (x, v), (xa, va) in zip(out[:4], out[4:]):
+        np.testing.assert_array_equal(x, xa)
+        np.testing.assert_array_equal(v, va)
+
+
+def test_sort_time_does_not_follow_the_square_of_the_cells():
+    """59,000 atoms in a box that they fill (2,700 cells) and in one six times as wide (600,000):
+    0.035 and 0.14 ms a full sort; 2.2 ms where every wavefront sums all cells before its own."""
+    host = _host()
+    s = S.make_system(100, 19300, seed=2)
+    best = []
+    for x in (s, _in_larger_box(s, 6.0)):
+        e = host.Engine([host.ReplicaSpec(x, temp=300.0, gamma_ps=1.0, seed=3)])
+        try:
+            e.init()
+            e.minimize(20)
+            best.append(min(e.profile_step(4, full_rebuild=True)["sort+gather"] for _ in range(3)))
+        finally:
+            e.close()
+    print(f"[many cells] full sort {best[0]:.3f} ms, in a larger box {best[1]:.3f} ms", flush=True)
+    assert best[1] < 12.0 * best[0]
