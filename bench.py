@@ -521,6 +521,7 @@ def main():
     ms_p, pairs_p = eng.profile_nonbond(10)
     temp_p = float(eng.temperatures()[0])
     phases_p = eng.profile_step(30)
+    lanes_p = eng.config()["lanes"]
     state_c2 = eng.state()[0]
     log(f"[plain] {plain_rate / 1e6:.1f} Matom-steps/s  ({1e3 * dt_plain / K:.3f} ms/step, "
         f"pair kernel {ms_p:.3f} ms, {pairs_p / plain_sys.np:.1f} pairs/atom in cutoff, T {temp_p:.1f} K)")
@@ -549,6 +550,7 @@ def main():
     batched_rate = natoms * K / dt_b
     rebuilds = eng.rebuilds() - b0
     temps_b = eng.temperatures()
+    lanes_b = eng.config()["lanes"]
     ms_b, pairs_b = eng.profile_nonbond(10)
     ms_copy = eng.profile_copy(1 << 30, 10)
     snap = (eng.state(), eng.forces(), eng.steps())
@@ -570,7 +572,7 @@ def main():
             e1.set_steps([snap[2][k]])
             if tune_b is not None:
                 e1.set_skin(tune_b[0])
-                e1.set_tuning(tune_b[1], host.PAIR_BLOCK, tune_b[3])
+                e1.set_tuning(-1, host.PAIR_BLOCK, tune_b[3])   # lanes by the replica's own size
                 e1.set_bonded_mode(tune_b[4])
                 e1.set_graph_steps(tune_b[5])
             e1.resume([snap[1][k]])
@@ -593,7 +595,7 @@ def main():
         SV.relax(pool, args.minimize)
         reqs = SV.poisson_stream(pool, args.serve_rate, args.serve_seconds)
         nreq = len(reqs)
-        tuning = None if tune_b is None else (tune_b[0], tune_b[1], tune_b[3], tune_b[4], tune_b[5])
+        tuning = None if tune_b is None else (tune_b[0], -1, tune_b[3], tune_b[4], tune_b[5])
         srv = SV.SegmentServer(segment=100, tuning=tuning)
         res, wall, atom_steps = srv.serve(reqs)
         lat = np.array([r.latency_ms for r in res])
@@ -648,13 +650,13 @@ def main():
             "replicas": len(reps), "atoms": natoms,
             "temperature_K_mean": round(float(temps_b.mean()), 1),
             "phase_ms_eager": {k: round(v, 4) for k, v in phases_b.items()},
-            "tuning": None if tune_b is None else {"skin": tune_b[0], "lanes": tune_b[1],
+            "tuning": None if tune_b is None else {"skin": tune_b[0], "lanes": lanes_b,
                                                    "list_waves": tune_b[3], "bonded_mode": tune_b[4],
                                                    "steps_per_graph": tune_b[5]},
             "preparation": f"minimize {args.minimize}, Langevin gamma 20/ps for {args.equil} steps "
                            "(untimed)",
             "plain": {"workload": f"the same {len(reps)} replicas, one system per launch (one engine "
-                                  f"each, hipGraph steps, mixed precision, batched tuning), {kp} "
+                                  f"each, hipGraph steps, mixed precision, batched tuning with lanes by size), {kp} "
                                   "timed steps each",
                       "value": round(per_launch_rate / 1e6, 3), "unit": "Matom-steps/s"},
             "plain_c2": {"workload": "204,000-atom glycine/water, FP64 pair math and state",
@@ -662,7 +664,7 @@ def main():
                       "ms_per_step": round(1e3 * dt_plain / K, 4), "dtype": "f64",
                       "temperature_K": round(temp_p, 1),
                       "phase_ms_eager": {k: round(v, 4) for k, v in phases_p.items()},
-                      "tuning": None if tune_p is None else {"skin": tune_p[0], "lanes": tune_p[1],
+                      "tuning": None if tune_p is None else {"skin": tune_p[0], "lanes": lanes_p,
                                                              "list_waves": tune_p[3],
                                                              "bonded_mode": tune_p[4],
                                                              "steps_per_graph": tune_p[5]}},

@@ -368,6 +368,9 @@ int sofia_profile_step(sofia_ctx *ctx, int32_t nsteps, int32_t full_rebuild, dou
  * the mixed pair kernel (64..1024 in steps of 64; the FP64 and Ewald kernels take at most
  * 256 of them), waves per block in the list build. */
 int sofia_set_tuning(sofia_ctx *ctx, int32_t lanes_per_atom, int32_t block, int32_t list_waves);
+/* The pair kernel's lanes and block chosen by kernel and number of atoms, as they are until
+ * sofia_set_tuning is called; waves per block in the list build as given. */
+int sofia_set_tuning_by_size(sofia_ctx *ctx, int32_t list_waves);
 /* Engine Verlet skin in A (list radius rc + skin; default: the reference's pad).  The
  * engine's lists hold every pair inside the cutoff whatever the skin, so the skin changes
  * only speed (longer lists against more frequent rebuilds), never the trajectory.  Takes

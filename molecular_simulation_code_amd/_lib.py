@@ -119,6 +119,7 @@ SIGNATURES = {
     "sofia_get_replica_steps": [_vp, _vp],
     "sofia_profile_nonbond": [_vp, _i32, _vp, _vp],
     "sofia_set_tuning": [_vp, _i32, _i32, _i32],
+    "sofia_set_tuning_by_size": [_vp, _i32],
     "sofia_set_skin": [_vp, _d],
     "sofia_set_bonded_mode": [_vp, _i32],
     "sofia_profile_step": [_vp, _i32, _i32, _vp],

@@ -2391,6 +2391,13 @@ int sofia_set_tuning(sofia_ctx *c, int32_t lanes, int32_t block, int32_t list_wa
     return SOFIA_OK;
 }
 
+int sofia_set_tuning_by_size(sofia_ctx *c, int32_t list_waves) {
+    TRY(sofia_set_tuning(c, 16, 256, list_waves));
+    c->lanes = -1;
+    c->block = 0;
+    return SOFIA_OK;
+}
+
 int sofia_profile_step(sofia_ctx *c, int32_t nsteps, int32_t full_rebuild, double *phase_ms) {
     if (!c || !phase_ms || nsteps < 1) return fail(SOFIA_E_ARG, "bad argument");
     if (!c->engine_ready) return fail(SOFIA_E_STATE, "call sofia_md_init first");

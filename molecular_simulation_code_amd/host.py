@@ -688,7 +688,12 @@ class Engine:
             pass
 
     def set_tuning(self, lanes: int, block: int, list_waves: int):
-        check(lib().sofia_set_tuning(self.ctx, lanes, block, list_waves))
+        """Pair-kernel lanes per atom (0: the compacting mixed kernel; -1: lanes and block by
+        the engine's size), block, list waves."""
+        if lanes == -1:
+            check(lib().sofia_set_tuning_by_size(self.ctx, list_waves))
+        else:
+            check(lib().sofia_set_tuning(self.ctx, lanes, block, list_waves))
 
     def tune_key(self) -> str:
         """The autotune cache bucket of this engine: precision, electrostatics, replica
@@ -702,8 +707,9 @@ class Engine:
 
     def autotune(self, steps: int = 80, skins=(1.0, 1.3, 1.6, 2.0, 2.5), lanes=(0, 8, 16, 32),
                  waves=(4, 8, 16), graph_steps=(1, 20), cache: bool = True):
-        """Pick the Verlet skin and the pair kernel's lanes per atom on the current state.
-        First the list build's waves per workgroup on full rebuilds; then, for each skin, the
+        """Pick the Verlet skin and the pair kernel's lanes per atom on the current state;
+        lanes -1 stands for lanes and block by size, as of an engine that nobody tunes, and is
+        always among the candidates.  First the list build's waves per workgroup on full rebuilds; then, for each skin, the
         lanes by timing the pair kernel alone, and the skins compared on whole MD steps (list
         length against rebuild rate); then the bonded evaluation (per-kind kernels or
         molecule bundles) on eager steps, and the MD steps per captured graph on whole
@@ -733,6 +739,9 @@ class Engine:
             t_w[w] = self.profile_step(3, full_rebuild=True)["list build"]
         self.tune_log["list_ms"] = t_w
         w = min(t_w, key=t_w.get)
+        self.set_tuning(-1, 0, w)
+        by_size = self.config()["lanes"]
+        lanes = (-1, *(L for L in lanes if L != by_size))
         for sk in skins:
             self.set_skin(sk)
             t_l = {}

@@ -628,3 +628,31 @@ def test_sort_time_does_not_follow_the_square_of_the_cells():
             e.close()
     print(f"[many cells] full sort {best[0]:.3f} ms, in a larger box {best[1]:.3f} ms", flush=True)
     assert best[1] < 12.0 * best[0]
+
+
+@pytest.mark.parametrize("ng,nw", [(40, 1530), (160, 6130)])
+def test_a_tuned_small_engine_is_no_slower_than_an_untuned_one(ng, nw):
+    """The tuner times the layout by size beside the fixed ones, at 5,000 and 20,000 atoms, and
+    takes the fastest: its pair launch (best of 5 x 50, same skin) is within 6 %, twice what such
+    a timing varies by, of the untuned engine's."""
+    host = _host()
+    s = S.make_system(ng, nw, seed=8)
+    ms, forces = [], []
+    for tuned in (False, True):
+        e = _one(host, s.copy())
+        try:
+            e.set_skin(2.0)
+            e.init()
+            e.minimize(30)
+            forces.append(e.forces()[0])
+            if tuned:
+                picked = e.autotune(steps=20, skins=(2.0,), cache=False)
+                t = e.tune_log["pair_ms"][2.0]
+                assert -1 in t and e.config()["lanes"] not in set(t) - {picked[1]} and picked[1] == min(t, key=t.get)
+                print(f"[tuned] {s.np} atoms: {picked}, {e.tune_log['pair_ms']}", flush=True)
+            ms.append(min(e.profile_nonbond(50)[0] for _ in range(5)))
+        finally:
+            e.close()
+    print(f"[tuned] {s.np} atoms: untuned {1e3 * ms[0]:.1f} us, tuned {1e3 * ms[1]:.1f} us", flush=True)
+    np.testing.assert_array_equal(*forces)
+    assert ms[1] <= 1.06 * ms[0]
