@@ -886,7 +886,8 @@ class Engine:
 
     def state(self):
         """FP64 positions/velocities per replica, in each replica's own original atom
-        order (global_id order)."""
+        order (global_id order).  A replica's arrays are rows of the whole batch's: copy what is
+        to outlast the others."""
         x = np.empty((self.N, 3), f64)
         v = np.empty((self.N, 3), f64)
         if self._ordered(x=x, v=v):
@@ -905,7 +906,7 @@ class Engine:
 
     def forces(self):
         """Total force per replica after the last step (global_id order): the force the
-        next step's first half-kick uses."""
+        next step's first half-kick uses.  Rows of the whole batch's, as in state()."""
         f = np.empty((self.N, 3), f64)
         if self._ordered(f=f):
             return [t[0] for t in self._split((f,))]

@@ -76,6 +76,12 @@ class _Slot:
     f: np.ndarray | None = None      # total force after the last step (None before the first)
 
 
+def _own(a: np.ndarray) -> np.ndarray:
+    """The array, or a copy where it is part of a larger one (a replica's rows of a batch's
+    state): what is kept past the batch holds no other replica's memory."""
+    return a if a.base is None or a.base.nbytes == a.nbytes else a.copy()
+
+
 class SegmentServer:
     """Admission budget: hbm_budget_gb, or (None) 85 % of the GPU memory free when the server
     starts, read from the device.  A request's footprint is its atoms times bytes_per_atom;
@@ -144,7 +150,7 @@ class SegmentServer:
 
     def _result(self, s, now, energies, state):
         return Result(s.req.rid, s.req.system.np, s.req.arrival, s.admitted, now, s.clusters,
-                      energies, state)
+                      energies.copy(), None if state is None else tuple(_own(a) for a in state))
 
     def _serve_cohorts(self, requests, realtime: bool):
         t0 = time.perf_counter()
@@ -268,8 +274,7 @@ class SegmentServer:
                 states = eng.state() if self.keep_state else None
                 for k in finished:
                     s = active[k]
-                    results.append(Result(s.req.rid, s.req.system.np, s.req.arrival, s.admitted, now,
-                                          s.clusters, energies[k], states[k] if states else None))
+                    results.append(self._result(s, now, energies[k], states[k] if states else None))
                     used -= self.footprint(s.req)
                 keep = [k for k in range(len(active)) if k not in set(finished)]
                 if keep:
@@ -290,8 +295,8 @@ class SegmentServer:
         forces = eng.forces()
         steps = eng.steps()
         for k, s in enumerate(slots):
-            s.x, s.v = states[k]
-            s.f = forces[k]
+            s.x, s.v = (_own(a) for a in states[k])
+            s.f = _own(forces[k])
             s.step = int(steps[k])
 
 

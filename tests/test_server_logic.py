@@ -163,3 +163,43 @@ def test_autotune_cache_survives_the_process_and_buckets_by_size_and_density(mon
     assert key(204000, 127.3) != key(1020000, 217.7)    # another size
     assert key(204000, 127.3) != key(204000, 127.3, nrep=4)
     assert key(204000, 127.3) != key(204000, 140.0)     # another density
+
+
+@pytest.mark.parametrize("policy", ["cohort", "rebatch"])
+def test_kept_states_hold_no_other_replicas_memory(fake, monkeypatch, policy):
+    """An engine hands out each replica's state and forces as rows of the whole batch's arrays.
+    What the server keeps past the batch, in results and in the slots of requests that go on,
+    are arrays of their own (a lone replica's rows are the whole array already)."""
+    class Rows(_FakeEngine):
+        def _rows(self):
+            n = [r.system.np for r in self.reps]
+            whole = np.zeros((sum(n), 3))
+            off = np.concatenate([[0], np.cumsum(n)])
+            return [whole[a:b] for a, b in zip(off[:-1], off[1:])]
+
+        def state(self):
+            return list(zip(self._rows(), self._rows()))
+
+        def forces(self):
+            return self._rows()
+
+        def put_state(self, xv):
+            super().put_state(xv)
+            for x, v in xv:
+                kept.extend([x, v])
+
+        def resume(self, forces):
+            super().resume(forces)
+            kept.extend(f for f in forces if f is not None)
+
+    kept = []
+    monkeypatch.setattr(SV, "Engine", Rows)
+    srv = SV.SegmentServer(hbm_budget_gb=100.0, segment=50, keep_state=True, policy=policy, max_cohorts=1)
+    srv._calibrated = True
+    res, _, _ = srv.serve(_stream([1000, 2000, 3000, 4000], [0.0, 0.0, 0.0, 1.0], [50, 100, 200, 150]),
+                          realtime=False)
+    for r in res:
+        kept.extend([*r.state, r.energies])
+    assert len(kept) > 20
+    for a in kept:
+        assert a.base is None or a.base.nbytes == a.nbytes
