@@ -104,13 +104,6 @@ __global__ void k_fix_to_aos(int32_t n, const long long *__restrict__ f, float *
     for (int c = 0; c < 3; ++c) out[3 * (size_t)i + c] = (float)((double)f[(size_t)c * n + i] * FIX_INV);
 }
 
-__global__ void k_f64_to_aos(int32_t n, const double *__restrict__ f, float *__restrict__ out) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) out[3 * (size_t)i + c] = (float)f[(size_t)c * n + i];
-}
-
 // ------------------------------------------------------------------ drop-in (real*4 state)
 __global__ void k_nve_v32(int32_t n, float dt_partial, const float4 *__restrict__ pos4,
                           const double *__restrict__ mass, float *__restrict__ v,
@@ -979,10 +972,6 @@ void launch_zero_forces(sofia_ctx *c, long long *f, bool energies) {
 
 void launch_fix_to_coords(sofia_ctx *c, const long long *f, float *out) {
     hipLaunchKernelGGL(k_fix_to_aos, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N, f, out);
-}
-
-void launch_f64_to_coords(sofia_ctx *c, const double *f, float *out) {
-    hipLaunchKernelGGL(k_f64_to_aos, dim3(nblocks(c->N, 256)), dim3(256), 0, c->stream, c->N, f, out);
 }
 
 void launch_nve_v32(sofia_ctx *c, float dt_partial, const float *ff) {

@@ -465,10 +465,7 @@ __global__ void k_list_done(int32_t nrep, int32_t *__restrict__ rebuild, int32_t
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int mx = *maxcnt;
     if (t == 0) hw->maxcnt = mx;
-    if (mx <= na && t <= nrep) {
-        if (t < nrep && rebuild[t]) nbuilds[t] += 1;
-        rebuild[t] = 0;   // [nrep] is `any`
-    }
+    if (mx <= na && t <= nrep) finish_rebuild(t, nrep, rebuild, nbuilds);
     if (local && t < n) local[t] = tt[t] - reps[rep[t]].atom0 + 1;
 }
 

@@ -318,7 +318,6 @@ int record_bytes(const sofia_ctx *c);
 // integration (k_integrate.hip)
 void launch_zero_forces(sofia_ctx *c, long long *f, bool energies);
 void launch_fix_to_coords(sofia_ctx *c, const long long *f, float *out_aos);
-void launch_f64_to_coords(sofia_ctx *c, const double *f, float *out_aos);
 void launch_nve_v32(sofia_ctx *c, float dt_partial, const float *ff_aos);
 void launch_nve_x32(sofia_ctx *c);
 void launch_pbc32(sofia_ctx *c);
