@@ -56,19 +56,14 @@ def _profile_json(name):
         return None
 
 
-def traffic_bytes():
-    """HBM bytes per pair-kernel launch on the batched workload, from the committed
-    rocprofv3 FETCH_SIZE / WRITE_SIZE summary (counters scaled by the calibration copy), or
-    None when no such summary exists."""
-    d = _profile_json("pair_kernel_batched64_traffic.json")
-    return None if d is None else d.get("traffic_bytes_per_launch")
-
-
-def valu_counters():
-    """VALU issue rate (instructions over the one-per-CU-per-cycle ceiling) and the FP32 /
-    FP64 / integer instruction mix of the pair kernel on the batched workload, from the
-    committed rocprofv3 counter summary, or None."""
-    return _profile_json("pair_kernel_batched64_valu.json")
+def counters(name, skin):
+    """The committed rocprofv3 summary `name` of the pair kernel on the batched workload, at the
+    profiled skin nearest to the timed run's (its "skin" and "workload" say which), or {}."""
+    d = _profile_json(name)
+    if d is None or skin is None:
+        return {}
+    return {"kernel": d["kernel"], **min(d["by_skin"], key=lambda e: abs(e["skin"] - skin)),
+            **({"note": d["note"]} if "note" in d else {})}
 
 
 def log(*a):
@@ -550,7 +545,7 @@ def main():
     batched_rate = natoms * K / dt_b
     rebuilds = eng.rebuilds() - b0
     temps_b = eng.temperatures()
-    lanes_b = eng.config()["lanes"]
+    lanes_b, skin_b = (eng.config()[k] for k in ("lanes", "skin"))
     ms_b, pairs_b = eng.profile_nonbond(10)
     ms_copy = eng.profile_copy(1 << 30, 10)
     snap = (eng.state(), eng.forces(), eng.steps())
@@ -629,7 +624,9 @@ def main():
 
     flops = FLOP_PER_PAIR * pairs_b
     achieved = flops / (ms_b * 1e-3)
-    valu = valu_counters()
+    # HBM bytes a launch (FETCH_SIZE / WRITE_SIZE scaled by the calibration copy); VALU issue and mix
+    traffic = counters("pair_kernel_batched64_traffic.json", skin_b)
+    valu = counters("pair_kernel_batched64_valu.json", skin_b)
     line = {
         "metric": METRIC,
         "value": round(batched_rate / 1e6, 3),
@@ -699,10 +696,9 @@ def main():
         "roofline": {"bound": "valu", "achieved": achieved / 1e12, "peak": PEAK_FP32 / 1e12,
                      "unit": "TFLOP/s", "frac": achieved / PEAK_FP32,
                      "peak_unpacked": PEAK_FP32_UNPACKED / 1e12,
-                     "frac_unpacked": achieved / PEAK_FP32_UNPACKED, "traffic": traffic_bytes(),
-                     "traffic_workload": (_profile_json("pair_kernel_batched64_traffic.json")
-                                          or {}).get("workload"),
-                     "valu_counters": valu,
+                     "frac_unpacked": achieved / PEAK_FP32_UNPACKED, "traffic": traffic.get("traffic_bytes_per_launch"),
+                     "traffic_workload": traffic.get("workload"),
+                     "valu_counters": valu or None,
                      "kernel": PAIR_KERNEL, "ms_per_launch": ms_b,
                      "pairs_in_cutoff_per_launch": pairs_b, "flop_per_pair": FLOP_PER_PAIR},
         "cpu_baseline": cpu,

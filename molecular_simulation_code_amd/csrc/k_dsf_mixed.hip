@@ -2,17 +2,17 @@
 // lj_cut_coul_dsf_nonewton_NOMIC (Source/mod_force_nonbond.f90:105-196) with FP32 pair
 // arithmetic and exact per-atom force sums.
 //
-// Positions.  Before a launch, k_fixpos writes each atom as one 16-byte record: three
-// unsigned 32-bit fractions of its replica's box, X = round(x 2^32 / box) mod 2^32, with the
-// atom type in the low 6 bits of X (the x resolution becomes 2^-26 box, 3e-6 A at 217 A,
-// finer than a float32 coordinate there), and the charge.  The difference of two such
-// words taken in 32-bit integers is already the minimum image (the box maps to 2^32
-// exactly), so the pair loop has no rint/fma wrap; the integer difference is converted to
-// float and scaled by box 2^-32.  Fixed point also removes the cancellation of FP32
-// coordinates near the box edge: separations carry full FP32 relative precision.  One
-// gather per list entry brings position, type and charge.  When every atom of a type carries
-// the same charge the record drops the charge (12 bytes) and C q_i q_j comes from a
-// per-type-pair table in LDS, formed as the kernel would form it from the charges.
+// Positions.  Each atom is one 16-byte record, which the engine's launches write along with the
+// positions (write_record; k_fixpos where no step precedes the pair launch): three unsigned
+// 32-bit fractions of its replica's box, X = round(x 2^32 / box) mod 2^32, with the atom type in
+// the low 6 bits of X (the x resolution becomes 2^-26 box, 3e-6 A at 217 A, finer than a float32
+// coordinate there), and the charge.  The difference of two such words taken in 32-bit integers
+// is already the minimum image (the box maps to 2^32 exactly), so the pair loop has no rint/fma
+// wrap; the integer difference is converted to float and scaled by box 2^-32.  Fixed point also
+// removes the cancellation of FP32 coordinates near the box edge: separations carry full FP32
+// relative precision.  One gather per list entry brings position, type and charge.  When every
+// atom of a type carries the same charge the record drops the charge (12 bytes) and C q_i q_j
+// comes from a per-type-pair table in LDS, formed as the kernel would form it from the charges.
 //
 // Pair math (force over r):
 //   dr6i = (1/r^2)^3, 0 beyond rcut2;  F_LJ/r = dr6i (lj1 dr6i - lj2) / r^2

@@ -65,12 +65,13 @@ k_chunk_sums(int32_t ncell, const int32_t *__restrict__ any, const int32_t *__re
     chunk[blockIdx.x] = s;
 }
 
-// Atoms of a cell in descending old index (the chain order of the reference's linked cells),
-// by ranking, which is deterministic.  A wavefront owns `per` consecutive cells; it finds
-// their first atom by summing the replica's counts before its first cell (a scan kernel of one
+// Atoms of a cell in descending old index (the chain order of the reference's linked cells), by
+// ranking, which is deterministic.  A wavefront owns `per` consecutive cells; it finds their
+// first atom by summing the replica's counts before its first cell (a scan kernel of one
 // workgroup per replica in the launch sequence cost every step more than these sums cost the
-// steps that rebuild), by runs of cells where k_chunk_sums counted those.  A cell with more atoms than a bucket holds first gathers them, from its
-// bucket and the list of atoms past full buckets, where its places will be (in fat).
+// steps that rebuild), by runs of cells where k_chunk_sums counted those.  A cell with more atoms
+// than a bucket holds first gathers them, from its bucket and the list of atoms past full
+// buckets, where its places will be (in fat).
 __global__ void __launch_bounds__(256)
 k_sort_gather(int32_t ncell, int32_t per, int32_t split, const int32_t *__restrict__ cell_rep,
               const RepInfo *__restrict__ reps, const int32_t *__restrict__ rebuild,

@@ -101,7 +101,8 @@ k_nonbond(int32_t n, const float4 *__restrict__ pos4, const float *__restrict__ 
     const double2 *ljrow64 = s_lj64 + 2 * (ti * P.ntypes - 1);
     // QT (charges by atom type): C qi qj from a type-pair table, formed as from the atoms'
     // charges, instead of a second gather per entry: Ewald at 20,000 atoms 31.3 -> 28.9 us;
-    // FP64 at 204,000, bound by FP64 issue, 446 -> 441 us, with energies 603 -> 540
+    // FP64 at 204,000, bound by FP64 issue (VALU busy 90 % of the launch), 446 -> 441 us, with
+    // energies 603 -> 540
     const double *qqrow = s_qq + ti * P.ntypes - 1;
     const float4 *ptrow = s_pt + ti * P.ntypes - 1;
 
